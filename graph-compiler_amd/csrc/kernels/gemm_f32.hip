@@ -1,12 +1,11 @@
-// f32 GEMM (f32 multiply-add throughout: vector FMAs, or the f32 matrix
-// instruction on whole tiles; no reduced precision) and the
-// batch-reduce microkernel with the reference's operand layouts.
+// f32 GEMM on the f32 matrix instruction (f32 multiply-add throughout; no
+// reduced precision) and the batch-reduce microkernel with the reference's
+// operand layouts.
 //
-// gemm_f32_kernel: C[M,N] = act(beta*C + A.B + bias), arbitrary element strides
-// on A and B so that transpose_a / transpose_b of onednn_graph.matmul
+// gemm_f32_mfma_kernel, gemm_f32_small_kernel: C[M,N] = act(beta*C + A.B + bias),
+// any sizes; either operand contiguous along k or along its own dimension, so
+// that transpose_a / transpose_b of onednn_graph.matmul
 // (lib/gc/Transforms/OneDNNGraphToLinalg.cpp:421-499) need no copy.
-// 64/32/16-square workgroup tiles, 32-deep K slices through LDS with register
-// prefetch, k ascending per output element.
 //
 // brgemm_kernel: C[m*LDC+n] (+)= sum_i sum_k a(i,m,k) * b(i,k,n) with
 //   f32 : b at i*stride_b + k*LDB + n
@@ -20,180 +19,344 @@
 // f32 results equal the reference's bit for bit; bf16 products are exact in f32
 // and integer sums are exact anyway.
 #include "common.hpp"
+#include <math.h>
 #include <type_traits>
 #include "gemm_params.h"
 
 namespace gcmi {
 
-// BT x BT workgroup tile (BT = 64, 32 or 16: small problems take small tiles so
-// that more compute units take part), 256 threads, (BT/16)^2 outputs per thread,
-// 32-deep K slices through LDS.  The next slice is fetched into registers while
-// the current one is multiplied, so global latency is paid once, not per slice.
-template <int BT> __global__ __launch_bounds__(256) void gemm_f32_kernel(F32GemmParams p) {
-  constexpr int BK = 32, MT = BT / 16, PER = BT * BK / 256; // elements per thread per operand slice
-  __shared__ float As[BK][BT + 4];
-  __shared__ float Bs[BK][BT + 4];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int64_t m0 = (int64_t)blockIdx.y * BT, n0 = (int64_t)blockIdx.x * BT;
-  p.A += (int64_t)blockIdx.z * p.a_bs, p.B += (int64_t)blockIdx.z * p.b_bs, p.C += (int64_t)blockIdx.z * p.c_bs;
-  // slice element e of this thread: (row/col within the tile, k within the slice);
-  // the contiguous direction of each operand runs along consecutive threads
-  int am[PER], ak[PER], bn[PER], bk[PER];
-#pragma unroll
-  for (int e = 0; e < PER; e++) {
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4))); // 16 bytes from any 4-byte aligned address
+
+// One operand's side of a K slice: fetched to registers (float4 chunks, one slice ahead), stashed in LDS, read back as
+// matrix operands.  KC: the operand is contiguous along k and lies in LDS as [row][k] -- one ds_read_b128 gives a lane
+// the four k it contributes to a step (k = 4 * (lane / MT) + 0 .. 3: 8 or 16 deep for 32 x 32 or 16 x 16 products); else it is contiguous along its own
+// dimension, lies in LDS as [k][column] and is read with four ds_read_b32.  Both sides use the same k in the same
+// matrix instruction, which is all a sum needs, so neither layout is transposed on the way.
+// Rows or chunks past the edge read the last valid ones instead (their products land in results nobody stores); a
+// chunk cut by the edge reads the last four and moves them into place.
+template <int BX, int BK, bool KC> struct F32Tile {
+  // four floats of padding spread the rows over the banks (exchanging chunks within unpadded rows: 3 % slower)
+  static constexpr int PITCH = KC ? BK + 4 : BX + 4, SIZE = KC ? BX * PITCH : BK * PITCH;
+  static constexpr int PER = BX * BK / 4 / 256; // chunks per thread and slice
+  static_assert(PER >= 1, "a slice is at least one chunk per thread");
+  const float *src[PER]; // next slice's chunk
+  int shift;             // !KC: places the chunk was moved back because the edge cuts it (the same for all chunks)
+  bool cut;              // !KC: some chunk of this tile is cut (wave-uniform)
+  int64_t step, ks;      // elements from slice to slice, from k to k
+  f32x4_t r[2][PER];     // two slices in flight
+
+  static __device__ __forceinline__ int x_of(int e) {
     const int idx = threadIdx.x + 256 * e;
-    if (p.a_cs == 1) {
-      ak[e] = idx % BK;
-      am[e] = idx / BK;
-    } else {
-      am[e] = idx % BT;
-      ak[e] = idx / BT;
-    }
-    if (p.b_rs == 1 && p.b_cs != 1) {
-      bk[e] = idx % BK;
-      bn[e] = idx / BK;
-    } else {
-      bn[e] = idx % BT;
-      bk[e] = idx / BT;
-    }
+    return KC ? idx / (BK / 4) : 4 * (idx % (BX / 4));
   }
-  float ra[PER], rb[PER];
-  auto fetch = [&](int64_t k0) {
+  static __device__ __forceinline__ int k_of(int e) {
+    const int idx = threadIdx.x + 256 * e;
+    return KC ? 4 * (idx % (BK / 4)) : idx / (BX / 4);
+  }
+  __device__ __forceinline__ void init(const float *base, int64_t x0, int64_t X, int64_t xs, int64_t kstride) {
+    ks = kstride, step = (int64_t)BK * kstride, shift = 0, cut = !KC && X - x0 < BX && X % 4 != 0;
+    static_assert(KC || 256 % (BX / 4) == 0, "all chunks of a thread cover the same columns");
 #pragma unroll
     for (int e = 0; e < PER; e++) {
-      const int64_t gm = m0 + am[e], gk = k0 + ak[e];
-      ra[e] = (gm < p.M && gk < p.K) ? p.A[gm * p.a_rs + gk * p.a_cs] : 0.0f;
-      const int64_t gn = n0 + bn[e], gk2 = k0 + bk[e];
-      rb[e] = (gn < p.N && gk2 < p.K) ? p.B[gk2 * p.b_rs + gn * p.b_cs] : 0.0f;
+      int64_t g = x0 + x_of(e);
+      if constexpr (KC) {
+        g = g < X ? g : X - 1;
+      } else { // X >= 4
+        const int64_t left = X - g;
+        shift = left > 0 && left < 4 ? 4 - (int)left : 0;
+        g = left >= 4 ? g : X - 4;
+      }
+      src[e] = base + g * xs + k_of(e) * kstride;
     }
+  }
+  __device__ __forceinline__ void fetch(int q) { // a whole slice, into register set q
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      r[q][e] = *reinterpret_cast<const f32x4u_t *>(src[e]);
+      src[e] += step;
+    }
+  }
+  __device__ __forceinline__ void fetch_tail(int q, int left) { // the last `left` < BK k, zero behind them
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        r[q][e][c] = k_of(e) + (KC ? c : 0) < left ? src[e][c] : 0.0f;
+    }
+  }
+  __device__ __forceinline__ void stash(int q, float *lds) {
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      f32x4_t v = r[q][e];
+      if constexpr (KC) {
+        *reinterpret_cast<f32x4_t *>(&lds[x_of(e) * PITCH + k_of(e)]) = v;
+      } else {
+        if (cut) {
+          const f32x4_t u = v;
+          v[0] = shift == 0 ? u[0] : shift == 1 ? u[1] : shift == 2 ? u[2] : u[3];
+          v[1] = shift == 0 ? u[1] : shift == 1 ? u[2] : u[3];
+          v[2] = shift == 0 ? u[2] : u[3];
+        }
+        *reinterpret_cast<f32x4_t *>(&lds[k_of(e) * PITCH + x_of(e)]) = v;
+      }
+    }
+  }
+  // the four operand values of row/column x at k .. k + 3
+  static __device__ __forceinline__ f32x4_t frag(const float *lds, int x, int k) {
+    if constexpr (KC)
+      return *reinterpret_cast<const f32x4_t *>(&lds[x * PITCH + k]);
+    f32x4_t v;
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      v[c] = lds[(k + c) * PITCH + x];
+    return v;
+  }
+};
+
+// One result: beta, bias, activation.
+__device__ __forceinline__ void f32_store(const F32GemmParams &p, int64_t m, int64_t n, float x) {
+  if (p.beta != 0.0f)
+    x = x + p.C[m * p.ldc + n];
+  if (p.bias)
+    x = x + p.bias[n];
+  p.C[m * p.ldc + n] = apply_act(x, p.act);
+}
+
+// BM x BN tile of a workgroup of 4 waves, WM x WN of them over the tile and WK over a slice of BK k (their partial sums
+// are added through LDS at the end).  v_mfma_f32_32x32x2_f32: 256 flop per clock and compute unit (157 TFLOP/s), twice
+// the vector ALU; a 64 x 64 tile needs 16 bytes per clock of operands, so nothing but the issue of these instructions
+// should bound it.  MT: side of the matrix instruction's tile (16: the k of a step and their order are those of the
+// small kernel below).  Two slices are in flight in registers behind the one in LDS (with one: 8 % slower, a load then has
+// less time than memory takes), the barrier of a slice lies between its last products with the writes in front and the
+// next slice's first reads behind it.  At 4096^3 the matrix pipes are 90 % busy: 1025 us = 134 TFLOP/s (1230 us when A
+// was transposed on its way into LDS, one slice ahead, reads waited for in front of every product).  1111 tokens
+// through 1000 x 3000 x 1000 x 500: 71 + 77 + 22 us (150 + 288 + 62 on vector FMAs, which were all that sizes off the
+// tile took).  v_mfma_f32_16x16x4_f32 in the large tiles: up to 10 % slower (more registers); in the 32 x 32 tile level.
+template <int MT, int BM, int BN, int WM, int WN, int WK, int BK, bool AKC, bool BKC>
+__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(F32GemmParams p) {
+  constexpr int TM = BM / WM / MT, TN = BN / WN / MT, KW = BK / WK; // MT x MT tiles of a wave, its k of a slice
+  constexpr int DEEP = 256 / MT, STEPS = KW / DEEP, R = MT * MT / 64; // k of a step, results per lane and tile
+  static_assert(WM * WN * WK == 4 && KW % DEEP == 0, "4 waves, whole steps");
+  typedef float acc_t __attribute__((ext_vector_type(R)));
+  typedef F32Tile<BM, BK, AKC> TA;
+  typedef F32Tile<BN, BK, BKC> TB;
+  constexpr int STAGE = TA::SIZE + TB::SIZE;
+  constexpr int RED = (WK - 1) * BM * BN;
+  __shared__ __attribute__((aligned(16))) float smem[2 * STAGE > RED ? 2 * STAGE : RED];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wk = wave % WK, wn = (wave / WK) % WN, wm = wave / (WK * WN);
+  const int lx = lane % MT, lk = lane / MT;
+  // workgroup i runs on XCD i % 8: each XCD walks its own run of tiles, columns of 8 tile rows at a time
+  const int64_t mt = (p.M + BM - 1) / BM, nt = (p.N + BN - 1) / BN, tiles = mt * nt;
+  const int64_t t = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (t >= tiles)
+    return;
+  const int64_t group = t / (8 * nt), rows = mt - 8 * group < 8 ? mt - 8 * group : 8, in = t - group * 8 * nt;
+  const int64_t m0 = (8 * group + in % rows) * BM, n0 = in / rows * BN;
+  p.A += (int64_t)blockIdx.z * p.a_bs, p.B += (int64_t)blockIdx.z * p.b_bs, p.C += (int64_t)blockIdx.z * p.c_bs;
+  TA ta;
+  TB tb;
+  ta.init(p.A, m0, p.M, p.a_rs, p.a_cs);
+  tb.init(p.B, n0, p.N, p.b_cs, p.b_rs);
+  acc_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        acc[i][j][r] = 0.0f;
+  const int xa = wm * TM * MT + lx, xb = wn * TN * MT + lx;
+  f32x4_t a[2][TM], b[2][TN]; // operands of this step and the next
+  auto load = [&](int q, int step) { // of the slice in slot q
+    const float *as = smem + q * STAGE, *bs = as + TA::SIZE;
+    const int s = (q * STEPS + step) & 1, k = wk * KW + DEEP * step + 4 * lk;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+      a[s][i] = TA::frag(as, xa + i * MT, k);
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+      b[s][j] = TB::frag(bs, xb + j * MT, k);
   };
-  float acc[MT][MT] = {};
-  fetch(0);
-  for (int64_t k0 = 0; k0 < p.K; k0 += BK) {
+  auto products = [&](int s, int c) {
 #pragma unroll
-    for (int e = 0; e < PER; e++) {
-      As[ak[e]][am[e]] = ra[e];
-      Bs[bk[e]][bn[e]] = rb[e];
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+        if constexpr (MT == 32)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][i][c], b[s][j][c], acc[i][j], 0, 0, 0);
+        else
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][i][c], b[s][j][c], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0); // reads and writes keep their places between the products
+  };
+  // slice s lies in slot s % 2 (offset 0 or STAGE); slice s + 1 is in register set (s + 1) % 2 or on its way there,
+  // slice s + 2 is requested into set s % 2 at the start: two slices' worth of products to hide a load behind
+  const int64_t whole = p.K / BK;
+  const int tail = (int)(p.K - whole * BK);
+  const int64_t slices = whole + (tail ? 1 : 0);
+  auto fetch = [&](int q, int64_t s) {
+    if (s < whole)
+      ta.fetch(q), tb.fetch(q);
+    else if (s < slices)
+      ta.fetch_tail(q, tail), tb.fetch_tail(q, tail);
+  };
+  auto stash = [&](int q) {
+    ta.stash(q, smem + q * STAGE);
+    tb.stash(q, smem + q * STAGE + TA::SIZE);
+  };
+  auto slice = [&](int q, bool next) {
+#pragma unroll
+    for (int step = 0; step < STEPS - 1; step++) {
+      load(q, step + 1);
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        products((q * STEPS + step) & 1, c);
     }
-    __syncthreads();
-    if (k0 + BK < p.K)
-      fetch(k0 + BK);
-#pragma unroll
-    for (int k = 0; k < BK; k++) { // k ascending per output element
-      float a[MT], b[MT];
-#pragma unroll
-      for (int i = 0; i < MT; i++)
-        a[i] = As[k][ty * MT + i];
-#pragma unroll
-      for (int j = 0; j < MT; j++)
-        b[j] = Bs[k][tx * MT + j];
-#pragma unroll
-      for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < MT; j++)
-          acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+    const int last = (q * STEPS + STEPS - 1) & 1;
+    products(last, 0);
+    if (next)
+      stash(q ^ 1);
+    products(last, 1);
+    if (next) {
+      __syncthreads();
+      load(q ^ 1, 0); // the next slice's first operands, under the last products of this one
     }
+    products(last, 2);
+    products(last, 3);
+  };
+  if (slices > 0) {
+    fetch(0, 0);
+    fetch(1, 1);
+    stash(0);
     __syncthreads();
+    load(0, 0);
+    int64_t s = 0;
+    for (; s + 3 < whole; s += 2) {
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        ta.fetch(q), tb.fetch(q);
+        __builtin_amdgcn_sched_barrier(0);
+        slice(q, true);
+      }
+    }
+    for (; s < slices; s += 2) {
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        if (s + q < slices) {
+          fetch(q, s + q + 2);
+          slice(q, s + q + 1 < slices);
+        }
+    }
   }
+  if constexpr (WK > 1)
+    __syncthreads(); // the operand slots become the reduction's
+  if constexpr (WK > 1) { // the waves' shares of K, added in ascending order of wk
+    float *mine = smem + (wm * WN + wn) * (WK - 1) * TM * TN * R * 64 + lane;
+    if (wk > 0) {
 #pragma unroll
-  for (int i = 0; i < MT; i++) {
-    int64_t m = m0 + ty * MT + i;
-    if (m >= p.M)
-      continue;
+      for (int i = 0; i < TM; i++)
 #pragma unroll
-    for (int j = 0; j < MT; j++) {
-      int64_t n = n0 + tx * MT + j;
-      if (n >= p.N)
-        continue;
-      float x = acc[i][j];
-      if (p.beta != 0.0f)
-        x = x + p.C[m * p.ldc + n];
-      if (p.bias)
-        x = x + p.bias[n];
-      p.C[m * p.ldc + n] = apply_act(x, p.act);
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int r = 0; r < R; r++)
+            mine[(((wk - 1) * TM + i) * TN + j) * R * 64 + r * 64] = acc[i][j][r];
+    }
+    __syncthreads();
+    if (wk > 0)
+      return;
+#pragma unroll
+    for (int w = 0; w < WK - 1; w++)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int r = 0; r < R; r++)
+            acc[i][j][r] += mine[((w * TM + i) * TN + j) * R * 64 + r * 64];
+  }
+  // lane (lx, lk) holds column lx and rows 8 * (r / 4) + 4 * lk + r % 4 of every tile
+#pragma unroll
+  for (int j = 0; j < TN; j++) {
+    const int64_t n = n0 + (wn * TN + j) * MT + lx;
+    if (n < p.N) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          const int64_t m = m0 + (wm * TM + i) * MT + 8 * (r >> 2) + 4 * lk + (r & 3);
+          if (m < p.M)
+            f32_store(p, m, n, acc[i][j][r]);
+        }
     }
   }
 }
 
-// The same GEMM on the matrix cores for whole 128 x 128 tiles of row-major operands: v_mfma_f32_32x32x2_f32 multiplies
-// and adds in f32 (no reduced precision), 256 flop per clock and compute unit against 128 for the vector ALU's FMA.
-// 256 threads = 4 waves as 2 x 2, a wave owns 64 x 64 = four 32 x 32 tiles (64 accumulator registers); 16-deep K
-// slices through LDS, the next slice prefetched into registers.  A is stored k-major in LDS ([k][m]) so that a
-// fragment read (lane = row, k = lane / 32) is one conflict-free ds_read_b32 per tile, B as it lies in memory.
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(F32GemmParams p) {
-  constexpr int BT = 128, BK = 16;
-  __shared__ float As[BK][BT + 4];
-  __shared__ float Bs[BK][BT + 4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-  const int l32 = lane & 31, lh = lane >> 5;
-  const int64_t m0 = (int64_t)blockIdx.y * BT, n0 = (int64_t)blockIdx.x * BT;
+// Small problems: what counts is the chain launch -> loads -> sums -> store.  A workgroup owns one 16 x 16 tile, its
+// four waves take every fourth 16-deep step of K straight from memory into v_mfma_f32_16x16x4_f32 operands (lane l:
+// row/column l % 16, and k = 4 * (l / 16) .. + 3 of the step as four operand values), eight steps in flight per wave,
+// no LDS and no barrier until the four partial sums are added.  128 x 512 x 256 (128 workgroups) in 7.2 us per call (10.6 as
+// 16 x 16 tiles of vector FMAs over LDS slices of 32 k with a barrier each).
+template <bool AKC, bool BKC> __global__ __launch_bounds__(256) void gemm_f32_small_kernel(F32GemmParams p) {
+  constexpr int U = 8;
+  __shared__ float red[3][256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lq = lane >> 4;
+  const int64_t nt = (p.N + 15) / 16, m0 = blockIdx.x / nt * 16, n0 = blockIdx.x % nt * 16;
   p.A += (int64_t)blockIdx.z * p.a_bs, p.B += (int64_t)blockIdx.z * p.b_bs, p.C += (int64_t)blockIdx.z * p.c_bs;
-  // slice loads, 16 bytes per thread and operand piece: A 128 rows x 16 k = 512 float4 (two per thread: row = idx / 4,
-  // k = 4 * (idx % 4)), B 16 k x 128 n = 512 float4 (k = idx / 32, n = 4 * (idx % 32))
-  f32x4_t ra[2], rb[2];
-  auto fetch = [&](int64_t k0) {
-#pragma unroll
-    for (int e = 0; e < 2; e++) {
-      const int idx = tid + 256 * e;
-      ra[e] = *reinterpret_cast<const f32x4_t *>(p.A + (m0 + idx / 4) * p.a_rs + k0 + 4 * (idx % 4));
-      rb[e] = *reinterpret_cast<const f32x4_t *>(p.B + (k0 + idx / 32) * p.b_rs + n0 + 4 * (idx % 32));
+  const int64_t ga = m0 + l16 < p.M ? m0 + l16 : p.M - 1, gb = n0 + l16 < p.N ? n0 + l16 : p.N - 1;
+  const float *a = p.A + ga * p.a_rs + 4 * lq * p.a_cs, *b = p.B + gb * p.b_cs + 4 * lq * p.b_rs;
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto load = [&](const float *s, int64_t ks, int64_t left, bool contig) -> f32x4_t {
+    f32x4_t v;
+    if (left >= 4) {
+      if (contig)
+        v = *reinterpret_cast<const f32x4u_t *>(s);
+      else
+        for (int c = 0; c < 4; c++)
+          v[c] = s[c * ks];
+    } else {
+      for (int c = 0; c < 4; c++)
+        v[c] = c < left ? s[c * ks] : 0.0f;
     }
+    return v;
   };
-  f32x16_t acc[2][2];
+  int64_t k = 16 * wave;
+  for (; k + 64 * (U - 1) + 16 <= p.K; k += 64 * U) {
+    f32x4_t va[U], vb[U];
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+    for (int u = 0; u < U; u++) {
+      va[u] = load(a + (k + 64 * u) * p.a_cs, p.a_cs, 4, AKC);
+      vb[u] = load(b + (k + 64 * u) * p.b_rs, p.b_rs, 4, BKC);
+    }
+    __builtin_amdgcn_sched_barrier(0); // all loads first
 #pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++)
-        acc[i][j][r] = 0.0f;
-  fetch(0);
-  for (int64_t k0 = 0; k0 < p.K; k0 += BK) {
-#pragma unroll
-    for (int e = 0; e < 2; e++) {
-      const int idx = tid + 256 * e;
+    for (int u = 0; u < U; u++)
 #pragma unroll
       for (int c = 0; c < 4; c++)
-        As[4 * (idx % 4) + c][idx / 4] = ra[e][c];
-      *reinterpret_cast<f32x4_t *>(&Bs[idx / 32][4 * (idx % 32)]) = rb[e];
-    }
-    __syncthreads();
-    if (k0 + BK < p.K)
-      fetch(k0 + BK);
-#pragma unroll
-    for (int ks = 0; ks < BK; ks += 2) { // k ascending per output element
-      float a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-        a[i] = As[ks + lh][wm * 64 + i * 32 + l32];
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-        b[j] = Bs[ks + lh][wn * 64 + j * 32 + l32];
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u][c], vb[u][c], acc, 0, 0, 0);
   }
-  // lane (l32, lh) holds column l32 and rows 8 * (r / 4) + 4 * lh + r % 4 of every tile: 32 lanes write 128 bytes
+  for (; k < p.K; k += 64) {
+    const f32x4_t va = load(a + k * p.a_cs, p.a_cs, p.K - k - 4 * lq, AKC);
+    const f32x4_t vb = load(b + k * p.b_rs, p.b_rs, p.K - k - 4 * lq, BKC);
 #pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const int64_t n = n0 + wn * 64 + j * 32 + l32;
-    const float bias = p.bias ? p.bias[n] : 0.0f;
+    for (int c = 0; c < 4; c++)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[c], vb[c], acc, 0, 0, 0);
+  }
+  if (wave > 0)
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int r = 0; r < 4; r++)
+      red[wave - 1][r * 64 + lane] = acc[r];
+  __syncthreads();
+  if (wave > 0)
+    return;
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int64_t m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-        float x = acc[i][j][r];
-        if (p.beta != 0.0f)
-          x = x + p.C[m * p.ldc + n];
-        if (p.bias)
-          x = x + bias;
-        p.C[m * p.ldc + n] = apply_act(x, p.act);
-      }
+  for (int r = 0; r < 4; r++) {
+    float x = acc[r];
+#pragma unroll
+    for (int w = 0; w < 3; w++)
+      x += red[w][r * 64 + lane];
+    const int64_t m = m0 + 4 * lq + r, n = n0 + l16; // lane l holds column l % 16 and rows 4 * (l / 16) + r
+    if (m < p.M && n < p.N)
+      f32_store(p, m, n, x);
   }
 }
 
@@ -340,34 +503,57 @@ __global__ __launch_bounds__(256) void brgemm_kernel(BrgemmParams p) {
 
 using namespace gcmi;
 
+// the kernel of one tile for the four operand layouts (A along k: + 2, B along k: + 1)
+#define F32_LAYOUTS(...)                                                                                              \
+  {gemm_f32_mfma_kernel<__VA_ARGS__, false, false>, gemm_f32_mfma_kernel<__VA_ARGS__, false, true>,                   \
+   gemm_f32_mfma_kernel<__VA_ARGS__, true, false>, gemm_f32_mfma_kernel<__VA_ARGS__, true, true>}
+
 extern "C" int gcmi_launch_gemm_f32(const F32GemmParams *pp, hipStream_t stream) {
   F32GemmParams p = *pp;
   if (p.M <= 0 || p.N <= 0)
     return 0;
-  // the largest tile that still gives every compute unit a workgroup
   const int64_t nbatch = p.batch > 1 ? p.batch : 1;
   if (nbatch > 65535)
     return 2;
-  // whole 128 x 128 tiles of row-major operands with 16-byte aligned rows, and enough of them: the matrix cores
-  auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-  if (p.a_cs == 1 && p.b_cs == 1 && p.M % 128 == 0 && p.N % 128 == 0 && p.K % 16 == 0 && p.K > 0 && p.a_rs % 4 == 0 &&
-      p.b_rs % 4 == 0 && al16(p.A) && al16(p.B) && (nbatch == 1 || (p.a_bs % 4 == 0 && p.b_bs % 4 == 0)) &&
-      (p.M / 128) * (p.N / 128) * nbatch >= 64 && p.M / 128 <= 65535) {
-    dim3 grid((unsigned)(p.N / 128), (unsigned)(p.M / 128), (unsigned)nbatch);
-    hipLaunchKernelGGL(gemm_f32_mfma_kernel, grid, dim3(256), 0, stream, p);
+  // The tile by estimated time (ns per k, measured on one MI355X; two constants where a lone workgroup of a compute
+  // unit is slower than one of several): tiles are dealt out evenly, a compute unit is done when the one with the most
+  // is.  1111 x 1000, K 3000, in us: 128 x 128 198, 64 x 64 100, 32 x 32 77; 4096^3: 1025, 1051, 1218; 1000 x 1000 x
+  // 1000: 75, 24-26, 29; 300 x 300, K 1000: 73, 23, 11.4 and 8.3 with 16 x 16 tiles.
+  // The two small tiles add an element's products in the same order, and so do the two large ones: which pair is
+  // taken depends on one matrix, so a batch has the bits of its matrices multiplied one by one.
+  const double cus = gcmi_num_cus(), k = (double)p.K * 1e-3;
+  auto tiles = [&](int64_t bm, int64_t bn) { return (double)(((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn)); };
+  auto us = [&](int tile, double batches) {
+    const double n = batches * tiles(tile, tile) / cus; // per compute unit
+    switch (tile) {
+    case 16: return 2.0 + k * 2.7 * fmax(1.0, n);
+    case 32: return 4.0 + k * 4.5 * ceil(n);
+    case 64: return 4.0 + k * fmax(18.0, 15.5 * ceil(n));
+    default: return 5.0 + k * fmax(63.0, 60.0 * ceil(n));
+    }
+  };
+  // 16 bytes along m (A stored [K,M]) or n (B stored [K,N]) are a chunk of the tiles from 32 x 32 on: one must exist
+  const bool akc = p.a_cs == 1, bkc = p.b_rs == 1 && p.b_cs != 1, chunk = (akc || p.M >= 4) && (bkc || p.N >= 4);
+  const bool large = chunk && fmin(us(64, 1), us(128, 1)) < fmin(us(16, 1), us(32, 1));
+  const int tile = large ? (us(128, nbatch) < us(64, nbatch) ? 128 : 64) : chunk && us(32, nbatch) < us(16, nbatch) ? 32 : 16;
+  const int layout = (akc ? 2 : 0) + (bkc ? 1 : 0);
+  if (tile == 16) {
+    const int64_t all = ((p.N + 15) / 16) * ((p.M + 15) / 16);
+    if (all >= 1 << 24) // threads of a grid dimension
+      return 2;
+    const dim3 grid((unsigned)all, 1, (unsigned)nbatch);
+    void (*const kernel[4])(F32GemmParams) = {gemm_f32_small_kernel<false, false>, gemm_f32_small_kernel<false, true>,
+                                              gemm_f32_small_kernel<true, false>, gemm_f32_small_kernel<true, true>};
+    hipLaunchKernelGGL(kernel[layout], grid, dim3(256), 0, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : 5;
   }
-  auto tiles = [&](int bt) { return ((p.N + bt - 1) / bt) * ((p.M + bt - 1) / bt) * nbatch; };
-  const int bt = tiles(64) >= 256 ? 64 : tiles(32) >= 256 ? 32 : 16;
-  dim3 grid((unsigned)((p.N + bt - 1) / bt), (unsigned)((p.M + bt - 1) / bt), (unsigned)nbatch), block(256);
-  if (grid.y > 65535)
+  static void (*const kernels[3][4])(F32GemmParams) = {F32_LAYOUTS(16, 32, 32, 1, 1, 4, 64),
+                                                       F32_LAYOUTS(32, 64, 64, 2, 2, 1, 32),
+                                                       F32_LAYOUTS(32, 128, 128, 2, 2, 1, 16)};
+  const int64_t per_xcd = (((p.M + tile - 1) / tile) * ((p.N + tile - 1) / tile) + 7) / 8;
+  if (per_xcd * 8 >= 1 << 24)
     return 2;
-  if (bt == 64)
-    hipLaunchKernelGGL(gemm_f32_kernel<64>, grid, block, 0, stream, p);
-  else if (bt == 32)
-    hipLaunchKernelGGL(gemm_f32_kernel<32>, grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL(gemm_f32_kernel<16>, grid, block, 0, stream, p);
+  hipLaunchKernelGGL(kernels[tile == 32 ? 0 : tile == 64 ? 1 : 2][layout], dim3((unsigned)(per_xcd * 8), 1, (unsigned)nbatch), dim3(256), 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : 5;
 }
 
