@@ -44,14 +44,17 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
   const int64_t m0 = (int64_t)tm * T128_B, n0 = (int64_t)tn * T128_B;
   const int64_t lda_b = p.lda * ES, ldb_b = p.ldb * ES;
   const int64_t b_step = TB ? (int64_t)KB : (int64_t)BK * ldb_b;
-  int KT = (int)(p.K / BK); // k-blocks: a positive multiple of NST (checked by the launcher)
-  int64_t k_first = 0;      // first k-block of this workgroup
+  const int all_groups = (int)((p.K + NST * BK - 1) / (NST * BK)), k_left = (int)(p.K % (NST * BK));
+  int KT = all_groups * NST; // k-blocks: a positive multiple of NST
+  int64_t k_first = 0;       // first k-block of this workgroup
+  bool k_tail = k_left != 0; // this workgroup has the incomplete last ring group: computed first (fill_ring_k_tail)
   if (p.splits > 1) {
     // K slices: blockIdx.y is the slice, whole ring groups each (they differ by at most one group); its f32 sums go
     // to the workspace as they are, the second kernel adds the slices and runs the epilogue
-    const int slice = blockIdx.y, groups = KT / NST;
+    const int slice = blockIdx.y, groups = all_groups;
     const int g0 = (int)((int64_t)slice * groups / p.splits), g1 = (int)((int64_t)(slice + 1) * groups / p.splits);
     k_first = (int64_t)g0 * NST, KT = (g1 - g0) * NST;
+    k_tail = k_tail && g1 == groups;
     p.C = p.partial + (int64_t)slice * p.M * p.N, p.ldc = p.N, p.out_dt = DT_F32;
     p.bias = nullptr, p.act = ACT_NONE, p.residual = nullptr;
   } else {
@@ -66,6 +69,7 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
 
   // this wave's two DMA instructions per operand and stage: 1 KiB each = 16 rows of A (or of B stored [N,K]), 4 k-rows of B
   uint32_t a_src[2], b_src[2];
+  int a_k[2], b_k[2]; // the first k of the lane's 16 bytes inside a k-block
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const int d = wave * 2 + i;
@@ -75,6 +79,7 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
     const int krow = d * (1024 / B_ROW_BYTES) + lane / B_CPR;
     const int cb = min((lane % B_CPR) ^ b_swz(krow), cols_in * ES / 16 - 1);
     b_src[i] = TB ? (uint32_t)(min(row, cols_in - 1) * ldb_b + c * 16) : (uint32_t)(krow * ldb_b + cb * 16);
+    a_k[i] = c * 16 / ES, b_k[i] = TB ? a_k[i] : krow;
   }
   auto issue = [&](char *__restrict__ stage, const char *a_base, const char *b_base) {
 #pragma unroll
@@ -165,9 +170,18 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
         cp_cs = p.comp * p.colsum[n0 + tid];
     }
   }
+  int first_request = NST - 1; // the k-block that the first stage requests
+  if (k_tail) { // all four slots are filled here; k-blocks 4.. are the whole ones from k_first on
+    const int64_t k_full = p.K - k_left - k_first * BK;
+    fill_ring_k_tail<ES, TB, 2, STAGE, A_BYTES>(smem, wave, lane, a_ptr + k_full * ES, b_ptr + (TB ? k_full * ES : k_full * ldb_b),
+                                                b_step, k_left, a_src, b_src, a_k, b_k);
+    first_request = NST;
+    a_ptr -= NST * KB, b_ptr -= NST * b_step;
+  } else {
 #pragma unroll
-  for (int d = 0; d < NST - 1; d++)
-    issue(smem + d * STAGE, a_ptr + d * KB, b_ptr + d * b_step);
+    for (int d = 0; d < NST - 1; d++)
+      issue(smem + d * STAGE, a_ptr + d * KB, b_ptr + d * b_step);
+  }
   if (tid < T128_B) {
     colp[tid] = cp_bias;
     if (ES == 1) {
@@ -183,12 +197,14 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
   // One stage: k-block kt is in the `cur` registers.  Request block kt+NST-1 into the slot block kt-1 was read from
   // (every wave's reads of it had returned before it passed the previous barrier); wait for this wave's share of
   // block kt+1 and for its own LDS reads; barrier: block kt+1 is visible; read its fragments under the MFMAs of kt.
-  auto stage = [&](auto has_fill, auto has_next, auto behindc, const char *__restrict__ nxt, char *__restrict__ fill,
+  auto stage = [&](auto has_fill, auto has_next, auto behindc, int kf, const char *__restrict__ nxt, char *__restrict__ fill,
                    const char *a_fill, const char *b_fill, uint4(&ca)[4], uint4(&cb)[4], uint4(&na)[4], uint4(&nb)[4]) {
     constexpr bool HAS_FILL = decltype(has_fill)::value, HAS_NEXT = decltype(has_next)::value;
     constexpr int BEHIND = decltype(behindc)::value;
-    if constexpr (HAS_FILL)
-      issue(fill, a_fill, b_fill);
+    if constexpr (HAS_FILL) {
+      if (kf >= first_request)
+        issue(fill, a_fill, b_fill);
+    }
     if constexpr (HAS_NEXT) {
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEHIND * 4) : "memory");
       __builtin_amdgcn_s_barrier();
@@ -216,10 +232,10 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
       constexpr int nxt = (st + 1) % NST, fill = (st + NST - 1) % NST;
       const int kf = kt0 + st + NST - 1;
       if constexpr (st % 2 == 0)
-        stage(T{}, T{}, std::integral_constant<int, NST - 2>{}, smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB,
+        stage(T{}, T{}, std::integral_constant<int, NST - 2>{}, st == 0 ? kf : NST, smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB,
               b_ptr + kf * b_step, fa0, fb0, fa1, fb1);
       else
-        stage(T{}, T{}, std::integral_constant<int, NST - 2>{}, smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB,
+        stage(T{}, T{}, std::integral_constant<int, NST - 2>{}, st == 0 ? kf : NST, smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB,
               b_ptr + kf * b_step, fa1, fb1, fa0, fb0);
     });
   }
@@ -230,10 +246,10 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
     const int kf = kt0 + st + NST - 1;
     if constexpr (st % 2 == 0)
       stage(std::integral_constant<bool, st == 0>{}, std::integral_constant<bool, (st < NST - 1)>{}, std::integral_constant<int, behind>{},
-            smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB, b_ptr + kf * b_step, fa0, fb0, fa1, fb1);
+            kf, smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB, b_ptr + kf * b_step, fa0, fb0, fa1, fb1);
     else
       stage(std::integral_constant<bool, st == 0>{}, std::integral_constant<bool, (st < NST - 1)>{}, std::integral_constant<int, behind>{},
-            smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB, b_ptr + kf * b_step, fa1, fb1, fa0, fb0);
+            kf, smem + nxt * STAGE, smem + fill * STAGE, a_ptr + (int64_t)kf * KB, b_ptr + kf * b_step, fa1, fb1, fa0, fb0);
   });
 
   // the accumulator regions lie over the ring: every wave's reads of the last block must have returned

@@ -1446,6 +1446,49 @@ __device__ __forceinline__ void w4_epilogue_half_any(const GemmParams &p, int ki
 #undef GCMI_W4_CASE
 }
 
+// K not a whole number of ring groups (four k-blocks of 64 bytes): the incomplete group [k_full, K) is the FIRST one
+// computed, and this puts it into the ring's four slots before the main loop starts: whole k-blocks by DMA, the block
+// that K ends in through registers with zeros behind K (in both operands, so no product of theirs counts, whatever the
+// memory behind K holds), zero blocks without a load.  The main loop then requests from k = 0 on; its steady state
+// knows nothing of the tail.  (A tail handled behind the loop would need the accumulators outside the assembly.)
+// Before, every K that is no multiple of 128 bf16 / 256 bytes went to the bounds-checked kernel: 1237 x 4096 x 1376
+// ([N,K] weights) took 89.7 us there, 29.5 us as 320 tiles of 128 x 128.
+// a_src / b_src: the lane's byte offset per DMA instruction; a_chunk / b_kpos: what decides whether it lies before K.
+template <int ES, bool TB, int NDMA, int STAGE, int A_BYTES, typename OffA, typename OffB>
+__device__ __forceinline__ void fill_ring_k_tail(char *smem, int wave, int lane, const char *a_tail, const char *b_tail,
+                                                 int64_t b_step, int k_left, const OffA &a_src, const OffB &b_src,
+                                                 const int (&a_k)[NDMA], const int (&b_k)[NDMA]) {
+  constexpr int BK = 64 / ES;
+#pragma unroll 1
+  for (int blk = 0; blk < 4; blk++, k_left -= BK, a_tail += 64, b_tail += b_step) {
+    char *st = smem + blk * STAGE + wave * NDMA * 1024;
+    if (k_left >= BK) {
+#pragma unroll
+      for (int i = 0; i < NDMA; i++) {
+        __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(a_tail + (uint32_t)a_src[i]), (GCMI_LDS void *)(st + i * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(b_tail + (uint32_t)b_src[i]),
+                                         (GCMI_LDS void *)(st + A_BYTES + i * 1024), 16, 0, 0);
+      }
+      continue;
+    }
+    uint4 va[NDMA], vb[NDMA];
+#pragma unroll
+    for (int i = 0; i < NDMA; i++) {
+      va[i] = vb[i] = make_uint4(0, 0, 0, 0);
+      if (a_k[i] < k_left)
+        va[i] = *reinterpret_cast<const uint4 *>(a_tail + (uint32_t)a_src[i]);
+      if (b_k[i] < k_left)
+        vb[i] = *reinterpret_cast<const uint4 *>(b_tail + (uint32_t)b_src[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NDMA; i++) {
+      *reinterpret_cast<uint4 *>(st + i * 1024 + lane * 16) = va[i];
+      *reinterpret_cast<uint4 *>(st + A_BYTES + i * 1024 + lane * 16) = vb[i];
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+}
+
 template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gemm_tile256_w4_kernel(GemmParams p) {
   // B stored [N,K]: bf16 only.  (The same loop for 8-bit operands -- plain 16-byte fragment reads in place of the
   // transposing ones -- was measured against [K,N] on one board and is no faster: 166.9-168.9 against 167.2-168.6 us
@@ -1489,6 +1532,7 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
   // chunk's columns): their products land in accumulators that the epilogue never stores.
   const int rows_in = (int)min((int64_t)G_BM, p.M - m0), cols_in = (int)min((int64_t)G_BN, p.N - n0);
   i32x4_t a_off, b_off;
+  int a_k[4], b_k[4]; // the first k of the lane's 16 bytes inside a k-block
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int row = (wave * 4 + i) * FG::A_ROWS_PER_DMA + lane / FG::A_CPR;
@@ -1497,6 +1541,7 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
     const int krow = (wave * 4 + i) * FG::B_ROWS_PER_DMA + lane / FG::B_CPR;
     const int cb = min((lane % FG::B_CPR) ^ ((krow % FG::RG) * FG::CW), cols_in * ES / 16 - 1);
     b_off[i] = TB ? (int)(min(row, cols_in - 1) * ldb_b + c * 16) : (int)(krow * ldb_b + cb * 16);
+    a_k[i] = c * 16 / ES, b_k[i] = TB ? a_k[i] : krow;
   }
   // fragment addresses as in gemm_tile256_mi16_kernel: A tile `it` = rows wm*128 + 16*it .., B tile `jt` = columns
   // wn*128 + 16*jt ..; slots 2 and 3 through a second base (an instruction's offset field has 16 bits)
@@ -1542,7 +1587,17 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
   uint64_t a_ptr = (uint64_t)(reinterpret_cast<const char *>(p.A) + m0 * lda_b);
   uint64_t b_ptr = (uint64_t)(reinterpret_cast<const char *>(p.B) + (TB ? n0 * ldb_b : n0 * ES));
   uint64_t b_step = TB ? (uint64_t)FG::KB : (uint64_t)(FG::BK * ldb_b);
-  int trips = (int)(p.K / FG::BK) / 4 - 1; // k-blocks: a positive multiple of 4 (checked by the launcher)
+  // (a row of A is shorter than 2^31 bytes, so K fits 32 bits; inputs of the assembly in scalar registers)
+  const int K32 = (int)p.K;
+  int trips = __builtin_amdgcn_readfirstlane((K32 - 1) >> (ES == 2 ? 7 : 8)); // ring groups of four k-blocks, less the last one
+  const int k_left = __builtin_amdgcn_readfirstlane(K32 & (4 * FG::BK - 1));
+  const int ring_filled = k_left;
+  if (k_left) {
+    const int64_t k_full = p.K - k_left;
+    fill_ring_k_tail<ES, TB, 4, FG::STAGE_BYTES, FG::A_BYTES>(
+        smem, wave, lane, reinterpret_cast<const char *>(a_ptr) + k_full * ES,
+        reinterpret_cast<const char *>(b_ptr) + (TB ? k_full * ES : k_full * ldb_b), (int64_t)b_step, k_left, a_off, b_off, a_k, b_k);
+  }
   const uint32_t dma_lds = lds0 + (uint32_t)wave * 4096u;
   const uint32_t a_xor = p.a_xor;
   // where this lane writes its accumulators for the epilogue: row lane%16 (+ 16*it), 16-byte chunk lane/16 (+ 4*jt)
@@ -1552,7 +1607,7 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
 #define GCMI_W4_OPERANDS                                                                                              \
   : "+{s[40:41]}"(a_ptr), "+{s[42:43]}"(b_ptr), "+{s46}"(trips)                                                       \
   : "{v[0:3]}"(a_off), "{v[4:7]}"(b_off), "{v[8:9]}"(a_ld), "{v[10:17]}"(b_ld0), "{v[18:25]}"(b_ld2),                \
-    "{s[44:45]}"(b_step), "{s47}"(dma_lds), "{s48}"(a_xor), "{v26}"(dump_ld)                                        \
+    "{s[44:45]}"(b_step), "{s47}"(dma_lds), "{s48}"(a_xor), "{s50}"(ring_filled), "{v26}"(dump_ld)                   \
   : "memory", "scc", "s49", GCMI_W4_CLOBBERS
 #ifdef GCMI_W4_TIMING // measurement builds: core clock cycles and 100 MHz ticks spent in the main loop
   const long long tick0 = clock64(), wall0 = wall_clock64();
@@ -1739,10 +1794,13 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
   const int res_es = p.residual_dt == DT_BF16 ? 2 : 4;
   // the kernels for whole tiles read four residual elements with one load
   const bool res_vec = !p.residual || (al16(p.residual) && (p.ldr * res_es) % 16 == 0);
-  const bool aligned = p.K % KGROUP == 0 && p.K > 0 && al16(p.A) && al16(p.B) && al16(p.C) && res_vec &&
+  // K: whole 16-byte chunks; the 4-wave kernel and the 128 x 128 one take an incomplete last ring group themselves,
+  // the others need whole groups
+  const bool k_whole = p.K % KGROUP == 0;
+  const bool aligned = p.K % (16 / ES) == 0 && p.K > 0 && al16(p.A) && al16(p.B) && al16(p.C) && res_vec &&
                        (p.lda * ES) % 16 == 0 && (p.ldb * ES) % 16 == 0 && (p.ldc * out_es) % 16 == 0 &&
                        p.lda * ES * G_BM < (int64_t)1 << 31 && p.ldb * ES * (p.trans_b ? G_BN : BK) < (int64_t)1 << 31;
-  const bool fast_but_m = aligned && p.N % G_BN == 0;
+  const bool fast_but_m = aligned && k_whole && p.N % G_BN == 0;
   if (p.trans_b && ES != 2)
     return 3;
   if (p.residual && (ES != 2 || (p.residual_dt != DT_BF16 && p.residual_dt != DT_F32) || p.out_dt == DT_S32))
@@ -1758,9 +1816,9 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
   else if (!((p.a_bs * ES) % 16 == 0 && (p.b_bs * ES) % 16 == 0 && (p.c_bs * out_es) % 16 == 0 &&
              (!p.residual || (p.c_bs * res_es) % 16 == 0)))
     fast = false; // every batch's operands must keep the alignment the fast path loads with
-  // Any M, N a whole number of 16-byte chunks: the 4-wave kernel still takes it; its edge tiles clamp their loads
+  // Any M, N and K whole numbers of 16-byte chunks: the 4-wave kernel still takes it; its edge tiles clamp their loads
   // and store what lies inside C.
-  const bool ragged = !fast && aligned && p.N % (16 / ES) == 0 && (p.M % G_BM != 0 || p.N % G_BN != 0) &&
+  const bool ragged = !fast && aligned && p.N % (16 / ES) == 0 && (p.M % G_BM != 0 || p.N % G_BN != 0 || !k_whole) &&
                       (nbatch == 1 || ((p.a_bs * ES) % 16 == 0 && (p.b_bs * ES) % 16 == 0 && (p.c_bs * out_es) % 16 == 0 &&
                                        (!p.residual || (p.c_bs * res_es) % 16 == 0)));
   if (p.group_m <= 0)
@@ -1785,7 +1843,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
   const bool slices_can = ES == 2 && fast_but_m && p.out_dt != DT_S32 && nbatch == 1; // the 256-wide kernels: whole column tiles
   const int64_t nblk128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
   const int n_cu = gcmi_num_cus();
-  const int groups = (int)(p.K / KGROUP);
+  const int groups = (int)((p.K + KGROUP - 1) / KGROUP);
   int plan = PLAN_TILE256, splits = 1;
   if (p.cfg_tile == 128) {
     if (t128_can && nblk128 <= 0x7fffffff)

@@ -19,6 +19,8 @@ Register contract with the kernel (inputs in fixed registers, see the constraint
   s47       LDS address of this wave's 4 KiB share of slot 0's A tile (DMA target)
   s48       int8: 0x80808080 when A is u8 (the bytes are flipped to s8 on the way into the MFMA), else 0
   s49       scratch (keeps m0)
+  s50       not 0: the four slots hold k-blocks 0..3 already (an incomplete group of K, zero-filled by the set-up, which
+            has waited for them) and s[40:43] point at k-block 4: nothing is requested before the loop
   v26       LDS address at which this lane writes accumulator tile (0, 0) for the epilogue
   a[0:255]  out: accumulator tile (jt, it) = a[(jt*8+it)*4 : +4]
   v[32:63], v[64:95]    A fragments (8 row tiles x 4 registers) of even / odd k-blocks
@@ -191,6 +193,8 @@ def gen(es, tb):
 
     emit("s_mov_b32 s49, m0")  # m0 carries the DMA's LDS address in here; the compiler's value is put back
     # prologue: request k-blocks 0..3, clear the accumulators while they fly, take block 0 into registers
+    emit("s_cmp_lg_u32 s50, 0")
+    emit("s_cbranch_scc1 .LW4_FILLED_%=")
     for d in range(4):
         for i in range(8):
             m0, ld = dma(d, i)
@@ -199,6 +203,7 @@ def gen(es, tb):
             emit(ld)
         for ins in advance("a") + advance("b"):
             emit(ins)
+    emit(".LW4_FILLED_%=:")
     for r in range(256):
         emit("v_accvgpr_write_b32 a%d, 0" % r)
     emit("s_waitcnt vmcnt(24) lgkmcnt(0)")
