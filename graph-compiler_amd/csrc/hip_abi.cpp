@@ -32,6 +32,7 @@ int64_t gcmi_launch_gemm_bf16_workspace(const GemmParams *p);
 int gcmi_launch_gemm_bf16_config(const GemmParams *p, GemmTileConfig *cfg);
 int gcmi_launch_gemm_int8_config(const GemmParams *p, GemmTileConfig *cfg);
 int64_t gcmi_launch_mha_workspace(const MhaParams *p);
+int64_t gcmi_launch_mha_partial_bytes(const MhaParams *p);
 int gcmi_noalloc_scratch(void **ptr, size_t *bytes);
 }
 
@@ -138,6 +139,40 @@ int ws_acquire(size_t bytes, hipStream_t stream, LibraryWorkspace **out, void **
 void ws_release(LibraryWorkspace *w, hipStream_t stream) {
   w->used = true, w->last = stream;
   w->mu.unlock();
+}
+
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return stream == nullptr; // the null stream while another one is being captured: leave everything alone
+  }
+  return cap != hipStreamCaptureStatusNone;
+}
+
+// For calls that can do without: nothing is taken, and no error left, where the call's stream or the last user's is
+// being captured or the memory cannot be had.
+bool ws_try_acquire(size_t bytes, hipStream_t stream, LibraryWorkspace **out, void **ptr) {
+  if (capturing(stream))
+    return false;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
+    return false;
+  {
+    std::lock_guard<std::mutex> g(g_ws[dev].mu);
+    LibraryWorkspace &w = g_ws[dev];
+    if (w.used && !same_stream_for_sure(w.last, stream) && capturing(w.last))
+      return false;
+  }
+  // a first allocation must not break a capture that another thread has under way
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const int rc = ws_acquire(bytes, stream, out, ptr);
+  if (relaxed)
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (rc)
+    (void)hipGetLastError();
+  return rc == 0;
 }
 } // namespace
 
@@ -618,6 +653,14 @@ int mha_any(const void *Q, const void *K, const void *V, const float *mask, int6
     if (int rc = ws_acquire((size_t)want, (hipStream_t)stream, &lw, &lp))
       return rc;
     p.tile_class = (uint8_t *)lp, p.tile_class_cap = want;
+  }
+  // few queries of few heads: with scratch memory the keys are cut over workgroups.  Only where the library's own can be
+  // had without disturbing anyone (not under capture); otherwise the call runs in one piece as it is.
+  const int64_t cut = ws_from == Ws::Library && !lw ? gcmi_launch_mha_partial_bytes(&p) : 0;
+  if (cut > 0) {
+    void *lp = nullptr;
+    if (ws_try_acquire((size_t)cut, (hipStream_t)stream, &lw, &lp))
+      p.partial = (float *)lp;
   }
   int rc = gcmi_launch_mha_fwd(&p, (hipStream_t)stream);
   if (lw)
