@@ -82,22 +82,37 @@ bool same_stream_for_sure(hipStream_t a, hipStream_t b) {
   return a == b && a != nullptr && a != hipStreamPerThread && a != hipStreamLegacy;
 }
 
-// Takes the device's buffer (at least `bytes`) for one call on `stream`; the lock is held until release().
-int ws_acquire(size_t bytes, hipStream_t stream, LibraryWorkspace **out, void **ptr) {
-  // Under stream capture nothing here is legal (allocation, device-wide waits), and a captured graph would keep the
-  // address of a buffer that later calls share: such callers bring their own workspace.
+enum class Capture { No, Yes, Unknown };
+Capture capture_state(hipStream_t stream) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
     (void)hipGetLastError();
-    cap = hipStreamCaptureStatusNone;
+    return Capture::Unknown; // the null stream while another one is being captured, or a stream that no longer exists
   }
-  if (cap != hipStreamCaptureStatusNone)
+  return cap == hipStreamCaptureStatusNone ? Capture::No : Capture::Yes;
+}
+bool in_capture(hipStream_t stream) {
+  const Capture c = capture_state(stream);
+  return c == Capture::Yes || (c == Capture::Unknown && stream == nullptr);
+}
+
+// Takes the device's buffer (at least `bytes`) for one call on `stream`; the lock is held until release().  Returns ST_OK
+// with *out null where the call has to do without: the last user's stream is being captured (this call can neither be
+// put behind its work nor be drawn into its graph), or `optional` and the buffer cannot be had.  Everything is decided
+// under the one lock and for the one buffer that is then handed out.
+int ws_acquire(size_t bytes, hipStream_t stream, bool optional, LibraryWorkspace **out, void **ptr) {
+  *out = nullptr, *ptr = nullptr;
+  // Under stream capture nothing here is legal (allocation, device-wide waits), and a captured graph would keep the
+  // address of a buffer that later calls share: such callers bring their own workspace.
+  if (!optional && capture_state(stream) == Capture::Yes)
     return fail(ST_INVALID, "this call needs scratch memory and its stream is being captured: use the entry point that takes "
                             "a workspace (gcmi_gemm_bf16_ws / gcmi_mha_fwd_bf16_ws) or gcmi_gemm_bf16_noalloc");
+  if (in_capture(stream))
+    return ST_OK;
   // the buffer of the device the stream belongs to (the current device for the null and per-thread streams)
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
-    return fail(ST_RUNTIME, "workspace: no current device");
+    return optional ? ST_OK : fail(ST_RUNTIME, "workspace: no current device");
   if (stream != nullptr && stream != hipStreamPerThread && stream != hipStreamLegacy) {
     hipDevice_t sdev = 0;
     if (hipStreamGetDevice(stream, &sdev) == hipSuccess && (int)sdev >= 0 && (int)sdev < 64)
@@ -105,14 +120,23 @@ int ws_acquire(size_t bytes, hipStream_t stream, LibraryWorkspace **out, void **
     else
       (void)hipGetLastError();
   }
+  // a first allocation must not break a capture that another thread has under way
+  struct Relaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~Relaxed() {
+      if (set)
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+  } relaxed;
   LibraryWorkspace &w = g_ws[dev];
-  w.mu.lock();
+  std::unique_lock<std::mutex> lock(w.mu);
   if (w.cap < bytes) {
     const size_t want = bytes < ((size_t)8 << 20) ? ((size_t)8 << 20) : bytes;
     void *fresh = nullptr;
     if (hipMalloc(&fresh, want) != hipSuccess) {
-      w.mu.unlock();
-      return fail(1, "workspace: hipMalloc of %zu bytes failed", want);
+      (void)hipGetLastError();
+      return optional ? ST_OK : fail(1, "workspace: hipMalloc of %zu bytes failed", want);
     }
     if (w.ptr)
       w.retired.push_back(w.ptr); // never freed: see above
@@ -121,58 +145,31 @@ int ws_acquire(size_t bytes, hipStream_t stream, LibraryWorkspace **out, void **
   }
   if (!w.done && hipEventCreateWithFlags(&w.done, hipEventDisableTiming) != hipSuccess) {
     w.done = nullptr;
-    w.mu.unlock();
-    return fail(ST_RUNTIME, "workspace: hipEventCreate failed");
+    (void)hipGetLastError();
+    return optional ? ST_OK : fail(ST_RUNTIME, "workspace: hipEventCreate failed");
   }
   // A caller on another stream than the last user's waits for everything that stream has been given so far (the
   // marker is recorded now, behind the last user's kernels: nothing is recorded per call, so a single-stream caller
   // pays for no event).  A stream that no longer exists: wait for the device.
   if (w.used && !same_stream_for_sure(w.last, stream)) {
-    if (hipEventRecord(w.done, w.last) != hipSuccess || hipStreamWaitEvent(stream, w.done, 0) != hipSuccess) {
+    if (in_capture(w.last))
+      return ST_OK;
+    const bool marked = hipEventRecord(w.done, w.last) == hipSuccess;
+    // its owner does not hold this lock: had a capture begun by now, the marker might be a part of it
+    if (marked && in_capture(w.last))
+      return ST_OK;
+    if (!marked || hipStreamWaitEvent(stream, w.done, 0) != hipSuccess) {
       (void)hipGetLastError();
       (void)hipDeviceSynchronize();
     }
   }
+  lock.release(); // held on: ws_release
   *out = &w, *ptr = w.ptr;
   return ST_OK;
 }
 void ws_release(LibraryWorkspace *w, hipStream_t stream) {
   w->used = true, w->last = stream;
   w->mu.unlock();
-}
-
-bool capturing(hipStream_t stream) {
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
-    (void)hipGetLastError();
-    return stream == nullptr; // the null stream while another one is being captured: leave everything alone
-  }
-  return cap != hipStreamCaptureStatusNone;
-}
-
-// For calls that can do without: nothing is taken, and no error left, where the call's stream or the last user's is
-// being captured or the memory cannot be had.
-bool ws_try_acquire(size_t bytes, hipStream_t stream, LibraryWorkspace **out, void **ptr) {
-  if (capturing(stream))
-    return false;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
-    return false;
-  {
-    std::lock_guard<std::mutex> g(g_ws[dev].mu);
-    LibraryWorkspace &w = g_ws[dev];
-    if (w.used && !same_stream_for_sure(w.last, stream) && capturing(w.last))
-      return false;
-  }
-  // a first allocation must not break a capture that another thread has under way
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-  const int rc = ws_acquire(bytes, stream, out, ptr);
-  if (relaxed)
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (rc)
-    (void)hipGetLastError();
-  return rc == 0;
 }
 } // namespace
 
@@ -373,11 +370,12 @@ int gemm_bf16_any(bool trans_b, const void *A, const void *B, void *C, int64_t M
   }
   LibraryWorkspace *lw = nullptr;
   void *lp = nullptr;
-  if (int rc = ws_acquire((size_t)want * 4, (hipStream_t)stream, &lw, &lp))
+  if (int rc = ws_acquire((size_t)want * 4, (hipStream_t)stream, false, &lw, &lp))
     return rc;
-  p.partial = (float *)lp, p.partial_cap = want;
+  p.partial = (float *)lp, p.partial_cap = lw ? want : 0; // without: K is not sliced
   const int rc = launched(gcmi_launch_gemm_bf16(&p, (hipStream_t)stream), "gemm_bf16");
-  ws_release(lw, (hipStream_t)stream);
+  if (lw)
+    ws_release(lw, (hipStream_t)stream);
   return rc;
 }
 } // namespace
@@ -650,17 +648,17 @@ int mha_any(const void *Q, const void *K, const void *V, const float *mask, int6
     p.tile_class = (uint8_t *)ws, p.tile_class_cap = (int64_t)ws_bytes;
   } else if (want > 0) {
     void *lp = nullptr;
-    if (int rc = ws_acquire((size_t)want, (hipStream_t)stream, &lw, &lp))
+    if (int rc = ws_acquire((size_t)want, (hipStream_t)stream, false, &lw, &lp))
       return rc;
-    p.tile_class = (uint8_t *)lp, p.tile_class_cap = want;
+    p.tile_class = (uint8_t *)lp, p.tile_class_cap = lw ? want : 0; // without: every tile is read, the result is the same
   }
   // few queries of few heads: with scratch memory the keys are cut over workgroups.  Only where the library's own can be
   // had without disturbing anyone (not under capture); otherwise the call runs in one piece as it is.
   const int64_t cut = ws_from == Ws::Library && !lw ? gcmi_launch_mha_partial_bytes(&p) : 0;
   if (cut > 0) {
     void *lp = nullptr;
-    if (ws_try_acquire((size_t)cut, (hipStream_t)stream, &lw, &lp))
-      p.partial = (float *)lp;
+    (void)ws_acquire((size_t)cut, (hipStream_t)stream, true, &lw, &lp);
+    p.partial = (float *)lp;
   }
   int rc = gcmi_launch_mha_fwd(&p, (hipStream_t)stream);
   if (lw)
