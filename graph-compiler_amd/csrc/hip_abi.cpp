@@ -28,7 +28,7 @@ int gcmi_launch_brgemm(const void *A, const void *B, void *C, int64_t M, int64_t
                        int64_t LDB, int64_t LDC, int64_t stride_a, int64_t stride_b, int num, int beta_zero, int dtA,
                        int dtB, hipStream_t stream);
 int gcmi_launch_mha_fwd(const MhaParams *p, hipStream_t stream);
-int64_t gcmi_launch_gemm_bf16_workspace(const GemmParams *p);
+int64_t gcmi_launch_gemm_bf16_workspace(const GemmParams *p, int *optional);
 int gcmi_launch_gemm_bf16_config(const GemmParams *p, GemmTileConfig *cfg);
 int gcmi_launch_gemm_int8_config(const GemmParams *p, GemmTileConfig *cfg);
 int64_t gcmi_launch_mha_workspace(const MhaParams *p);
@@ -336,7 +336,8 @@ int gemm_bf16_any(bool trans_b, const void *A, const void *B, void *C, int64_t M
     (void)apply_matmul_config(matmul_config, M, N, K, p, &why); // not usable: ignored, as in the reference
   }
   // K-sliced shapes (a short A against wide weights) pass f32 partial sums through a workspace
-  const int64_t want = gcmi_launch_gemm_bf16_workspace(&p);
+  int optional = 0;
+  const int64_t want = gcmi_launch_gemm_bf16_workspace(&p, &optional);
   if (want <= 0)
     return launched(gcmi_launch_gemm_bf16(&p, (hipStream_t)stream), "gemm_bf16");
   if (ws_from == Ws::Caller) { // what the caller brought, however little: the launcher cuts fewer slices, or none
@@ -370,7 +371,7 @@ int gemm_bf16_any(bool trans_b, const void *A, const void *B, void *C, int64_t M
   }
   LibraryWorkspace *lw = nullptr;
   void *lp = nullptr;
-  if (int rc = ws_acquire((size_t)want * 4, (hipStream_t)stream, false, &lw, &lp))
+  if (int rc = ws_acquire((size_t)want * 4, (hipStream_t)stream, optional != 0, &lw, &lp))
     return rc;
   p.partial = (float *)lp, p.partial_cap = lw ? want : 0; // without: K is not sliced
   const int rc = launched(gcmi_launch_gemm_bf16(&p, (hipStream_t)stream), "gemm_bf16");
@@ -393,7 +394,8 @@ extern "C" size_t gcmi_gemm_bf16_workspace_bytes_cfg(int64_t M, int64_t N, int64
     const char *why;
     (void)apply_matmul_config(matmul_config, M, N, K, p, &why);
   }
-  const int64_t want = gcmi_launch_gemm_bf16_workspace(&p);
+  int optional = 0;
+  const int64_t want = gcmi_launch_gemm_bf16_workspace(&p, &optional);
   return want > 0 ? (size_t)want * 4 : 0;
 }
 
