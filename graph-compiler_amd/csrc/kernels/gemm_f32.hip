@@ -300,7 +300,10 @@ template <bool AKC, bool BKC> __global__ __launch_bounds__(256) void gemm_f32_sm
   constexpr int U = 8;
   __shared__ float red[3][256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lq = lane >> 4;
-  const int64_t nt = (p.N + 15) / 16, m0 = blockIdx.x / nt * 16, n0 = blockIdx.x % nt * 16;
+  const int64_t nt = (p.N + 15) / 16, t = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+  if (t >= (p.M + 15) / 16 * nt)
+    return;
+  const int64_t m0 = t / nt * 16, n0 = t % nt * 16;
   p.A += (int64_t)blockIdx.z * p.a_bs, p.B += (int64_t)blockIdx.z * p.b_bs, p.C += (int64_t)blockIdx.z * p.c_bs;
   const int64_t ga = m0 + l16 < p.M ? m0 + l16 : p.M - 1, gb = n0 + l16 < p.N ? n0 + l16 : p.N - 1;
   const float *a = p.A + ga * p.a_rs + 4 * lq * p.a_cs, *b = p.B + gb * p.b_cs + 4 * lq * p.b_rs;
@@ -535,13 +538,13 @@ extern "C" int gcmi_launch_gemm_f32(const F32GemmParams *pp, hipStream_t stream)
   // 16 bytes along m (A stored [K,M]) or n (B stored [K,N]) are a chunk of the tiles from 32 x 32 on: one must exist
   const bool akc = p.a_cs == 1, bkc = p.b_rs == 1 && p.b_cs != 1, chunk = (akc || p.M >= 4) && (bkc || p.N >= 4);
   const bool large = chunk && fmin(us(64, 1), us(128, 1)) < fmin(us(16, 1), us(32, 1));
-  const int tile = large ? (us(128, nbatch) < us(64, nbatch) ? 128 : 64) : chunk && us(32, nbatch) < us(16, nbatch) ? 32 : 16;
+  int tile = large ? (us(128, nbatch) < us(64, nbatch) ? 128 : 64) : chunk && us(32, nbatch) < us(16, nbatch) ? 32 : 16;
   const int layout = (akc ? 2 : 0) + (bkc ? 1 : 0);
   if (tile == 16) {
-    const int64_t all = ((p.N + 15) / 16) * ((p.M + 15) / 16);
-    if (all >= 1 << 24) // threads of a grid dimension
+    const int64_t all = ((p.N + 15) / 16) * ((p.M + 15) / 16), gx = all < 1 << 23 ? all : 1 << 23; // 2^32 threads a dimension
+    if ((all + gx - 1) / gx > 65535)
       return 2;
-    const dim3 grid((unsigned)all, 1, (unsigned)nbatch);
+    const dim3 grid((unsigned)gx, (unsigned)((all + gx - 1) / gx), (unsigned)nbatch);
     void (*const kernel[4])(F32GemmParams) = {gemm_f32_small_kernel<false, false>, gemm_f32_small_kernel<false, true>,
                                               gemm_f32_small_kernel<true, false>, gemm_f32_small_kernel<true, true>};
     hipLaunchKernelGGL(kernel[layout], grid, dim3(256), 0, stream, p);
@@ -550,7 +553,10 @@ extern "C" int gcmi_launch_gemm_f32(const F32GemmParams *pp, hipStream_t stream)
   static void (*const kernels[3][4])(F32GemmParams) = {F32_LAYOUTS(16, 32, 32, 1, 1, 4, 64),
                                                        F32_LAYOUTS(32, 64, 64, 2, 2, 1, 32),
                                                        F32_LAYOUTS(32, 128, 128, 2, 2, 1, 16)};
-  const int64_t per_xcd = (((p.M + tile - 1) / tile) * ((p.N + tile - 1) / tile) + 7) / 8;
+  auto per_xcd_of = [&](int t) { return (((p.M + t - 1) / t) * ((p.N + t - 1) / t) + 7) / 8; };
+  while (tile < 128 && per_xcd_of(tile) * 8 >= 1 << 24) // too many for a grid dimension: a question of one matrix as well
+    tile *= 2;
+  const int64_t per_xcd = per_xcd_of(tile);
   if (per_xcd * 8 >= 1 << 24)
     return 2;
   hipLaunchKernelGGL(kernels[tile == 32 ? 0 : tile == 64 ? 1 : 2][layout], dim3((unsigned)(per_xcd * 8), 1, (unsigned)nbatch), dim3(256), 0, stream, p);
