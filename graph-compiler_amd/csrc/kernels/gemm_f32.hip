@@ -296,13 +296,15 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(F32GemmParams p) {
 // row/column l % 16, and k = 4 * (l / 16) .. + 3 of the step as four operand values), eight steps in flight per wave,
 // no LDS and no barrier until the four partial sums are added.  128 x 512 x 256 (128 workgroups) in 7.2 us per call (10.6 as
 // 16 x 16 tiles of vector FMAs over LDS slices of 32 k with a barrier each).
+static constexpr int64_t F32_SMALL_GRID = 1 << 23; // workgroups of a grid's first dimension, at most: 2^32 threads are too many
 template <bool AKC, bool BKC> __global__ __launch_bounds__(256) void gemm_f32_small_kernel(F32GemmParams p) {
   constexpr int U = 8;
   __shared__ float red[3][256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lq = lane >> 4;
-  const int64_t nt = (p.N + 15) / 16, t = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
-  if (t >= (p.M + 15) / 16 * nt)
-    return;
+  // The size of the grid is a constant, and workgroups past the last tile (a grid of more than one row) compute rows that
+  // nobody stores: reading the size, or leaving early, puts a second wait for kernel arguments in front of the loads of
+  // every workgroup (0.2 us a launch).
+  const int64_t nt = (p.N + 15) / 16, t = blockIdx.x + (int64_t)blockIdx.y * F32_SMALL_GRID;
   const int64_t m0 = t / nt * 16, n0 = t % nt * 16;
   p.A += (int64_t)blockIdx.z * p.a_bs, p.B += (int64_t)blockIdx.z * p.b_bs, p.C += (int64_t)blockIdx.z * p.c_bs;
   const int64_t ga = m0 + l16 < p.M ? m0 + l16 : p.M - 1, gb = n0 + l16 < p.N ? n0 + l16 : p.N - 1;
@@ -541,7 +543,7 @@ extern "C" int gcmi_launch_gemm_f32(const F32GemmParams *pp, hipStream_t stream)
   int tile = large ? (us(128, nbatch) < us(64, nbatch) ? 128 : 64) : chunk && us(32, nbatch) < us(16, nbatch) ? 32 : 16;
   const int layout = (akc ? 2 : 0) + (bkc ? 1 : 0);
   if (tile == 16) {
-    const int64_t all = ((p.N + 15) / 16) * ((p.M + 15) / 16), gx = all < 1 << 23 ? all : 1 << 23; // 2^32 threads a dimension
+    const int64_t all = ((p.N + 15) / 16) * ((p.M + 15) / 16), gx = all < F32_SMALL_GRID ? all : F32_SMALL_GRID;
     if ((all + gx - 1) / gx > 65535)
       return 2;
     const dim3 grid((unsigned)gx, (unsigned)((all + gx - 1) / gx), (unsigned)nbatch);
