@@ -24,6 +24,7 @@ int gcmi_launch_gemm_bf16(const GemmParams *p, hipStream_t stream);
 int gcmi_launch_gemm_int8(const GemmParams *p, hipStream_t stream);
 int gcmi_launch_colsum_s8(const void *W, int64_t K, int64_t N, int64_t ldw, void *out, hipStream_t stream);
 int gcmi_launch_gemm_f32(const F32GemmParams *p, hipStream_t stream);
+int gcmi_launch_gemm_f32_config(const F32GemmParams *p, GemmTileConfig *cfg);
 int gcmi_launch_brgemm(const void *A, const void *B, void *C, int64_t M, int64_t N, int64_t K, int64_t LDA,
                        int64_t LDB, int64_t LDC, int64_t stride_a, int64_t stride_b, int num, int beta_zero, int dtA,
                        int dtB, hipStream_t stream);
@@ -435,6 +436,15 @@ extern "C" int gcmi_gemm_tile_config_query(int a_dtype, int64_t M, int64_t N, in
   if (!out || M <= 0 || N <= 0 || K <= 0)
     return fail(ST_INVALID, "gemm_tile_config_query: bad arguments");
   const bool i8 = a_dtype == GCMI_S8 || a_dtype == GCMI_U8;
+  static_assert(sizeof(gcmi_gemm_tile_config) == sizeof(GemmTileConfig), "the public struct mirrors GemmTileConfig");
+  if (a_dtype == GCMI_F32) { // A stored [M,K]; no MatmulConfig steers these
+    F32GemmParams f{};
+    f.M = M, f.N = N, f.K = K, f.a_rs = K, f.a_cs = 1, f.b_rs = trans_b ? 1 : N, f.b_cs = trans_b ? K : 1;
+    GemmTileConfig c{};
+    (void)gcmi_launch_gemm_f32_config(&f, &c);
+    memcpy(out, &c, sizeof(c));
+    return ST_OK;
+  }
   if (!i8 && a_dtype != GCMI_BF16)
     return fail(ST_UNIMPL, "gemm_tile_config_query: a_dtype %d", a_dtype);
   GemmParams p{};
@@ -452,7 +462,6 @@ extern "C" int gcmi_gemm_tile_config_query(int a_dtype, int64_t M, int64_t N, in
   const int rc = i8 ? gcmi_launch_gemm_int8_config(&p, &c) : gcmi_launch_gemm_bf16_config(&p, &c);
   if (rc)
     return fail(rc, "gemm_tile_config_query: no kernel takes this call");
-  static_assert(sizeof(gcmi_gemm_tile_config) == sizeof(GemmTileConfig), "the public struct mirrors GemmTileConfig");
   memcpy(out, &c, sizeof(c));
   return ST_OK;
 }

@@ -365,6 +365,96 @@ template <bool AKC, bool BKC> __global__ __launch_bounds__(256) void gemm_f32_sm
   }
 }
 
+// A short K (see f32_plan): products on the vector ALU.  BT x BT workgroup tile (BT = 64, 32 or 16: small problems
+// take small tiles so that more compute units take part), 256 threads, (BT/16)^2 outputs per thread, 32-deep K slices
+// through LDS: with one slice a workgroup is one load, one barrier and one store, where the matrix kernels' slices of 32
+// and 64 k come half empty.
+template <int BT> __global__ __launch_bounds__(256) void gemm_f32_fma_kernel(F32GemmParams p) {
+  constexpr int BK = 32, MT = BT / 16, PER = BT * BK / 256; // elements per thread per operand slice
+  __shared__ float As[BK][BT + 4];
+  __shared__ float Bs[BK][BT + 4];
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  const int64_t m0 = (int64_t)blockIdx.y * BT, n0 = (int64_t)blockIdx.x * BT;
+  p.A += (int64_t)blockIdx.z * p.a_bs, p.B += (int64_t)blockIdx.z * p.b_bs, p.C += (int64_t)blockIdx.z * p.c_bs;
+  // slice element e of this thread: (row/col within the tile, k within the slice);
+  // the contiguous direction of each operand runs along consecutive threads
+  int am[PER], ak[PER], bn[PER], bk[PER];
+#pragma unroll
+  for (int e = 0; e < PER; e++) {
+    const int idx = threadIdx.x + 256 * e;
+    if (p.a_cs == 1) {
+      ak[e] = idx % BK;
+      am[e] = idx / BK;
+    } else {
+      am[e] = idx % BT;
+      ak[e] = idx / BT;
+    }
+    if (p.b_rs == 1 && p.b_cs != 1) {
+      bk[e] = idx % BK;
+      bn[e] = idx / BK;
+    } else {
+      bn[e] = idx % BT;
+      bk[e] = idx / BT;
+    }
+  }
+  float ra[PER], rb[PER];
+  auto fetch = [&](int64_t k0) {
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      const int64_t gm = m0 + am[e], gk = k0 + ak[e];
+      ra[e] = (gm < p.M && gk < p.K) ? p.A[gm * p.a_rs + gk * p.a_cs] : 0.0f;
+      const int64_t gn = n0 + bn[e], gk2 = k0 + bk[e];
+      rb[e] = (gn < p.N && gk2 < p.K) ? p.B[gk2 * p.b_rs + gn * p.b_cs] : 0.0f;
+    }
+  };
+  float acc[MT][MT] = {};
+  fetch(0);
+  for (int64_t k0 = 0; k0 < p.K; k0 += BK) {
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      As[ak[e]][am[e]] = ra[e];
+      Bs[bk[e]][bn[e]] = rb[e];
+    }
+    __syncthreads();
+    if (k0 + BK < p.K)
+      fetch(k0 + BK);
+#pragma unroll
+    for (int k = 0; k < BK; k++) { // k ascending per output element
+      float a[MT], b[MT];
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+        a[i] = As[k][ty * MT + i];
+#pragma unroll
+      for (int j = 0; j < MT; j++)
+        b[j] = Bs[k][tx * MT + j];
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+          acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    int64_t m = m0 + ty * MT + i;
+    if (m >= p.M)
+      continue;
+#pragma unroll
+    for (int j = 0; j < MT; j++) {
+      int64_t n = n0 + tx * MT + j;
+      if (n >= p.N)
+        continue;
+      float x = acc[i][j];
+      if (p.beta != 0.0f)
+        x = x + p.C[m * p.ldc + n];
+      if (p.bias)
+        x = x + p.bias[n];
+      p.C[m * p.ldc + n] = apply_act(x, p.act);
+    }
+  }
+}
+
 struct BrgemmParams {
   const void *A, *B;
   void *C;
@@ -513,6 +603,60 @@ using namespace gcmi;
   {gemm_f32_mfma_kernel<__VA_ARGS__, false, false>, gemm_f32_mfma_kernel<__VA_ARGS__, false, true>,                   \
    gemm_f32_mfma_kernel<__VA_ARGS__, true, false>, gemm_f32_mfma_kernel<__VA_ARGS__, true, true>}
 
+static bool f32_a_along_k(const F32GemmParams &p) { return p.a_cs == 1; }
+static bool f32_b_along_k(const F32GemmParams &p) { return p.b_rs == 1 && p.b_cs != 1; }
+struct F32Plan {
+  int tile;
+  bool vector; // gemm_f32_fma_kernel
+};
+// The tile by estimated time (us, fitted to graph-replayed launches of 1 .. 2048 rows, 16 .. 3000 columns and K 16 .. 3000 on
+// one MI355X; n tiles per compute unit, k = K / 1000; two constants where a lone workgroup of a compute unit is slower
+// than one of several): tiles are dealt out evenly, a compute unit is done when the one with the most is, and a tile
+// costs its start and its stores whatever K is.  1111 x 1000, K 3000, in us: 128 x 128 198, 64 x 64 100, 32 x 32 77;
+// 4096^3: 1025, 1051, 1218; 1000 x 1000 x 1000: 75, 24-26, 29; 300 x 300, K 1000: 73, 23, 11.4 and 8.3 with 16 x 16 tiles;
+// 1071 x 2048, K 16: 13, 8.7, 17, 17 (an estimate without the cost of a tile took 16 x 16 here).
+// The two small tiles add an element's products in the same order, and so do the two large ones, and the vector
+// kernel whatever its tile: which of the three is taken depends on one matrix, so a batch has the bits of its matrices
+// multiplied one by one.
+static F32Plan f32_plan(const F32GemmParams &p) {
+  const double cus = gcmi_num_cus(), k = (double)p.K * 1e-3, nbatch = (double)(p.batch > 1 ? p.batch : 1);
+  auto tiles = [&](int64_t t) { return (double)(((p.M + t - 1) / t) * ((p.N + t - 1) / t)); };
+  auto us = [&](int tile, double batches) {
+    const double n = batches * tiles(tile) / cus; // per compute unit
+    switch (tile) {
+    case 16: return 2.7 + fmax(3.8 * k, (0.38 + 2.7 * k) * n);
+    case 32: return 4.6 + (1.3 + 4.6 * k) * ceil(n);
+    case 64: return 4.5 + 1.1 * ceil(n) + k * fmax(18.3, 16.2 * ceil(n));
+    default: return 7.5 + 4.0 * ceil(n) + k * fmax(63.0, 60.0 * ceil(n));
+    }
+  };
+  // A K of one 32-deep slice and less than a round of 64 x 64 tiles: the vector kernel.  256 x 2048, K 32: 4.5 us, 5.6
+  // on the best matrix tile; 512 x 2048: 8.5 and 5.9; K 40: 5.9 and 6.6, but 256 x 3000 7.2 and 6.8, 512 x 1500 7.4 and 6.8.
+  if (p.K <= 32 && tiles(64) < cus && (p.M + 15) / 16 <= 65535)
+    return {tiles(64) * nbatch >= cus ? 64 : tiles(32) * nbatch >= cus ? 32 : 16, true};
+  // 16 bytes along m (A stored [K,M]) or n (B stored [K,N]) are a chunk of the tiles from 32 x 32 on: one must exist
+  const bool chunk = (f32_a_along_k(p) || p.M >= 4) && (f32_b_along_k(p) || p.N >= 4);
+  if (chunk && fmin(us(64, 1), us(128, 1)) < fmin(us(16, 1), us(32, 1)))
+    return {us(128, nbatch) < us(64, nbatch) ? 128 : 64, false};
+  return {chunk && us(32, nbatch) < us(16, nbatch) ? 32 : 16, false};
+}
+
+// what the launch below would choose (nothing is launched)
+extern "C" int gcmi_launch_gemm_f32_config(const F32GemmParams *p, GemmTileConfig *cfg) {
+  const F32Plan plan = f32_plan(*p);
+  GemmTileConfig c{};
+  c.kernel = GK_F32, c.bm = c.bn = plan.tile, c.split_k = 1, c.group_m = 8;
+  c.workgroups = (int32_t)(((p->M + plan.tile - 1) / plan.tile) * ((p->N + plan.tile - 1) / plan.tile));
+  c.stages = plan.vector || plan.tile == 16 ? 1 : 2;
+  c.kbytes = plan.vector ? 128 : plan.tile == 16 ? 0 : plan.tile == 32 ? 256 : plan.tile == 64 ? 128 : 64;
+  c.waves_m = c.waves_n = plan.tile >= 64 && !plan.vector ? 2 : 1;
+  c.wave_m = c.wave_n = plan.tile / c.waves_m;
+  if (!plan.vector)
+    c.mfma_m = c.mfma_n = plan.tile >= 64 ? 32 : 16, c.mfma_k = plan.tile >= 64 ? 2 : 4;
+  *cfg = c;
+  return 0;
+}
+
 extern "C" int gcmi_launch_gemm_f32(const F32GemmParams *pp, hipStream_t stream) {
   F32GemmParams p = *pp;
   if (p.M <= 0 || p.N <= 0)
@@ -520,28 +664,15 @@ extern "C" int gcmi_launch_gemm_f32(const F32GemmParams *pp, hipStream_t stream)
   const int64_t nbatch = p.batch > 1 ? p.batch : 1;
   if (nbatch > 65535)
     return 2;
-  // The tile by estimated time (ns per k, measured on one MI355X; two constants where a lone workgroup of a compute
-  // unit is slower than one of several): tiles are dealt out evenly, a compute unit is done when the one with the most
-  // is.  1111 x 1000, K 3000, in us: 128 x 128 198, 64 x 64 100, 32 x 32 77; 4096^3: 1025, 1051, 1218; 1000 x 1000 x
-  // 1000: 75, 24-26, 29; 300 x 300, K 1000: 73, 23, 11.4 and 8.3 with 16 x 16 tiles.
-  // The two small tiles add an element's products in the same order, and so do the two large ones: which pair is
-  // taken depends on one matrix, so a batch has the bits of its matrices multiplied one by one.
-  const double cus = gcmi_num_cus(), k = (double)p.K * 1e-3;
-  auto tiles = [&](int64_t bm, int64_t bn) { return (double)(((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn)); };
-  auto us = [&](int tile, double batches) {
-    const double n = batches * tiles(tile, tile) / cus; // per compute unit
-    switch (tile) {
-    case 16: return 2.0 + k * 2.7 * fmax(1.0, n);
-    case 32: return 4.0 + k * 4.5 * ceil(n);
-    case 64: return 4.0 + k * fmax(18.0, 15.5 * ceil(n));
-    default: return 5.0 + k * fmax(63.0, 60.0 * ceil(n));
-    }
-  };
-  // 16 bytes along m (A stored [K,M]) or n (B stored [K,N]) are a chunk of the tiles from 32 x 32 on: one must exist
-  const bool akc = p.a_cs == 1, bkc = p.b_rs == 1 && p.b_cs != 1, chunk = (akc || p.M >= 4) && (bkc || p.N >= 4);
-  const bool large = chunk && fmin(us(64, 1), us(128, 1)) < fmin(us(16, 1), us(32, 1));
-  int tile = large ? (us(128, nbatch) < us(64, nbatch) ? 128 : 64) : chunk && us(32, nbatch) < us(16, nbatch) ? 32 : 16;
-  const int layout = (akc ? 2 : 0) + (bkc ? 1 : 0);
+  const F32Plan plan = f32_plan(p);
+  int tile = plan.tile;
+  const int layout = (f32_a_along_k(p) ? 2 : 0) + (f32_b_along_k(p) ? 1 : 0);
+  if (plan.vector) {
+    const dim3 grid((unsigned)((p.N + tile - 1) / tile), (unsigned)((p.M + tile - 1) / tile), (unsigned)nbatch);
+    hipLaunchKernelGGL(tile == 64 ? gemm_f32_fma_kernel<64> : tile == 32 ? gemm_f32_fma_kernel<32> : gemm_f32_fma_kernel<16>, grid,
+                       dim3(256), 0, stream, p);
+    return hipGetLastError() == hipSuccess ? 0 : 5;
+  }
   if (tile == 16) {
     const int64_t all = ((p.N + 15) / 16) * ((p.M + 15) / 16), gx = all < F32_SMALL_GRID ? all : F32_SMALL_GRID;
     if ((all + gx - 1) / gx > 65535)

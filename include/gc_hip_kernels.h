@@ -149,7 +149,9 @@ int gcmi_gemm_bf16_ws(const void *A, const void *B, void *C, int64_t batch, int6
  * the 8-wave kernel with the LDS ring, with split_k > 1 followed by the second
  * pass), 5 tiles of 128 x 128 with 4 waves
  * of 64 x 64 (problems of few 256 x 256 tiles; with split_k > 1 kind 3 is
- * reported and bm = bn = 128 tells).
+ * reported and bm = bn = 128 tells), 6 the f32 kernels (a_dtype GCMI_F32, A
+ * stored [M,K]: bm = bn = 16, 32, 64 or 128, mfma_m = 0 for the vector kernel of
+ * a short K).
  *
  * matmul_config (may be NULL) is the reference's per-op override: the nine
  * integers {MThreads, NThreads, KThreads, MBlock, NBlock, KBlock,
