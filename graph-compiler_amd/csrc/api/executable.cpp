@@ -235,7 +235,8 @@ char *Executable::staging() {
   return staging_;
 }
 
-// Scratch of the steps whose kernels need some (partial sums of K-sliced GEMMs, mask tile classes of attention): a
+// Scratch of the steps whose kernels need some (partial sums of K-sliced GEMMs, mask tile classes of attention, partial
+// results of attention whose keys are cut over workgroups): a
 // slot of the step's own, alive for that step only, so it shares arena space with other temporaries.  Nothing is
 // shared between executables or streams: two executables may run side by side, as the reference's may
 // (thread-local scratch, lib/gc/ExecutionEngine/CPURuntime/Microkernel/BrgemmOnednn.cpp:70).
@@ -244,8 +245,8 @@ void Executable::plan_workspaces() {
     size_t bytes = 0;
     if (s.kind == Step::GemmBf16 && s.batch <= 1)
       bytes = gcmi_gemm_bf16_workspace_bytes_cfg(s.M, s.N, s.K, s.tb ? 1 : 0, s.mm_cfg.size() == 9 ? s.mm_cfg.data() : nullptr);
-    else if (s.kind == Step::Mha && s.mask >= 0 && s.ws < 0)
-      bytes = gcmi_mha_fwd_workspace_bytes(s.Sq, s.Sk, s.D, 1);
+    else if (s.kind == Step::Mha && s.ws < 0)
+      bytes = gcmi_mha_fwd_workspace_bytes_bh(s.BH, s.Sq, s.Sk, s.D, s.mask >= 0 ? 1 : 0);
     if (bytes)
       s.ws = new_slot(bytes);
   }

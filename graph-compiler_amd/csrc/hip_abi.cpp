@@ -626,6 +626,15 @@ extern "C" size_t gcmi_mha_fwd_workspace_bytes(int64_t Sq, int64_t Sk, int64_t D
   return want > 0 ? (size_t)want : 0;
 }
 
+extern "C" size_t gcmi_mha_fwd_workspace_bytes_bh(int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int has_mask) {
+  if (BH <= 0 || Sq <= 0 || Sk <= 0 || BH > 0x7fffffff || Sq > 0x7fffffff || Sk > 0x7fffffff)
+    return 0;
+  MhaParams p{};
+  p.BH = (int)BH, p.Sq = (int)Sq, p.Sk = (int)Sk, p.D = (int)D;
+  const int64_t cut = gcmi_launch_mha_partial_bytes(&p); // fewer than 128 queries; the mask's classes: 128 and more
+  return cut > 0 ? (size_t)cut : gcmi_mha_fwd_workspace_bytes(Sq, Sk, D, has_mask);
+}
+
 namespace {
 int mha_any(const void *Q, const void *K, const void *V, const float *mask, int64_t mask_ld, void *O, int64_t BH,
             int64_t Sq, int64_t Sk, int64_t D, float scale, int skip_masked, void *stream, Ws ws_from, void *ws,
@@ -663,10 +672,14 @@ int mha_any(const void *Q, const void *K, const void *V, const float *mask, int6
       return rc;
     p.tile_class = (uint8_t *)lp, p.tile_class_cap = lw ? want : 0; // without: every tile is read, the result is the same
   }
-  // few queries of few heads: with scratch memory the keys are cut over workgroups.  Only where the library's own can be
-  // had without disturbing anyone (not under capture); otherwise the call runs in one piece as it is.
-  const int64_t cut = ws_from == Ws::Library && !lw ? gcmi_launch_mha_partial_bytes(&p) : 0;
-  if (cut > 0) {
+  // few queries of few heads: with scratch memory the keys are cut over workgroups, into ranges that follow from the sizes.
+  // The caller's where it holds enough (and not classes that other calls read), else the library's where that can be had
+  // without disturbing anyone (not under capture); otherwise the call runs in one piece as it is.
+  const int64_t cut = gcmi_launch_mha_partial_bytes(&p);
+  if (cut > 0 && ws_from == Ws::Caller) {
+    if (ws && (int64_t)ws_bytes >= cut && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 && !p.classes_mode)
+      p.partial = (float *)ws;
+  } else if (cut > 0) {
     void *lp = nullptr;
     (void)ws_acquire((size_t)cut, (hipStream_t)stream, true, &lw, &lp);
     p.partial = (float *)lp;

@@ -273,10 +273,19 @@ int gcmi_mha_fwd_bf16_opt(const void *Q, const void *K, const void *V, const flo
                           int64_t BH, int64_t Sq, int64_t Sk, int64_t D, float scale, int skip_masked, void *stream);
 
 /*
- * The same with the workspace as an argument: one byte per (32 query rows x 64
- * keys) mask tile, gcmi_mha_fwd_workspace_bytes in all (0: the shape has no
- * use for one).  With NULL or too small a workspace every tile is read from
- * the mask and nothing is skipped; the result is the same.
+ * The same with the workspace as an argument (gcmi_mha_fwd_workspace_bytes_bh
+ * bytes; 0: the shape has no use for one).
+ * From 128 queries on: one byte per (32 query rows x 64 keys) mask tile
+ * (gcmi_mha_fwd_workspace_bytes gives this part alone).  With NULL or too small
+ * a workspace every tile is read from the mask and nothing is skipped; the
+ * result is the same.
+ * Fewer than 128 queries of few (batch, head): f32 partial results of the key
+ * ranges that are cut over workgroups.  The ranges depend on the sizes alone, so
+ * with a workspace of that size (16-byte aligned, and without
+ * GCMI_MHA_CLASSES_VALID, which makes it read-only) the result has the bits that
+ * the entry points without the argument give; with a smaller one the keys of a
+ * head stay in one workgroup: slower, the weights of later ranges rounded
+ * relative to another maximum, the sums in another order.
  *
  * A mask that does not change between calls (a constant of the partition, the
  * counterpart of the reference's constant-tensor cache, src/dnnl/JsonParser.cpp:
@@ -289,6 +298,7 @@ int gcmi_mha_fwd_bf16_opt(const void *Q, const void *K, const void *V, const flo
 #define GCMI_MHA_SKIP_MASKED 1
 #define GCMI_MHA_CLASSES_VALID 2
 size_t gcmi_mha_fwd_workspace_bytes(int64_t Sq, int64_t Sk, int64_t D, int has_mask);
+size_t gcmi_mha_fwd_workspace_bytes_bh(int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int has_mask);
 int gcmi_mha_classify_mask(const float *mask, int64_t mask_ld, int64_t Sq, int64_t Sk, int64_t D, void *workspace,
                            size_t workspace_bytes, void *stream);
 int gcmi_mha_fwd_bf16_ws(const void *Q, const void *K, const void *V, const float *mask, int64_t mask_ld, void *O,
