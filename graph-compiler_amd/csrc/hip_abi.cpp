@@ -60,17 +60,23 @@ namespace {
 // Where a call's scratch (partial sums of K-sliced GEMMs, mask tile classes of attention) comes from.
 enum class Ws { Library, Caller, Static };
 
-// Scratch of the entry points that take no workspace argument: one buffer per device, allocated at the first call
-// that needs it and grown on demand.  Every call on the device shares it, so its users are put in order: the mutex
-// is held while a call's kernels are enqueued, an event is recorded behind them, and a call on another stream
-// waits for that event first.
+// Scratch of the entry points that take no workspace argument: up to WS_BLOCKS buffers per device, allocated at the
+// first call that needs one more and grown on demand.  A stream keeps to the buffer that it used last, so callers on up to
+// that many streams never meet; beyond, a call takes the buffer that has not been handed out for longest and is put in
+// order behind the stream that used it: an event is recorded there and waited for.  The mutex is held while a call's
+// kernels are enqueued.
+static constexpr int WS_BLOCKS = 4;
 struct LibraryWorkspace {
+  struct Block {
+    void *ptr = nullptr;
+    size_t cap = 0;
+    hipEvent_t done = nullptr;
+    hipStream_t last = nullptr;
+    uint64_t used = 0; // number of the call that used it last, 0: none
+  } blocks[WS_BLOCKS];
   std::mutex mu;
-  void *ptr = nullptr;
-  size_t cap = 0;
-  hipEvent_t done = nullptr;
-  hipStream_t last = nullptr;
-  bool used = false;
+  uint64_t calls = 0;
+  Block *taken = nullptr; // by the call that holds the lock
   // Blocks that were outgrown.  They are kept until the process ends: a kernel enqueued earlier (or a HIP graph
   // captured from an earlier call through an entry point that did not refuse capture) may still name them.
   std::vector<void *> retired;
@@ -97,10 +103,10 @@ bool in_capture(hipStream_t stream) {
   return c == Capture::Yes || (c == Capture::Unknown && stream == nullptr);
 }
 
-// Takes the device's buffer (at least `bytes`) for one call on `stream`; the lock is held until release().  Returns ST_OK
-// with *out null where the call has to do without: the last user's stream is being captured (this call can neither be
-// put behind its work nor be drawn into its graph), or `optional` and the buffer cannot be had.  Everything is decided
-// under the one lock and for the one buffer that is then handed out.
+// Takes a buffer of the device (at least `bytes`) for one call on `stream`; the lock is held until release().  Returns
+// ST_OK with *out null where the call has to do without: the stream it would have to wait for is being captured (this call
+// can neither be put behind its work nor be drawn into its graph), or `optional` and no buffer can be had.  Everything is
+// decided under the one lock and for the one buffer that is then handed out.
 int ws_acquire(size_t bytes, hipStream_t stream, bool optional, LibraryWorkspace **out, void **ptr) {
   *out = nullptr, *ptr = nullptr;
   // Under stream capture nothing here is legal (allocation, device-wide waits), and a captured graph would keep the
@@ -132,44 +138,59 @@ int ws_acquire(size_t bytes, hipStream_t stream, bool optional, LibraryWorkspace
   } relaxed;
   LibraryWorkspace &w = g_ws[dev];
   std::unique_lock<std::mutex> lock(w.mu);
-  if (w.cap < bytes) {
+  // this stream's own block, else one that nobody has used, else the one that was used longest ago
+  LibraryWorkspace::Block *b = nullptr;
+  for (auto &x : w.blocks)
+    if (x.used && x.last == stream && (!b || x.used > b->used))
+      b = &x;
+  for (auto &x : w.blocks)
+    if (!b && !x.used)
+      b = &x;
+  if (!b) {
+    b = &w.blocks[0];
+    for (auto &x : w.blocks)
+      if (x.used < b->used)
+        b = &x;
+  }
+  if (b->cap < bytes) {
     const size_t want = bytes < ((size_t)8 << 20) ? ((size_t)8 << 20) : bytes;
     void *fresh = nullptr;
     if (hipMalloc(&fresh, want) != hipSuccess) {
       (void)hipGetLastError();
       return optional ? ST_OK : fail(1, "workspace: hipMalloc of %zu bytes failed", want);
     }
-    if (w.ptr)
-      w.retired.push_back(w.ptr); // never freed: see above
-    w.ptr = fresh, w.cap = want;
-    // the new block has no earlier user, but the order between callers is kept as it was (w.used, w.last)
+    if (b->ptr)
+      w.retired.push_back(b->ptr); // never freed: see above
+    b->ptr = fresh, b->cap = want;
+    // the new memory has no earlier user, but the order between callers is kept as it was (used, last)
   }
-  if (!w.done && hipEventCreateWithFlags(&w.done, hipEventDisableTiming) != hipSuccess) {
-    w.done = nullptr;
+  if (!b->done && hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess) {
+    b->done = nullptr;
     (void)hipGetLastError();
     return optional ? ST_OK : fail(ST_RUNTIME, "workspace: hipEventCreate failed");
   }
-  // A caller on another stream than the last user's waits for everything that stream has been given so far (the
-  // marker is recorded now, behind the last user's kernels: nothing is recorded per call, so a single-stream caller
-  // pays for no event).  A stream that no longer exists: wait for the device.
-  if (w.used && !same_stream_for_sure(w.last, stream)) {
-    if (in_capture(w.last))
+  // A caller on another stream than the block's last user waits for everything that stream has been given so far (the
+  // marker is recorded now, behind the last user's kernels: nothing is recorded per call, so a caller on a stream of its
+  // own pays for no event).  A stream that no longer exists: wait for the device.
+  if (b->used && !same_stream_for_sure(b->last, stream)) {
+    if (in_capture(b->last))
       return ST_OK;
-    const bool marked = hipEventRecord(w.done, w.last) == hipSuccess;
+    const bool marked = hipEventRecord(b->done, b->last) == hipSuccess;
     // its owner does not hold this lock: had a capture begun by now, the marker might be a part of it
-    if (marked && in_capture(w.last))
+    if (marked && in_capture(b->last))
       return ST_OK;
-    if (!marked || hipStreamWaitEvent(stream, w.done, 0) != hipSuccess) {
+    if (!marked || hipStreamWaitEvent(stream, b->done, 0) != hipSuccess) {
       (void)hipGetLastError();
       (void)hipDeviceSynchronize();
     }
   }
+  w.taken = b;
   lock.release(); // held on: ws_release
-  *out = &w, *ptr = w.ptr;
+  *out = &w, *ptr = b->ptr;
   return ST_OK;
 }
 void ws_release(LibraryWorkspace *w, hipStream_t stream) {
-  w->used = true, w->last = stream;
+  w->taken->used = ++w->calls, w->taken->last = stream;
   w->mu.unlock();
 }
 } // namespace
