@@ -651,6 +651,7 @@ extern "C" size_t gcmi_mha_fwd_workspace_bytes_bh(int64_t BH, int64_t Sq, int64_
   if (BH <= 0 || Sq <= 0 || Sk <= 0 || BH > 0x7fffffff || Sq > 0x7fffffff || Sk > 0x7fffffff)
     return 0;
   MhaParams p{};
+  p.mask = has_mask ? (const float *)(uintptr_t)256 : nullptr;
   p.BH = (int)BH, p.Sq = (int)Sq, p.Sk = (int)Sk, p.D = (int)D;
   const int64_t cut = gcmi_launch_mha_partial_bytes(&p); // fewer than 128 queries; the mask's classes: 128 and more
   return cut > 0 ? (size_t)cut : gcmi_mha_fwd_workspace_bytes(Sq, Sk, D, has_mask);
