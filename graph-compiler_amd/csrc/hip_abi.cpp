@@ -111,10 +111,11 @@ int ws_acquire(size_t bytes, hipStream_t stream, bool optional, LibraryWorkspace
   *out = nullptr, *ptr = nullptr;
   // Under stream capture nothing here is legal (allocation, device-wide waits), and a captured graph would keep the
   // address of a buffer that later calls share: such callers bring their own workspace.
-  if (!optional && capture_state(stream) == Capture::Yes)
+  const Capture own = capture_state(stream);
+  if (!optional && own == Capture::Yes)
     return fail(ST_INVALID, "this call needs scratch memory and its stream is being captured: use the entry point that takes "
                             "a workspace (gcmi_gemm_bf16_ws / gcmi_mha_fwd_bf16_ws) or gcmi_gemm_bf16_noalloc");
-  if (in_capture(stream))
+  if (own == Capture::Yes || (own == Capture::Unknown && stream == nullptr))
     return ST_OK;
   // the buffer of the device the stream belongs to (the current device for the null and per-thread streams)
   int dev = 0;
@@ -127,15 +128,6 @@ int ws_acquire(size_t bytes, hipStream_t stream, bool optional, LibraryWorkspace
     else
       (void)hipGetLastError();
   }
-  // a first allocation must not break a capture that another thread has under way
-  struct Relaxed {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    ~Relaxed() {
-      if (set)
-        (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-  } relaxed;
   LibraryWorkspace &w = g_ws[dev];
   std::unique_lock<std::mutex> lock(w.mu);
   // this stream's own block, else one that nobody has used, else the one that was used longest ago
@@ -152,6 +144,21 @@ int ws_acquire(size_t bytes, hipStream_t stream, bool optional, LibraryWorkspace
       if (x.used < b->used)
         b = &x;
   }
+  if (b->cap >= bytes && same_stream_for_sure(b->last, stream)) { // the usual call: nothing to allocate, nobody to wait for
+    w.taken = b;
+    lock.release(); // held on: ws_release
+    *out = &w, *ptr = b->ptr;
+    return ST_OK;
+  }
+  // what follows must not break a capture that another thread has under way
+  struct Relaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~Relaxed() {
+      if (set)
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+  } relaxed;
   if (b->cap < bytes) {
     const size_t want = bytes < ((size_t)8 << 20) ? ((size_t)8 << 20) : bytes;
     void *fresh = nullptr;
