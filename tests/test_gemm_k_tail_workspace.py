@@ -56,3 +56,10 @@ def test_k_tail_under_capture_and_without_allocation(gc, dev, M, N, K, trans_b):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(other, -want)
+
+
+@pytest.mark.parametrize("M,K,kernel", [(16, 16, 0), (31, 64, 0), (31, 72, 2), (31, 136, 2), (16, 128, 2)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_a_k_of_one_block_under_few_rows(gc, M, K, kernel, trans_b):
+    """Where the tile kernels' set-up costs more than the bounds-checked kernel's checks."""
+    assert gc.tile_config(M, 1000, K, trans_b=trans_b)[0].kernel == kernel
