@@ -4,8 +4,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# one row/column, less than a 16-byte chunk, one off a tile, K below, at and past a slice and past its steady loop;
-# sizes that reach each tile: 16 (small), 32 (>= 256 tiles of 32), 64 (960 x 1088 and up), 128 (whole multiples)
+# one row/column, less than a 16-byte chunk, one off a tile, K below, at and past a slice and past its steady loop, on
+# tiles of 16 and 64 and on the vector kernel (sizes chosen for each tile, ragged and strided: test_gpu_gemm_f32_edges.py)
 SHAPES = [(1, 1, 1), (3, 3, 70), (1, 300, 64), (17, 15, 16), (40, 50, 1030), (513, 547, 65), (545, 511, 400),
           (961, 1023, 33), (1023, 1090, 257), (1111, 1501, 31), (2049, 2050, 47), (2048, 2048, 128)]
 

@@ -51,6 +51,10 @@ def _pick(kernels, *parts):
     (("gemm_rows32_kernel", "ILi4E"), 2, 96 * 1024),    # 64 rows of A: three 32 KiB stages, one workgroup per compute unit
     (("gemm_rows32_kernel", "ILi8E"), 2, 144 * 1024),   # 128 rows of A: three 48 KiB stages
     (("gemm_tile128_kernel",), 2, 80 * 1024),           # small tiles: two workgroups per compute unit share its LDS
+    (("mha_few_kernel", "ELi128E"), 1, 160 * 1024),     # few queries: one workgroup per compute unit, 128 KiB of requests
+    (("mha_few_kernel", "ELi64E"), 2, 80 * 1024),       # head dim 64: two
+    (("gemm_f32_mfma_kernel",), 2, 80 * 1024),          # f32 tiles: two workgroups or more per compute unit
+    (("gemm_f32_small_kernel",), 2, 8 * 1024),
 ])
 def test_hot_kernels_have_no_scratch_and_keep_their_occupancy(kernels, parts, occupancy, max_lds):
     for name, r in _pick(kernels, *parts).items():
