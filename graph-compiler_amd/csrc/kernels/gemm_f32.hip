@@ -128,10 +128,9 @@ __device__ __forceinline__ void f32_store(const F32GemmParams &p, int64_t m, int
 // should bound it.  MT: side of the matrix instruction's tile (16: the k of a step and their order are those of the
 // small kernel below).  Two slices are in flight in registers behind the one in LDS (with one: 8 % slower, a load then has
 // less time than memory takes), the barrier of a slice lies between its last products with the writes in front and the
-// next slice's first reads behind it.  At 4096^3 the matrix pipes are 90 % busy: 1025 us = 134 TFLOP/s (1230 us when A
-// was transposed on its way into LDS, one slice ahead, reads waited for in front of every product).  1111 tokens
-// through 1000 x 3000 x 1000 x 500: 71 + 77 + 22 us (150 + 288 + 62 on vector FMAs, which were all that sizes off the
-// tile took).  v_mfma_f32_16x16x4_f32 in the large tiles: up to 10 % slower (more registers); in the 32 x 32 tile level.
+// next slice's first reads behind it.  At 4096^3 the matrix pipes are 84 % busy: 1034 us = 133 TFLOP/s (1056 us on the
+// same board when A was transposed on its way into LDS, one slice ahead).  1111 tokens through 1000 x 3000 x 1000 x 500:
+// 177 us (470 on vector FMAs, which were all that sizes off the tile took).  v_mfma_f32_16x16x4_f32 in the large tiles: up to 10 % slower (more registers); in the 32 x 32 tile level.
 template <int MT, int BM, int BN, int WM, int WN, int WK, int BK, bool AKC, bool BKC>
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(F32GemmParams p) {
   constexpr int TM = BM / WM / MT, TN = BN / WN / MT, KW = BK / WK; // MT x MT tiles of a wave, its k of a slice
@@ -613,7 +612,7 @@ struct F32Plan {
 // one MI355X; n tiles per compute unit, k = K / 1000; two constants where a lone workgroup of a compute unit is slower
 // than one of several): tiles are dealt out evenly, a compute unit is done when the one with the most is, and a tile
 // costs its start and its stores whatever K is.  1111 x 1000, K 3000, in us: 128 x 128 198, 64 x 64 100, 32 x 32 77;
-// 4096^3: 1025, 1051, 1218; 1000 x 1000 x 1000: 75, 24-26, 29; 300 x 300, K 1000: 73, 23, 11.4 and 8.3 with 16 x 16 tiles;
+// 4096^3: 1034, 1051, 1218; 1000 x 1000 x 1000: 75, 24-26, 29; 300 x 300, K 1000: 73, 23, 11.4 and 8.3 with 16 x 16 tiles;
 // 1071 x 2048, K 16: 13, 8.7, 17, 17 (an estimate without the cost of a tile took 16 x 16 here).
 // The two small tiles add an element's products in the same order, and so do the two large ones, and the vector
 // kernel whatever its tile: which of the three is taken depends on one matrix, so a batch has the bits of its matrices

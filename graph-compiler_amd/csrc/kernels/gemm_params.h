@@ -96,8 +96,9 @@ struct MhaParams {
   // 1: tile_class already holds the classes of this mask (an earlier call's classification pass for the same mask,
   // shape and buffer): the pass is not launched again.  2: launch the pass only, no attention kernel.
   int32_t classes_mode;
-  // few queries (Sq < 128): f32 partial results when the keys are cut over workgroups (set by the launcher where
-  // `partial` holds the gcmi_launch_mha_partial_bytes the call asks for; null: not cut)
+  // few queries (Sq < 128): where the keys are cut over workgroups, their f32 partial results, as many bytes as
+  // gcmi_launch_mha_partial_bytes says (the caller's of the launcher; null: not cut), and the number of key ranges (the
+  // launcher's)
   float *partial;
   int32_t key_splits;
 };

@@ -1453,7 +1453,8 @@ __device__ __forceinline__ void w4_epilogue_half_any(const GemmParams &p, int ki
 // knows nothing of the tail.  (A tail handled behind the loop would need the accumulators outside the assembly.)
 // Before, every K that is no multiple of 128 bf16 / 256 bytes went to the bounds-checked kernel: 1237 x 4096 x 1376
 // ([N,K] weights) took 89.7 us there, 29.5 us as 320 tiles of 128 x 128.
-// a_src / b_src: the lane's byte offset per DMA instruction; a_chunk / b_kpos: what decides whether it lies before K.
+// a_src / b_src: the lane's byte offset per DMA instruction; a_k / b_k: its first k inside a block, which decides whether
+// it lies before K.
 template <int ES, bool TB, int NDMA, int STAGE, int A_BYTES, typename OffA, typename OffB>
 __device__ __forceinline__ void fill_ring_k_tail(char *smem, int wave, int lane, const char *a_tail, const char *b_tail,
                                                  int64_t b_step, int k_left, const OffA &a_src, const OffB &b_src,
@@ -1971,8 +1972,8 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
   }
   // Whole tiles: 4 waves of 128 x 128 unless the caller asks for 8 waves of 128 x 64.  Results of 8-bit operands
   // leave the 4-wave kernel as bf16, f32 or as the raw s32 accumulators (same main loop, the epilogue is a plain
-  // store).  Tiles that stick out of C (`ragged`): the 4-wave kernel.  Anything else (a K tail, unaligned rows): the
-  // bounds-checked kernel.
+  // store).  Tiles that stick out of C and a K that ends inside a ring group (`ragged`): the 4-wave kernel.  Anything
+  // else (a K or N of no whole 16-byte chunks, unaligned rows): the bounds-checked kernel.
   const bool w4_can = fast || ragged;
   const bool use_w4 = w4_can && (p.cfg_waves != 8 || !fast);
   const bool tiled = fast || use_w4; // one of the kernels with the LDS ring

@@ -5,16 +5,26 @@
  * hipStream_t passed as void* (NULL = the default stream).  Calls are
  * asynchronous on `stream`.
  *
- * Scratch memory.  Two kinds of call need device memory beyond their operands:
- * K-sliced GEMMs (too few 256 x 256 tiles for the GPU, e.g. a short A against
- * wide weights or 1024 x 1024 x 8192: f32 partial sums) and masked
- * attention (one byte per mask tile).  Each entry point says where it comes
- * from:
- *   - plain entry points (gcmi_gemm_bf16, gcmi_mha_fwd_bf16, ...): a workspace
- *     the library allocates per device at the first call that needs one and
- *     grows on demand (hipMalloc under a lock).  Calls that use it are put in
- *     order across streams (an event behind each, waited for by the next call
- *     on another stream), so they are safe from any number of host threads;
+ * Scratch memory.  Three kinds of call need device memory beyond their
+ * operands: K-sliced GEMMs (too few 256 x 256 tiles for the GPU, e.g. a short A
+ * against wide weights or 1024 x 1024 x 8192: f32 partial sums), masked
+ * attention of 128 queries or more (one byte per mask tile) and attention of
+ * fewer queries of few heads, masked or not (f32 partial results of key ranges).
+ * Each entry point says where it comes from:
+ *   - plain entry points (gcmi_gemm_bf16, gcmi_mha_fwd_bf16, ...): up to four
+ *     buffers per device that the library allocates at the first call that needs
+ *     one more and grows on demand (hipMalloc under a lock).  A stream keeps to
+ *     the buffer it used last; with more than four streams a call waits for what
+ *     the stream that used its buffer has been given by then.  Safe from any
+ *     number of host threads.  A call whose stream is being captured gets none:
+ *     masked attention of 128 queries or more and K-sliced GEMMs are then
+ *     refused, but for GEMMs whose K is no multiple of 128 (with [N,K] weights
+ *     and up to 64 rows: of 64), which run in one pass, and attention of fewer
+ *     queries, which keeps the keys of a head in one workgroup.  These two also
+ *     do without where memory cannot be had, and every kind does where the
+ *     stream it would have to wait for is being captured.  Without, sums are
+ *     added in another order and a result may differ in its last bits from that
+ *     of a call with the buffer;
  *   - *_ws entry points: a workspace the caller brings (size from the
  *     *_workspace_bytes query).  Nothing is shared: calls with different
  *     workspaces may overlap on different streams.  This is what a compiled
@@ -68,6 +78,7 @@ const char *gcmi_last_error(void);
  * compute units), K is cut into slices over workgroups and a second kernel adds
  * the f32 partial sums in a fixed order (results do not vary from run to run).
  * The partial sums go through the library workspace (see "Scratch memory").
+ * Not under stream capture: see there.
  */
 int gcmi_gemm_bf16(const void *A, const void *B, void *C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                    int64_t ldc, const void *bias, int bias_dtype, int act, int out_dtype, void *stream);
@@ -191,7 +202,8 @@ int gcmi_gemm_tile_config_query(int a_dtype, int64_t M, int64_t N, int64_t K, in
  * holds until the process ends; the call allocates nothing and frees nothing.
  * A shape whose K slices need more than that (gcmi_gemm_bf16_workspace_bytes)
  * is refused with status 2 and a message; shapes that are not K-sliced need no
- * scratch and are never refused.  Every call on a device shares that device's
+ * scratch and are never refused, nor is a K that is no multiple of 128 (its
+ * slices always fit).  Every call on a device shares that device's
  * array: calls that overlap in time on one device (different streams) race;
  * calls on one stream are safe.  Results equal gcmi_gemm_bf16's bit for bit.
  */
