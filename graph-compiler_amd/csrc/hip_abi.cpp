@@ -83,11 +83,11 @@ struct LibraryWorkspace {
 };
 LibraryWorkspace g_ws[64];
 
-// hipStreamPerThread is one handle value for a different stream in every thread, and the legacy null stream
-// synchronises with others by rules of its own: a comparison of handles says nothing about them.
-bool same_stream_for_sure(hipStream_t a, hipStream_t b) {
-  return a == b && a != nullptr && a != hipStreamPerThread && a != hipStreamLegacy;
-}
+// hipStreamPerThread is one handle value for a different stream in every thread: a comparison says nothing about it.  The
+// null stream is one stream per device, whichever thread names it, and the buffers here are per device: its calls follow
+// one another.  (With an event and a wait for each of its calls, attention of 1 query of 8 heads over 2000 keys took 13.2 us
+// on it, 10.1 on a stream of its own; 10.3 now.)
+bool same_stream_for_sure(hipStream_t a, hipStream_t b) { return a == b && a != hipStreamPerThread; }
 
 enum class Capture { No, Yes, Unknown };
 Capture capture_state(hipStream_t stream) {
@@ -144,7 +144,7 @@ int ws_acquire(size_t bytes, hipStream_t stream, bool optional, LibraryWorkspace
       if (x.used < b->used)
         b = &x;
   }
-  if (b->cap >= bytes && same_stream_for_sure(b->last, stream)) { // the usual call: nothing to allocate, nobody to wait for
+  if (b->used && b->cap >= bytes && same_stream_for_sure(b->last, stream)) { // the usual call: nothing to allocate, nobody to wait for
     w.taken = b;
     lock.release(); // held on: ws_release
     *out = &w, *ptr = b->ptr;

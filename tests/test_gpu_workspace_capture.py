@@ -115,3 +115,32 @@ def test_more_streams_than_blocks(gc, dev):
     for row in outs:
         for o, w in zip(row, want):
             assert torch.equal(o, w)
+
+
+def test_null_stream_calls_follow_one_another(gc, dev):
+    """Calls on the null stream, from two host threads, share its buffer without waits; other streams in between."""
+    import threading
+    g = torch.Generator(device=dev).manual_seed(6)
+    bf = lambda *s: torch.randn(*s, device=dev, generator=g).to(torch.bfloat16)  # noqa: E731
+    K, V = bf(1, 8, 3000, 128), bf(1, 8, 3000, 128)
+    Qs = [bf(1, 8, 1, 128) for _ in range(3)]
+    want = [gc.mha_fwd_bf16(q, K, V) for q in Qs]
+    outs = [[torch.zeros_like(q) for _ in range(40)] for q in Qs]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def calls(i, stream):
+        with torch.cuda.stream(stream):
+            for o in outs[i]:
+                gc.mha_fwd_bf16(Qs[i], K, V, out=o)
+
+    null = torch.cuda.default_stream()
+    assert null.cuda_stream == 0
+    threads = [threading.Thread(target=calls, args=a) for a in ((0, null), (1, null), (2, side))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i, w in enumerate(want):
+        assert all(torch.equal(o, w) for o in outs[i]), i
