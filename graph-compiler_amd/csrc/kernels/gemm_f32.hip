@@ -296,54 +296,115 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(F32GemmParams p) {
 // no LDS and no barrier until the four partial sums are added.  128 x 512 x 256 (128 workgroups) in 7.2 us per call (10.6 as
 // 16 x 16 tiles of vector FMAs over LDS slices of 32 k with a barrier each).
 static constexpr int64_t F32_SMALL_GRID = 1 << 23; // workgroups of a grid's first dimension, at most: 2^32 threads are too many
-template <bool AKC, bool BKC> __global__ __launch_bounds__(256) void gemm_f32_small_kernel(F32GemmParams p) {
+// WIDE: a lane's place in a step may lie more than 2^31 bytes behind the step's first element; else it is a 32-bit offset on
+// a scalar address (with 64-bit addresses in the lanes the sixteen steps in flight take all 256 registers, and one
+// workgroup a compute unit; with offsets two or more).
+template <bool AKC, bool BKC, bool WIDE> __global__ __launch_bounds__(256) void gemm_f32_small_kernel(F32GemmParams p) {
   constexpr int U = 8;
   __shared__ float red[3][256];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lq = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, lq = lane >> 4;
   // The size of the grid is a constant, and workgroups past the last tile (a grid of more than one row) compute rows that
   // nobody stores: reading the size, or leaving early, puts a second wait for kernel arguments in front of the loads of
   // every workgroup (0.2 us a launch).
   const int64_t nt = (p.N + 15) / 16, t = blockIdx.x + (int64_t)blockIdx.y * F32_SMALL_GRID;
   const int64_t m0 = t / nt * 16, n0 = t % nt * 16;
-  p.A += (int64_t)blockIdx.z * p.a_bs, p.B += (int64_t)blockIdx.z * p.b_bs, p.C += (int64_t)blockIdx.z * p.c_bs;
-  const int64_t ga = m0 + l16 < p.M ? m0 + l16 : p.M - 1, gb = n0 + l16 < p.N ? n0 + l16 : p.N - 1;
-  const float *a = p.A + ga * p.a_rs + 4 * lq * p.a_cs, *b = p.B + gb * p.b_cs + 4 * lq * p.b_rs;
+  p.C += (int64_t)blockIdx.z * p.c_bs;
+  // rows past the last one read the last one (a tile past the last one: its own rows' clamp)
+  const int64_t ma = m0 < p.M ? m0 : p.M - 1;
+  const int ra = ma + l16 < p.M ? l16 : (int)(p.M - 1 - ma), rb = n0 + l16 < p.N ? l16 : (int)(p.N - 1 - n0);
+  typedef typename std::conditional<WIDE, int64_t, uint32_t>::type off_t;
+  const float *a = p.A + (int64_t)blockIdx.z * p.a_bs + ma * p.a_rs, *b = p.B + (int64_t)blockIdx.z * p.b_bs + n0 * p.b_cs;
+  const off_t la = 4 * ((off_t)ra * (off_t)p.a_rs + (off_t)(4 * lq) * (off_t)p.a_cs);
+  const off_t lb = 4 * ((off_t)rb * (off_t)p.b_cs + (off_t)(4 * lq) * (off_t)p.b_rs);
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  auto load = [&](const float *s, int64_t ks, int64_t left, bool contig) -> f32x4_t {
+  auto at = [](const float *s, off_t o) { return reinterpret_cast<const float *>(reinterpret_cast<const char *>(s) + o); };
+  auto load = [&](const float *s, off_t o, int64_t ks, bool contig) -> f32x4_t {
     f32x4_t v;
-    if (left >= 4) {
-      if (contig)
-        v = *reinterpret_cast<const f32x4u_t *>(s);
-      else
-        for (int c = 0; c < 4; c++)
-          v[c] = s[c * ks];
-    } else {
+    if (contig)
+      v = *reinterpret_cast<const f32x4u_t *>(at(s, o));
+    else
       for (int c = 0; c < 4; c++)
-        v[c] = c < left ? s[c * ks] : 0.0f;
-    }
+        v[c] = *at(s + c * ks, o);
     return v;
   };
-  int64_t k = 16 * wave;
-  for (; k + 64 * (U - 1) + 16 <= p.K; k += 64 * U) {
-    f32x4_t va[U], vb[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      va[u] = load(a + (k + 64 * u) * p.a_cs, p.a_cs, 4, AKC);
-      vb[u] = load(b + (k + 64 * u) * p.b_rs, p.b_rs, 4, BKC);
-    }
-    __builtin_amdgcn_sched_barrier(0); // all loads first
+  auto load_end = [&](const float *s, off_t o, int64_t ks, int left) -> f32x4_t {
+    f32x4_t v;
+    for (int c = 0; c < 4; c++)
+      v[c] = c < left ? *at(s + c * ks, o) : 0.0f;
+    return v;
+  };
+  // This wave's whole steps are wave, wave + 4, ...; the step that K ends inside of, if it does, is behind some wave's last.
+  // Eight steps are multiplied (a chain of 32 sums, half as long as a load takes) while the next eight are on their way,
+  // and what is left of K is one more round of loads.
+  const int steps = (int)((p.K / 16 - wave + 3) >> 2), left = (int)(p.K & 15);
+  const bool ends = left != 0 && (int)((p.K >> 4) & 3) == wave;
+  const int64_t a_step = 64 * p.a_cs, b_step = 64 * p.b_rs;
+  a += 16 * wave * p.a_cs, b += 16 * wave * p.b_rs;
+  f32x4_t va[2][U], vb[2][U], ea, eb;
+  // (the addresses are scalars that go from step to step: worked out ahead, as the compiler would, they fill the registers)
+  auto step = [&](f32x4_t &x, f32x4_t &y) {
+    x = load(a, la, p.a_cs, AKC), y = load(b, lb, p.b_rs, BKC);
+    a += a_step, b += b_step;
+    asm volatile("" : "+s"(a), "+s"(b));
+  };
+  auto fetch = [&](int q) { // U steps
 #pragma unroll
     for (int u = 0; u < U; u++)
-#pragma unroll
-      for (int c = 0; c < 4; c++)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u][c], vb[u][c], acc, 0, 0, 0);
-  }
-  for (; k < p.K; k += 64) {
-    const f32x4_t va = load(a + k * p.a_cs, p.a_cs, p.K - k - 4 * lq, AKC);
-    const f32x4_t vb = load(b + k * p.b_rs, p.b_rs, p.K - k - 4 * lq, BKC);
+      step(va[q][u], vb[q][u]);
+    __builtin_amdgcn_sched_barrier(0); // all loads first
+  };
+  auto product = [&](const f32x4_t &x, const f32x4_t &y) {
 #pragma unroll
     for (int c = 0; c < 4; c++)
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[c], vb[c], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[c], y[c], acc, 0, 0, 0);
+  };
+  auto products = [&](int q) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      product(va[q][u], vb[q][u]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto fetch_rest = [&](int q, int n) { // n steps, fewer than U, and the end of K
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+      if (u < n)
+        step(va[q][u], vb[q][u]);
+    if (ends) {
+      ea = load_end(a, la, p.a_cs, left - 4 * lq);
+      eb = load_end(b, lb, p.b_rs, left - 4 * lq);
+    }
+  };
+  auto products_rest = [&](int q, int n) {
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+      if (u < n)
+        product(va[q][u], vb[q][u]);
+    if (ends)
+      product(ea, eb);
+  };
+  if (steps < U) {
+    fetch_rest(0, steps);
+    products_rest(0, steps);
+  } else {
+    int n = steps - U; // steps not asked for yet
+    fetch(0);
+    for (; n >= 2 * U; n -= 2 * U) {
+      fetch(1);
+      products(0);
+      fetch(0);
+      products(1);
+    }
+    if (n >= U) {
+      fetch(1);
+      products(0);
+      fetch_rest(0, n - U);
+      products(1);
+      products_rest(0, n - U);
+    } else {
+      fetch_rest(1, n);
+      products(0);
+      products_rest(1, n);
+    }
   }
   if (wave > 0)
 #pragma unroll
@@ -677,9 +738,14 @@ extern "C" int gcmi_launch_gemm_f32(const F32GemmParams *pp, hipStream_t stream)
     if ((all + gx - 1) / gx > 65535)
       return 2;
     const dim3 grid((unsigned)gx, (unsigned)((all + gx - 1) / gx), (unsigned)nbatch);
-    void (*const kernel[4])(F32GemmParams) = {gemm_f32_small_kernel<false, false>, gemm_f32_small_kernel<false, true>,
-                                              gemm_f32_small_kernel<true, false>, gemm_f32_small_kernel<true, true>};
-    hipLaunchKernelGGL(kernel[layout], grid, dim3(256), 0, stream, p);
+    // the last byte that a lane reads of a step, counted from the step's first
+    auto far = [](int64_t xs, int64_t ks) { return 4 * (15 * xs + 15 * ks + 1) >= (int64_t)1 << 31; };
+    const bool wide = far(p.a_rs, p.a_cs) || far(p.b_cs, p.b_rs);
+    void (*const kernel[8])(F32GemmParams) = {gemm_f32_small_kernel<false, false, false>, gemm_f32_small_kernel<false, true, false>,
+                                              gemm_f32_small_kernel<true, false, false>, gemm_f32_small_kernel<true, true, false>,
+                                              gemm_f32_small_kernel<false, false, true>, gemm_f32_small_kernel<false, true, true>,
+                                              gemm_f32_small_kernel<true, false, true>, gemm_f32_small_kernel<true, true, true>};
+    hipLaunchKernelGGL(kernel[layout + (wide ? 4 : 0)], grid, dim3(256), 0, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : 5;
   }
   static void (*const kernels[3][4])(F32GemmParams) = {F32_LAYOUTS(16, 32, 32, 1, 1, 4, 64),
