@@ -292,15 +292,16 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(F32GemmParams p) {
 
 // Small problems: what counts is the chain launch -> loads -> sums -> store.  A workgroup owns one 16 x 16 tile, its
 // four waves take every fourth 16-deep step of K straight from memory into v_mfma_f32_16x16x4_f32 operands (lane l:
-// row/column l % 16, and k = 4 * (l / 16) .. + 3 of the step as four operand values), eight steps in flight per wave,
+// row/column l % 16, and k = 4 * (l / 16) .. + 3 of the step as four operand values), up to eight steps in flight per wave,
 // no LDS and no barrier until the four partial sums are added.  128 x 512 x 256 (128 workgroups) in 7.2 us per call (10.6 as
-// 16 x 16 tiles of vector FMAs over LDS slices of 32 k with a barrier each).
+// 16 x 16 tiles of vector FMAs over LDS slices of 32 k with a barrier each).  Kernel alone: 154 x 737, K 1872 16.7 us, 1000 x
+// 64, K 3000 13.2 (18.2 and 15.0 when a wave waited for eight steps at a time and then took the rest of K step by step);
+// sixteen steps in flight are the slower choice where workgroups share a compute unit (18.3, 13.6).
 static constexpr int64_t F32_SMALL_GRID = 1 << 23; // workgroups of a grid's first dimension, at most: 2^32 threads are too many
 // WIDE: a lane's place in a step may lie more than 2^31 bytes behind the step's first element; else it is a 32-bit offset on
-// a scalar address (with 64-bit addresses in the lanes the sixteen steps in flight take all 256 registers, and one
-// workgroup a compute unit; with offsets two or more).
+// a scalar address (with 64-bit addresses in the lanes every load in flight takes two registers more).
 template <bool AKC, bool BKC, bool WIDE> __global__ __launch_bounds__(256) void gemm_f32_small_kernel(F32GemmParams p) {
-  constexpr int U = 8;
+  constexpr int U = 4;
   __shared__ float red[3][256];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, lq = lane >> 4;
   // The size of the grid is a constant, and workgroups past the last tile (a grid of more than one row) compute rows that
@@ -334,8 +335,8 @@ template <bool AKC, bool BKC, bool WIDE> __global__ __launch_bounds__(256) void 
     return v;
   };
   // This wave's whole steps are wave, wave + 4, ...; the step that K ends inside of, if it does, is behind some wave's last.
-  // Eight steps are multiplied (a chain of 32 sums, half as long as a load takes) while the next eight are on their way,
-  // and what is left of K is one more round of loads.
+  // Four steps are multiplied (a chain of 16 sums) while the next four are on their way, and what is left of K is one more
+  // round of loads.
   const int steps = (int)((p.K / 16 - wave + 3) >> 2), left = (int)(p.K & 15);
   const bool ends = left != 0 && (int)((p.K >> 4) & 3) == wave;
   const int64_t a_step = 64 * p.a_cs, b_step = 64 * p.b_rs;
