@@ -4,8 +4,13 @@
 #include "gemm_rows32.hpp"
 #include "gemm_skinny.hpp"
 
+extern "C" int gcmi_launch_few_rows(const gcmi::GemmParams *p, int es, hipStream_t stream, int dry, gcmi::GemmTileConfig *cfg); // gemm_few_rows.hip
+
 extern "C" int gcmi_launch_gemm_bf16(const gcmi::GemmParams *p, hipStream_t stream) {
   int rc = gcmi::launch_rows32(p, stream);
+  if (rc >= 0)
+    return rc;
+  rc = gcmi_launch_few_rows(p, 2, stream, 0, nullptr);
   if (rc >= 0)
     return rc;
   rc = gcmi::launch_skinny_nt(p, stream);
@@ -23,6 +28,8 @@ extern "C" int64_t gcmi_launch_gemm_bf16_workspace(const gcmi::GemmParams *p, in
   *optional = 0;
   if (gcmi::launch_rows32(p, nullptr, &want) >= 0)
     return want;
+  if (gcmi_launch_few_rows(p, 2, nullptr, 1, nullptr) >= 0)
+    return 0;
   if (gcmi::launch_skinny_nt(p, nullptr, &want) >= 0)
     return want;
   gcmi::launch_tile256<2>(p, nullptr, &want);
@@ -33,6 +40,8 @@ extern "C" int64_t gcmi_launch_gemm_bf16_workspace(const gcmi::GemmParams *p, in
 // what the launch above would choose (nothing is launched)
 extern "C" int gcmi_launch_gemm_bf16_config(const gcmi::GemmParams *p, gcmi::GemmTileConfig *cfg) {
   if (gcmi::launch_rows32(p, (hipStream_t)-1, nullptr, cfg) >= 0)
+    return 0;
+  if (gcmi_launch_few_rows(p, 2, nullptr, 1, cfg) >= 0)
     return 0;
   if (gcmi::launch_skinny_nt(p, (hipStream_t)-1, nullptr, cfg) >= 0)
     return 0;

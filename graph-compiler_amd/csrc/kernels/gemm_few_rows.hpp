@@ -1,0 +1,389 @@
+// GEMMs of few rows of A (up to 256) against weights that are no stream worth slicing: bf16 x bf16 with weights stored
+// [K,N] or [N,K], and 8-bit x s8 with weights stored [K,N].  C[M,N] = epilogue(A . W) in ONE launch.
+// What bounds such a call is the way launch -> loads -> sums -> store, once: the tile kernels' workgroup walks all of K
+// through one ring behind barriers (a 256 x 256 tile takes 60 us for 2 x 5456, K 3264, on 22 compute units), and K slices
+// over workgroups cost a second launch.  Here K is cut over the waves of a workgroup:
+//   * a workgroup has 16 * NT columns and 16 * MT rows; wave w takes stages w, w + W, ... of 128 bytes of K per row, each
+//     into an LDS ring of its own by global_load_lds_dwordx4, D stages deep: no barrier and no wait for another wave until
+//     the W partial sums are added (ascending, a fixed order: results do not depend on timing).  The waves' stages lie
+//     beside each other in memory, so eight of them read runs of 1 KiB of every row.  (Deeper rings, sixteen waves or stages
+//     of 64 bytes: no difference to 5 % slower; it is the number of lines a compute unit looks up that counts.)
+//   * the smallest tile that fits the GPU in one round, so that as many compute units as there are pull on the weights.  A
+//     run of neighbouring tiles goes to one XCD, whose L2 reads a line of [K,N] weights once for all of them (with the
+//     tiles dealt out over the XCDs, 8-bit 30 x 4960, K 3232 took 24.3 us, 9.2 now; 30 x 11008, K 4096 19.3 and 12.4).
+//   * rows of 128 bytes (A, [N,K] weights) lie at chunk ^ row % 8; k-rows of [K,N] weights are read through the transposing
+//     LDS loads, at a chunk that spreads them over the banks.
+// The columns' bias, scale and column sums are fetched before the loop by the wave that finishes them.
+// The k that a wave owns and the order of the sums depend on M and N only: both layouts of the weights, and a matrix alone
+// or in a batch, give the same bits.
+// Measured, us per call, graph-replayed over 64 MB of weights: bf16 [N,K] 3 x 1712, K 2736 48 -> 6; 19 x 1648, K 3592 63.4 ->
+// 7.7; 13 x 1792, K 1856 8.4 (two launches) -> 5.0; [K,N] 10 x 320, K 3200 53 -> 8.5; 8-bit 10 x 512, K 3776 36 -> 7.7; 32 x
+// 11008, K 4096 20.0 -> 12.5 (3.7 TB/s of weights).
+#pragma once
+#include "gemm_tile256.hpp"
+
+namespace gcmi {
+
+template <int ES, bool TB, int MT, int NT, int W, int D> struct FewRows {
+  static constexpr int STEPS = 2, KB = 64 * STEPS, BK = KB / ES; // MFMA steps, bytes and elements of K per stage
+  static constexpr int A_BYTES = 16 * MT * KB, STAGE = A_BYTES + 16 * NT * KB;
+  static constexpr int NA = STEPS * MT, NB = STEPS * NT, PER = NA + NB; // requests per stage: 1 KiB each
+  static constexpr int RING = D * STAGE, SMEM = W * RING;
+  static constexpr int BROW = 16 * NT * ES;                   // bytes of a k-row of [K,N] weights
+  static_assert(W * MT * NT * 1024 <= SMEM, "the partial sums lie over the rings");
+  static_assert(D * PER <= 63, "requests in flight are counted in six bits");
+  static_assert(W % NT == 0, "a wave finishes tiles of one column group");
+  // where the 16-byte chunk of a row of KB bytes lies inside it (rows 16 apart alike)
+  static __device__ __forceinline__ int row_swz(int row) { return row & 7; }
+  // where the 16-byte chunk of a k-row lies inside it
+  static __device__ __forceinline__ int swz(int krow) {
+    if constexpr (ES == 2 && NT == 4) // 8 chunks; a transposing read takes 4 k-rows per 16 lanes, 8 apart
+      return (((krow >> 1) & 1) | (((krow >> 3) & 1) << 1)) << 1;
+    else if constexpr (ES == 1 && NT == 4) // 4 chunks; 8 k-rows per 16 lanes, 16 apart
+      return ((krow >> 2) & 1) | (((krow >> 4) & 1) << 1);
+    else
+      return 0;
+  }
+};
+
+// one row quad of an 8-bit product: the 4-wave tile kernels' epilogue
+template <bool TAME>
+__device__ __forceinline__ void few_rows_store_int8(const GemmParams &p, const i32x4_t &c, int64_t m, int64_t n, const f32x4_t &bias4,
+                                                    const f32x4_t &scale4, const i32x4_t &cs4) {
+#define GCMI_FEW_CASE(ACT, OUT, K)                                                                                    \
+  case (int)ACT + 8 * K:                                                                                              \
+    w4_epilogue_row<1, ACT, OUT, false, false, false, TAME>(p, c, m, n, bias4, scale4, cs4);                          \
+    break;
+  const int out_kind = p.out_dt == DT_BF16 ? 0 : (p.out_dt == DT_S32 ? 2 : 1);
+  switch ((out_kind == 2 ? (int)ACT_NONE : p.act) + 8 * out_kind) {
+    GCMI_FEW_CASE(ACT_RELU, DT_BF16, 0)
+    GCMI_FEW_CASE(ACT_GELU_ERF, DT_BF16, 0)
+    GCMI_FEW_CASE(ACT_GELU_TANH, DT_BF16, 0)
+    GCMI_FEW_CASE(ACT_SIGMOID, DT_BF16, 0)
+    GCMI_FEW_CASE(ACT_NONE, DT_F32, 1)
+    GCMI_FEW_CASE(ACT_RELU, DT_F32, 1)
+    GCMI_FEW_CASE(ACT_GELU_ERF, DT_F32, 1)
+    GCMI_FEW_CASE(ACT_GELU_TANH, DT_F32, 1)
+    GCMI_FEW_CASE(ACT_SIGMOID, DT_F32, 1)
+    GCMI_FEW_CASE(ACT_NONE, DT_S32, 2)
+  default:
+    w4_epilogue_row<1, ACT_NONE, DT_BF16, false, false, false, TAME>(p, c, m, n, bias4, scale4, cs4);
+    break;
+  }
+#undef GCMI_FEW_CASE
+}
+
+template <int ES, bool TB, int MT, int NT, int W, int D> __global__ __launch_bounds__(64 * W) void gemm_few_rows_kernel(GemmParams p) {
+  static_assert(!TB || ES == 2, "weights stored [N,K]: bf16 only");
+  typedef FewRows<ES, TB, MT, NT, W, D> F;
+  constexpr int STEPS = F::STEPS;
+  typedef typename std::conditional<ES == 2, f32x4_t, i32x4_t>::type acc4_t;
+  __shared__ __align__(1024) char smem[F::SMEM];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g16 = lane >> 4;
+  const int tiles_m = (int)((p.M + 16 * MT - 1) / (16 * MT)), tiles_n = (int)((p.N + 16 * NT - 1) / (16 * NT));
+  // workgroup i runs on XCD i % 8: each XCD walks its own run of panels (the grid is rounded up to whole runs)
+  const int tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3), tm = tile % tiles_m, tn = tile / tiles_m;
+  if (tn >= tiles_n)
+    return;
+  const int64_t m0 = (int64_t)tm * 16 * MT, n0 = (int64_t)tn * 16 * NT;
+  const int rows_in = (int)min((int64_t)16 * MT, p.M - m0), cols_in = (int)min((int64_t)16 * NT, p.N - n0);
+  const int64_t bz = blockIdx.y; // strided batch
+  p.A = reinterpret_cast<const char *>(p.A) + bz * p.a_bs * ES;
+  p.B = reinterpret_cast<const char *>(p.B) + bz * p.b_bs * ES;
+  p.C = reinterpret_cast<char *>(p.C) + bz * p.c_bs * (p.out_dt == DT_BF16 ? 2 : 4);
+  if (ES == 2 && p.residual)
+    p.residual = reinterpret_cast<const char *>(p.residual) + bz * p.c_bs * (p.residual_dt == DT_BF16 ? 2 : 4);
+  const int64_t lda_b = p.lda * ES, ldb_b = p.ldb * ES;
+
+  // what belongs to the columns that this wave finishes, as it lies in memory (looked at behind the loop)
+  typedef uint16_t u16x4u_t __attribute__((ext_vector_type(4), aligned(2)));
+  typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+  typedef int i32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+  const int64_t nw = n0 + 16 * (wave % NT) + 4 * g16;
+  const bool finishes = wave < MT * NT && nw < p.N; // N is a multiple of 4
+  u16x4u_t bias16 = {0, 0, 0, 0};
+  f32x4u_t bias32 = {0.f, 0.f, 0.f, 0.f}, scale4 = {1.f, 1.f, 1.f, 1.f};
+  i32x4u_t sums4 = {0, 0, 0, 0};
+  if (finishes) {
+    if (p.bias && p.bias_dt == DT_BF16)
+      bias16 = *reinterpret_cast<const u16x4u_t *>(reinterpret_cast<const uint16_t *>(p.bias) + nw);
+    if (p.bias && p.bias_dt != DT_BF16)
+      bias32 = *reinterpret_cast<const f32x4u_t *>(reinterpret_cast<const float *>(p.bias) + nw);
+    if (ES == 1 && p.scale)
+      scale4 = *reinterpret_cast<const f32x4u_t *>(p.scale + nw);
+    if (ES == 1 && p.colsum)
+      sums4 = *reinterpret_cast<const i32x4u_t *>(p.colsum + nw);
+  }
+
+  const int stages = (int)((p.K + F::BK - 1) / F::BK), n_st = (stages - wave + W - 1) / W; // this wave's
+  const int k_end = (int)(p.K - (int64_t)(stages - 1) * F::BK);                            // elements of the last stage
+  // requests: 8 rows of 128 bytes, or 1024 / BROW k-rows.  Rows, chunks and k-rows outside read the last ones inside.
+  uint32_t a_src[F::NA], b_src[F::NB];
+  auto offsets = [&](int k_in) {
+    constexpr int CPR = F::KB / 16, RPR = 64 / CPR; // chunks of a row, rows of a request
+    const int chunks = k_in * ES / 16, row = lane / CPR, c = min((lane % CPR) ^ F::row_swz(row), chunks - 1);
+#pragma unroll
+    for (int i = 0; i < F::NA; i++)
+      a_src[i] = (uint32_t)(min(RPR * i + row, rows_in - 1) * lda_b + c * 16);
+#pragma unroll
+    for (int i = 0; i < F::NB; i++) {
+      if constexpr (TB) {
+        b_src[i] = (uint32_t)(min(RPR * i + row, cols_in - 1) * ldb_b + c * 16);
+      } else {
+        constexpr int CPR = F::BROW / 16; // chunks of a k-row
+        const int krow = i * (64 / CPR) + lane / CPR, cb = (lane % CPR) ^ F::swz(krow);
+        b_src[i] = (uint32_t)(min(krow, k_in - 1) * ldb_b + min(cb, cols_in * ES / 16 - 1) * 16);
+      }
+    }
+  };
+  const int64_t b_step = TB ? (int64_t)F::KB : (int64_t)F::BK * ldb_b;
+  const char *a_ptr = reinterpret_cast<const char *>(p.A) + m0 * lda_b + (int64_t)wave * F::KB;
+  const char *b_ptr = reinterpret_cast<const char *>(p.B) + (TB ? n0 * ldb_b : n0 * ES) + wave * b_step;
+  char *const ring = smem + wave * F::RING;
+  // (written as assembly: of requests that the compiler knows it awaits all in flight before every read of LDS)
+  const uint32_t ring_at = (uint32_t)(uintptr_t)(GCMI_LDS char *)ring;
+  auto request = [&](const char *base, uint32_t off, uint32_t at) { // 16 bytes per lane from base + off to LDS at + 16 * lane
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(at) : "m0", "memory");
+  };
+  auto issue = [&](int st, int i) { // this wave's stage i, to the slot at st
+    if (wave + i * W == stages - 1)
+      offsets(k_end);
+    const char *a = a_ptr + (int64_t)i * (W * F::KB), *b = b_ptr + i * (W * b_step);
+#pragma unroll
+    for (int r = 0; r < F::NA; r++)
+      request(a, a_src[r], ring_at + st + r * 1024);
+#pragma unroll
+    for (int r = 0; r < F::NB; r++)
+      request(b, b_src[r], ring_at + st + F::A_BYTES + r * 1024);
+  };
+  acc4_t acc[NT][MT]; // rows 16 * it + lane % 16, columns 16 * jt + 4 * (lane / 16) .. + 3 (weights as first operand)
+#pragma unroll
+  for (int jt = 0; jt < NT; jt++)
+#pragma unroll
+    for (int it = 0; it < MT; it++)
+      acc[jt][it] = acc4_t{0, 0, 0, 0};
+  uint4 fa[STEPS][MT], fb[STEPS][NT];
+  auto read = [&](const char *st) {
+#pragma unroll
+    for (int u = 0; u < STEPS; u++) {
+      const int at = r16 * F::KB + (((4 * u + g16) ^ F::row_swz(r16)) << 4);
+#pragma unroll
+      for (int it = 0; it < MT; it++)
+        fa[u][it] = *reinterpret_cast<const uint4 *>(st + at + it * 16 * F::KB);
+#pragma unroll
+      for (int jt = 0; jt < NT; jt++) {
+        if constexpr (TB) {
+          fb[u][jt] = *reinterpret_cast<const uint4 *>(st + F::A_BYTES + at + jt * 16 * F::KB);
+        } else {
+          // the 16 lanes of a group hand the transposing read RG k-rows x 16 columns in 8-byte pieces
+          constexpr int RG = ES == 2 ? 4 : 8;
+          const int kk = ES == 2 ? r16 >> 2 : r16 >> 1, cc = ES == 2 ? r16 & 3 : r16 & 1;
+          const int chunk = ES == 2 ? 2 * jt + (cc >> 1) : jt, sub = ES == 2 ? (cc & 1) * 8 : cc * 8;
+          const int krow = (64 / ES) * u + 2 * RG * g16 + kk;
+          const char *q = st + F::A_BYTES + sub;
+          const uint2 lo = MfmaOp<ES>::tr_read(q + krow * F::BROW + ((chunk ^ F::swz(krow)) << 4));
+          const uint2 hi = MfmaOp<ES>::tr_read(q + (krow + RG) * F::BROW + ((chunk ^ F::swz(krow + RG)) << 4));
+          fb[u][jt] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        }
+      }
+    }
+  };
+  const uint32_t a_xor = p.a_xor;
+  auto products = [&]() {
+#pragma unroll
+    for (int u = 0; u < STEPS; u++)
+#pragma unroll
+      for (int it = 0; it < MT; it++) {
+        if constexpr (ES == 2) {
+#pragma unroll
+          for (int jt = 0; jt < NT; jt++)
+            acc[jt][it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fb[u][jt]),
+                                                                  __builtin_bit_cast(bf16x8_t, fa[u][it]), acc[jt][it], 0, 0, 0);
+        } else {
+          const uint4 f = make_uint4(fa[u][it].x ^ a_xor, fa[u][it].y ^ a_xor, fa[u][it].z ^ a_xor, fa[u][it].w ^ a_xor);
+#pragma unroll
+          for (int jt = 0; jt < NT; jt++)
+            acc[jt][it] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4_t, fb[u][jt]), __builtin_bit_cast(i32x4_t, f),
+                                                                acc[jt][it], 0, 0, 0);
+        }
+      }
+  };
+  // what lies behind K in the last stage: zeros in the weights, and for bf16 in A (an infinity times zero would be a NaN;
+  // 8-bit bytes of A are any byte)
+  auto cut = [&]() {
+#pragma unroll
+    for (int u = 0; u < STEPS; u++)
+      if ((4 * u + g16) * (16 / ES) >= k_end) {
+#pragma unroll
+        for (int jt = 0; jt < NT; jt++)
+          fb[u][jt] = make_uint4(0, 0, 0, 0);
+        if constexpr (ES == 2)
+#pragma unroll
+          for (int it = 0; it < MT; it++)
+            fa[u][it] = make_uint4(0, 0, 0, 0);
+      }
+  };
+  offsets(F::BK);
+#pragma unroll
+  for (int d = 0; d < D; d++)
+    if (d < n_st)
+      issue(d * F::STAGE, d);
+  int slot = 0;
+  for (int i = 0; i < n_st; i++) {
+    // stage i has landed (the D - 1 behind it may be in flight; near the end fewer were asked for and all are awaited)
+    if (i + D - 1 < n_st)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * F::PER) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int st = slot * F::STAGE;
+    read(ring + st);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the reads are over: the slot is free
+    if (i + D < n_st)
+      issue(st, i + D);
+    if (k_end < F::BK && wave + i * W == stages - 1)
+      cut();
+    products();
+    slot = slot + 1 < D ? slot + 1 : 0;
+  }
+  // the waves' sums, in ascending order; a wave finishes every W-th tile
+  __syncthreads();
+  acc4_t *red = reinterpret_cast<acc4_t *>(smem);
+#pragma unroll
+  for (int it = 0; it < MT; it++)
+#pragma unroll
+    for (int jt = 0; jt < NT; jt++)
+      red[(wave * MT * NT + it * NT + jt) * 64 + lane] = acc[jt][it];
+  __syncthreads();
+  f32x4_t bias4;
+  i32x4_t cs4;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    bias4[e] = !p.bias ? -0.0f : p.bias_dt == DT_BF16 ? bf16_bits_to_f32(bias16[e]) : bias32[e]; // absent: nothing is added, not even to -0.0
+    cs4[e] = p.comp * sums4[e];
+  }
+  bool tame = ES == 1; // see w4_epilogue_half
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    tame = tame && fabsf(scale4[e]) < 0x1p90f && fabsf(bias4[e]) < 0x1p120f;
+#pragma unroll 1
+  for (int t = wave; t < MT * NT; t += W) {
+    acc4_t v = red[t * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < W; w++) {
+      const acc4_t o = red[(w * MT * NT + t) * 64 + lane];
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        v[e] += o[e];
+    }
+    const int64_t m = m0 + 16 * (t / NT) + r16;
+    if (m >= p.M || !finishes)
+      continue;
+    if constexpr (ES == 2)
+      epilogue_store4(p, v, m, nw, bias4);
+    else if (tame)
+      few_rows_store_int8<true>(p, v, m, nw, bias4, scale4, cs4);
+    else
+      few_rows_store_int8<false>(p, v, m, nw, bias4, scale4, cs4);
+  }
+}
+
+// The tile: 16 * mt rows and 16 * nt columns per workgroup.  A workgroup's time is that of its operands (about 45 KB a us
+// past 3 us), so the tile with the fewest of them wins that needs no second round of workgroups; a second round costs a
+// workgroup's time again.
+struct FewRowsTile {
+  int mt, nt, waves, stages; // waves that share K, stages of a wave's ring
+  int64_t blocks, rounds;
+};
+static FewRowsTile few_rows_tile(int64_t M, int64_t N) {
+  const int64_t n_cu = gcmi_num_cus();
+  FewRowsTile best{};
+  int64_t best_cost = INT64_MAX;
+  for (int mt = 4; mt >= 1; mt /= 2) // (of equal tiles the one with more rows: the weights are read by fewer workgroups)
+    for (int nt = 1; nt <= 4; nt *= 2) {
+      const int64_t blocks = ((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)), rounds = (blocks + n_cu - 1) / n_cu;
+      const int64_t cost = rounds * (mt + nt);
+      if (cost < best_cost || (cost == best_cost && blocks < best.blocks)) {
+        const int waves = nt == 1 && mt < 4 ? 8 : 4;
+        best = {mt, nt, waves, waves == 8 || mt + nt == 8 ? 2 : 3, blocks, rounds};
+        best_cost = cost;
+      }
+    }
+  return best;
+}
+
+// Where this kernel is the faster one, measured over 1 to 256 rows, 64 to 11008 columns and K 64 to 4096 (us, graph-replayed,
+// the other kernel / this):
+//   * bf16 below 32 rows, where the others walk K in one workgroup per 256 columns or slice it: 3 x 1712, K 2736 48 / 6;
+//     10 x 640, K 3968 8.0 / 5.6.  Wide weights (4 Mi and more of them, K in whole groups of 128) stream (gemm_rows32.hpp).
+//   * more rows while one round of workgroups, or two of small ones, holds them (rounds * (mt + nt) <= 12): 83 x 768, K 3136
+//     12.0 / 8.5; 8-bit 83 x 768, K 3136 18.8 / 8.5; 80 x 10384, K 1072 13.3 / 12.1; past that 128 x 128 tiles re-read the
+//     operands less often (8-bit 234 x 10816, K 3584 23.5 / 31.8).
+//   * a K of 136 bf16 or less stays with the tile kernels, as do more than 128 bf16 rows over a K with an incomplete group
+//     and just 32 rows over 2 Mi weights and more: calls whose kernel, or whose workspace, is part of what the tests hold
+//     fast.
+template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRowsTile &t) {
+  if (p.K * ES <= 272 || (p.M >= 32 && t.rounds * (t.mt + t.nt) > 12))
+    return false;
+  if (ES == 1 || p.M < 32)
+    return true;
+  const bool groups = p.K % 128 == 0;
+  if (p.M == 32)
+    return p.N * p.K < (int64_t)1 << 21;
+  return groups ? p.N * p.K < (int64_t)1 << 22 : p.M <= 128;
+}
+
+// Takes the call when the shape is this kernel's (returns -1 otherwise: the other kernels handle it).
+template <int ES> static int launch_few_rows(const GemmParams *pp, hipStream_t stream, bool dry, GemmTileConfig *cfg = nullptr) {
+  GemmParams p = *pp;
+  const int out_es = p.out_dt == DT_BF16 ? 2 : 4, res_es = p.residual_dt == DT_BF16 ? 2 : 4;
+  auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  if (p.cfg_tile || p.cfg_split_k || p.cfg_waves) // a caller's MatmulConfig names another kernel's tile
+    return -1;
+  if (p.M < 1 || p.M > 256 || p.K < 1 || p.K % (16 / ES) != 0 || p.N % (ES == 2 && p.trans_b ? 4 : 16 / ES) != 0 || !al16(p.A) || !al16(p.B) ||
+      !al16(p.C) || (p.lda * ES) % 16 != 0 || (p.ldb * ES) % 16 != 0 || (p.ldc * out_es) % 16 != 0 || (ES == 1 && (p.trans_b || p.residual)) ||
+      (ES == 2 && p.out_dt == DT_S32) || (p.residual && p.residual_dt != DT_BF16 && p.residual_dt != DT_F32))
+    return -1;
+  const int64_t nbatch = p.batch > 1 ? p.batch : 1;
+  if (nbatch > 65535 || p.N > (int64_t)1 << 28 || p.K > (int64_t)1 << 30)
+    return -1;
+  if (nbatch == 1)
+    p.a_bs = p.b_bs = p.c_bs = 0;
+  else if ((p.a_bs * ES) % 16 != 0 || (p.b_bs * ES) % 16 != 0 || (p.c_bs * out_es) % 16 != 0 || (p.residual && (p.c_bs * res_es) % 16 != 0))
+    return -1;
+  // a stage's rows reachable with 32-bit byte offsets
+  if (p.lda * ES * 64 >= (int64_t)1 << 31 || p.ldb * ES * (p.trans_b ? 64 : 128) >= (int64_t)1 << 31)
+    return -1;
+  const FewRowsTile t = few_rows_tile(p.M, p.N);
+  if (!few_rows_wanted<ES>(p, t))
+    return -1;
+  if (cfg) {
+    GemmTileConfig c{};
+    c.kernel = GK_FEW_ROWS, c.bm = 16 * t.mt, c.bn = 16 * t.nt, c.kbytes = 128, c.stages = t.stages;
+    c.waves_m = c.waves_n = 1, c.wave_m = c.bm, c.wave_n = c.bn, c.mfma_m = c.mfma_n = 16, c.mfma_k = 64 / ES;
+    c.split_k = 1, c.group_m = 1, c.workgroups = (int32_t)t.blocks;
+    *cfg = c;
+  }
+  if (dry)
+    return 0;
+  const dim3 grid((unsigned)((t.blocks + 7) / 8 * 8), (unsigned)nbatch), block(64 * t.waves);
+#define GCMI_FEW_LAUNCH(TB, MT, NT, W, D)                                                                                \
+  if (t.mt == MT && t.nt == NT)                                                                                           \
+    hipLaunchKernelGGL((gemm_few_rows_kernel<ES, TB, MT, NT, W, D>), grid, block, 0, stream, p);
+#define GCMI_FEW_ALL(TB)                                                                                              \
+  GCMI_FEW_LAUNCH(TB, 1, 1, 8, 2) GCMI_FEW_LAUNCH(TB, 2, 1, 8, 2) GCMI_FEW_LAUNCH(TB, 4, 1, 4, 3)            \
+  GCMI_FEW_LAUNCH(TB, 1, 2, 4, 3) GCMI_FEW_LAUNCH(TB, 2, 2, 4, 3) GCMI_FEW_LAUNCH(TB, 4, 2, 4, 3)            \
+  GCMI_FEW_LAUNCH(TB, 1, 4, 4, 3) GCMI_FEW_LAUNCH(TB, 2, 4, 4, 3) GCMI_FEW_LAUNCH(TB, 4, 4, 4, 2)
+  if (ES == 2 && p.trans_b) {
+    if constexpr (ES == 2) {
+      GCMI_FEW_ALL(true)
+    }
+  } else {
+    GCMI_FEW_ALL(false)
+  }
+#undef GCMI_FEW_ALL
+#undef GCMI_FEW_LAUNCH
+  return hipGetLastError() == hipSuccess ? 0 : 5;
+}
+
+} // namespace gcmi

@@ -33,48 +33,6 @@ namespace gcmi {
 
 static constexpr int R32_BM = 32, R32_BN = 64, R32_KB = 256, R32_NST = 3;
 
-// Four results of row m, columns n .. n+3, from their f32 sums: the rounding points of a bf16 graph (after the
-// matmul and after every op, lib/gc/Transforms/Pipeline.cpp:79-95), or one f32 epilogue.
-__device__ __forceinline__ void rows32_store4(const GemmParams &p, const f32x4_t &v, int64_t m, int64_t n) {
-  float o32[4];
-  uint16_t o16[4];
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    float b = 0.0f;
-    if (p.bias)
-      b = p.bias_dt == DT_BF16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t *>(p.bias)[n + c])
-                               : reinterpret_cast<const float *>(p.bias)[n + c];
-    float x = v[c], r = 0.0f;
-    if (p.residual)
-      r = p.residual_dt == DT_BF16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t *>(p.residual)[m * p.ldr + n + c])
-                                   : reinterpret_cast<const float *>(p.residual)[m * p.ldr + n + c];
-    if (p.out_dt == DT_BF16) {
-      x = round_bf16(x);
-      if (p.bias)
-        x = round_bf16(x + b);
-      if (p.act != ACT_NONE)
-        x = round_bf16(apply_act(x, p.act));
-      if (p.residual)
-        x = round_bf16(x + r);
-    } else {
-      if (p.bias)
-        x = x + b;
-      x = apply_act(x, p.act);
-      if (p.residual) { // kept apart from the activation's last multiply: the sum equals a separate add
-#pragma clang fp contract(off)
-        x = x + r;
-      }
-    }
-    o32[c] = x;
-    o16[c] = f32_to_bf16_bits(x);
-  }
-  if (p.out_dt == DT_BF16)
-    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.C) + m * p.ldc + n) =
-        make_uint2(o16[0] | ((uint32_t)o16[1] << 16), o16[2] | ((uint32_t)o16[3] << 16));
-  else
-    *reinterpret_cast<f32x4_t *>(reinterpret_cast<float *>(p.C) + m * p.ldc + n) = f32x4_t{o32[0], o32[1], o32[2], o32[3]};
-}
-
 // MT: 16-row tiles of A (2: up to 32 rows; 4: up to 64; 8: up to 128, with an A tile of 16 / 32 KiB per stage)
 // TB: the weights are stored [N,K]; else [K,N]: a stage's weights are then 128 k-rows of 128 bytes (the panel's 64
 // columns), requested 8 k-rows at a time (whole lines again) and read through the transposing LDS load; a k-row's 8
@@ -209,7 +167,7 @@ template <int MT, bool TB> __global__ __launch_bounds__(512, 1) void gemm_rows32
       if (p.splits > 1)
         *reinterpret_cast<f32x4_t *>(part + m * p.N + n0 + col) = v;
       else
-        rows32_store4(p, v, m, n0 + col);
+        epilogue_store4(p, v, m, n0 + col, epilogue_bias4(p, n0 + col));
     }
   }
 }

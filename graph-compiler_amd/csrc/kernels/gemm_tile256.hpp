@@ -1658,6 +1658,54 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
 
 #include "gemm_tile128.hpp"
 
+// Four results of row m, columns n .. n+3, from their f32 sums: the rounding points of a bf16 graph (after the
+// matmul and after every op, lib/gc/Transforms/Pipeline.cpp:79-95), or one f32 epilogue.
+__device__ __forceinline__ f32x4_t epilogue_bias4(const GemmParams &p, int64_t n) {
+  f32x4_t b = {0.f, 0.f, 0.f, 0.f};
+  if (p.bias)
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      b[c] = p.bias_dt == DT_BF16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t *>(p.bias)[n + c])
+                                  : reinterpret_cast<const float *>(p.bias)[n + c];
+  return b;
+}
+__device__ __forceinline__ void epilogue_store4(const GemmParams &p, const f32x4_t &v, int64_t m, int64_t n, const f32x4_t &b4) {
+  float o32[4];
+  uint16_t o16[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const float b = b4[c];
+    float x = v[c], r = 0.0f;
+    if (p.residual)
+      r = p.residual_dt == DT_BF16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t *>(p.residual)[m * p.ldr + n + c])
+                                   : reinterpret_cast<const float *>(p.residual)[m * p.ldr + n + c];
+    if (p.out_dt == DT_BF16) {
+      x = round_bf16(x);
+      if (p.bias)
+        x = round_bf16(x + b);
+      if (p.act != ACT_NONE)
+        x = round_bf16(apply_act(x, p.act));
+      if (p.residual)
+        x = round_bf16(x + r);
+    } else {
+      if (p.bias)
+        x = x + b;
+      x = apply_act(x, p.act);
+      if (p.residual) { // kept apart from the activation's last multiply: the sum equals a separate add
+#pragma clang fp contract(off)
+        x = x + r;
+      }
+    }
+    o32[c] = x;
+    o16[c] = f32_to_bf16_bits(x);
+  }
+  if (p.out_dt == DT_BF16)
+    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.C) + m * p.ldc + n) =
+        make_uint2(o16[0] | ((uint32_t)o16[1] << 16), o16[2] | ((uint32_t)o16[3] << 16));
+  else
+    *reinterpret_cast<f32x4_t *>(reinterpret_cast<float *>(p.C) + m * p.ldc + n) = f32x4_t{o32[0], o32[1], o32[2], o32[3]};
+}
+
 // Second pass of split-K: out = epilogue(sum over slices of the f32 partials), slices added in ascending
 // order (deterministic), the same rounding points as the fused epilogue.  One thread per 4 columns; the
 // loads of eight slices are in flight together.

@@ -1,0 +1,29 @@
+"""Which GEMMs of few rows take the kernel that cuts K over the waves of a workgroup, and with which tile (asked of the
+launcher, no GPU needed)."""
+import pytest
+
+
+@pytest.mark.parametrize("M,N,K,kernel,bm,bn", [
+    (1, 640, 576, 7, 16, 16), (31, 4096, 4032, 7, 32, 16), (31, 4200, 4032, 7, 32, 32), (17, 16384, 200, 7, 32, 64),
+    (31, 4096, 4096, 4, 32, 64), (31, 1000, 136, 2, 256, 256),          # a stream of weights; a short K
+    (46, 192, 2792, 7, 16, 16), (62, 1208, 3432, 7, 32, 16), (64, 4096, 1000, 7, 32, 32), (64, 4096, 4072, 7, 32, 32),
+    (32, 4096, 1376, 3, 128, 128), (32, 2048, 1016, 7, 16, 16), (33, 2048, 1024, 7, 16, 32), (128, 1288, 200, 7, 32, 32), (129, 1024, 4072, 3, 128, 128), (256, 1024, 512, 7, 32, 32),
+    (257, 1024, 512, 5, 128, 128)])
+def test_bf16(gc, M, N, K, kernel, bm, bn):
+    for tb in (False, True):
+        c = gc.tile_config(M, N, K, trans_b=tb)[0]
+        assert (c.kernel, c.bm, c.bn) == (kernel, bm, bn)
+        if kernel == 7:  # one launch: no partial sums
+            assert c.split_k == 1 and gc.lib().gcmi_gemm_bf16_workspace_bytes(M, N, K, int(tb)) == 0
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [(1, 512, 512, 7), (32, 11008, 4096, 7), (256, 896, 2112, 7), (234, 10816, 3584, 5),
+                                          (300, 272, 512, 5), (32, 512, 272, 5), (20, 512, 520, 0)])
+def test_int8(gc, M, N, K, kernel):
+    for dt in (gc.U8, gc.S8):
+        assert gc.tile_config(M, N, K, a_dtype=dt)[0].kernel == kernel
+
+
+def test_a_matmul_config_names_another_kernel(gc):
+    cfg = [1, 1, 1, 128, 128, 64, 64, 64, 32]
+    assert gc.tile_config(40, 1024, 1024, matmul_config=cfg)[0].kernel == 5

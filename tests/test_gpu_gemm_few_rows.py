@@ -1,0 +1,119 @@
+"""Up to 256 rows of A in one launch (K over the waves of a workgroup): every tile of the kernel at its edges, ends of K
+inside a stage, strided operands, every epilogue, special values behind K, and both layouts of the weights."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FEW = 7
+# every tile of 16, 32 and 64 rows and columns, whole and cut, one and two rounds of workgroups; K in whole stages (64 bf16,
+# 128 bytes), one chunk into and one chunk short of one, and fewer stages than waves
+SHAPES = [(1, 640, 576), (3, 1712, 2736), (16, 24, 144), (17, 1000, 1080), (32, 2048, 1016), (33, 520, 1544), (64, 2008, 640),
+          (50, 8, 4096), (5, 8200, 264), (31, 9000, 200), (64, 8208, 328), (9, 16400, 160), (20, 17000, 232), (48, 16376, 168), (128, 1288, 200), (97, 3000, 392), (256, 1000, 256), (65, 520, 4088)]
+
+
+def _ints(shape, lo, hi, dev, g, dt):
+    return torch.randint(lo, hi, shape, device=dev, generator=g, dtype=torch.int32).to(dt)
+
+
+def _padded(t, pad, fill):
+    """The same values inside rows that are `pad` elements longer, `fill` between and behind them."""
+    full = torch.full((t.shape[0] + 1, t.shape[1] + pad), fill, device=t.device, dtype=t.dtype)
+    full[:t.shape[0], :t.shape[1]] = t
+    return full[:t.shape[0], :t.shape[1]]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_bf16_exact_on_integers(gc, dev, M, N, K, trans_b):
+    """NaN in what lies behind the rows and the columns of the operands: none of it may be used."""
+    assert gc.tile_config(M, N, K, trans_b=trans_b, out_dtype=gc.F32)[0].kernel == FEW
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    A, W = _ints((M, K), -3, 4, dev, g, torch.bfloat16), _ints((K, N), -3, 4, dev, g, torch.bfloat16)
+    want = A.float() @ W.float()
+    Ap, Wp = _padded(A, 8, float("nan")), _padded(W.t().contiguous() if trans_b else W, 8, float("nan"))
+    guard = torch.full((M + 2, N + 4), 7.0, device=dev)
+    out = guard[1:M + 1, :N]
+    (gc.gemm_bf16_nt if trans_b else gc.gemm_bf16)(Ap, Wp, out_dtype=gc.F32, out=out)
+    assert torch.equal(out, want)
+    assert (guard[0] == 7.0).all() and (guard[M + 1] == 7.0).all() and (guard[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 1712, 2736), (32, 2048, 1016), (64, 8208, 328), (20, 17000, 232)])
+def test_bf16_rounding_points_and_layouts(gc, dev, M, N, K):
+    """Bias, activation and residual against float64 rounded where a bf16 graph rounds; [N,K] and [K,N] weights, and a batch
+    of such matrices, give the same bits."""
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    A = torch.randn(M, K, device=dev, generator=g).to(torch.bfloat16)
+    W = (torch.randn(K, N, device=dev, generator=g) * 0.05).to(torch.bfloat16)
+    bias, res = torch.randn(N, device=dev, generator=g).to(torch.bfloat16), torch.randn(M, N, device=dev, generator=g).to(torch.bfloat16)
+    acc = A.double() @ W.double()
+    r = lambda t: t.to(torch.bfloat16).double()  # noqa: E731
+    gelu = lambda t: 0.5 * t * (1.0 + torch.special.erf(t / 2.0 ** 0.5))  # noqa: E731
+    want = r(r(gelu(r(r(acc) + bias.double()))) + res.double())
+    nn = gc.gemm_bf16_residual(A, W, res, bias=bias, act="gelu_erf")
+    mag = torch.maximum(acc.abs(), torch.maximum(want.abs(), res.double().abs())) + 1.0
+    assert float(((nn.double() - want).abs() / mag).max()) < 2.0 ** -7
+    nt = gc.gemm_bf16_residual(A, W.t().contiguous(), res, trans_b=True, bias=bias, act="gelu_erf")
+    assert torch.equal(nn, nt)
+    f32 = gc.gemm_bf16(A, W, bias, "sigmoid", gc.F32)
+    # K + 1 additions of exact products, each rounded once; the sigmoid's slope is at most a quarter and its own error 1e-6
+    tol = 0.25 * (K + 1) * 2.0 ** -24 * (A.double().abs() @ W.double().abs() + bias.double().abs()) + 1e-6
+    assert ((f32.double() - torch.sigmoid(acc + bias.double())).abs() <= tol).all()
+    batch = gc.gemm_batched(torch.stack([A, -A, A]), W, bias=bias, act="relu")
+    for i, a in enumerate((A, -A, A)):
+        assert torch.equal(batch[i], gc.gemm_bf16(a, W, bias, "relu"))
+
+
+def test_bf16_special_values(gc, dev):
+    """An infinity reaches its own row or column as it is, also in the chunks that stand in for what lies behind K."""
+    M, N, K = 18, 520, 1032
+    A, W = torch.ones(M, K, device=dev, dtype=torch.bfloat16), torch.ones(K, N, device=dev, dtype=torch.bfloat16)
+    A[2, K - 1], W[K - 1, 5], W[3, 7] = float("inf"), float("-inf"), float("nan")
+    for out in (gc.gemm_bf16(A, W), gc.gemm_bf16_nt(A, W.t().contiguous())):
+        assert out[:, 7].isnan().all() and out[2, 5] == float("-inf")
+        assert (out[2, [c for c in range(N) if c not in (5, 7)]] == float("inf")).all()
+        assert (out[[m for m in range(M) if m != 2], 5] == float("-inf")).all()
+        rest = out[[m for m in range(M) if m != 2]][:, [c for c in range(N) if c not in (5, 7)]]
+        assert (rest == K).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 640, 512), (8, 672, 1856), (17, 1008, 1040), (32, 11008, 4096), (64, 4096, 528), (22, 16, 4080),
+                                   (40, 9008, 272 + 16), (12, 16400, 400), (64, 16368, 336), (200, 1040, 528), (256, 3008, 304)])
+@pytest.mark.parametrize("a_dtype", [torch.uint8, torch.int8])
+def test_int8_exact_and_epilogues(gc, dev, M, N, K, a_dtype):
+    u8 = a_dtype is torch.uint8
+    assert gc.tile_config(M, N, K, a_dtype=gc.U8 if u8 else gc.S8)[0].kernel == FEW
+    g = torch.Generator(device=dev).manual_seed(K + N)
+    A = _padded(_ints((M, K), 0 if u8 else -128, 256 if u8 else 128, dev, g, a_dtype), 16, 77)
+    W = _padded(_ints((K, N), -128, 128, dev, g, torch.int8), 16, 99)
+    zp = 131 if u8 else 0
+    cs = gc.colsum_s8(W)
+    acc = (A.double() - zp) @ W.double()
+    raw = torch.full((M + 2, N), 7, device=dev, dtype=torch.int32)
+    gc.gemm_int8(A, W, cs, zp, None, None, None, gc.S32, out=raw[1:M + 1])
+    assert torch.equal(raw[1:M + 1].double(), A.double() @ W.double()) and (raw[0] == 7).all() and (raw[M + 1] == 7).all()
+    scale = (torch.rand(N, device=dev, generator=g) + 0.5) / (60.0 * K ** 0.5)
+    bias = torch.randn(N + 1, device=dev, generator=g)[1:]  # not 16-byte aligned
+    pre = acc * scale.double() + bias.double()
+    f = {None: lambda x: x, "relu": torch.relu, "sigmoid": torch.sigmoid, "gelu_erf": torch.nn.functional.gelu,
+         "gelu_tanh": lambda x: torch.nn.functional.gelu(x, approximate="tanh")}
+    for act, fn in f.items():
+        # the accumulators are exact: a conversion, a product and a sum in f32, and the activation's own error
+        y32 = gc.gemm_int8(A, W, cs, zp, scale, bias, act, gc.F32)
+        assert ((y32.double() - fn(pre)).abs() <= 1.13 * 2.0 ** -22 * ((acc * scale.double()).abs() + bias.double().abs()) + 2e-6).all()
+        y16 = gc.gemm_int8(A, W, cs, zp, scale, bias, act, gc.BF16)
+        # one rounding to bf16; the short GELU is good to 2^-11.9
+        assert ((y16.double() - fn(pre)).abs() <= 2.0 ** -8 * 1.1 * fn(pre).abs() + 2e-6).all()
+
+
+def test_int8_special_scales(gc, dev):
+    """Scales and biases that leave the range of f32 take the epilogue that looks for NaN."""
+    M, N, K = 4, 48, 512
+    A, W = torch.full((M, K), 3, device=dev, dtype=torch.uint8), torch.ones(K, N, device=dev, dtype=torch.int8)
+    scale, bias = torch.ones(N, device=dev), torch.zeros(N, device=dev)
+    scale[0], scale[1], bias[1], bias[2], scale[20] = float("inf"), float("inf"), float("-inf"), float("nan"), 1e38
+    out = gc.gemm_int8(A, W, gc.colsum_s8(W), 0, scale, bias, "relu", gc.BF16)
+    assert (out[:, 0] == float("inf")).all() and out[:, 1].isnan().all() and out[:, 2].isnan().all()
+    assert (out[:, 20] == float("inf")).all() and (out[:, 3:20] == 3 * K).all()
+    assert (out[:, 1].view(torch.int16) == 0x7FC0).all() and (out[:, 2].view(torch.int16) == 0x7FC0).all()
