@@ -316,14 +316,14 @@ static FewRowsTile few_rows_tile(int64_t M, int64_t N) {
 // the other kernel / this):
 //   * bf16 below 32 rows, where the others walk K in one workgroup per 256 columns or slice it: 3 x 1712, K 2736 48 / 6;
 //     10 x 640, K 3968 8.0 / 5.6.  Wide weights (4 Mi and more of them, K in whole groups of 128) stream (gemm_rows32.hpp).
-//   * more rows while one round of workgroups, or two of small ones, holds them (rounds * (mt + nt) <= 12): 83 x 768, K 3136
-//     12.0 / 8.5; 8-bit 83 x 768, K 3136 18.8 / 8.5; 80 x 10384, K 1072 13.3 / 12.1; past that 128 x 128 tiles re-read the
-//     operands less often (8-bit 234 x 10816, K 3584 23.5 / 31.8).
+//   * more rows while one round of workgroups, or two of small ones with 8-bit operands, holds them (rounds * (mt + nt)): 83 x
+//     768, K 3136 12.0 / 8.5; 8-bit 83 x 768, K 3136 18.8 / 8.5; 80 x 10384, K 1072 13.3 / 12.1; past that 128 x 128 tiles
+//     re-read the operands less often (8-bit 234 x 10816, K 3584 23.5 / 31.8; bf16 150 x 5736, K 512 8.9 / 10.8).
 //   * a K of 136 bf16 or less stays with the tile kernels, as do more than 128 bf16 rows over a K with an incomplete group
 //     and just 32 rows over 2 Mi weights and more: calls whose kernel, or whose workspace, is part of what the tests hold
 //     fast.
 template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRowsTile &t) {
-  if (p.K * ES <= 272 || (p.M >= 32 && t.rounds * (t.mt + t.nt) > 12))
+  if (p.K * ES <= 272 || (p.M >= 32 && t.rounds * (t.mt + t.nt) > (ES == 2 ? 8 : 12)))
     return false;
   if (ES == 1 || p.M < 32)
     return true;

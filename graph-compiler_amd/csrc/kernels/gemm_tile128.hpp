@@ -1,7 +1,9 @@
-// The 128 x 128 tile kernel.  Included by gemm_tile256.hpp (inside namespace gcmi, behind the pieces it shares with
-// the 256 x 256 kernels: tile_of_block, MfmaOp, the 4-wave kernel's epilogue); the launcher there chooses between the
-// tiles.
+// The 128 x 128 tile kernel and its taller forms (pieces it shares with the 256 x 256 kernels: tile_of_block, MfmaOp, the
+// 4-wave kernel's epilogue); the launcher in gemm_tile256.hpp chooses between the tiles.
 #pragma once
+#include "gemm_tile256.hpp"
+
+namespace gcmi {
 
 // ---------------------------------------------------------------------------
 // 128 x 128 tiles for problems whose 256 x 256 tiles would leave most of the GPU idle (a 256 x 256 tile keeps
@@ -14,21 +16,29 @@
 // barrier per stage.  Rows past M and columns past N (N a multiple of 8) are fetched from the last row / chunk
 // inside and never stored.  The epilogue is the 4-wave kernel's: accumulators through a wave-private LDS region,
 // then rows of four columns per lane.  blockIdx.y: the batch, or with GemmParams::splits the K slice.
-static constexpr int T128_B = 128, T128_KB = 64, T128_NST = 4;
-static constexpr int T128_A_BYTES = T128_B * T128_KB, T128_STAGE_BYTES = 2 * T128_A_BYTES;
-static constexpr int T128_DUMP_WAVE_BYTES = 64 * W4_DUMP_PITCH; // 17408 per wave
-static constexpr int T128_SMEM_BYTES = 4 * T128_DUMP_WAVE_BYTES + 3 * 256 * 4; // accumulator regions / ring, column parameters
-static_assert(T128_NST * T128_STAGE_BYTES <= 4 * T128_DUMP_WAVE_BYTES, "the ring overlaps the column parameters");
+// LDS bounds the loop (a stage of 128 rows: 32 KiB of fragment reads and 16 KiB of requests for 256 cycles of MFMAs), so a
+// taller wave tile gets more out of it: 96 or 128 rows per wave read 14 or 12 bytes where 64 rows read 16.  That is what the
+// forms of 192 and 256 rows are for, with one workgroup per compute unit: 1.5 and 1.85 us per 128 of K against 1.12 (one
+// workgroup) and 1.9 to 2.17 (two on a compute unit) at 128 rows.
+template <int MI> struct T128 {
+  static constexpr int BM = 32 * MI, A_BYTES = BM * T128_KB, STAGE_BYTES = A_BYTES + T128_B * T128_KB;
+  static constexpr int DUMP_WAVE_BYTES = 16 * MI * W4_DUMP_PITCH;      // 17408 per wave at 128 rows
+  static constexpr int SMEM_BYTES = 4 * DUMP_WAVE_BYTES + 3 * 256 * 4; // accumulator regions / ring, column parameters
+  static_assert(T128_NST * STAGE_BYTES <= 4 * DUMP_WAVE_BYTES, "the ring overlaps the column parameters");
+  static_assert(MI % 2 == 0, "every wave requests as many rows of A");
+};
 
-template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void gemm_tile128_kernel(GemmParams p) {
+// MI: 16-row tiles of a wave; the workgroup's tile has 32 * MI rows (128, 192 or 256) and 128 columns
+template <bool TB, int ES, int MI> __device__ __forceinline__ void tile128_body(GemmParams p) {
   static_assert(!TB || ES == 2, "B stored [N,K]: bf16 only");
-  constexpr int KB = T128_KB, BK = KB / ES, NST = T128_NST, A_BYTES = T128_A_BYTES, STAGE = T128_STAGE_BYTES;
+  constexpr int KB = T128_KB, BK = KB / ES, NST = T128_NST, BM = T128<MI>::BM, A_BYTES = T128<MI>::A_BYTES, STAGE = T128<MI>::STAGE_BYTES;
+  constexpr int NA = MI / 2, NB = 2, PER = NA + NB; // requests of 1 KiB per wave and stage
   // a k-row of the B tile: 256 bytes of bf16 (4 k-rows per transposing read, chunk ^ 4 * (k % 4)) or 128 bytes of
   // int8 (8 k-rows per read, chunk ^ 2 * (k % 8 / 2): the read of 8 k-rows x 16 columns touches every bank once)
   constexpr int RG = ES == 2 ? 4 : 8, B_ROW_BYTES = T128_B * ES, B_CPR = B_ROW_BYTES / 16;
   typedef typename std::conditional<ES == 2, f32x4_t, i32x4_t>::type acc4_t;
-  __shared__ __align__(1024) char smem[T128_SMEM_BYTES];
-  float *colp = reinterpret_cast<float *>(smem + 4 * T128_DUMP_WAVE_BYTES); // [0..127] bias, [256..] scale, [512..] comp * colsum
+  __shared__ __align__(1024) char smem[T128<MI>::SMEM_BYTES];
+  float *colp = reinterpret_cast<float *>(smem + 4 * T128<MI>::DUMP_WAVE_BYTES); // [0..127] bias, [256..] scale, [512..] comp * colsum
   auto b_swz = [](int krow) { return ES == 2 ? (krow % 4) * 4 : ((krow % 8) >> 1) * 2; };
 
   const int tid = threadIdx.x;
@@ -37,11 +47,11 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
   const int wm = wave >> 1, wn = wave & 1;
   const int r16 = lane & 15, g16 = lane >> 4;
 
-  const int tiles_m = (int)((p.M + T128_B - 1) / T128_B), tiles_n = (int)((p.N + T128_B - 1) / T128_B);
+  const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + T128_B - 1) / T128_B);
   int tm, tn;
   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, p.group_m, tm, tn);
   tm = __builtin_amdgcn_readfirstlane(tm), tn = __builtin_amdgcn_readfirstlane(tn);
-  const int64_t m0 = (int64_t)tm * T128_B, n0 = (int64_t)tn * T128_B;
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * T128_B;
   const int64_t lda_b = p.lda * ES, ldb_b = p.ldb * ES;
   const int64_t b_step = TB ? (int64_t)KB : (int64_t)BK * ldb_b;
   const int all_groups = (int)((p.K + NST * BK - 1) / (NST * BK)), k_left = (int)(p.K % (NST * BK));
@@ -65,34 +75,38 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
     if (p.residual)
       p.residual = reinterpret_cast<const char *>(p.residual) + bz * p.c_bs * (p.residual_dt == DT_BF16 ? 2 : 4);
   }
-  const int rows_in = (int)min((int64_t)T128_B, p.M - m0), cols_in = (int)min((int64_t)T128_B, p.N - n0);
+  const int rows_in = (int)min((int64_t)BM, p.M - m0), cols_in = (int)min((int64_t)T128_B, p.N - n0);
 
-  // this wave's two DMA instructions per operand and stage: 1 KiB each = 16 rows of A (or of B stored [N,K]), 4 k-rows of B
-  uint32_t a_src[2], b_src[2];
-  int a_k[2], b_k[2]; // the first k of the lane's 16 bytes inside a k-block
+  // this wave's DMA instructions per stage, MI / 2 for A and two for B: 1 KiB each = 16 rows of A (or of B stored [N,K]), 4
+  // k-rows of B
+  uint32_t a_src[NA], b_src[NB];
+  int a_k[NA], b_k[NB]; // the first k of the lane's 16 bytes inside a k-block
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int d = wave * 2 + i;
-    const int row = d * 16 + lane / 4;
-    const int c = (lane % 4) ^ ((row >> 2) & 3);
+  for (int i = 0; i < NA; i++) {
+    const int row = (wave * NA + i) * 16 + lane / 4, c = (lane % 4) ^ ((row >> 2) & 3);
     a_src[i] = (uint32_t)(min(row, rows_in - 1) * lda_b + c * 16);
+    a_k[i] = c * 16 / ES;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    const int d = wave * NB + i, row = d * 16 + lane / 4, c = (lane % 4) ^ ((row >> 2) & 3);
     const int krow = d * (1024 / B_ROW_BYTES) + lane / B_CPR;
     const int cb = min((lane % B_CPR) ^ b_swz(krow), cols_in * ES / 16 - 1);
     b_src[i] = TB ? (uint32_t)(min(row, cols_in - 1) * ldb_b + c * 16) : (uint32_t)(krow * ldb_b + cb * 16);
-    a_k[i] = c * 16 / ES, b_k[i] = TB ? a_k[i] : krow;
+    b_k[i] = TB ? c * 16 / ES : krow;
   }
   auto issue = [&](char *__restrict__ stage, const char *a_base, const char *b_base) {
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < NA; i++)
       __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(a_base + a_src[i]),
-                                       (GCMI_LDS void *)(stage + (wave * 2 + i) * 1024), 16, 0, 0);
+                                       (GCMI_LDS void *)(stage + (wave * NA + i) * 1024), 16, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < NB; i++)
       __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(b_base + b_src[i]),
-                                       (GCMI_LDS void *)(stage + A_BYTES + (wave * 2 + i) * 1024), 16, 0, 0);
+                                       (GCMI_LDS void *)(stage + A_BYTES + (wave * NB + i) * 1024), 16, 0, 0);
   };
-  // fragment reads as in gemm_tile256_mi16_kernel: A tile `it` = rows wm*64 + 16*it .., B tile `jt` = columns wn*64 + 16*jt ..
-  const int row_a = wm * 64 + r16;
+  // fragment reads as in gemm_tile256_mi16_kernel: A tile `it` = rows wm*16*MI + 16*it .., B tile `jt` = columns wn*64 + 16*jt ..
+  const int row_a = wm * 16 * MI + r16;
   const uint32_t a_ld = (uint32_t)(row_a * KB + ((g16 ^ ((row_a >> 2) & 3)) << 4));
   uint32_t b_ld[4];
   {
@@ -110,9 +124,9 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
       }
     }
   }
-  auto load_frags = [&](const char *__restrict__ st, uint4(&a)[4], uint4(&b)[4]) {
+  auto load_frags = [&](const char *__restrict__ st, uint4(&a)[MI], uint4(&b)[4]) {
 #pragma unroll
-    for (int it = 0; it < 4; it++)
+    for (int it = 0; it < MI; it++)
       a[it] = *reinterpret_cast<const uint4 *>(st + a_ld + it * (16 * KB));
 #pragma unroll
     for (int jt = 0; jt < 4; jt++) {
@@ -125,26 +139,26 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
       }
     }
   };
-  acc4_t acc[4][4]; // [jt][it]: rows 16*it + lane%16, columns 16*jt + 4*(lane/16) .. +3 (B fragment as first operand)
+  acc4_t acc[4][MI]; // [jt][it]: rows 16*it + lane%16, columns 16*jt + 4*(lane/16) .. +3 (B fragment as first operand)
 #pragma unroll
   for (int jt = 0; jt < 4; jt++)
 #pragma unroll
-    for (int it = 0; it < 4; it++)
+    for (int it = 0; it < MI; it++)
       acc[jt][it] = acc4_t{0, 0, 0, 0};
   const uint32_t a_xor = p.a_xor;
-  auto mfma_all = [&](const uint4(&a)[4], const uint4(&b)[4]) {
+  auto mfma_all = [&](const uint4(&a)[MI], const uint4(&b)[4]) {
     if constexpr (ES == 2) {
 #pragma unroll
       for (int jt = 0; jt < 4; jt++)
 #pragma unroll
-        for (int it = 0; it < 4; it++)
+        for (int it = 0; it < MI; it++)
           acc[jt][it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b[jt]),
                                                                 __builtin_bit_cast(bf16x8_t, a[it]), acc[jt][it], 0, 0, 0);
     } else {
       // row tile by row tile; its bytes are flipped (u8 activations: a - 128 as s8 == a ^ 0x80) just before its four
       // MFMAs, a whole stage after they were read, so no flip waits for LDS
 #pragma unroll
-      for (int it = 0; it < 4; it++) {
+      for (int it = 0; it < MI; it++) {
         const uint4 f = make_uint4(a[it].x ^ a_xor, a[it].y ^ a_xor, a[it].z ^ a_xor, a[it].w ^ a_xor);
 #pragma unroll
         for (int jt = 0; jt < 4; jt++)
@@ -173,7 +187,7 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
   int first_request = NST - 1; // the k-block that the first stage requests
   if (k_tail) { // all four slots are filled here; k-blocks 4.. are the whole ones from k_first on
     const int64_t k_full = p.K - k_left - k_first * BK;
-    fill_ring_k_tail<ES, TB, 2, STAGE, A_BYTES>(smem, wave, lane, a_ptr + k_full * ES, b_ptr + (TB ? k_full * ES : k_full * ldb_b),
+    fill_ring_k_tail<ES, TB, NA, NB, STAGE, A_BYTES>(smem, wave, lane, a_ptr + k_full * ES, b_ptr + (TB ? k_full * ES : k_full * ldb_b),
                                                 b_step, k_left, a_src, b_src, a_k, b_k);
     first_request = NST;
     a_ptr -= NST * KB, b_ptr -= NST * b_step;
@@ -189,16 +203,19 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
       reinterpret_cast<int *>(colp)[512 + tid] = cp_cs;
     }
   }
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * 4) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * PER) : "memory");
   __builtin_amdgcn_s_barrier();
-  uint4 fa0[4], fb0[4], fa1[4], fb1[4];
+  uint4 fa0[MI], fb0[4], fa1[MI], fb1[4];
   load_frags(smem, fa0, fb0);
 
   // One stage: k-block kt is in the `cur` registers.  Request block kt+NST-1 into the slot block kt-1 was read from
   // (every wave's reads of it had returned before it passed the previous barrier); wait for this wave's share of
   // block kt+1 and for its own LDS reads; barrier: block kt+1 is visible; read its fragments under the MFMAs of kt.
+  // (Measured and not kept: the barrier in front of the request, so that a block's reads are waited for one stage later:
+  // 8 % slower at K 11008, the requests go out later; a ring of seven or eight slots: level at best.)
+  constexpr int N_DS = MI + (TB ? 4 : 8); // LDS reads of a block's fragments
   auto stage = [&](auto has_fill, auto has_next, auto behindc, int kf, const char *__restrict__ nxt, char *__restrict__ fill,
-                   const char *a_fill, const char *b_fill, uint4(&ca)[4], uint4(&cb)[4], uint4(&na)[4], uint4(&nb)[4]) {
+                   const char *a_fill, const char *b_fill, uint4(&ca)[MI], uint4(&cb)[4], uint4(&na)[MI], uint4(&nb)[4]) {
     constexpr bool HAS_FILL = decltype(has_fill)::value, HAS_NEXT = decltype(has_next)::value;
     constexpr int BEHIND = decltype(behindc)::value;
     if constexpr (HAS_FILL) {
@@ -206,15 +223,14 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
         issue(fill, a_fill, b_fill);
     }
     if constexpr (HAS_NEXT) {
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEHIND * 4) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEHIND * PER) : "memory");
       __builtin_amdgcn_s_barrier();
       load_frags(nxt, na, nb);
     }
     mfma_all(ca, cb);
     // MFMA, two LDS reads, MFMA, two LDS reads ... then the remaining MFMAs
     if constexpr (HAS_NEXT) {
-      constexpr int N_DS = TB ? 8 : 12;
-      static_for<0, 16>([&](auto ic) {
+      static_for<0, 4 * MI>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         constexpr int left = N_DS - 2 * i;
@@ -254,16 +270,22 @@ template <bool TB = false, int ES = 2> __global__ __launch_bounds__(256, 2) void
 
   // the accumulator regions lie over the ring: every wave's reads of the last block must have returned
   __syncthreads();
-  char *dump = smem + wave * T128_DUMP_WAVE_BYTES;
+  char *dump = smem + wave * T128<MI>::DUMP_WAVE_BYTES;
 #pragma unroll
   for (int jt = 0; jt < 4; jt++)
 #pragma unroll
-    for (int it = 0; it < 4; it++)
+    for (int it = 0; it < MI; it++)
       *reinterpret_cast<acc4_t *>(dump + (it * 16 + r16) * W4_DUMP_PITCH + (jt * 16 + 4 * g16) * 4) = acc[jt][it];
   const int out_kind = p.out_dt == DT_BF16 ? 0 : ((ES == 1 && p.out_dt == DT_S32) ? 2 : 1);
   const int kind = (out_kind == 2 ? (int)ACT_NONE : p.act) + 8 * out_kind;
-  if (rows_in < T128_B || cols_in < T128_B)
-    w4_epilogue_half_any<ES, true, 64, 64>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, rows_in, cols_in);
+  if (rows_in < BM || cols_in < T128_B)
+    w4_epilogue_half_any<ES, true, 16 * MI, 64>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, rows_in, cols_in);
   else
-    w4_epilogue_half_any<ES, false, 64, 64>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, T128_B, T128_B);
+    w4_epilogue_half_any<ES, false, 16 * MI, 64>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, BM, T128_B);
 }
+
+template <bool TB, int ES> __global__ __launch_bounds__(256, 2) void gemm_tile128_kernel(GemmParams p) { tile128_body<TB, ES, 4>(p); }
+// 192 or 256 rows: one workgroup per compute unit (107 and 142 KiB of LDS)
+template <bool TB, int ES, int MI> __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams p) { tile128_body<TB, ES, MI>(p); }
+
+} // namespace gcmi

@@ -1453,39 +1453,44 @@ __device__ __forceinline__ void w4_epilogue_half_any(const GemmParams &p, int ki
 // knows nothing of the tail.  (A tail handled behind the loop would need the accumulators outside the assembly.)
 // Before, every K that is no multiple of 128 bf16 / 256 bytes went to the bounds-checked kernel: 1237 x 4096 x 1376
 // ([N,K] weights) took 89.7 us there, 29.5 us as 320 tiles of 128 x 128.
-// a_src / b_src: the lane's byte offset per DMA instruction; a_k / b_k: its first k inside a block, which decides whether
+// a_src / b_src: the lane's byte offset per DMA instruction (NA and NB of them per wave and block); a_k / b_k: its first k inside a block, which decides whether
 // it lies before K.
-template <int ES, bool TB, int NDMA, int STAGE, int A_BYTES, typename OffA, typename OffB>
+template <int ES, bool TB, int NA, int NB, int STAGE, int A_BYTES, typename OffA, typename OffB>
 __device__ __forceinline__ void fill_ring_k_tail(char *smem, int wave, int lane, const char *a_tail, const char *b_tail,
                                                  int64_t b_step, int k_left, const OffA &a_src, const OffB &b_src,
-                                                 const int (&a_k)[NDMA], const int (&b_k)[NDMA]) {
+                                                 const int (&a_k)[NA], const int (&b_k)[NB]) {
   constexpr int BK = 64 / ES;
 #pragma unroll 1
   for (int blk = 0; blk < 4; blk++, k_left -= BK, a_tail += 64, b_tail += b_step) {
-    char *st = smem + blk * STAGE + wave * NDMA * 1024;
+    char *sa = smem + blk * STAGE + wave * NA * 1024, *sb = smem + blk * STAGE + A_BYTES + wave * NB * 1024;
     if (k_left >= BK) {
 #pragma unroll
-      for (int i = 0; i < NDMA; i++) {
-        __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(a_tail + (uint32_t)a_src[i]), (GCMI_LDS void *)(st + i * 1024), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(b_tail + (uint32_t)b_src[i]),
-                                         (GCMI_LDS void *)(st + A_BYTES + i * 1024), 16, 0, 0);
-      }
+      for (int i = 0; i < NA; i++)
+        __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(a_tail + (uint32_t)a_src[i]), (GCMI_LDS void *)(sa + i * 1024), 16, 0, 0);
+#pragma unroll
+      for (int i = 0; i < NB; i++)
+        __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(b_tail + (uint32_t)b_src[i]), (GCMI_LDS void *)(sb + i * 1024), 16, 0, 0);
       continue;
     }
-    uint4 va[NDMA], vb[NDMA];
+    uint4 va[NA], vb[NB];
 #pragma unroll
-    for (int i = 0; i < NDMA; i++) {
-      va[i] = vb[i] = make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < NA; i++) {
+      va[i] = make_uint4(0, 0, 0, 0);
       if (a_k[i] < k_left)
         va[i] = *reinterpret_cast<const uint4 *>(a_tail + (uint32_t)a_src[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      vb[i] = make_uint4(0, 0, 0, 0);
       if (b_k[i] < k_left)
         vb[i] = *reinterpret_cast<const uint4 *>(b_tail + (uint32_t)b_src[i]);
     }
 #pragma unroll
-    for (int i = 0; i < NDMA; i++) {
-      *reinterpret_cast<uint4 *>(st + i * 1024 + lane * 16) = va[i];
-      *reinterpret_cast<uint4 *>(st + A_BYTES + i * 1024 + lane * 16) = vb[i];
-    }
+    for (int i = 0; i < NA; i++)
+      *reinterpret_cast<uint4 *>(sa + i * 1024 + lane * 16) = va[i];
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+      *reinterpret_cast<uint4 *>(sb + i * 1024 + lane * 16) = vb[i];
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 }
@@ -1595,7 +1600,7 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
   const int ring_filled = k_left;
   if (k_left) {
     const int64_t k_full = p.K - k_left;
-    fill_ring_k_tail<ES, TB, 4, FG::STAGE_BYTES, FG::A_BYTES>(
+    fill_ring_k_tail<ES, TB, 4, 4, FG::STAGE_BYTES, FG::A_BYTES>(
         smem, wave, lane, reinterpret_cast<const char *>(a_ptr) + k_full * ES,
         reinterpret_cast<const char *>(b_ptr) + (TB ? k_full * ES : k_full * ldb_b), (int64_t)b_step, k_left, a_off, b_off, a_k, b_k);
   }
@@ -1656,7 +1661,6 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
 #endif
 }
 
-#include "gemm_tile128.hpp"
 
 // Four results of row m, columns n .. n+3, from their f32 sums: the rounding points of a bf16 graph (after the
 // matmul and after every op, lib/gc/Transforms/Pipeline.cpp:79-95), or one f32 epilogue.
@@ -1794,6 +1798,13 @@ static void launch_splitk_reduce(const GemmParams &p, hipStream_t stream) {
   }
 }
 
+// 128 columns, 128 rows or more: gemm_tile128.hpp
+static constexpr int T128_B = 128, T128_KB = 64, T128_NST = 4;
+
+} // namespace gcmi
+extern "C" int gcmi_launch_tile128(const gcmi::GemmParams *p, int es, int rows, unsigned grid_x, unsigned grid_y, hipStream_t stream);
+namespace gcmi {
+
 // Host-side launch of the 256x256 tile kernels for one element size.
 // want != null: nothing is launched; *want receives the floats of workspace this call would use if it had them.
 // cfg != null: receives what was (or would be) chosen.
@@ -1808,6 +1819,17 @@ static inline double gcmi_us_per_group_256(double load) { // one workgroup per c
   if (load <= 1.0)
     return 2.1 + 0.65 * (load - 0.5) / 0.5;
   return 2.75;
+}
+// Taller tiles of 128 columns (one workgroup per compute unit): fewer fragment reads per product than 128 rows, so where 128
+// rows make more than a round and 192 or 256 do not, they are ahead (64 random such sizes: 1.14 times on the average, at most
+// 1.5; 8-bit ones with a short K down to 0.93).  128 / 192 / 256 rows in one pass, us: 1237 x 4096, K 1376 29.3 / 22.5 / 27.5; 305 x 11008, K 4096 69.5 / 56.3 / 63.8; 483 x 11008 73.1 / - / 67.3; where 128 rows fit one
+// round they stay: 1000 x 4096, K 4096 38.6 / 47.8 / 59.4.
+static inline double gcmi_us_per_group_tall(int rows) { return rows == 192 ? 1.5 : 1.85; }
+static inline double gcmi_us_fixed_tall(int rows, int es) { return (rows == 192 ? 5.0 : 6.0) + (es == 1 ? 1.0 : 0.0); } // (8-bit: the longer epilogue, alone on its unit)
+// A K past 8192 costs 128 rows more per group (1.39 us at K 11008: 1000 x 4096 123.6 us, 112.8 as two slices of 256 rows;
+// 483 x 4096 74.8 in two slices, 65.5 in four of 256 rows).
+static inline double gcmi_us_per_group_128_long_k(int64_t K) {
+  return K <= 8192 ? 0.0 : K >= 11008 ? 0.27 : 0.27 * (double)(K - 8192) / 2816.0;
 }
 static inline double gcmi_us_per_group_128(double load) { // up to two workgroups per compute unit
   if (load <= 0.25)
@@ -1893,7 +1915,8 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
                                         (!p.residual || (p.c_bs * res_es) % 16 == 0));
   const bool t128_can = aligned && p.N % (16 / ES) == 0 && (ES == 2 ? p.out_dt != DT_S32 : !p.trans_b) && batch_ok;
   const bool slices_can = ES == 2 && fast_but_m && p.out_dt != DT_S32 && nbatch == 1; // the 256-wide kernels: whole column tiles
-  const int64_t nblk128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
+  int rows128 = 128; // of the 128-column tile
+  int64_t nblk128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
   const int n_cu = gcmi_num_cus();
   const int groups = (int)((p.K + KGROUP - 1) / KGROUP);
   int plan = PLAN_TILE256, splits = 1;
@@ -1910,10 +1933,18 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     const double w256 = (double)(nblk * nbatch) / n_cu, w128 = (double)(nblk128 * nbatch) / n_cu;
     double best = GCMI_US_FIXED_256 + gcmi_us_per_group_256(w256) * groups; // one pass, less than one round
     const bool small_tile = p.M >= 32 && t128_can; // shorter: most of a 128-row tile would be padding
+    const double long_k = ES == 2 ? gcmi_us_per_group_128_long_k(p.K) : 0.0; // (of two workgroups on a compute unit, both)
+    // taller tiles: at least two rows of them, in one round
+    auto tall_tiles = [&](int rows) { return ((p.M + rows - 1) / rows) * ((p.N + 127) / 128) * nbatch; };
     if (small_tile) {
-      const double t = GCMI_US_FIXED_128 + gcmi_us_per_group_128(w128) * groups * (double)((nblk128 * nbatch + 2 * n_cu - 1) / (2 * n_cu));
+      const double t = GCMI_US_FIXED_128 + (gcmi_us_per_group_128(w128) + (w128 <= 1.0 ? 1 : 2) * long_k) * groups * (double)((nblk128 * nbatch + 2 * n_cu - 1) / (2 * n_cu));
       if (t < best)
         best = t, plan = PLAN_TILE128;
+      for (int rows = 192; rows <= 256; rows += 64) {
+        const double u = gcmi_us_fixed_tall(rows, ES) + gcmi_us_per_group_tall(rows) * groups;
+        if (p.M > rows && tall_tiles(rows) <= n_cu && u < best)
+          best = u, plan = PLAN_TILE128, rows128 = rows;
+      }
     }
     best *= GCMI_ONE_PASS_MARGIN;
     if (ES == 2 && nbatch == 1 && (small_tile || p.M > 128)) {
@@ -1925,11 +1956,19 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
             best = t, plan = PLAN_SLICES_TILE256, splits = s;
         }
         if (small_tile && nblk128 * s <= 2 * n_cu) {
-          const double t = GCMI_US_FIXED_128 + gcmi_us_per_group_128(w128 * s) * ((groups + s - 1) / s) + through_memory;
+          const double t = GCMI_US_FIXED_128 + (gcmi_us_per_group_128(w128 * s) + (nblk128 * s <= n_cu ? 1 : 2) * long_k) * ((groups + s - 1) / s) + through_memory;
           if (t < best)
-            best = t, plan = PLAN_SLICES_TILE128, splits = s;
+            best = t, plan = PLAN_SLICES_TILE128, splits = s, rows128 = 128;
         }
       }
+      double tall_best = best * (splits > 1 ? GCMI_ONE_PASS_MARGIN : 1.0); // against other slices they too must be clearly ahead
+      for (int s = 2; small_tile && s <= groups; s++)
+        for (int rows = 192; rows <= 256; rows += 64) {
+          const double t = gcmi_us_fixed_tall(rows, ES) + gcmi_us_per_group_tall(rows) * ((groups + s - 1) / s) + GCMI_US_SECOND_PASS +
+                           GCMI_US_PER_SLICE_MOUT * s * mn;
+          if (p.M > rows && tall_tiles(rows) * s <= n_cu && t < tall_best)
+            tall_best = best = t, plan = PLAN_SLICES_TILE128, splits = s, rows128 = rows;
+        }
     }
     if (nbatch == 1 && p.M <= 128 && slices_can && nblk * 2 <= n_cu) { // a short A: 1.35 (32 rows) to 2 us (128) per group
       const double per_group = 1.35 + 0.65 * (double)((p.M + 31) / 32 - 1) / 3.0;
@@ -1941,6 +1980,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
       }
     }
   }
+  nblk128 = ((p.M + rows128 - 1) / rows128) * ((p.N + 127) / 128);
   if (splits > 1) {
     if (want)
       *want = (int64_t)splits * p.M * p.N;
@@ -1957,8 +1997,8 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     const int tiles = (int)(by128 ? nblk128 : nblk);
     c.kernel = GK_SPLITK, c.split_k = splits, c.workgroups = tiles * splits;
     if (by128) {
-      c.bm = c.bn = 128, c.kbytes = T128_KB, c.stages = T128_NST;
-      c.waves_m = c.waves_n = 2, c.wave_m = c.wave_n = 64, c.mfma_m = c.mfma_n = 16, c.mfma_k = 32;
+      c.bm = rows128, c.bn = 128, c.kbytes = T128_KB, c.stages = T128_NST;
+      c.waves_m = c.waves_n = 2, c.wave_m = rows128 / 2, c.wave_n = 64, c.mfma_m = c.mfma_n = 16, c.mfma_k = 32;
     } else if (by256) {
       c.kbytes = 64, c.stages = 4, c.waves_m = 2, c.waves_n = 2, c.wave_m = 128, c.wave_n = 128;
       c.mfma_m = c.mfma_n = 16, c.mfma_k = 64 / ES;
@@ -1975,11 +2015,9 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     p.partial = ws;
     if constexpr (ES == 2) {
       if (by128) { // the kernel cuts K itself: blockIdx.y = slice
-        const dim3 grid((unsigned)tiles, (unsigned)splits);
-        if (p.trans_b)
-          hipLaunchKernelGGL(gemm_tile128_kernel<true>, grid, dim3(256), 0, stream, p);
-        else
-          hipLaunchKernelGGL(gemm_tile128_kernel<false>, grid, dim3(256), 0, stream, p);
+        const int rc = gcmi_launch_tile128(&p, ES, rows128, (unsigned)tiles, (unsigned)splits, stream);
+        if (rc)
+          return rc;
       } else if (by256) { // equal slices as a strided batch with f32 results
         GemmParams q = p;
         q.K = p.K / splits, q.batch = splits;
@@ -2002,21 +2040,14 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     return hipGetLastError() == hipSuccess ? 0 : 5;
   }
   if (plan == PLAN_TILE128) {
-    c.kernel = GK_TILE128, c.bm = c.bn = 128, c.kbytes = T128_KB, c.stages = T128_NST;
-    c.waves_m = c.waves_n = 2, c.wave_m = c.wave_n = 64, c.mfma_m = c.mfma_n = 16, c.mfma_k = 64 / ES;
+    c.kernel = GK_TILE128, c.bm = rows128, c.bn = 128, c.kbytes = T128_KB, c.stages = T128_NST;
+    c.waves_m = c.waves_n = 2, c.wave_m = rows128 / 2, c.wave_n = 64, c.mfma_m = c.mfma_n = 16, c.mfma_k = 64 / ES;
     c.workgroups = (int32_t)nblk128;
     if (cfg)
       *cfg = c;
     if (dry)
       return 0;
-    const dim3 grid((unsigned)nblk128, (unsigned)nbatch);
-    if (p.trans_b) {
-      if constexpr (ES == 2)
-        hipLaunchKernelGGL((gemm_tile128_kernel<true, 2>), grid, dim3(256), 0, stream, p);
-    } else {
-      hipLaunchKernelGGL((gemm_tile128_kernel<false, ES>), grid, dim3(256), 0, stream, p);
-    }
-    return hipGetLastError() == hipSuccess ? 0 : 5;
+    return gcmi_launch_tile128(&p, ES, rows128, (unsigned)nblk128, (unsigned)nbatch, stream);
   }
   // Whole tiles: 4 waves of 128 x 128 unless the caller asks for 8 waves of 128 x 64.  Results of 8-bit operands
   // leave the 4-wave kernel as bf16, f32 or as the raw s32 accumulators (same main loop, the epilogue is a plain
@@ -2075,17 +2106,15 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
       if (p.residual)
         rest.residual = reinterpret_cast<const char *>(p.residual) + m1 * p.ldr * res_es;
     }
-    const dim3 hgrid((unsigned)(nblk - nblk % n_cu)), tgrid((unsigned)(4 * (nblk % n_cu)));
+    const dim3 hgrid((unsigned)(nblk - nblk % n_cu));
     if (p.trans_b) {
       if constexpr (ES == 2) {
         hipLaunchKernelGGL((gemm_tile256_w4_kernel<ES, true>), hgrid, dim3(256), 0, stream, head);
-        hipLaunchKernelGGL((gemm_tile128_kernel<true, 2>), tgrid, dim3(256), 0, stream, rest);
       }
     } else {
       hipLaunchKernelGGL(gemm_tile256_w4_kernel<ES>, hgrid, dim3(256), 0, stream, head);
-      hipLaunchKernelGGL((gemm_tile128_kernel<false, ES>), tgrid, dim3(256), 0, stream, rest);
     }
-    return hipGetLastError() == hipSuccess ? 0 : 5;
+    return gcmi_launch_tile128(&rest, ES, 128, (unsigned)(4 * (nblk % n_cu)), 1, stream);
   }
   dim3 grid((unsigned)nblk, (unsigned)nbatch), block(G_THREADS);
   if (use_w4) {

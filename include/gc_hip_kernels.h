@@ -159,8 +159,9 @@ int gcmi_gemm_bf16_ws(const void *A, const void *B, void *C, int64_t batch, int6
  * kernel (up to 128 rows of A against wide weights in either layout; bn = 64:
  * the 8-wave kernel with the LDS ring, with split_k > 1 followed by the second
  * pass), 5 tiles of 128 x 128 with 4 waves
- * of 64 x 64 (problems of few 256 x 256 tiles; with split_k > 1 kind 3 is
- * reported and bm = bn = 128 tells), 6 the f32 kernels (a_dtype GCMI_F32, A
+ * of 64 x 64, or of 192 or 256 x 128 with one workgroup per compute unit
+ * (problems of few 256 x 256 tiles; with split_k > 1 kind 3 is reported and
+ * bn = 128 tells), 6 the f32 kernels (a_dtype GCMI_F32, A
  * stored [M,K]: bm = bn = 16, 32, 64 or 128, mfma_m = 0 for the vector kernel of
  * a short K), 7 few rows of A (up to 256) in one launch: K over the waves of a
  * workgroup, which all have the wave tile wave_m x wave_n.
