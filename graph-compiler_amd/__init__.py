@@ -135,46 +135,66 @@ def check(rc, what=""):
         raise GcError("%s failed with status %d: %s" % (what, rc, lib().gcmi_last_error().decode()))
 
 
-def _stream():
+# A call of a small GEMM or attention is bound by the host: 10.4 us around a kernel of 4 to 5.  So the helpers below hand plain
+# integers to ctypes (it converts them as it does c_void_p objects), ask torch for the stream's handle without building a
+# Stream object, and read shape and strides once (6.9 us).
+_torch = None
+
+
+def _load_torch():
+    global _torch
     import torch
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _torch = torch
+    return torch
+
+
+def _stream():
+    """The current stream of the current device, as an integer."""
+    torch = _torch or _load_torch()
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+def _result(A, M, N, out_dtype):
+    return _torch.empty((M, N), dtype=_torch.bfloat16 if out_dtype == BF16 else _torch.float32, device=A.device)
+
+
+def _bias_dt(bias):
+    return BF16 if bias is None or bias.dtype is _torch.bfloat16 else F32
 
 
 def gemm_bf16(A, B, bias=None, act=None, out_dtype=BF16, out=None):
     """A [M,K], B [K,N] torch.bfloat16 cuda tensors (row strides may exceed the row)."""
-    import torch
-    M, K = A.shape
-    K2, N = B.shape
-    assert K == K2 and (A.stride(1) == 1 or K == 1) and (B.stride(1) == 1 or N == 1)
+    _torch or _load_torch()
+    (M, K), (K2, N) = A.shape, B.shape
+    (lda, ca), (ldb, cb) = A.stride(), B.stride()
+    assert K == K2 and (ca == 1 or K == 1) and (cb == 1 or N == 1)
     if out is None:
-        out = torch.empty((M, N), device=A.device, dtype=torch.bfloat16 if out_dtype == BF16 else torch.float32)
-    bdt = BF16
-    if bias is not None:
-        bdt = BF16 if bias.dtype == torch.bfloat16 else F32
-    check(lib().gcmi_gemm_bf16(_ptr(A), _ptr(B), _ptr(out), M, N, K, A.stride(0) if M > 1 else K,
-                               B.stride(0) if K > 1 else N, out.stride(0) if M > 1 else N, _ptr(bias), bdt,
-                               ACT[act], out_dtype, _stream()), "gcmi_gemm_bf16")
+        out = _result(A, M, N, out_dtype)
+    rc = (_lib or lib()).gcmi_gemm_bf16(A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, lda if M > 1 else K, ldb if K > 1 else N,
+                                        out.stride(0) if M > 1 else N, _ptr(bias), _bias_dt(bias), ACT[act], out_dtype, _stream())
+    if rc:
+        check(rc, "gcmi_gemm_bf16")
     return out
 
 
 def gemm_bf16_nt(A, Bt, bias=None, act=None, out_dtype=BF16, out=None):
     """A [M,K], Bt [N,K] (the weight as torch.nn.Linear stores it): A @ Bt.T without a transposed copy."""
-    import torch
-    M, K = A.shape
-    N, K2 = Bt.shape
-    assert K == K2 and (A.stride(1) == 1 or K == 1) and (Bt.stride(1) == 1 or K == 1)
+    _torch or _load_torch()
+    (M, K), (N, K2) = A.shape, Bt.shape
+    (lda, ca), (ldb, cb) = A.stride(), Bt.stride()
+    assert K == K2 and (ca == 1 or K == 1) and (cb == 1 or K == 1)
     if out is None:
-        out = torch.empty((M, N), device=A.device, dtype=torch.bfloat16 if out_dtype == BF16 else torch.float32)
-    bdt = BF16
-    if bias is not None:
-        bdt = BF16 if bias.dtype == torch.bfloat16 else F32
-    check(lib().gcmi_gemm_bf16_nt(_ptr(A), _ptr(Bt), _ptr(out), M, N, K, A.stride(0) if M > 1 else K,
-                                  Bt.stride(0) if N > 1 else K, out.stride(0) if M > 1 else N, _ptr(bias), bdt,
-                                  ACT[act], out_dtype, _stream()), "gcmi_gemm_bf16_nt")
+        out = _result(A, M, N, out_dtype)
+    rc = (_lib or lib()).gcmi_gemm_bf16_nt(A.data_ptr(), Bt.data_ptr(), out.data_ptr(), M, N, K, lda if M > 1 else K, ldb if N > 1 else K,
+                                           out.stride(0) if M > 1 else N, _ptr(bias), _bias_dt(bias), ACT[act], out_dtype, _stream())
+    if rc:
+        check(rc, "gcmi_gemm_bf16_nt")
     return out
 
 
@@ -271,7 +291,7 @@ def gemm_f32(A, B, bias=None, act=None, trans_a=False, trans_b=False, out=None):
 
 def mha_fwd_bf16(Q, K, V, mask=None, scale=None, out=None, skip_masked=True):
     """Q [B,H,Sq,D], K,V [B,H,Sk,D] contiguous bf16; mask f32 [Sq,Sk] or None."""
-    import torch
+    torch = _torch or _load_torch()
     Bn, H, Sq, D = Q.shape
     Sk = K.shape[2]
     assert Q.is_contiguous() and K.is_contiguous() and V.is_contiguous()
@@ -279,9 +299,10 @@ def mha_fwd_bf16(Q, K, V, mask=None, scale=None, out=None, skip_masked=True):
         scale = 1.0 / (D ** 0.5)
     if out is None:
         out = torch.empty_like(Q)
-    mld = 0 if mask is None else mask.stride(0)
-    check(lib().gcmi_mha_fwd_bf16_opt(_ptr(Q), _ptr(K), _ptr(V), _ptr(mask), mld, _ptr(out), Bn * H, Sq, Sk, D,
-                                      float(scale), int(bool(skip_masked)), _stream()), "gcmi_mha_fwd_bf16")
+    rc = (_lib or lib()).gcmi_mha_fwd_bf16_opt(Q.data_ptr(), K.data_ptr(), V.data_ptr(), _ptr(mask), 0 if mask is None else mask.stride(0),
+                                               out.data_ptr(), Bn * H, Sq, Sk, D, float(scale), int(bool(skip_masked)), _stream())
+    if rc:
+        check(rc, "gcmi_mha_fwd_bf16")
     return out
 
 
