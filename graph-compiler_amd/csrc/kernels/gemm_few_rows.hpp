@@ -1,4 +1,4 @@
-// GEMMs of few rows of A (up to 256) against weights that are no stream worth slicing: bf16 x bf16 with weights stored
+// GEMMs of few rows of A (up to 256; 2048 of 8 bits) against weights that are no stream worth slicing: bf16 x bf16 with weights stored
 // [K,N] or [N,K], and 8-bit x s8 with weights stored [K,N].  C[M,N] = epilogue(A . W) in ONE launch.
 // What bounds such a call is the way launch -> loads -> sums -> store, once: the tile kernels' workgroup walks all of K
 // through one ring behind barriers (a 256 x 256 tile takes 60 us for 2 x 5456, K 3264, on 22 compute units), and K slices
@@ -319,12 +319,16 @@ static FewRowsTile few_rows_tile(int64_t M, int64_t N) {
 //   * more rows while one round of workgroups, or two of small ones with 8-bit operands, holds them (rounds * (mt + nt)): 83 x
 //     768, K 3136 12.0 / 8.5; 8-bit 83 x 768, K 3136 18.8 / 8.5; 80 x 10384, K 1072 13.3 / 12.1; past that 128 x 128 tiles
 //     re-read the operands less often (8-bit 234 x 10816, K 3584 23.5 / 31.8; bf16 150 x 5736, K 512 8.9 / 10.8).
+//   * 8-bit operands, for which the tile kernels have no K slices, up to 2048 rows while one round holds them: 45 random sizes
+//     of 257 to 2000 rows 1.75 times on the average (679 x 608, K 3568 23.6 / 11.1; 1328 x 768, K 976 11.0 / 8.1).
 //   * a K of 136 bf16 or less stays with the tile kernels, as do more than 128 bf16 rows over a K with an incomplete group
 //     and just 32 rows over 2 Mi weights and more: calls whose kernel, or whose workspace, is part of what the tests hold
 //     fast.
 template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRowsTile &t) {
   if (p.K * ES <= 272 || (p.M >= 32 && t.rounds * (t.mt + t.nt) > (ES == 2 ? 8 : 12)))
     return false;
+  if (p.M > 256) // 8-bit operands
+    return t.rounds == 1 && p.N >= 512 && p.K <= 4096;
   if (ES == 1 || p.M < 32)
     return true;
   const bool groups = p.K % 128 == 0;
@@ -340,7 +344,7 @@ template <int ES> static int launch_few_rows(const GemmParams *pp, hipStream_t s
   auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   if (p.cfg_tile || p.cfg_split_k || p.cfg_waves) // a caller's MatmulConfig names another kernel's tile
     return -1;
-  if (p.M < 1 || p.M > 256 || p.K < 1 || p.K % (16 / ES) != 0 || p.N % (ES == 2 && p.trans_b ? 4 : 16 / ES) != 0 || !al16(p.A) || !al16(p.B) ||
+  if (p.M < 1 || p.M > (ES == 1 ? 2048 : 256) || p.K < 1 || p.K % (16 / ES) != 0 || p.N % (ES == 2 && p.trans_b ? 4 : 16 / ES) != 0 || !al16(p.A) || !al16(p.B) ||
       !al16(p.C) || (p.lda * ES) % 16 != 0 || (p.ldb * ES) % 16 != 0 || (p.ldc * out_es) % 16 != 0 || (ES == 1 && (p.trans_b || p.residual)) ||
       (ES == 2 && p.out_dt == DT_S32) || (p.residual && p.residual_dt != DT_BF16 && p.residual_dt != DT_F32))
     return -1;

@@ -163,7 +163,7 @@ int gcmi_gemm_bf16_ws(const void *A, const void *B, void *C, int64_t batch, int6
  * (problems of few 256 x 256 tiles; with split_k > 1 kind 3 is reported and
  * bn = 128 tells), 6 the f32 kernels (a_dtype GCMI_F32, A
  * stored [M,K]: bm = bn = 16, 32, 64 or 128, mfma_m = 0 for the vector kernel of
- * a short K), 7 few rows of A (up to 256) in one launch: K over the waves of a
+ * a short K), 7 few rows of A (up to 256, 2048 of 8 bits) in one launch: K over the waves of a
  * workgroup, which all have the wave tile wave_m x wave_n.
  *
  * matmul_config (may be NULL) is the reference's per-op override: the nine

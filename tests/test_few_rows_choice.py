@@ -17,7 +17,8 @@ def test_bf16(gc, M, N, K, kernel, bm, bn):
             assert c.split_k == 1 and gc.lib().gcmi_gemm_bf16_workspace_bytes(M, N, K, int(tb)) == 0
 
 
-@pytest.mark.parametrize("M,N,K,kernel", [(1, 512, 512, 7), (32, 11008, 4096, 7), (256, 896, 2112, 7), (234, 10816, 3584, 5),
+@pytest.mark.parametrize("M,N,K,kernel", [(1, 512, 512, 7), (32, 11008, 4096, 7), (256, 896, 2112, 7), (234, 10816, 3584, 5), (257, 3264, 4096, 7), (257, 3280, 4096, 5),
+                                          (2048, 512, 528, 7), (2049, 512, 528, 5), (1024, 1024, 4096, 7), (1024, 1024, 4112, 5), (700, 496, 1024, 5),
                                           (300, 272, 512, 5), (32, 512, 272, 5), (20, 512, 520, 0)])
 def test_int8(gc, M, N, K, kernel):
     for dt in (gc.U8, gc.S8):

@@ -79,7 +79,8 @@ def test_bf16_special_values(gc, dev):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 640, 512), (8, 672, 1856), (17, 1008, 1040), (32, 11008, 4096), (64, 4096, 528), (22, 16, 4080),
-                                   (40, 9008, 272 + 16), (12, 16400, 400), (64, 16368, 336), (200, 1040, 528), (256, 3008, 304)])
+                                   (40, 9008, 272 + 16), (12, 16400, 400), (64, 16368, 336), (200, 1040, 528), (256, 3008, 304),
+                                   (257, 3264, 4096), (700, 1008, 1040), (2048, 512, 528)])
 @pytest.mark.parametrize("a_dtype", [torch.uint8, torch.int8])
 def test_int8_exact_and_epilogues(gc, dev, M, N, K, a_dtype):
     u8 = a_dtype is torch.uint8
