@@ -1,0 +1,33 @@
+"""Masked attention over few key blocks runs without the pass that classifies the mask's tiles: the bits of the calls that have
+classes, on both sides of the line and with masks that leave rows, tiles and single entries out."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Sq,Sk", [(128, 64), (130, 129), (200, 384), (384, 384), (256, 385), (385, 385)])
+@pytest.mark.parametrize("kind", ["causal", "zero", "tiles", "values"])
+def test_the_bits_of_the_classified_call(gc, dev, D, Sq, Sk, kind):
+    g = torch.Generator(device=dev).manual_seed(Sq + Sk)
+    q, k, v = (torch.randn(2, 3, s, D, device=dev, generator=g).bfloat16() for s in (Sq, Sk, Sk))
+    mask = torch.zeros(Sq, Sk, device=dev)
+    if kind == "causal":
+        mask = torch.triu(torch.full((Sq, Sk), float("-inf"), device=dev), diagonal=1 + max(0, Sk - Sq))
+    elif kind == "tiles":  # whole tiles of -inf, never a whole row
+        mask[:, 64:192] = float("-inf")
+        mask[:, Sk - 1] = 0.0
+    elif kind == "values":
+        mask = torch.randn(Sq, Sk, device=dev, generator=g)
+        mask[5, 3:] = float("-inf")
+    out = gc.mha_fwd_bf16(q, k, v, mask)
+    classes = gc.mha_mask_classes(mask, Sq, Sk, D)
+    assert classes is not None
+    assert torch.equal(out, gc.mha_fwd_bf16_classified(q, k, v, mask, classes))
+    assert torch.equal(out, gc.mha_fwd_bf16(q, k, v, mask, skip_masked=False))
+    s = q.double() @ k.double().transpose(-1, -2) * D ** -0.5 + mask.double()
+    ref = torch.softmax(s, -1) @ v.double()
+    # weights and result rounded to bf16 (2^-9 each), the exponentials' own error far below
+    mag = torch.softmax(s, -1) @ v.double().abs() + ref.abs()
+    assert ((out.double() - ref).abs() <= 2.0 ** -8 * mag + 1e-6).all()
