@@ -82,13 +82,17 @@ template <int ES, bool TB, int MT, int NT, int W, int D> __global__ __launch_bou
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g16 = lane >> 4;
   const int tiles_m = (int)((p.M + 16 * MT - 1) / (16 * MT)), tiles_n = (int)((p.N + 16 * NT - 1) / (16 * NT));
-  // workgroup i runs on XCD i % 8: each XCD walks its own run of panels (the grid is rounded up to whole runs)
-  const int tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3), tm = tile % tiles_m, tn = tile / tiles_m;
-  if (tn >= tiles_n)
+  // workgroup i runs on XCD i % 8: each XCD walks its own run of panels (the grid is rounded up to whole runs), through the
+  // matrices of a batch one after the other: with a grid of their own, rounded up each, 84 matrices of three tiles met on
+  // three XCDs (84 x 46 x 176, K 960 25 us)
+  const int tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3), tm = tile % tiles_m;
+  int tn = tile / tiles_m, bz = 0; // bz: strided batch
+  if (p.batch > 1)
+    bz = tn / tiles_n, tn -= bz * tiles_n;
+  if (tn >= tiles_n || (p.batch > 1 && bz >= p.batch))
     return;
   const int64_t m0 = (int64_t)tm * 16 * MT, n0 = (int64_t)tn * 16 * NT;
   const int rows_in = (int)min((int64_t)16 * MT, p.M - m0), cols_in = (int)min((int64_t)16 * NT, p.N - n0);
-  const int64_t bz = blockIdx.y; // strided batch
   p.A = reinterpret_cast<const char *>(p.A) + bz * p.a_bs * ES;
   p.B = reinterpret_cast<const char *>(p.B) + bz * p.b_bs * ES;
   p.C = reinterpret_cast<char *>(p.C) + bz * p.c_bs * (p.out_dt == DT_BF16 ? 2 : 4);
@@ -295,13 +299,13 @@ struct FewRowsTile {
   int mt, nt, waves, stages; // waves that share K, stages of a wave's ring
   int64_t blocks, rounds;
 };
-static FewRowsTile few_rows_tile(int64_t M, int64_t N) {
+static FewRowsTile few_rows_tile(int64_t M, int64_t N, int64_t nbatch) {
   const int64_t n_cu = gcmi_num_cus();
   FewRowsTile best{};
   int64_t best_cost = INT64_MAX;
   for (int mt = 4; mt >= 1; mt /= 2) // (of equal tiles the one with more rows: the weights are read by fewer workgroups)
     for (int nt = 1; nt <= 4; nt *= 2) {
-      const int64_t blocks = ((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)), rounds = (blocks + n_cu - 1) / n_cu;
+      const int64_t blocks = ((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)), rounds = (blocks * nbatch + n_cu - 1) / n_cu;
       const int64_t cost = rounds * (mt + nt);
       if (cost < best_cost || (cost == best_cost && blocks < best.blocks)) {
         const int waves = nt == 1 && mt < 4 ? 8 : 4;
@@ -358,7 +362,9 @@ template <int ES> static int launch_few_rows(const GemmParams *pp, hipStream_t s
   // a stage's rows reachable with 32-bit byte offsets
   if (p.lda * ES * 64 >= (int64_t)1 << 31 || p.ldb * ES * (p.trans_b ? 64 : 128) >= (int64_t)1 << 31)
     return -1;
-  const FewRowsTile t = few_rows_tile(p.M, p.N);
+  const FewRowsTile t = few_rows_tile(p.M, p.N, nbatch);
+  if (t.blocks * nbatch > (int64_t)1 << 22) // (a grid has less than 2^32 threads)
+    return -1;
   if (!few_rows_wanted<ES>(p, t))
     return -1;
   if (cfg) {
@@ -370,7 +376,7 @@ template <int ES> static int launch_few_rows(const GemmParams *pp, hipStream_t s
   }
   if (dry)
     return 0;
-  const dim3 grid((unsigned)((t.blocks + 7) / 8 * 8), (unsigned)nbatch), block(64 * t.waves);
+  const dim3 grid((unsigned)((t.blocks * nbatch + 7) / 8 * 8)), block(64 * t.waves);
 #define GCMI_FEW_LAUNCH(TB, MT, NT, W, D)                                                                                \
   if (t.mt == MT && t.nt == NT)                                                                                           \
     hipLaunchKernelGGL((gemm_few_rows_kernel<ES, TB, MT, NT, W, D>), grid, block, 0, stream, p);

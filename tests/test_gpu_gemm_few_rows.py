@@ -41,8 +41,7 @@ def test_bf16_exact_on_integers(gc, dev, M, N, K, trans_b):
 
 @pytest.mark.parametrize("M,N,K", [(3, 1712, 2736), (32, 2048, 1016), (64, 8208, 328), (20, 17000, 232)])
 def test_bf16_rounding_points_and_layouts(gc, dev, M, N, K):
-    """Bias, activation and residual against float64 rounded where a bf16 graph rounds; [N,K] and [K,N] weights, and a batch
-    of such matrices, give the same bits."""
+    """Bias, activation and residual against float64 rounded where a bf16 graph rounds; [N,K] and [K,N] weights give the same bits."""
     g = torch.Generator(device=dev).manual_seed(N + K)
     A = torch.randn(M, K, device=dev, generator=g).to(torch.bfloat16)
     W = (torch.randn(K, N, device=dev, generator=g) * 0.05).to(torch.bfloat16)
@@ -60,9 +59,21 @@ def test_bf16_rounding_points_and_layouts(gc, dev, M, N, K):
     # K + 1 additions of exact products, each rounded once; the sigmoid's slope is at most a quarter and its own error 1e-6
     tol = 0.25 * (K + 1) * 2.0 ** -24 * (A.double().abs() @ W.double().abs() + bias.double().abs()) + 1e-6
     assert ((f32.double() - torch.sigmoid(acc + bias.double())).abs() <= tol).all()
-    batch = gc.gemm_batched(torch.stack([A, -A, A]), W, bias=bias, act="relu")
-    for i, a in enumerate((A, -A, A)):
-        assert torch.equal(batch[i], gc.gemm_bf16(a, W, bias, "relu"))
+
+
+@pytest.mark.parametrize("nb,M,N,K", [(3, 3, 1712, 2736), (84, 46, 176, 960), (7, 1, 96, 1064), (300, 20, 24, 144), (9, 64, 520, 328)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_bf16_batches_exact_on_integers(gc, dev, nb, M, N, K, trans_b):
+    """Matrices of one and several tiles, whole and cut, their workgroups in one run over the XCDs; one B for all, or each its own."""
+    g = torch.Generator(device=dev).manual_seed(nb + N)
+    A, W = _ints((nb, M, K), -3, 4, dev, g, torch.bfloat16), _ints((nb, K, N), -3, 4, dev, g, torch.bfloat16)
+    guard = torch.full((nb * M * N + 64,), 7.0, device=dev, dtype=torch.bfloat16)
+    out = guard[32:32 + nb * M * N].view(nb, M, N)
+    for B in (W, W[0]):
+        gc.gemm_batched(A, (B.transpose(-2, -1) if trans_b else B).contiguous(), trans_b, out=out)
+        want = torch.stack([A[i].float() @ (B[i] if B.dim() == 3 else B).float() for i in range(nb)])
+        assert torch.equal(out, want.to(torch.bfloat16))
+        assert (guard[:32] == 7.0).all() and (guard[-32:] == 7.0).all()
 
 
 def test_bf16_special_values(gc, dev):
