@@ -7,11 +7,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("Sq,Sk", [(128, 64), (130, 129), (200, 384), (384, 384), (256, 385), (385, 385)])
+@pytest.mark.parametrize("H,Sq,Sk", [(3, 128, 64), (3, 130, 129), (3, 200, 256), (3, 256, 256), (3, 256, 257), (3, 385, 385),
+                                     (128, 128, 128), (129, 128, 128), (32, 256, 256), (33, 200, 256)])
 @pytest.mark.parametrize("kind", ["causal", "zero", "tiles", "values"])
-def test_the_bits_of_the_classified_call(gc, dev, D, Sq, Sk, kind):
-    g = torch.Generator(device=dev).manual_seed(Sq + Sk)
-    q, k, v = (torch.randn(2, 3, s, D, device=dev, generator=g).bfloat16() for s in (Sq, Sk, Sk))
+def test_the_bits_of_the_classified_call(gc, dev, D, H, Sq, Sk, kind):
+    g = torch.Generator(device=dev).manual_seed(H + Sq + Sk)
+    q, k, v = (torch.randn(2, H, s, D, device=dev, generator=g).bfloat16() for s in (Sq, Sk, Sk))
     mask = torch.zeros(Sq, Sk, device=dev)
     if kind == "causal":
         mask = torch.triu(torch.full((Sq, Sk), float("-inf"), device=dev), diagonal=1 + max(0, Sk - Sq))
