@@ -1,6 +1,7 @@
-// bf16 x bf16 -> f32 GEMMs: the 256x256 MFMA tile kernels (gemm_tile256.hpp) and the streaming kernels for a short
-// A against [N,K] weights (gemm_rows32.hpp: up to 32 rows; gemm_skinny.hpp: up to 64 rows where a caller's slice
-// count asks for it, and the shapes the former does not take).
+// bf16 x bf16 -> f32 GEMMs: the MFMA tile kernels (gemm_tile256.hpp, gemm_tile128.hpp) and those for a short A:
+// gemm_rows32.hpp streams wide weights past up to 128 rows, gemm_few_rows.hpp takes up to 256 rows in one launch where a
+// round of its tiles holds them, gemm_skinny.hpp [N,K] weights where a caller's slice count asks for it and the shapes
+// the others do not take.
 #include "gemm_rows32.hpp"
 #include "gemm_skinny.hpp"
 

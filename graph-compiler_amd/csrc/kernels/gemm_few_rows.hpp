@@ -1,5 +1,6 @@
-// GEMMs of few rows of A (up to 256; 2048 of 8 bits) against weights that are no stream worth slicing: bf16 x bf16 with weights stored
-// [K,N] or [N,K], and 8-bit x s8 with weights stored [K,N].  C[M,N] = epilogue(A . W) in ONE launch.
+// GEMMs of few rows of A (up to 256; 2048 of 8 bits) against weights that are no stream worth slicing: bf16 x bf16 with weights
+// stored [K,N] or [N,K], and 8-bit x s8 with weights stored [K,N], alone or in a strided batch.  C[M,N] = epilogue(A . W) in
+// ONE launch.
 // What bounds such a call is the way launch -> loads -> sums -> store, once: the tile kernels' workgroup walks all of K
 // through one ring behind barriers (a 256 x 256 tile takes 60 us for 2 x 5456, K 3264, on 22 compute units), and K slices
 // over workgroups cost a second launch.  Here K is cut over the waves of a workgroup:
@@ -14,8 +15,8 @@
 //   * rows of 128 bytes (A, [N,K] weights) lie at chunk ^ row % 8; k-rows of [K,N] weights are read through the transposing
 //     LDS loads, at a chunk that spreads them over the banks.
 // The columns' bias, scale and column sums are fetched before the loop by the wave that finishes them.
-// The k that a wave owns and the order of the sums depend on M and N only: both layouts of the weights, and a matrix alone
-// or in a batch, give the same bits.
+// The k that a wave owns and the order of the sums depend on M, N and the size of the batch only: both layouts of the weights
+// give the same bits.
 // Measured, us per call, graph-replayed over 64 MB of weights: bf16 [N,K] 3 x 1712, K 2736 48 -> 6; 19 x 1648, K 3592 63.4 ->
 // 7.7; 13 x 1792, K 1856 8.4 (two launches) -> 5.0; [K,N] 10 x 320, K 3200 53 -> 8.5; 8-bit 10 x 512, K 3776 36 -> 7.7; 32 x
 // 11008, K 4096 20.0 -> 12.5 (3.7 TB/s of weights).

@@ -1822,8 +1822,9 @@ static inline double gcmi_us_per_group_256(double load) { // one workgroup per c
 }
 // Taller tiles of 128 columns (one workgroup per compute unit): fewer fragment reads per product than 128 rows, so where 128
 // rows make more than a round and 192 or 256 do not, they are ahead (64 random such sizes: 1.14 times on the average, at most
-// 1.5; 8-bit ones with a short K down to 0.93).  128 / 192 / 256 rows in one pass, us: 1237 x 4096, K 1376 29.3 / 22.5 / 27.5; 305 x 11008, K 4096 69.5 / 56.3 / 63.8; 483 x 11008 73.1 / - / 67.3; where 128 rows fit one
-// round they stay: 1000 x 4096, K 4096 38.6 / 47.8 / 59.4.
+// 1.5; 8-bit ones with a short K down to 0.93).  128 / 192 / 256 rows in one pass, us: 1237 x 4096, K 1376 29.3 / 22.5 / 27.5;
+// 305 x 11008, K 4096 69.5 / 56.3 / 63.8; 483 x 11008 73.1 / - / 67.3; where 128 rows fit one round they stay: 1000 x 4096,
+// K 4096 38.6 / 47.8 / 59.4.
 static inline double gcmi_us_per_group_tall(int rows) { return rows == 192 ? 1.5 : 1.85; }
 static inline double gcmi_us_fixed_tall(int rows, int es) { return (rows == 192 ? 5.0 : 6.0) + (es == 1 ? 1.0 : 0.0); } // (8-bit: the longer epilogue, alone on its unit)
 // A K past 8192 costs 128 rows more per group (1.39 us at K 11008: 1000 x 4096 123.6 us, 112.8 as two slices of 256 rows;
@@ -1928,7 +1929,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
       splits = p.cfg_split_k < groups ? p.cfg_split_k : groups;
       plan = p.M > 128 && groups % splits == 0 ? PLAN_SLICES_TILE256 : PLAN_SLICES_SHORT_A;
     }
-  } else if (aligned && nblk * nbatch < n_cu) { // (8-bit operands: the small tile in one pass is the only alternative)
+  } else if (aligned && nblk * nbatch < n_cu) { // (8-bit operands: smaller tiles in one pass are the only alternative here)
     const double mn = (double)p.M * (double)p.N / 1048576.0;
     const double w256 = (double)(nblk * nbatch) / n_cu, w128 = (double)(nblk128 * nbatch) / n_cu;
     double best = GCMI_US_FIXED_256 + gcmi_us_per_group_256(w256) * groups; // one pass, less than one round
