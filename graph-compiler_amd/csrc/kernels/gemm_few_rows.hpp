@@ -324,13 +324,19 @@ static FewRowsTile few_rows_tile(int64_t M, int64_t N, int64_t nbatch) {
 //   * more rows while one round of workgroups, or two of small ones with 8-bit operands, holds them (rounds * (mt + nt)): 83 x
 //     768, K 3136 12.0 / 8.5; 8-bit 83 x 768, K 3136 18.8 / 8.5; 80 x 10384, K 1072 13.3 / 12.1; past that 128 x 128 tiles
 //     re-read the operands less often (8-bit 234 x 10816, K 3584 23.5 / 31.8; bf16 150 x 5736, K 512 8.9 / 10.8).
+//     The largest tiles with a bf16 K of 256 or less, or of up to four whole groups, leave a wave two stages at most: 177 x 3328,
+//     K 256 6.8 / 7.8; 112 x 7072, K 384 8.1 / 8.8; 10 matrices of 189 x 448, K 256 6.4 / 7.6; with a longer K or a tail 92
+//     random sizes 1.0 to 1.3 times (96 x 7032, K 616 12.5 / 10.0).
 //   * 8-bit operands, for which the tile kernels have no K slices, up to 2048 rows while one round holds them: 45 random sizes
 //     of 257 to 2000 rows 1.75 times on the average (679 x 608, K 3568 23.6 / 11.1; 1328 x 768, K 976 11.0 / 8.1).
 //   * a K of 136 bf16 or less stays with the tile kernels, as do more than 128 bf16 rows over a K with an incomplete group
 //     and just 32 rows over 2 Mi weights and more: calls whose kernel, or whose workspace, is part of what the tests hold
 //     fast.
 template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRowsTile &t) {
-  if (p.K * ES <= 272 || (p.M >= 32 && t.rounds * (t.mt + t.nt) > (ES == 2 ? 8 : 12)))
+  const int64_t cost = t.rounds * (t.mt + t.nt);
+  if (p.K * ES <= 272 || (p.M >= 32 && cost > (ES == 2 ? 8 : 12)))
+    return false;
+  if (ES == 2 && p.M >= 32 && cost > 6 && (p.K <= 256 || (p.K <= 512 && p.K % 128 == 0)))
     return false;
   if (p.M > 256) // 8-bit operands
     return t.rounds == 1 && p.N >= 512 && p.K <= 4096;
