@@ -8,7 +8,7 @@ import pytest
     (31, 4096, 4096, 4, 32, 64), (31, 1000, 136, 2, 256, 256),          # a stream of weights; a short K
     (46, 192, 2792, 7, 16, 16), (62, 1208, 3432, 7, 32, 16), (64, 4096, 1000, 7, 32, 32), (64, 4096, 4072, 7, 32, 32),
     (32, 4096, 1376, 3, 128, 128), (32, 2048, 1016, 7, 16, 16), (33, 2048, 1024, 7, 16, 32), (128, 1288, 200, 7, 32, 32), (129, 1024, 4072, 3, 128, 128), (256, 1024, 512, 7, 32, 32),
-    (257, 1024, 512, 5, 128, 128), (64, 8208, 328, 7, 64, 64), (64, 8208, 256, 5, 128, 128), (64, 7000, 512, 5, 128, 128), (64, 8208, 520, 7, 64, 64)])
+    (257, 1024, 512, 5, 128, 128), (64, 8208, 328, 7, 64, 64), (64, 8208, 256, 5, 128, 128), (96, 6000, 512, 5, 128, 128), (64, 8208, 520, 7, 64, 64)])
 def test_bf16(gc, M, N, K, kernel, bm, bn):
     for tb in (False, True):
         c = gc.tile_config(M, N, K, trans_b=tb)[0]
