@@ -23,6 +23,8 @@
 #include <type_traits>
 #include "gemm_params.h"
 
+#define GCMI_GLB __attribute__((address_space(1)))
+
 namespace gcmi {
 
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4))); // 16 bytes from any 4-byte aligned address
@@ -293,10 +295,10 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(F32GemmParams p) {
 // Small problems: what counts is the chain launch -> loads -> sums -> store.  A workgroup owns one 16 x 16 tile, its
 // four waves take every fourth 16-deep step of K straight from memory into v_mfma_f32_16x16x4_f32 operands (lane l:
 // row/column l % 16, and k = 4 * (l / 16) .. + 3 of the step as four operand values), up to eight steps in flight per wave,
-// no LDS and no barrier until the four partial sums are added.  128 x 512 x 256 (128 workgroups) in 7.2 us per call (10.6 as
-// 16 x 16 tiles of vector FMAs over LDS slices of 32 k with a barrier each).  Kernel alone: 154 x 737, K 1872 16.7 us, 1000 x
-// 64, K 3000 13.2 (18.2 and 15.0 when a wave waited for eight steps at a time and then took the rest of K step by step);
-// sixteen steps in flight are the slower choice where workgroups share a compute unit (18.3, 13.6).
+// no LDS and no barrier until the four partial sums are added.  Kernel alone, us: 128 x 256, K 512 (128 workgroups) 4.15, 532 x
+// 492, K 1068 17.0, 154 x 737, K 1872 16.0, 1000 x 64, K 3000 12.6 (4.31, 20.0, 18.1 and 15.1 when a wave waited for eight steps
+// at a time and then took the rest of K step by step; 4.50, 20.7, 16.6 and 13.3 when all but its first step's loads were flat
+// ones, each wait for all of them); sixteen steps in flight are the slower choice where workgroups share a compute unit.
 static constexpr int64_t F32_SMALL_GRID = 1 << 23; // workgroups of a grid's first dimension, at most: 2^32 threads are too many
 // WIDE: a lane's place in a step may lie more than 2^31 bytes behind the step's first element; else it is a 32-bit offset on
 // a scalar address (with 64-bit addresses in the lanes every load in flight takes two registers more).
@@ -313,25 +315,34 @@ template <bool AKC, bool BKC, bool WIDE> __global__ __launch_bounds__(256) void 
   // rows past the last one read the last one (a tile past the last one: its own rows' clamp)
   const int64_t ma = m0 < p.M ? m0 : p.M - 1;
   const int ra = ma + l16 < p.M ? l16 : (int)(p.M - 1 - ma), rb = n0 + l16 < p.N ? l16 : (int)(p.N - 1 - n0);
+  // (global by their type: behind the pins below the compiler cannot tell, and waits for all flat loads together)
   typedef typename std::conditional<WIDE, int64_t, uint32_t>::type off_t;
-  const float *a = p.A + (int64_t)blockIdx.z * p.a_bs + ma * p.a_rs, *b = p.B + (int64_t)blockIdx.z * p.b_bs + n0 * p.b_cs;
-  const off_t la = 4 * ((off_t)ra * (off_t)p.a_rs + (off_t)(4 * lq) * (off_t)p.a_cs);
-  const off_t lb = 4 * ((off_t)rb * (off_t)p.b_cs + (off_t)(4 * lq) * (off_t)p.b_rs);
+  typedef GCMI_GLB const char *mem_t;
+  mem_t a = (mem_t)(p.A + (int64_t)blockIdx.z * p.a_bs + ma * p.a_rs), b = (mem_t)(p.B + (int64_t)blockIdx.z * p.b_bs + n0 * p.b_cs);
+  off_t la[AKC ? 1 : 4], lb[BKC ? 1 : 4]; // the lane's four k, or its four contiguous ones
+#pragma unroll
+  for (int c = 0; c < (AKC ? 1 : 4); c++)
+    la[c] = 4 * ((off_t)ra * (off_t)p.a_rs + (off_t)(4 * lq + c) * (off_t)(AKC ? 1 : p.a_cs));
+#pragma unroll
+  for (int c = 0; c < (BKC ? 1 : 4); c++)
+    lb[c] = 4 * ((off_t)rb * (off_t)p.b_cs + (off_t)(4 * lq + c) * (off_t)(BKC ? 1 : p.b_rs));
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  auto at = [](const float *s, off_t o) { return reinterpret_cast<const float *>(reinterpret_cast<const char *>(s) + o); };
-  auto load = [&](const float *s, off_t o, int64_t ks, bool contig) -> f32x4_t {
-    f32x4_t v;
-    if (contig)
-      v = *reinterpret_cast<const f32x4u_t *>(at(s, o));
+  auto load = [](mem_t s, const auto &o) -> f32x4_t {
+    if constexpr (sizeof(o) == sizeof(off_t))
+      return *(GCMI_GLB const f32x4u_t *)(s + o[0]);
     else
-      for (int c = 0; c < 4; c++)
-        v[c] = *at(s + c * ks, o);
-    return v;
+      return f32x4_t{*(GCMI_GLB const float *)(s + o[0]), *(GCMI_GLB const float *)(s + o[1]), *(GCMI_GLB const float *)(s + o[2]),
+                     *(GCMI_GLB const float *)(s + o[3])};
   };
-  auto load_end = [&](const float *s, off_t o, int64_t ks, int left) -> f32x4_t {
+  auto load_end = [](mem_t s, const auto &o, int left) -> f32x4_t {
     f32x4_t v;
-    for (int c = 0; c < 4; c++)
-      v[c] = c < left ? *at(s + c * ks, o) : 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      constexpr bool contig = sizeof(o) == sizeof(off_t);
+      v[c] = 0.0f;
+      if (c < left)
+        v[c] = *(GCMI_GLB const float *)(contig ? s + o[0] + 4 * c : s + o[contig ? 0 : c]);
+    }
     return v;
   };
   // This wave's whole steps are wave, wave + 4, ...; the step that K ends inside of, if it does, is behind some wave's last.
@@ -339,16 +350,25 @@ template <bool AKC, bool BKC, bool WIDE> __global__ __launch_bounds__(256) void 
   // round of loads.
   const int steps = (int)((p.K / 16 - wave + 3) >> 2), left = (int)(p.K & 15);
   const bool ends = left != 0 && (int)((p.K >> 4) & 3) == wave;
-  const int64_t a_step = 64 * p.a_cs, b_step = 64 * p.b_rs;
-  a += 16 * wave * p.a_cs, b += 16 * wave * p.b_rs;
+  const int64_t a_step = 256 * (AKC ? 1 : p.a_cs), b_step = 256 * (BKC ? 1 : p.b_rs);
+  a += 64 * wave * (AKC ? 1 : p.a_cs), b += 64 * wave * (BKC ? 1 : p.b_rs);
   f32x4_t va[2][U], vb[2][U], ea, eb;
-  // (the addresses are scalars that go from step to step: worked out ahead, as the compiler would, they fill the registers)
+  // (the addresses are scalars that go from step to step, the lane's offsets 32 bits beside them: worked out or widened ahead,
+  // as the compiler would, they fill the registers)
   auto step = [&](f32x4_t &x, f32x4_t &y) {
-    x = load(a, la, p.a_cs, AKC), y = load(b, lb, p.b_rs, BKC);
+    x = load(a, la), y = load(b, lb);
     a += a_step, b += b_step;
     asm volatile("" : "+s"(a), "+s"(b));
   };
   auto fetch = [&](int q) { // U steps
+    if constexpr (!WIDE) {
+#pragma unroll
+      for (auto &o : la)
+        asm volatile("" : "+v"(o));
+#pragma unroll
+      for (auto &o : lb)
+        asm volatile("" : "+v"(o));
+    }
 #pragma unroll
     for (int u = 0; u < U; u++)
       step(va[q][u], vb[q][u]);
@@ -371,8 +391,8 @@ template <bool AKC, bool BKC, bool WIDE> __global__ __launch_bounds__(256) void 
       if (u < n)
         step(va[q][u], vb[q][u]);
     if (ends) {
-      ea = load_end(a, la, p.a_cs, left - 4 * lq);
-      eb = load_end(b, lb, p.b_rs, left - 4 * lq);
+      ea = load_end(a, la, left - 4 * lq);
+      eb = load_end(b, lb, left - 4 * lq);
     }
   };
   auto products_rest = [&](int q, int n) {
