@@ -94,6 +94,7 @@ struct MhaParams {
   uint8_t *tile_class;
   int64_t tile_class_cap;
   int32_t skip_masked; // 1: tiles whose mask is all -inf are not computed (the result is the same)
+  int32_t find_hidden; // the launcher's: no classes, but the kernel looks for the tiles to leave out itself (few key blocks)
   // 1: tile_class already holds the classes of this mask (an earlier call's classification pass for the same mask,
   // shape and buffer): the pass is not launched again.  2: launch the pass only, no attention kernel.
   int32_t classes_mode;

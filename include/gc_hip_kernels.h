@@ -273,7 +273,9 @@ int gcmi_mha_fwd_bf16(const void *Q, const void *K, const void *V, const float *
 /*
  * The same with the block-skipping switch exposed.  When a mask is given, one
  * pass over it classifies every (32 query rows x 64 keys) tile as all 0, all
- * -inf or general; constant tiles cost no mask traffic in the main kernel.
+ * -inf or general; constant tiles cost no mask traffic in the main kernel.  (Up
+ * to two blocks of keys for few workgroups: the main kernel looks for the -inf
+ * tiles itself, in one launch.)
  * skip_masked != 0 (what gcmi_mha_fwd_bf16 uses): a block of 64 keys whose
  * tiles are -inf for all 128 query rows of a workgroup is not visited at all --
  * it contributes exp(-inf) = 0 to every sum, so the result is bit-identical.
