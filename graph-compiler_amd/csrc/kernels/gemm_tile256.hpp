@@ -1916,20 +1916,15 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
                                         (!p.residual || (p.c_bs * res_es) % 16 == 0));
   const bool t128_can = aligned && p.N % (16 / ES) == 0 && (ES == 2 ? p.out_dt != DT_S32 : !p.trans_b) && batch_ok;
   const bool slices_can = ES == 2 && fast_but_m && p.out_dt != DT_S32 && nbatch == 1; // the 256-wide kernels: whole column tiles
-  int rows128 = 128; // of the 128-column tile
-  int64_t nblk128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
   const int n_cu = gcmi_num_cus();
   const int groups = (int)((p.K + KGROUP - 1) / KGROUP);
-  int plan = PLAN_TILE256, splits = 1;
-  if (p.cfg_tile == 128) {
-    if (t128_can && nblk128 <= 0x7fffffff)
-      plan = PLAN_TILE128, c.from_attrs = 1;
-  } else if (p.cfg_tile == 256) {
-    if (slices_can && p.cfg_split_k > 1) {
-      splits = p.cfg_split_k < groups ? p.cfg_split_k : groups;
-      plan = p.M > 128 && groups % splits == 0 ? PLAN_SLICES_TILE256 : PLAN_SLICES_SHORT_A;
-    }
-  } else if (aligned && nblk * nbatch < n_cu) { // (8-bit operands: smaller tiles in one pass are the only alternative here)
+  struct Choice {
+    int plan, splits, rows128; // rows of the 128-column tile
+  };
+  // The choice by the estimates, with slices whose partial sums fit `cap` floats.
+  auto choose = [&](int64_t cap) -> Choice {
+    Choice ch{PLAN_TILE256, 1, 128};
+    const int64_t nblk128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
     const double mn = (double)p.M * (double)p.N / 1048576.0;
     const double w256 = (double)(nblk * nbatch) / n_cu, w128 = (double)(nblk128 * nbatch) / n_cu;
     double best = GCMI_US_FIXED_256 + gcmi_us_per_group_256(w256) * groups; // one pass, less than one round
@@ -1937,60 +1932,78 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     const double long_k = ES == 2 ? gcmi_us_per_group_128_long_k(p.K) : 0.0; // (of two workgroups on a compute unit, both)
     // taller tiles: at least two rows of them, in one round
     auto tall_tiles = [&](int rows) { return ((p.M + rows - 1) / rows) * ((p.N + 127) / 128) * nbatch; };
+    auto fits = [&](int s) { return (int64_t)s * p.M * p.N <= cap; };
     if (small_tile) {
       const double t = GCMI_US_FIXED_128 + (gcmi_us_per_group_128(w128) + (w128 <= 1.0 ? 1 : 2) * long_k) * groups * (double)((nblk128 * nbatch + 2 * n_cu - 1) / (2 * n_cu));
       if (t < best)
-        best = t, plan = PLAN_TILE128;
+        best = t, ch.plan = PLAN_TILE128;
       for (int rows = 192; rows <= 256; rows += 64) {
         const double u = gcmi_us_fixed_tall(rows, ES) + gcmi_us_per_group_tall(rows) * groups;
         if (p.M > rows && tall_tiles(rows) <= n_cu && u < best)
-          best = u, plan = PLAN_TILE128, rows128 = rows;
+          best = u, ch = {PLAN_TILE128, 1, rows};
       }
     }
     best *= GCMI_ONE_PASS_MARGIN;
     if (ES == 2 && nbatch == 1 && (small_tile || p.M > 128)) {
-      for (int s = 2; s <= groups; s++) {
+      for (int s = 2; s <= groups && fits(s); s++) {
         const double through_memory = GCMI_US_SECOND_PASS + GCMI_US_PER_SLICE_MOUT * s * mn;
         if (slices_can && p.M > 128 && groups % s == 0 && nblk * s <= n_cu) {
           const double t = GCMI_US_FIXED_256 + gcmi_us_per_group_256(w256 * s) * (groups / s) + through_memory;
           if (t < best)
-            best = t, plan = PLAN_SLICES_TILE256, splits = s;
+            best = t, ch = {PLAN_SLICES_TILE256, s, 128};
         }
         if (small_tile && nblk128 * s <= 2 * n_cu) {
           const double t = GCMI_US_FIXED_128 + (gcmi_us_per_group_128(w128 * s) + (nblk128 * s <= n_cu ? 1 : 2) * long_k) * ((groups + s - 1) / s) + through_memory;
           if (t < best)
-            best = t, plan = PLAN_SLICES_TILE128, splits = s, rows128 = 128;
+            best = t, ch = {PLAN_SLICES_TILE128, s, 128};
         }
       }
-      double tall_best = best * (splits > 1 ? GCMI_ONE_PASS_MARGIN : 1.0); // against other slices they too must be clearly ahead
-      for (int s = 2; small_tile && s <= groups; s++)
+      double tall_best = best * (ch.splits > 1 ? GCMI_ONE_PASS_MARGIN : 1.0); // against other slices they too must be clearly ahead
+      for (int s = 2; small_tile && s <= groups && fits(s); s++)
         for (int rows = 192; rows <= 256; rows += 64) {
           const double t = gcmi_us_fixed_tall(rows, ES) + gcmi_us_per_group_tall(rows) * ((groups + s - 1) / s) + GCMI_US_SECOND_PASS +
                            GCMI_US_PER_SLICE_MOUT * s * mn;
           if (p.M > rows && tall_tiles(rows) * s <= n_cu && t < tall_best)
-            tall_best = best = t, plan = PLAN_SLICES_TILE128, splits = s, rows128 = rows;
+            tall_best = best = t, ch = {PLAN_SLICES_TILE128, s, rows};
         }
     }
     if (nbatch == 1 && p.M <= 128 && slices_can && nblk * 2 <= n_cu) { // a short A: 1.35 (32 rows) to 2 us (128) per group
       const double per_group = 1.35 + 0.65 * (double)((p.M + 31) / 32 - 1) / 3.0;
       const int smax = n_cu / (int)nblk < groups ? n_cu / (int)nblk : groups;
-      for (int s = 2; s <= smax; s++) {
+      for (int s = 2; s <= smax && fits(s); s++) {
         const double t = 7.0 + per_group * ((groups + s - 1) / s) + GCMI_US_PER_SLICE_MOUT * s * mn;
         if (t < best)
-          best = t, plan = PLAN_SLICES_SHORT_A, splits = s;
+          best = t, ch = {PLAN_SLICES_SHORT_A, s, 128};
       }
     }
+    return ch;
+  };
+  Choice chosen{PLAN_TILE256, 1, 128};
+  if (p.cfg_tile == 128) {
+    if (t128_can && ((p.M + 127) / 128) * ((p.N + 127) / 128) <= 0x7fffffff)
+      chosen.plan = PLAN_TILE128, c.from_attrs = 1;
+  } else if (p.cfg_tile == 256) {
+    if (slices_can && p.cfg_split_k > 1) {
+      chosen.splits = p.cfg_split_k < groups ? p.cfg_split_k : groups;
+      chosen.plan = p.M > 128 && groups % chosen.splits == 0 ? PLAN_SLICES_TILE256 : PLAN_SLICES_SHORT_A;
+    }
+  } else if (aligned && nblk * nbatch < n_cu) { // (8-bit operands: smaller tiles in one pass are the only alternative here)
+    chosen = choose(INT64_MAX);
   }
-  nblk128 = ((p.M + rows128 - 1) / rows128) * ((p.N + 127) / 128);
-  if (splits > 1) {
+  if (chosen.splits > 1) {
     if (want)
-      *want = (int64_t)splits * p.M * p.N;
-    // less workspace than that: fewer slices, or none
-    while (splits > 1 && ((int64_t)splits * p.M * p.N > ws_cap || (plan == PLAN_SLICES_TILE256 && groups % splits != 0)))
-      splits--;
-    if (splits == 1)
-      plan = plan == PLAN_SLICES_TILE128 ? PLAN_TILE128 : PLAN_TILE256;
+      *want = (int64_t)chosen.splits * p.M * p.N;
+    // less workspace than that: what is best with what there is; of a caller's slices fewer, or none
+    if (p.cfg_tile == 0 && (int64_t)chosen.splits * p.M * p.N > ws_cap)
+      chosen = choose(ws_cap);
+    while (chosen.splits > 1 &&
+           ((int64_t)chosen.splits * p.M * p.N > ws_cap || (chosen.plan == PLAN_SLICES_TILE256 && groups % chosen.splits != 0)))
+      chosen.splits--;
+    if (chosen.splits == 1 && p.cfg_tile != 0)
+      chosen.plan = PLAN_TILE256;
   }
+  const int plan = chosen.plan, splits = chosen.splits, rows128 = chosen.rows128;
+  const int64_t nblk128 = ((p.M + rows128 - 1) / rows128) * ((p.N + 127) / 128);
   if (want && !cfg)
     return 0;
   if (splits > 1) {
