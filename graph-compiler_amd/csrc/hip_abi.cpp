@@ -390,7 +390,7 @@ int gemm_bf16_any(bool trans_b, const void *A, const void *B, void *C, int64_t M
     size_t sb = 0;
     if (gcmi_noalloc_scratch(&sp, &sb) != 0)
       return fail(ST_RUNTIME, "gemm_bf16_noalloc: the address of the static scratch array is not available");
-    if ((size_t)want * 4 > sb)
+    if ((size_t)want * 4 > sb && !optional)
       return fail(ST_INVALID,
                   "gemm_bf16_noalloc: %lld x %lld x %lld needs %lld bytes of scratch for its K slices, the static "
                   "buffer holds %zu; use gcmi_gemm_bf16 (library workspace) or gcmi_gemm_bf16_ws",

@@ -22,8 +22,8 @@ extern "C" int gcmi_launch_gemm_bf16(const gcmi::GemmParams *p, hipStream_t stre
 
 // Floats of workspace (GemmParams::partial) the launch above would use for this call: 0 when K is not sliced.
 // *optional: the call is one that has to run without as well (in one pass, the sums in another order): a K with an
-// incomplete ring group, which the tile kernels slice like any other K, but which no entry point may refuse under
-// stream capture, as it does a K of whole groups.
+// incomplete ring group, which the tile kernels slice like any other K, or a call that is sliced only since there are tiles of
+// more than 128 rows.  No entry point may refuse these under stream capture, as it does the others with a K of whole groups.
 extern "C" int64_t gcmi_launch_gemm_bf16_workspace(const gcmi::GemmParams *p, int *optional) {
   int64_t want = 0;
   *optional = 0;
@@ -33,8 +33,9 @@ extern "C" int64_t gcmi_launch_gemm_bf16_workspace(const gcmi::GemmParams *p, in
     return 0;
   if (gcmi::launch_skinny_nt(p, nullptr, &want) >= 0)
     return want;
-  gcmi::launch_tile256<2>(p, nullptr, &want);
-  *optional = p->K % (256 / 2) != 0;
+  bool one_pass_too = false;
+  gcmi::launch_tile256<2>(p, nullptr, &want, nullptr, &one_pass_too);
+  *optional = p->K % (256 / 2) != 0 || one_pass_too;
   return want;
 }
 

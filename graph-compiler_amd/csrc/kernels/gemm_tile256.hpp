@@ -1806,7 +1806,9 @@ extern "C" int gcmi_launch_tile128(const gcmi::GemmParams *p, int es, int rows, 
 namespace gcmi {
 
 // Host-side launch of the 256x256 tile kernels for one element size.
-// want != null: nothing is launched; *want receives the floats of workspace this call would use if it had them.
+// want != null: nothing is launched; *want receives the floats of workspace this call would use if it had them, *optional whether
+// it is one that the taller tiles brought to slices: without them it runs in one pass, so no entry point may refuse it for
+// want of a workspace.
 // cfg != null: receives what was (or would be) chosen.
 // Estimates behind the choice of tile and K slices for bf16 problems that do not fill the GPU with 256 x 256 tiles,
 // in microseconds, fitted to graph-replayed timings on a 256-CU board (load = workgroups / compute units).  One ring
@@ -1847,10 +1849,11 @@ static constexpr double GCMI_US_PER_SLICE_MOUT = 1.7;  // partial sums written a
 static constexpr double GCMI_ONE_PASS_MARGIN = 0.9;    // slices must win by this factor
 enum GemmPlan { PLAN_TILE256 = 0, PLAN_TILE128, PLAN_SLICES_SHORT_A, PLAN_SLICES_TILE256, PLAN_SLICES_TILE128 };
 template <int ES>
-static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *want = nullptr, GemmTileConfig *cfg = nullptr) {
+static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *want = nullptr, GemmTileConfig *cfg = nullptr,
+                          bool *optional = nullptr) {
   GemmParams p = *pp;
   if (want)
-    *want = 0;
+    *want = 0, *optional = false;
   const bool dry = want != nullptr || (cfg != nullptr && stream == (hipStream_t)-1);
   const int64_t ws_cap = want ? INT64_MAX : (p.partial ? p.partial_cap : 0);
   float *const ws = p.partial;
@@ -1921,15 +1924,16 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
   struct Choice {
     int plan, splits, rows128; // rows of the 128-column tile
   };
-  // The choice by the estimates, with slices whose partial sums fit `cap` floats.
-  auto choose = [&](int64_t cap) -> Choice {
+  // The choice by the estimates, with slices whose partial sums fit `cap` floats.  taller: the tiles of 192 and 256 rows, and what
+  // a long K costs those of 128, take part.
+  auto choose = [&](bool taller, int64_t cap) -> Choice {
     Choice ch{PLAN_TILE256, 1, 128};
     const int64_t nblk128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
     const double mn = (double)p.M * (double)p.N / 1048576.0;
     const double w256 = (double)(nblk * nbatch) / n_cu, w128 = (double)(nblk128 * nbatch) / n_cu;
     double best = GCMI_US_FIXED_256 + gcmi_us_per_group_256(w256) * groups; // one pass, less than one round
     const bool small_tile = p.M >= 32 && t128_can; // shorter: most of a 128-row tile would be padding
-    const double long_k = ES == 2 ? gcmi_us_per_group_128_long_k(p.K) : 0.0; // (of two workgroups on a compute unit, both)
+    const double long_k = ES == 2 && taller ? gcmi_us_per_group_128_long_k(p.K) : 0.0; // (of two workgroups on a compute unit, both)
     // taller tiles: at least two rows of them, in one round
     auto tall_tiles = [&](int rows) { return ((p.M + rows - 1) / rows) * ((p.N + 127) / 128) * nbatch; };
     auto fits = [&](int s) { return (int64_t)s * p.M * p.N <= cap; };
@@ -1937,7 +1941,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
       const double t = GCMI_US_FIXED_128 + (gcmi_us_per_group_128(w128) + (w128 <= 1.0 ? 1 : 2) * long_k) * groups * (double)((nblk128 * nbatch + 2 * n_cu - 1) / (2 * n_cu));
       if (t < best)
         best = t, ch.plan = PLAN_TILE128;
-      for (int rows = 192; rows <= 256; rows += 64) {
+      for (int rows = 192; taller && rows <= 256; rows += 64) {
         const double u = gcmi_us_fixed_tall(rows, ES) + gcmi_us_per_group_tall(rows) * groups;
         if (p.M > rows && tall_tiles(rows) <= n_cu && u < best)
           best = u, ch = {PLAN_TILE128, 1, rows};
@@ -1959,7 +1963,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
         }
       }
       double tall_best = best * (ch.splits > 1 ? GCMI_ONE_PASS_MARGIN : 1.0); // against other slices they too must be clearly ahead
-      for (int s = 2; small_tile && s <= groups && fits(s); s++)
+      for (int s = 2; taller && small_tile && s <= groups && fits(s); s++)
         for (int rows = 192; rows <= 256; rows += 64) {
           const double t = gcmi_us_fixed_tall(rows, ES) + gcmi_us_per_group_tall(rows) * ((groups + s - 1) / s) + GCMI_US_SECOND_PASS +
                            GCMI_US_PER_SLICE_MOUT * s * mn;
@@ -1988,14 +1992,16 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
       chosen.plan = p.M > 128 && groups % chosen.splits == 0 ? PLAN_SLICES_TILE256 : PLAN_SLICES_SHORT_A;
     }
   } else if (aligned && nblk * nbatch < n_cu) { // (8-bit operands: smaller tiles in one pass are the only alternative here)
-    chosen = choose(INT64_MAX);
+    chosen = choose(true, INT64_MAX);
+    if (want && chosen.splits > 1)
+      *optional = choose(false, INT64_MAX).splits == 1;
   }
   if (chosen.splits > 1) {
     if (want)
       *want = (int64_t)chosen.splits * p.M * p.N;
     // less workspace than that: what is best with what there is; of a caller's slices fewer, or none
     if (p.cfg_tile == 0 && (int64_t)chosen.splits * p.M * p.N > ws_cap)
-      chosen = choose(ws_cap);
+      chosen = choose(true, ws_cap);
     while (chosen.splits > 1 &&
            ((int64_t)chosen.splits * p.M * p.N > ws_cap || (chosen.plan == PLAN_SLICES_TILE256 && groups % chosen.splits != 0)))
       chosen.splits--;

@@ -19,10 +19,11 @@
  *     number of host threads.  A call whose stream is being captured gets none:
  *     masked attention of 128 queries or more and K-sliced GEMMs are then
  *     refused, but for GEMMs whose K is no multiple of 128 (with [N,K] weights
- *     and up to 64 rows: of 64), which run in one pass, and attention of fewer
- *     queries, which keeps the keys of a head in one workgroup.  These two also
- *     do without where memory cannot be had, and every kind does where the
- *     stream it would have to wait for is being captured.  Without, sums are
+ *     and up to 64 rows: of 64) or that are sliced only because of tiles of more
+ *     than 128 rows, which run in one pass, and attention of fewer queries,
+ *     which keeps the keys of a head in one workgroup.  These also do without
+ *     where memory cannot be had, and every kind does where the stream it would
+ *     have to wait for is being captured.  Without, sums are
  *     added in another order and a result may differ in its last bits from that
  *     of a call with the buffer;
  *   - *_ws entry points: a workspace the caller brings (size from the
@@ -203,11 +204,14 @@ int gcmi_gemm_tile_config_query(int a_dtype, int64_t M, int64_t N, int64_t K, in
  * gcmi_noalloc_scratch_bytes() = 32 MiB that every device the library runs on
  * holds until the process ends; the call allocates nothing and frees nothing.
  * A shape whose K slices need more than that (gcmi_gemm_bf16_workspace_bytes)
- * is refused with status 2 and a message; shapes that are not K-sliced need no
+ * is refused with status 2 and a message, unless it is one that runs in one pass
+ * under stream capture (see "Scratch memory"); shapes that are not K-sliced need no
  * scratch and are never refused, nor is a K that is no multiple of 128 (its
  * slices always fit).  Every call on a device shares that device's
  * array: calls that overlap in time on one device (different streams) race;
- * calls on one stream are safe.  Results equal gcmi_gemm_bf16's bit for bit.
+ * calls on one stream are safe.  Results equal gcmi_gemm_bf16's bit for bit
+ * (where the slices fit: a call that takes fewer than it could has its sums in
+ * another order).
  */
 size_t gcmi_noalloc_scratch_bytes(void);
 int gcmi_gemm_bf16_noalloc(const void *A, const void *B, void *C, int64_t M, int64_t N, int64_t K, int64_t lda,
