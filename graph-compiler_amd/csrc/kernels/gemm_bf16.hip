@@ -5,13 +5,37 @@
 #include "gemm_rows32.hpp"
 #include "gemm_skinny.hpp"
 
-extern "C" int gcmi_launch_few_rows(const gcmi::GemmParams *p, int es, hipStream_t stream, int dry, gcmi::GemmTileConfig *cfg); // gemm_few_rows.hip
+extern "C" int gcmi_launch_few_rows(const gcmi::GemmParams *p, int es, hipStream_t stream, int dry, gcmi::GemmTileConfig *cfg,
+                                    int slices); // gemm_few_rows.hip
+
+// Floats of workspace that the kernels behind the few-row one would use for this call; *optional: see the query below.
+static int64_t slices_want(const gcmi::GemmParams *p, bool *optional) {
+  int64_t want = 0;
+  *optional = false;
+  if (gcmi::launch_skinny_nt(p, nullptr, &want) >= 0)
+    return want;
+  gcmi::launch_tile256<2>(p, nullptr, &want, nullptr, optional);
+  *optional = *optional || p->K % (256 / 2) != 0;
+  return want;
+}
+
+// A call of few rows.  One with a long K is left to K slices where another kernel has them and two of them at least fit the
+// workspace.
+static int launch_few(const gcmi::GemmParams *p, hipStream_t stream, bool dry, gcmi::GemmTileConfig *cfg) {
+  const int rc = gcmi_launch_few_rows(p, 2, stream, dry, cfg, 1);
+  if (rc >= 0 || gcmi_launch_few_rows(p, 2, nullptr, 1, nullptr, 0) < 0)
+    return rc;
+  bool optional;
+  if (p->partial && p->partial_cap >= 2 * p->M * p->N && slices_want(p, &optional) > 0)
+    return -1;
+  return gcmi_launch_few_rows(p, 2, stream, dry, cfg, 0);
+}
 
 extern "C" int gcmi_launch_gemm_bf16(const gcmi::GemmParams *p, hipStream_t stream) {
   int rc = gcmi::launch_rows32(p, stream);
   if (rc >= 0)
     return rc;
-  rc = gcmi_launch_few_rows(p, 2, stream, 0, nullptr);
+  rc = launch_few(p, stream, false, nullptr);
   if (rc >= 0)
     return rc;
   rc = gcmi::launch_skinny_nt(p, stream);
@@ -22,20 +46,19 @@ extern "C" int gcmi_launch_gemm_bf16(const gcmi::GemmParams *p, hipStream_t stre
 
 // Floats of workspace (GemmParams::partial) the launch above would use for this call: 0 when K is not sliced.
 // *optional: the call is one that has to run without as well (in one pass, the sums in another order): a K with an
-// incomplete ring group, which the tile kernels slice like any other K, or a call that is sliced only since there are tiles of
-// more than 128 rows.  No entry point may refuse these under stream capture, as it does the others with a K of whole groups.
+// incomplete ring group, which the tile kernels slice like any other K, a call of few rows whose slices are only the faster
+// way, or one that is sliced only since there are tiles of more than 128 rows.  No entry point may refuse these under stream
+// capture, as it does the others with a K of whole groups.
 extern "C" int64_t gcmi_launch_gemm_bf16_workspace(const gcmi::GemmParams *p, int *optional) {
   int64_t want = 0;
   *optional = 0;
   if (gcmi::launch_rows32(p, nullptr, &want) >= 0)
     return want;
-  if (gcmi_launch_few_rows(p, 2, nullptr, 1, nullptr) >= 0)
+  if (gcmi_launch_few_rows(p, 2, nullptr, 1, nullptr, 1) >= 0)
     return 0;
-  if (gcmi::launch_skinny_nt(p, nullptr, &want) >= 0)
-    return want;
   bool one_pass_too = false;
-  gcmi::launch_tile256<2>(p, nullptr, &want, nullptr, &one_pass_too);
-  *optional = p->K % (256 / 2) != 0 || one_pass_too;
+  want = slices_want(p, &one_pass_too);
+  *optional = one_pass_too || gcmi_launch_few_rows(p, 2, nullptr, 1, nullptr, 0) >= 0;
   return want;
 }
 
@@ -43,7 +66,7 @@ extern "C" int64_t gcmi_launch_gemm_bf16_workspace(const gcmi::GemmParams *p, in
 extern "C" int gcmi_launch_gemm_bf16_config(const gcmi::GemmParams *p, gcmi::GemmTileConfig *cfg) {
   if (gcmi::launch_rows32(p, (hipStream_t)-1, nullptr, cfg) >= 0)
     return 0;
-  if (gcmi_launch_few_rows(p, 2, nullptr, 1, cfg) >= 0)
+  if (launch_few(p, nullptr, true, cfg) >= 0)
     return 0;
   if (gcmi::launch_skinny_nt(p, (hipStream_t)-1, nullptr, cfg) >= 0)
     return 0;

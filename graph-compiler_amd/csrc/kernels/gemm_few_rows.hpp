@@ -348,8 +348,33 @@ template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRows
   return groups ? p.N * p.K < (int64_t)1 << 22 : p.M <= 128;
 }
 
-// Takes the call when the shape is this kernel's (returns -1 otherwise: the other kernels handle it).
-template <int ES> static int launch_few_rows(const GemmParams *pp, hipStream_t stream, bool dry, GemmTileConfig *cfg = nullptr) {
+// A wave walks its share of K alone, a stage in about 0.85 us ([K,N]; 0.4 where N is no more than 40) or 0.35 ([N,K]; half as much
+// again with rows that are no whole lines), up to 1.3 on the larger tiles, while K slices over workgroups take their 10 to 15 us
+// and little more for a longer K.  So past a K they win, where another kernel has them.  Measured over 32 to 256 rows of 16 to
+// 8192 columns (530 random sizes), by the sixteenths of rows and columns of a tile, us, slices / this:
+//   [K,N] 2   112 x 528, K 5824 14.6 / 12.5   32 x 168, K 5968 12.8 / 14.2   169 x 168, K 7776 13.7 / 16.0  48 x 112, K 188208 37 / 302
+//         2, few columns   157 x 40, K 8704 14.4 / 11.9   143 x 16, K 13696 17.4 / 11.8   46 x 24, K 26112 25 / 23   256 x 32, K 24448 18 / 25
+//         3   48 x 2632, K 4840 16.2 / 14.9   214 x 408, K 5280 14.4 / 15.1     4   195 x 1088, K 5560 16.5 / 16.2
+//         6   250 x 1088, K 3840 16.6 / 14.7   96 x 3848, K 4792 19.7 / 22.2    8   242 x 2704, K 5376 24.6 / 24.7   202 x 3000, K 6968 26 / 32
+//   [N,K] 2   169 x 128, K 15872 17.2 / 15.4  63 x 448, K 19680 17.4 / 19.9   64 x 64, K 191744 35 / 125
+//         2, few columns   56 x 88, K 20992 23.5 / 16.7   127 x 64, K 23960 18.7 / 25.2
+//         3   121 x 640, K 13632 17.9 / 17.3   197 x 496, K 16808 22.1 / 26.9   4   160 x 824, K 10624 19.5 / 18.4   190 x 1112, K 21464 33 / 43
+//         6   253 x 1600, K 4224 17.2 / 13.6   96 x 3200, K 5704 19.8 / 23.4    8   139 x 4488, K 8704 32.4 / 29.6   200 x 2496, K 11648 30 / 36
+//   up to 32 rows against gemm_skinny.hpp ([N,K])   19 x 224, K 10048 9.5 / 8.9   15 x 320, K 13952 10.2 / 12.6
+//   and against slices of 256 columns ([K,N])       26 x 512, K 6016 13.6 / 12.8   4 x 256, K 9600 14.2 / 18.0
+static bool few_rows_slices_ahead(const GemmParams &p, const FewRowsTile &t) {
+  const int64_t cost = t.rounds * (t.mt + t.nt);
+  if (p.trans_b) {
+    const int64_t k = cost <= 2 ? (p.N <= 128 ? 23040 : 16384) : cost == 3 ? 13312 : cost == 4 ? 10240 : cost <= 6 ? 5120 : 8704;
+    return p.K > (p.M <= 32 && k > 10240 ? 10240 : k);
+  }
+  const int64_t k = cost <= 2 ? (p.N <= 24 ? 24576 : p.N <= 40 ? 16384 : 5888) : cost == 3 ? 5120 : cost == 4 ? 6144 : cost <= 6 ? 4608 : 5376;
+  return p.K > (p.M < 32 && k < 6144 ? 6144 : k);
+}
+
+// Takes the call when the shape is this kernel's (returns -1 otherwise: the other kernels handle it).  slices: another kernel cuts
+// this call's K over workgroups, and the workspace for it is there.
+template <int ES> static int launch_few_rows(const GemmParams *pp, hipStream_t stream, bool dry, GemmTileConfig *cfg, bool slices) {
   GemmParams p = *pp;
   const int out_es = p.out_dt == DT_BF16 ? 2 : 4, res_es = p.residual_dt == DT_BF16 ? 2 : 4;
   auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
@@ -372,7 +397,7 @@ template <int ES> static int launch_few_rows(const GemmParams *pp, hipStream_t s
   const FewRowsTile t = few_rows_tile(p.M, p.N, nbatch);
   if (t.blocks * nbatch > (int64_t)1 << 22) // (a grid has less than 2^32 threads)
     return -1;
-  if (!few_rows_wanted<ES>(p, t))
+  if (!few_rows_wanted<ES>(p, t) || (slices && few_rows_slices_ahead(p, t)))
     return -1;
   if (cfg) {
     GemmTileConfig c{};

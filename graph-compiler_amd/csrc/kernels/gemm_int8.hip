@@ -79,15 +79,15 @@ __global__ __launch_bounds__(256) void colsum_s8_wide_kernel(const int8_t *W, in
 
 using namespace gcmi;
 
-extern "C" int gcmi_launch_few_rows(const GemmParams *p, int es, hipStream_t stream, int dry, GemmTileConfig *cfg); // gemm_few_rows.hip
+extern "C" int gcmi_launch_few_rows(const GemmParams *p, int es, hipStream_t stream, int dry, GemmTileConfig *cfg, int slices); // gemm_few_rows.hip
 
 extern "C" int gcmi_launch_gemm_int8(const GemmParams *p, hipStream_t stream) {
-  const int rc = gcmi_launch_few_rows(p, 1, stream, 0, nullptr);
+  const int rc = gcmi_launch_few_rows(p, 1, stream, 0, nullptr, 0);
   return rc >= 0 ? rc : launch_tile256<1>(p, stream);
 }
 
 extern "C" int gcmi_launch_gemm_int8_config(const GemmParams *p, GemmTileConfig *cfg) {
-  if (gcmi_launch_few_rows(p, 1, nullptr, 1, cfg) >= 0)
+  if (gcmi_launch_few_rows(p, 1, nullptr, 1, cfg, 0) >= 0)
     return 0;
   return launch_tile256<1>(p, (hipStream_t)-1, nullptr, cfg);
 }

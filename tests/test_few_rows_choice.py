@@ -17,6 +17,22 @@ def test_bf16(gc, M, N, K, kernel, bm, bn):
             assert c.split_k == 1 and gc.lib().gcmi_gemm_bf16_workspace_bytes(M, N, K, int(tb)) == 0
 
 
+@pytest.mark.parametrize("trans_b,M,N,K,kernel", [
+    (0, 176, 192, 5888, 7), (0, 176, 192, 6016, 3), (0, 157, 40, 16384, 7), (0, 157, 40, 16512, 3), (0, 157, 24, 24576, 7), (0, 157, 24, 24704, 3),   # 16 x 16 tiles; few columns
+    (0, 48, 2632, 5112, 7), (0, 48, 2632, 5128, 3), (0, 50, 2056, 6136, 7), (0, 50, 2056, 6152, 3),     # larger ones
+    (0, 96, 3848, 4600, 7), (0, 96, 3848, 4616, 3), (0, 97, 6000, 5368, 7), (0, 97, 6000, 5384, 3),
+    (0, 26, 512, 6144, 7), (0, 26, 512, 6272, 3), (0, 16, 96, 65408, 7), (0, 1, 16, 1000000, 7),        # below 32 rows; nobody cuts K
+    (1, 192, 136, 16384, 7), (1, 192, 136, 16512, 3), (1, 192, 128, 23040, 7), (1, 192, 128, 23168, 3), (1, 121, 640, 13304, 7), (1, 121, 640, 13320, 3),
+    (1, 128, 1504, 10232, 7), (1, 128, 1504, 10248, 3), (1, 128, 3200, 5112, 7), (1, 128, 3200, 5128, 3),
+    (1, 19, 224, 10240, 7), (1, 19, 224, 10304, 4), (1, 19, 216, 40000, 7), (1, 100, 6000, 8696, 7), (1, 100, 6000, 8712, 3),
+    (0, 64, 64, 65408, 3), (1, 64, 64, 65408, 3), (0, 128, 64, 65408, 3), (0, 64, 512, 40008, 3), (1, 64, 512, 40008, 3)])
+def test_a_long_k_is_left_to_slices(gc, trans_b, M, N, K, kernel):
+    """Where another kernel cuts K over workgroups; it then has the workspace that it wants."""
+    c = gc.tile_config(M, N, K, trans_b=bool(trans_b))[0]
+    assert c.kernel == kernel and (c.split_k > 1) == (kernel != 7)
+    assert (gc.lib().gcmi_gemm_bf16_workspace_bytes(M, N, K, trans_b) > 0) == (kernel != 7)
+
+
 @pytest.mark.parametrize("M,N,K,kernel", [(1, 512, 512, 7), (32, 11008, 4096, 7), (256, 896, 2112, 7), (234, 10816, 3584, 5), (257, 3264, 4096, 7), (257, 3280, 4096, 5),
                                           (2048, 512, 528, 7), (2049, 512, 528, 5), (1024, 1024, 4096, 7), (1024, 1024, 4112, 5), (700, 496, 1024, 5),
                                           (300, 272, 512, 5), (32, 512, 272, 5), (20, 512, 520, 0)])

@@ -129,3 +129,34 @@ def test_int8_special_scales(gc, dev):
     assert (out[:, 0] == float("inf")).all() and out[:, 1].isnan().all() and out[:, 2].isnan().all()
     assert (out[:, 20] == float("inf")).all() and (out[:, 3:20] == 3 * K).all()
     assert (out[:, 1].view(torch.int16) == 0x7FC0).all() and (out[:, 2].view(torch.int16) == 0x7FC0).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 64, 65408), (33, 200, 20008), (19, 224, 20032), (7, 256, 16384), (5, 24, 50000)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_a_long_k_with_and_without_the_workspace(gc, dev, M, N, K, trans_b):
+    """K slices where another kernel has them and the buffer can be had; in one launch under capture and without a workspace."""
+    import ctypes as C
+    g = torch.Generator(device=dev).manual_seed(K)
+    A, W = _ints((M, K), -2, 3, dev, g, torch.bfloat16), _ints((K, N), -2, 3, dev, g, torch.bfloat16)
+    want = A.double() @ W.double()
+    B, f = (W.t().contiguous(), gc.gemm_bf16_nt) if trans_b else (W, gc.gemm_bf16)
+    assert torch.equal(f(A, B, out_dtype=gc.F32).double(), want)
+    out, none = torch.zeros(M, N, device=dev), torch.zeros(M, N, device=dev)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        graph = torch.cuda.CUDAGraph()
+        graph.capture_begin()
+        f(A, B, out_dtype=gc.F32, out=out)
+        graph.capture_end()
+    for _ in range(3):
+        out.zero_()
+        f(-A, B, out_dtype=gc.F32)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.double(), want)
+    gc.check(gc.lib().gcmi_gemm_bf16_ws(A.data_ptr(), B.data_ptr(), none.data_ptr(), 1, M, N, K, K, B.shape[1], N, 0, 0, 0, int(trans_b), None,
+                                        gc.BF16, 0, None, 0, gc.BF16, gc.F32, None, 0, None,
+                                        C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert torch.equal(none.double(), want)
