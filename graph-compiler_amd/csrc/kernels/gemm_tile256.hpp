@@ -1829,8 +1829,15 @@ static inline double gcmi_us_per_group_256(double load) { // one workgroup per c
 // K 4096 38.6 / 47.8 / 59.4.
 static inline double gcmi_us_per_group_tall(int rows) { return rows == 192 ? 1.5 : 1.85; }
 static inline double gcmi_us_fixed_tall(int rows, int es) { return (rows == 192 ? 5.0 : 6.0) + (es == 1 ? 1.0 : 0.0); } // (8-bit: the longer epilogue, alone on its unit)
-// A K past 8192 costs 128 rows more per group (1.39 us at K 11008: 1000 x 4096 123.6 us, 112.8 as two slices of 256 rows;
-// 483 x 4096 74.8 in two slices, 65.5 in four of 256 rows).
+// A long K beside wide weights costs 128 rows more per group than the estimate has, which was fitted to weights that the
+// last-level cache holds from call to call (256 MiB; 1.04 us at any K): from memory, as a model's weights come, a group takes
+// 1.38.  Up to a K of 8192 the choice is the same either way; past it taller tiles, which read them fewer times, are ahead.
+// 1000 x 4096 [N,K], one pass of 128 rows / two slices of 256, from memory (from the cache), us: K 6144 71.2 / 72.3 (57 / 68), 8192
+// 82.7 / 85.2 (68 / 83), 9728 107 / 102 (87 / 96), 11008 128 / 112 (105 / 106), 12288 139 / 122 (110 / 116), 14336 159 / 140, 16384 175 /
+// 159, 22016 249 / 214; [K,N] the two meet at 11008 (122 / 124) and 22016 has 234 / 219.  Random sizes of more than 256 rows and 512
+// columns or more, against the rules without this and without taller tiles: K 8200 to 24576 90 of them 1.13 times from the cache,
+// 1.15 from memory (0.87 to 1.6), K to 60000 24 of them 1.17 and 1.16.  Fewer rows or columns have weights or results so small that
+// it only made more slices of them: 26 sizes 0.95, down to 0.7.
 static inline double gcmi_us_per_group_128_long_k(int64_t K) {
   return K <= 8192 ? 0.0 : K >= 11008 ? 0.27 : 0.27 * (double)(K - 8192) / 2816.0;
 }
@@ -1933,7 +1940,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     const double w256 = (double)(nblk * nbatch) / n_cu, w128 = (double)(nblk128 * nbatch) / n_cu;
     double best = GCMI_US_FIXED_256 + gcmi_us_per_group_256(w256) * groups; // one pass, less than one round
     const bool small_tile = p.M >= 32 && t128_can; // shorter: most of a 128-row tile would be padding
-    const double long_k = ES == 2 && taller ? gcmi_us_per_group_128_long_k(p.K) : 0.0; // (of two workgroups on a compute unit, both)
+    const double long_k = ES == 2 && taller && p.M > 256 && p.N >= 512 ? gcmi_us_per_group_128_long_k(p.K) : 0.0; // (of two workgroups on a compute unit, both)
     // taller tiles: at least two rows of them, in one round
     auto tall_tiles = [&](int rows) { return ((p.M + rows - 1) / rows) * ((p.N + 127) / 128) * nbatch; };
     auto fits = [&](int s) { return (int64_t)s * p.M * p.N <= cap; };
