@@ -329,9 +329,12 @@ static FewRowsTile few_rows_tile(int64_t M, int64_t N, int64_t nbatch) {
 //     random sizes 1.0 to 1.3 times (96 x 7032, K 616 12.5 / 10.0).
 //   * 8-bit operands, for which the tile kernels have no K slices, up to 2048 rows while one round holds them: 45 random sizes
 //     of 257 to 2000 rows 1.75 times on the average (679 x 608, K 3568 23.6 / 11.1; 1328 x 768, K 976 11.0 / 8.1).
-//   * a K of 136 bf16 or less stays with the tile kernels, as do more than 128 bf16 rows over a K with an incomplete group
-//     and just 32 rows over 2 Mi weights and more: calls whose kernel, or whose workspace, is part of what the tests hold
-//     fast.
+//   * with a K that ends inside a group of 128 nothing streams, so these are taken whatever the weights' size, 32 rows (32 x 4096,
+//     K 1376 12.3 / 8.0, 32 x 6336, K 2136 14.4 / 10.4) and 129 to 256 (140 x 264, K 1048 9.8 / 5.5, 169 x 2400, K 1464 14.7 /
+//     10.0, 248 x 2656, K 776 13.3 / 10.5) like those between: 100 random sizes of them 1.5 times with [K,N] weights, 1.65 with
+//     [N,K]; a long K see below.
+//   * a K of 272 bytes or less is the tile kernels', which is no line by speed: this one would be ahead there as well, up to 31
+//     rows 9 to 14 us / 3 to 7, from 32 on 5.0 to 7.2 / 3.0 to 5.4 up to a cost of 6 (8-bit 8); at a bf16 cost of 8 5.7 / 6.9.
 template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRowsTile &t) {
   const int64_t cost = t.rounds * (t.mt + t.nt);
   if (p.K * ES <= 272 || (p.M >= 32 && cost > (ES == 2 ? 8 : 12)))
@@ -342,33 +345,37 @@ template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRows
     return t.rounds == 1 && p.N >= 512 && p.K <= 4096;
   if (ES == 1 || p.M < 32)
     return true;
-  const bool groups = p.K % 128 == 0;
-  if (p.M == 32)
-    return p.N * p.K < (int64_t)1 << 21;
-  return groups ? p.N * p.K < (int64_t)1 << 22 : p.M <= 128;
+  return p.K % 128 != 0 || p.N * p.K < (int64_t)1 << 22;
 }
 
 // A wave walks its share of K alone, a stage in about 0.85 us ([K,N]; 0.4 where N is no more than 40) or 0.35 ([N,K]; half as much
 // again with rows that are no whole lines), up to 1.3 on the larger tiles, while K slices over workgroups take their 10 to 15 us
 // and little more for a longer K.  So past a K they win, where another kernel has them.  Measured over 32 to 256 rows of 16 to
-// 8192 columns (530 random sizes), by the sixteenths of rows and columns of a tile, us, slices / this:
+// 8192 columns (530 random sizes from the cache, 240 wide ones, K 1000 to 10000, from memory too: m), by the sixteenths of rows and
+// columns of a tile, us, slices / this:
 //   [K,N] 2   112 x 528, K 5824 14.6 / 12.5   32 x 168, K 5968 12.8 / 14.2   169 x 168, K 7776 13.7 / 16.0  48 x 112, K 188208 37 / 302
 //         2, few columns   157 x 40, K 8704 14.4 / 11.9   143 x 16, K 13696 17.4 / 11.8   46 x 24, K 26112 25 / 23   256 x 32, K 24448 18 / 25
-//         3   48 x 2632, K 4840 16.2 / 14.9   214 x 408, K 5280 14.4 / 15.1     4   195 x 1088, K 5560 16.5 / 16.2
-//         6   250 x 1088, K 3840 16.6 / 14.7   96 x 3848, K 4792 19.7 / 22.2    8   242 x 2704, K 5376 24.6 / 24.7   202 x 3000, K 6968 26 / 32
+//         3   74 x 1488, K 4552 14.6 / 12.6 (m 16.2 / 16.4)   32 x 3840, K 4920 15.4 / 16.7 (m 16.6 / 24.1)   49 x 1880, K 5104 14.8 / 14.4 (m 15.5 / 17.7)
+//         4   100 x 1928, K 4320 15.9 / 15.8 (m 18.2 / 17.1)   55 x 2136, K 4744 15.1 / 16.4 (m 15.7 / 21.0)
+//         5   41 x 4400, K 3192 15.9 / 13.5 (m 16.7 / 17.4)   104 x 2200, K 5056 17.7 / 18.4 (m 18.6 / 23.0)
+//         6   119 x 2216, K 3136 16.0 / 14.0 (m 19.3 / 17.4)   206 x 1536, K 4304 16.4 / 15.7 (m 17.7 / 21.5)   102 x 2808, K 4600 17.7 / 19.0 (m 20.6 / 24.3)
+//         8   134 x 4112, K 3888 25.1 / 23.4 (m 25.3 / 24.4)   100 x 6208, K 3744 18.7 / 19.2 (m 21.3 / 23.8)   79 x 6216, K 4312 21.6 / 25.7 (m 24.3 / 28.8)
 //   [N,K] 2   169 x 128, K 15872 17.2 / 15.4  63 x 448, K 19680 17.4 / 19.9   64 x 64, K 191744 35 / 125
 //         2, few columns   56 x 88, K 20992 23.5 / 16.7   127 x 64, K 23960 18.7 / 25.2
-//         3   121 x 640, K 13632 17.9 / 17.3   197 x 496, K 16808 22.1 / 26.9   4   160 x 824, K 10624 19.5 / 18.4   190 x 1112, K 21464 33 / 43
-//         6   253 x 1600, K 4224 17.2 / 13.6   96 x 3200, K 5704 19.8 / 23.4    8   139 x 4488, K 8704 32.4 / 29.6   200 x 2496, K 11648 30 / 36
+//         3   121 x 640, K 13632 17.9 / 17.3   197 x 496, K 16808 22.1 / 26.9
+//         4   167 x 1224, K 8808 22.0 / 19.4 (m 23.4 / 23.5)   117 x 1336, K 9040 20.1 / 21.6 (m 24.4 / 26.9)   190 x 1112, K 21464 33 / 43
+//         6   120 x 3792, K 4744 20.3 / 18.9 (m 24.5 / 24.5)   128 x 3096, K 5600 19.4 / 20.3 (m 23.4 / 26.3)
+//         8   205 x 4088, K 4032 20.0 / 18.7 (m 23.0 / 21.2)   109 x 5160, K 4568 21.9 / 25.6 (m 27.9 / 33.4)   205 x 4008, K 9736 40 / 44; past the line 45
+//             sizes 0.92 times
 //   up to 32 rows against gemm_skinny.hpp ([N,K])   19 x 224, K 10048 9.5 / 8.9   15 x 320, K 13952 10.2 / 12.6
 //   and against slices of 256 columns ([K,N])       26 x 512, K 6016 13.6 / 12.8   4 x 256, K 9600 14.2 / 18.0
 static bool few_rows_slices_ahead(const GemmParams &p, const FewRowsTile &t) {
   const int64_t cost = t.rounds * (t.mt + t.nt);
   if (p.trans_b) {
-    const int64_t k = cost <= 2 ? (p.N <= 128 ? 23040 : 16384) : cost == 3 ? 13312 : cost == 4 ? 10240 : cost <= 6 ? 5120 : 8704;
+    const int64_t k = cost <= 2 ? (p.N <= 128 ? 23040 : 16384) : cost == 3 ? 13312 : cost == 4 ? 8832 : cost <= 6 ? 5120 : 3968;
     return p.K > (p.M <= 32 && k > 10240 ? 10240 : k);
   }
-  const int64_t k = cost <= 2 ? (p.N <= 24 ? 24576 : p.N <= 40 ? 16384 : 5888) : cost == 3 ? 5120 : cost == 4 ? 6144 : cost <= 6 ? 4608 : 5376;
+  const int64_t k = cost <= 2 ? (p.N <= 24 ? 24576 : p.N <= 40 ? 16384 : 5888) : cost == 3 ? 4608 : cost == 4 ? 4352 : cost == 5 ? 4096 : cost == 6 ? 3840 : 3584;
   return p.K > (p.M < 32 && k < 6144 ? 6144 : k);
 }
 

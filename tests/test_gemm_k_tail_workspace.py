@@ -17,7 +17,7 @@ def _status(gc, name, A, B, out, trans_b):
 
 
 # at most two workgroups per compute unit and 128 x 128 f32 sums of each
-@pytest.mark.parametrize("M,N,K", [(512, 4096, 16376), (300, 4000, 16000 + 8), (1024, 1024, 32760), (32, 4096, 1376),
+@pytest.mark.parametrize("M,N,K", [(512, 4096, 16376), (300, 4000, 16000 + 8), (1024, 1024, 32760), (32, 1096, 10248),
                                    (192, 4096, 4072)])
 @pytest.mark.parametrize("trans_b", [0, 1])
 def test_slices_fit_the_static_array(gc, M, N, K, trans_b):
@@ -26,7 +26,7 @@ def test_slices_fit_the_static_array(gc, M, N, K, trans_b):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(32, 4096, 1376), (64, 4096, 4072), (192, 4096, 4072), (512, 4096, 16376)])
+@pytest.mark.parametrize("M,N,K", [(32, 4096, 1376), (32, 1096, 10248), (64, 4096, 4072), (192, 4096, 4072), (512, 4096, 16376)])
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_k_tail_under_capture_and_without_allocation(gc, dev, M, N, K, trans_b):
     import torch

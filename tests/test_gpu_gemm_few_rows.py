@@ -9,7 +9,8 @@ FEW = 7
 # every tile of 16, 32 and 64 rows and columns, whole and cut, one and two rounds of workgroups; K in whole stages (64 bf16,
 # 128 bytes), one chunk into and one chunk short of one, and fewer stages than waves
 SHAPES = [(1, 640, 576), (3, 1712, 2736), (16, 24, 144), (17, 1000, 1080), (32, 2048, 1016), (33, 520, 1544), (64, 2008, 640),
-          (50, 8, 4096), (5, 8200, 264), (31, 9000, 200), (64, 8208, 328), (9, 16400, 160), (20, 17000, 232), (48, 16376, 296), (128, 1288, 200), (97, 3000, 392), (256, 1000, 256), (65, 520, 4088)]
+          (50, 8, 4096), (5, 8200, 264), (31, 9000, 200), (64, 8208, 328), (9, 16400, 160), (20, 17000, 232), (48, 16376, 296), (128, 1288, 200), (97, 3000, 392), (256, 1000, 256), (65, 520, 4088),
+          (32, 4096, 1376), (129, 1024, 4072), (140, 264, 1048), (251, 2648, 776)]
 
 
 def _ints(shape, lo, hi, dev, g, dt):
@@ -39,7 +40,7 @@ def test_bf16_exact_on_integers(gc, dev, M, N, K, trans_b):
     assert (guard[0] == 7.0).all() and (guard[M + 1] == 7.0).all() and (guard[:, N:] == 7.0).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(3, 1712, 2736), (32, 2048, 1016), (64, 8208, 328), (20, 17000, 232)])
+@pytest.mark.parametrize("M,N,K", [(3, 1712, 2736), (32, 2048, 1016), (64, 8208, 328), (20, 17000, 232), (32, 4096, 1376), (140, 264, 1048)])
 def test_bf16_rounding_points_and_layouts(gc, dev, M, N, K):
     """Bias, activation and residual against float64 rounded where a bf16 graph rounds; [N,K] and [K,N] weights give the same bits."""
     g = torch.Generator(device=dev).manual_seed(N + K)

@@ -38,7 +38,7 @@ def test_batches(gc, dev, nb, M, N, K, trans_b):
         assert torch.equal(out[i].double(), torch.relu(x + bias.double()) + res[i].double()), i
 
 
-@pytest.mark.parametrize("M,N,K", [(129, 1024, 4072), (140, 264, 1048), (32, 4096, 1376)])
+@pytest.mark.parametrize("M,N,K", [(129, 1024, 8840), (260, 264, 1048), (32, 1096, 10248)])
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("slices", [True, False])
 def test_slices(gc, dev, M, N, K, trans_b, slices):

@@ -43,7 +43,7 @@ def test_bf16_k_tail(gc, dev, K, tile, trans_b):
     assert torch.equal(out.double(), ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(129, 1024, 4072), (512, 512, 8168), (140, 264, 1048)])
+@pytest.mark.parametrize("M,N,K", [(129, 1024, 8840), (512, 512, 8168), (260, 264, 1048)])
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_bf16_k_tail_in_slices(gc, dev, M, N, K, trans_b):
     c = gc.tile_config(M, N, K, trans_b=trans_b)[0]

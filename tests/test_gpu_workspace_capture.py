@@ -66,9 +66,9 @@ def test_two_streams_do_not_wait_for_each_other(gc, dev):
     g = torch.Generator(device=dev).manual_seed(4)
     bf = lambda *s: torch.randn(*s, device=dev, generator=g).to(torch.bfloat16)  # noqa: E731
     Q, K, V = bf(1, 8, 1, 128), bf(1, 8, 4096, 128), bf(1, 8, 4096, 128)
-    A = torch.randint(-2, 3, (192, 4072), device=dev, generator=g).to(torch.bfloat16)
-    B = torch.randint(-2, 3, (4072, 1024), device=dev, generator=g).to(torch.bfloat16)
-    assert gc.lib().gcmi_gemm_bf16_workspace_bytes(192, 1024, 4072, 0) > 0
+    A = torch.randint(-2, 3, (192, 5640), device=dev, generator=g).to(torch.bfloat16)
+    B = torch.randint(-2, 3, (5640, 1024), device=dev, generator=g).to(torch.bfloat16)
+    assert gc.lib().gcmi_gemm_bf16_workspace_bytes(192, 1024, 5640, 0) > 0
     want = gc.mha_fwd_bf16(Q, K, V), gc.gemm_bf16(A, B, out_dtype=gc.F32)
     streams = [torch.cuda.Stream() for _ in range(2)]
     outs = [(torch.zeros_like(want[0]), torch.zeros_like(want[1])) for _ in streams]
