@@ -328,7 +328,11 @@ static FewRowsTile few_rows_tile(int64_t M, int64_t N, int64_t nbatch) {
 //     K 256 6.8 / 7.8; 112 x 7072, K 384 8.1 / 8.8; 10 matrices of 189 x 448, K 256 6.4 / 7.6; with a longer K or a tail 92
 //     random sizes 1.0 to 1.3 times (96 x 7032, K 616 12.5 / 10.0).
 //   * 8-bit operands, for which the tile kernels have no K slices, up to 2048 rows while one round holds them: 45 random sizes
-//     of 257 to 2000 rows 1.75 times on the average (679 x 608, K 3568 23.6 / 11.1; 1328 x 768, K 976 11.0 / 8.1).
+//     of 257 to 2000 rows 1.75 times on the average (679 x 608, K 3568 23.6 / 11.1; 1328 x 768, K 976 11.0 / 8.1).  In two rounds
+//     128 x 128 tiles are level or ahead up to a cost of 16 (562 x 2480, K 5184 32.4 / 34.3; 607 x 2976, K 25168 129 / 124), past it
+//     ahead (968 x 2128, K 4288 25.7 / 42.1).  The ends at 512 columns, K 4096 and 2048 rows are no lines by speed: 180 random sizes
+//     past them in one round, 16 to 2600 columns, K to 30000, 19000 rows, are 1.1 to 4.8 times ahead here too (257 x 1024, K 4112
+//     21.4 / 11.6; 257 x 496, K 2048 14.0 / 7.0; 1503 x 560, K 26368 117 / 71).
 //   * with a K that ends inside a group of 128 nothing streams, so these are taken whatever the weights' size, 32 rows (32 x 4096,
 //     K 1376 12.3 / 8.0, 32 x 6336, K 2136 14.4 / 10.4) and 129 to 256 (140 x 264, K 1048 9.8 / 5.5, 169 x 2400, K 1464 14.7 /
 //     10.0, 248 x 2656, K 776 13.3 / 10.5) like those between: 100 random sizes of them 1.5 times with [K,N] weights, 1.65 with

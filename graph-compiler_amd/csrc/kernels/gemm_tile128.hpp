@@ -16,9 +16,11 @@ namespace gcmi {
 // barrier per stage.  Rows past M and columns past N (N a multiple of 8) are fetched from the last row / chunk
 // inside and never stored.  The epilogue is the 4-wave kernel's: accumulators through a wave-private LDS region,
 // then rows of four columns per lane.  blockIdx.y: the batch, or with GemmParams::splits the K slice.
-// LDS bounds the loop (a stage of 128 rows: 32 KiB of fragment reads and 16 KiB of requests for 256 cycles of MFMAs), so a
-// taller wave tile gets more out of it: 96 or 128 rows per wave read 14 or 12 bytes where 64 rows read 16.  That is what the
-// forms of 192 and 256 rows are for, with one workgroup per compute unit: 1.5 and 1.85 us per 128 of K against 1.12 (one
+// A stage of 128 rows is 32 KiB of fragment reads and 16 KiB of requests (384 cycles of LDS) for 256 cycles of MFMAs; a taller
+// wave tile needs fewer: 96 or 128 rows per wave read 14 or 12 bytes where 64 rows read 16, and a barrier covers more products.
+// That is what the forms of 192 and 256 rows are for, with one workgroup per compute unit.  Nothing is saturated there (192
+// rows, 1237 x 4096, K 1376: matrix pipe busy 29 % of the cycles, LDS reads 27 %): one wave per SIMD waits for its reads, the
+// barrier and the epilogue in turn.  1.5 and 1.85 us per 128 of K against 1.12 (one
 // workgroup) and 1.9 to 2.17 (two on a compute unit) at 128 rows.
 template <int MI> struct T128 {
   static constexpr int BM = 32 * MI, A_BYTES = BM * T128_KB, STAGE_BYTES = A_BYTES + T128_B * T128_KB;

@@ -1824,7 +1824,7 @@ static inline double gcmi_us_per_group_256(double load) { // one workgroup per c
 }
 // Taller tiles of 128 columns (one workgroup per compute unit): fewer fragment reads per product than 128 rows, so where 128
 // rows make more than a round and 192 or 256 do not, they are ahead (64 random such sizes: 1.14 times on the average, at most
-// 1.5; 8-bit ones with a short K down to 0.93).  128 / 192 / 256 rows in one pass, us: 1237 x 4096, K 1376 29.3 / 22.5 / 27.5;
+// 1.5; 8-bit ones with K 1056 to 8112, 123 of them, 1.17, at least 0.95 from the cache and 0.81 from memory).  128 / 192 / 256 rows in one pass, us: 1237 x 4096, K 1376 29.3 / 22.5 / 27.5;
 // 305 x 11008, K 4096 69.5 / 56.3 / 63.8; 483 x 11008 73.1 / - / 67.3; where 128 rows fit one round they stay: 1000 x 4096,
 // K 4096 38.6 / 47.8 / 59.4.
 static inline double gcmi_us_per_group_tall(int rows) { return rows == 192 ? 1.5 : 1.85; }

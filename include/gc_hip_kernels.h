@@ -19,13 +19,13 @@
  *     number of host threads.  A call whose stream is being captured gets none:
  *     masked attention of 128 queries or more and K-sliced GEMMs are then
  *     refused, but for GEMMs whose K is no multiple of 128 (with [N,K] weights
- *     and up to 64 rows: of 64) or that are sliced only because of tiles of more
- *     than 128 rows, which run in one pass, and attention of fewer queries,
- *     which keeps the keys of a head in one workgroup.  These also do without
- *     where memory cannot be had, and every kind does where the stream it would
- *     have to wait for is being captured.  Without, sums are
- *     added in another order and a result may differ in its last bits from that
- *     of a call with the buffer;
+ *     and up to 64 rows: of 64), that are sliced only because of tiles of more
+ *     than 128 rows, or whose few rows one launch can take as well, which run in
+ *     one pass, and attention of fewer queries, which keeps the keys of a head in
+ *     one workgroup.  These also do without where memory cannot be had, and every
+ *     kind does where the stream it would have to wait for is being captured.
+ *     Without, sums are added in another order and a result may differ in its
+ *     last bits from that of a call with the buffer;
  *   - *_ws entry points: a workspace the caller brings (size from the
  *     *_workspace_bytes query).  Nothing is shared: calls with different
  *     workspaces may overlap on different streams.  This is what a compiled
