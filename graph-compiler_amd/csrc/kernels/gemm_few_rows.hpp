@@ -355,7 +355,7 @@ template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRows
 // A wave walks its share of K alone, a stage in about 0.85 us ([K,N]; 0.4 where N is no more than 40) or 0.35 ([N,K]; half as much
 // again with rows that are no whole lines), up to 1.3 on the larger tiles, while K slices over workgroups take their 10 to 15 us
 // and little more for a longer K.  So past a K they win, where another kernel has them.  Measured over 32 to 256 rows of 16 to
-// 8192 columns (530 random sizes from the cache, 240 wide ones, K 1000 to 10000, from memory too: m), by the sixteenths of rows and
+// 8192 columns (530 random sizes from the cache, 440, K 1000 to 14000, from memory too: m), by the sixteenths of rows and
 // columns of a tile, us, slices / this:
 //   [K,N] 2   112 x 528, K 5824 14.6 / 12.5   32 x 168, K 5968 12.8 / 14.2   169 x 168, K 7776 13.7 / 16.0  48 x 112, K 188208 37 / 302
 //         2, few columns   157 x 40, K 8704 14.4 / 11.9   143 x 16, K 13696 17.4 / 11.8   46 x 24, K 26112 25 / 23   256 x 32, K 24448 18 / 25
@@ -363,23 +363,26 @@ template <int ES> static bool few_rows_wanted(const GemmParams &p, const FewRows
 //         4   100 x 1928, K 4320 15.9 / 15.8 (m 18.2 / 17.1)   55 x 2136, K 4744 15.1 / 16.4 (m 15.7 / 21.0)
 //         5   41 x 4400, K 3192 15.9 / 13.5 (m 16.7 / 17.4)   104 x 2200, K 5056 17.7 / 18.4 (m 18.6 / 23.0)
 //         6   119 x 2216, K 3136 16.0 / 14.0 (m 19.3 / 17.4)   206 x 1536, K 4304 16.4 / 15.7 (m 17.7 / 21.5)   102 x 2808, K 4600 17.7 / 19.0 (m 20.6 / 24.3)
+//         6, full   37 x 7432, K 5344 25.1 / 21.9 (m 26.1 / 26.5)   40 x 7984, K 5720 27.2 / 24.1 (m 28.2 / 32.2)   56 x 7176, K 5512 25.5 / 26.2 (m 27.0 / 30.5)
 //         8   134 x 4112, K 3888 25.1 / 23.4 (m 25.3 / 24.4)   100 x 6208, K 3744 18.7 / 19.2 (m 21.3 / 23.8)   79 x 6216, K 4312 21.6 / 25.7 (m 24.3 / 28.8)
 //   [N,K] 2   169 x 128, K 15872 17.2 / 15.4  63 x 448, K 19680 17.4 / 19.9   64 x 64, K 191744 35 / 125
 //         2, few columns   56 x 88, K 20992 23.5 / 16.7   127 x 64, K 23960 18.7 / 25.2
-//         3   121 x 640, K 13632 17.9 / 17.3   197 x 496, K 16808 22.1 / 26.9
+//         3   120 x 544, K 10304 16.4 / 13.8 (m 17.2 / 17.7)   53 x 1352, K 11232 16.6 / 16.7 (m 17.6 / 22.9)   209 x 376, K 12552 18.6 / 21.8 (m 20.7 / 24.6)
 //         4   167 x 1224, K 8808 22.0 / 19.4 (m 23.4 / 23.5)   117 x 1336, K 9040 20.1 / 21.6 (m 24.4 / 26.9)   190 x 1112, K 21464 33 / 43
 //         6   120 x 3792, K 4744 20.3 / 18.9 (m 24.5 / 24.5)   128 x 3096, K 5600 19.4 / 20.3 (m 23.4 / 26.3)
+//         6, full   40 x 7640, K 6872 27.0 / 24.4 (m 34.7 / 29.9)   38 x 7928, K 10440 36.1 / 33.9 (m 53.9 / 49.9)   45 x 7600, K 11744 34.7 / 35.0 (m 47.9 / 52.4)
 //         8   205 x 4088, K 4032 20.0 / 18.7 (m 23.0 / 21.2)   109 x 5160, K 4568 21.9 / 25.6 (m 27.9 / 33.4)   205 x 4008, K 9736 40 / 44; past the line 45
 //             sizes 0.92 times
 //   up to 32 rows against gemm_skinny.hpp ([N,K])   19 x 224, K 10048 9.5 / 8.9   15 x 320, K 13952 10.2 / 12.6
 //   and against slices of 256 columns ([K,N])       26 x 512, K 6016 13.6 / 12.8   4 x 256, K 9600 14.2 / 18.0
 static bool few_rows_slices_ahead(const GemmParams &p, const FewRowsTile &t) {
   const int64_t cost = t.rounds * (t.mt + t.nt);
+  const bool full = p.M <= 64 && p.N >= 6784; // at a cost of 6: 64 x 32 tiles on nearly all compute units
   if (p.trans_b) {
-    const int64_t k = cost <= 2 ? (p.N <= 128 ? 23040 : 16384) : cost == 3 ? 13312 : cost == 4 ? 8832 : cost <= 6 ? 5120 : 3968;
+    const int64_t k = cost <= 2 ? (p.N <= 128 ? 23040 : 16384) : cost == 3 ? 11776 : cost == 4 ? 8832 : cost <= 6 ? (full ? 11264 : 5120) : 3968;
     return p.K > (p.M <= 32 && k > 10240 ? 10240 : k);
   }
-  const int64_t k = cost <= 2 ? (p.N <= 24 ? 24576 : p.N <= 40 ? 16384 : 5888) : cost == 3 ? 4608 : cost == 4 ? 4352 : cost == 5 ? 4096 : cost == 6 ? 3840 : 3584;
+  const int64_t k = cost <= 2 ? (p.N <= 24 ? 24576 : p.N <= 40 ? 16384 : 5888) : cost == 3 ? 4608 : cost == 4 ? 4352 : cost == 5 ? 4096 : cost == 6 ? (full ? 5376 : 3840) : 3584;
   return p.K > (p.M < 32 && k < 6144 ? 6144 : k);
 }
 
