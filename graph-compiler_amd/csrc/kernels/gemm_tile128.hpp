@@ -1,4 +1,4 @@
-// The 128 x 128 tile kernel and its taller forms (pieces it shares with the 256 x 256 kernels: tile_of_block, MfmaOp, the
+// The 128 x 128 tile kernel (pieces it shares with the 256 x 256 kernels: tile_of_block, MfmaOp, the
 // 4-wave kernel's epilogue); the launcher in gemm_tile256.hpp chooses between the tiles.
 #pragma once
 #include "gemm_tile256.hpp"
@@ -16,31 +16,26 @@ namespace gcmi {
 // barrier per stage.  Rows past M and columns past N (N a multiple of 8) are fetched from the last row / chunk
 // inside and never stored.  The epilogue is the 4-wave kernel's: accumulators through a wave-private LDS region,
 // then rows of four columns per lane.  blockIdx.y: the batch, or with GemmParams::splits the K slice.
-// A stage of 128 rows is 32 KiB of fragment reads and 16 KiB of requests (384 cycles of LDS) for 256 cycles of MFMAs; a taller
-// wave tile needs fewer: 96 or 128 rows per wave read 14 or 12 bytes where 64 rows read 16, and a barrier covers more products.
-// That is what the forms of 192 and 256 rows are for, with one workgroup per compute unit.  Nothing is saturated there (192
-// rows, 1237 x 4096, K 1376: matrix pipe busy 29 % of the cycles, LDS reads 27 %): one wave per SIMD waits for its reads, the
-// barrier and the epilogue in turn.  1.5 and 1.85 us per 128 of K against 1.12 (one
-// workgroup) and 1.9 to 2.17 (two on a compute unit) at 128 rows.
-template <int MI> struct T128 {
+// A stage is 32 KiB of fragment reads and 16 KiB of requests (384 cycles of LDS) for 256 cycles of MFMAs; a taller
+// wave tile needs fewer: 96 or 128 rows per wave read 14 or 12 bytes where 64 rows read 16 (gemm_tall_kernel).
+struct T128 {
+  static constexpr int MI = 4; // 16-row tiles of a wave
   static constexpr int BM = 32 * MI, A_BYTES = BM * T128_KB, STAGE_BYTES = A_BYTES + T128_B * T128_KB;
-  static constexpr int DUMP_WAVE_BYTES = 16 * MI * W4_DUMP_PITCH;      // 17408 per wave at 128 rows
+  static constexpr int DUMP_WAVE_BYTES = 16 * MI * W4_DUMP_PITCH;      // 17408 per wave
   static constexpr int SMEM_BYTES = 4 * DUMP_WAVE_BYTES + 3 * 256 * 4; // accumulator regions / ring, column parameters
   static_assert(T128_NST * STAGE_BYTES <= 4 * DUMP_WAVE_BYTES, "the ring overlaps the column parameters");
-  static_assert(MI % 2 == 0, "every wave requests as many rows of A");
 };
 
-// MI: 16-row tiles of a wave; the workgroup's tile has 32 * MI rows (128, 192 or 256) and 128 columns
-template <bool TB, int ES, int MI> __device__ __forceinline__ void tile128_body(GemmParams p) {
+template <bool TB, int ES> __global__ __launch_bounds__(256, 2) void gemm_tile128_kernel(GemmParams p) {
   static_assert(!TB || ES == 2, "B stored [N,K]: bf16 only");
-  constexpr int KB = T128_KB, BK = KB / ES, NST = T128_NST, BM = T128<MI>::BM, A_BYTES = T128<MI>::A_BYTES, STAGE = T128<MI>::STAGE_BYTES;
+  constexpr int KB = T128_KB, BK = KB / ES, NST = T128_NST, MI = T128::MI, BM = T128::BM, A_BYTES = T128::A_BYTES, STAGE = T128::STAGE_BYTES;
   constexpr int NA = MI / 2, NB = 2, PER = NA + NB; // requests of 1 KiB per wave and stage
   // a k-row of the B tile: 256 bytes of bf16 (4 k-rows per transposing read, chunk ^ 4 * (k % 4)) or 128 bytes of
   // int8 (8 k-rows per read, chunk ^ 2 * (k % 8 / 2): the read of 8 k-rows x 16 columns touches every bank once)
   constexpr int RG = ES == 2 ? 4 : 8, B_ROW_BYTES = T128_B * ES, B_CPR = B_ROW_BYTES / 16;
   typedef typename std::conditional<ES == 2, f32x4_t, i32x4_t>::type acc4_t;
-  __shared__ __align__(1024) char smem[T128<MI>::SMEM_BYTES];
-  float *colp = reinterpret_cast<float *>(smem + 4 * T128<MI>::DUMP_WAVE_BYTES); // [0..127] bias, [256..] scale, [512..] comp * colsum
+  __shared__ __align__(1024) char smem[T128::SMEM_BYTES];
+  float *colp = reinterpret_cast<float *>(smem + 4 * T128::DUMP_WAVE_BYTES); // [0..127] bias, [256..] scale, [512..] comp * colsum
   auto b_swz = [](int krow) { return ES == 2 ? (krow % 4) * 4 : ((krow % 8) >> 1) * 2; };
 
   const int tid = threadIdx.x;
@@ -272,7 +267,7 @@ template <bool TB, int ES, int MI> __device__ __forceinline__ void tile128_body(
 
   // the accumulator regions lie over the ring: every wave's reads of the last block must have returned
   __syncthreads();
-  char *dump = smem + wave * T128<MI>::DUMP_WAVE_BYTES;
+  char *dump = smem + wave * T128::DUMP_WAVE_BYTES;
 #pragma unroll
   for (int jt = 0; jt < 4; jt++)
 #pragma unroll
@@ -285,9 +280,5 @@ template <bool TB, int ES, int MI> __device__ __forceinline__ void tile128_body(
   else
     w4_epilogue_half_any<ES, false, 16 * MI, 64>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, BM, T128_B);
 }
-
-template <bool TB, int ES> __global__ __launch_bounds__(256, 2) void gemm_tile128_kernel(GemmParams p) { tile128_body<TB, ES, 4>(p); }
-// 192 or 256 rows: one workgroup per compute unit (107 and 142 KiB of LDS)
-template <bool TB, int ES, int MI> __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams p) { tile128_body<TB, ES, MI>(p); }
 
 } // namespace gcmi

@@ -1171,28 +1171,24 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(512, 1) void gem
 }
 
 // ---------------------------------------------------------------------------
-// The whole-tile kernel with one wave per SIMD: 4 waves as 2 x 2, each owning 128 x 128 of the 256 x 256 tile as
-// 8 x 8 tiles of 16 x 16 (v_mfma_f32_16x16x32_bf16 / v_mfma_i32_16x16x64_i8), 256 accumulator registers.  Against
+// The kernels with one wave per SIMD and a hand-placed main loop: 4 waves as 2 x 2, each owning MI x NJ tiles of 16 x 16
+// (v_mfma_f32_16x16x32_bf16 / v_mfma_i32_16x16x64_i8).  8 x 8: the 256 x 256 tile, 256 accumulator registers; against
 // the 8-wave kernel a multiply-accumulate costs a third less LDS read traffic (per k-step a wave reads 8 KiB of A
 // and 8 KiB of B for 64 MFMAs, not 8 + 4 KiB for 32), which is what counts on a board that holds its power limit
-// by lowering the clock.  With a single wave per SIMD nothing hides a stall, so every fragment is fetched a whole
-// stage ahead:
-//   stage s computes k-block s entirely from registers: A tiles in one of two register sets, B tiles in one set;
-//   its MFMAs run column tile by column tile, and between them the wave reads k-block s+1: one A tile per column
-//   tile into the other A set, and the B tile of a column as soon as that column's MFMAs are issued (column 7's
-//   goes to a spare register set, alternating by stage, so it can be fetched early as well).
-// Because a k-block sits in registers for the whole of its stage, its LDS slot is free during the stage: the ring
-// of 4 slots carries k-blocks s+1 .. s+4, and the DMA of block s+4 is issued at the start of stage s, three full
-// stages (about 3000 cycles) before the barrier that publishes it.  One barrier per stage, at its start:
-//   s_waitcnt vmcnt(2 stages) lgkmcnt(0)   own share of block s+1 has landed; own reads of block s have returned
-//   s_barrier                              block s+1 is visible to all; slot s may be overwritten
-// The main loop is assembly text written by gen_gemm_w4_mainloop.py (registers and issue order fixed by hand: the
-// compiler's allocator does not hold 64 accumulator tiles and three fragment sets without copies and spills);
+// by lowering the clock.  8 x 4 and 6 x 4: 256 and 192 rows by 128 columns, for problems that large tiles leave half the GPU idle.
+// With a single wave per SIMD nothing hides a stall, so every fragment is fetched a whole
+// stage ahead: stage t computes k-block t from registers, and between its MFMAs the wave reads k-block t+1 into the other
+// register set and requests what the LDS ring has room for, two to four stages ahead.  Operands whose rows run along K are
+// requested in pairs of k-blocks, 128 bytes of a row at a time (whole cache lines), B stored [K,N] block by block.
+// Against requests of single k-blocks (half lines, each line fetched from L2 twice: the line reads of L2 are what large tiles
+// then wait for) and, for the 128-column tiles, against a loop left to the compiler, us, weights [K,N] / [N,K], from memory:
+// 4096^3 99.3 -> 96.6 / 116 -> 94.5; 1000 x 11008, K 4096 (with its 172 tiles dealt to the XCDs in runs) 92 -> 78 / 118 -> 81;
+// 1000 x 4096, K 11008 (256 x 128, two slices) 117 -> 94 / 121 -> 97; 1237 x 4096, K 1376 (192 x 128) 26.4 -> 23.8 / 28.4 -> 25.8;
+// 8-bit 4096 x 4096 x 11008 with its epilogue 158.3 -> 155.8.
+// The main loop is assembly text written by gen_gemm_w4_mainloop.py, which has the details (registers and issue order fixed
+// by hand: the compiler's allocator does not hold 64 accumulator tiles and four fragment sets without copies and spills);
 // set-up and epilogue are the C++ below.
 #include "gemm_w4_mainloop.inc"
-#if defined(GCMI_W4_EXPERIMENT_OPTS) && !defined(GCMI_W4_ALLOW_EXPERIMENT)
-#error "gemm_w4_mainloop.inc was generated with experiment switches (some give wrong products): regenerate it without GCMI_W4_EXPERIMENT"
-#endif
 
 // Epilogue of gemm_tile256_w4_kernel.  The main loop's assembly ends by writing the raw accumulators of column
 // tiles 0-3 (the left 64 columns of the wave's 128 x 128) to a wave-private LDS region, 128 rows of 256 bytes at a
@@ -1451,7 +1447,7 @@ __device__ __forceinline__ void w4_epilogue_half_any(const GemmParams &p, int ki
 // computed, and this puts it into the ring's four slots before the main loop starts: whole k-blocks by DMA, the block
 // that K ends in through registers with zeros behind K (in both operands, so no product of theirs counts, whatever the
 // memory behind K holds), zero blocks without a load.  The main loop then requests from k = 0 on; its steady state
-// knows nothing of the tail.  (A tail handled behind the loop would need the accumulators outside the assembly.)
+// knows nothing of the tail.
 // Before, every K that is no multiple of 128 bf16 / 256 bytes went to the bounds-checked kernel: 1237 x 4096 x 1376
 // ([N,K] weights) took 89.7 us there, 29.5 us as 320 tiles of 128 x 128.
 // a_src / b_src: the lane's byte offset per DMA instruction (NA and NB of them per wave and block); a_k / b_k: its first k inside a block, which decides whether
@@ -1496,21 +1492,68 @@ __device__ __forceinline__ void fill_ring_k_tail(char *smem, int wave, int lane,
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 }
 
-template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gemm_tile256_w4_kernel(GemmParams p) {
+// K not a whole number of groups (two pairs of k-blocks, 256 bytes): the incomplete group [k_full, K) is the FIRST one
+// computed, and this puts it into slots 0 and 1 of the rings before the main loop starts: whole pairs (blocks of B stored
+// [K,N]) by DMA, the one that K ends in through registers with zeros behind K (in both operands, so no product of theirs
+// counts, whatever the memory behind K holds), zeros behind that without a load.  The pairs behind it are on their way already.
+template <int ES, bool TB, int MI, int NJ>
+__device__ __forceinline__ void w4_fill_k_tail(char *smem, int wave, int lane, const char *a_tail, const char *b_tail, int64_t b_step,
+                                               int k_left, const int (&a_off)[8], const int (&b_off)[8], const int (&a_k)[MI],
+                                               const int (&b_k)[TB ? NJ : NJ / 2]) {
+  constexpr int BK = 64 / ES, A_PAIR = MI * 4096, B_PAIR = NJ * 4096, NB = TB ? NJ : NJ / 2;
+  char *const sa = smem + wave * MI * 1024, *const sb = smem + W4Ring<ES, TB, MI, NJ>::DA * A_PAIR + wave * NB * 1024;
+  // one operand's requests of a pair or block: `left` of its k lie before K
+  auto fill = [&](auto nc, char *to, const char *from, const int (&off)[8], const auto &k, int whole, int left) {
+    constexpr int N = decltype(nc)::value;
+    if (left >= whole) {
+#pragma unroll
+      for (int i = 0; i < N; i++)
+        __builtin_amdgcn_global_load_lds((GCMI_GLB const void *)(from + (uint32_t)off[i]), (GCMI_LDS void *)(to + i * 1024), 16, 0, 0);
+      return;
+    }
+    uint4 v[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      v[i] = make_uint4(0, 0, 0, 0);
+      if (k[i] < left)
+        v[i] = *reinterpret_cast<const uint4 *>(from + (uint32_t)off[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++)
+      *reinterpret_cast<uint4 *>(to + i * 1024 + lane * 16) = v[i];
+  };
+#pragma unroll 1
+  for (int q = 0; q < 2; q++) {
+    const int left = k_left - q * 2 * BK;
+    fill(std::integral_constant<int, MI>{}, sa + q * A_PAIR, a_tail + q * 128, a_off, a_k, 2 * BK, left);
+    if constexpr (TB) {
+      fill(std::integral_constant<int, NB>{}, sb + q * B_PAIR, b_tail + q * 128, b_off, b_k, 2 * BK, left);
+    } else {
+#pragma unroll 1
+      for (int h = 0; h < 2; h++)
+        fill(std::integral_constant<int, NB>{}, sb + q * B_PAIR + h * (B_PAIR / 2), b_tail + (2 * q + h) * b_step, b_off, b_k, BK, left - h * BK);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+}
+
+template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_body(GemmParams p) {
   // B stored [N,K]: bf16 only.  (The same loop for 8-bit operands -- plain 16-byte fragment reads in place of the
   // transposing ones -- was measured against [K,N] on one board and is no faster: 166.9-168.9 against 167.2-168.6 us
   // for the 4096 x 4096 x 11008 layer; an 8-bit weight stored [N,K] is copied once instead.)
   static_assert(!TB || ES == 2, "B stored [N,K]: bf16 only");
-  typedef FastGemm<ES, 2, 4, false, TB> FG; // 4 waves: 4 DMA instructions per operand, wave and stage
-  static_assert(FG::NST == 4 && FG::NDMA == 4 && FG::STAGE_BYTES == 32768 && FG::A_BYTES == 16384, "the assembly's ring");
+  typedef W4Ring<ES, TB, MI, NJ> Ring;
+  constexpr int BM = 32 * MI, BN = 32 * NJ, BK = 64 / ES, NB = TB ? NJ : NJ / 2;
+  constexpr int A_PAIR = BM * 128, B_PAIR = BN * 128, RING = Ring::DA * A_PAIR + Ring::DB * B_PAIR;
+  constexpr int DUMP_WAVE = 16 * MI * W4_DUMP_PITCH, EPILOGUE = 4 * DUMP_WAVE + 3 * 256 * 4;
+  constexpr int B_ROW = BN * ES, B_CPR = B_ROW / 16, RG = ES == 2 ? 4 : 8; // B stored [K,N]: bytes and chunks of a k-row, k-rows per transposing read
 #ifdef GCMI_W4_TIMING
   const long long wall_entry = wall_clock64();
   float *const timing_out = p.partial;
 #endif
-  // one array: the ring (128 KiB; the epilogue's 4 x 34 KiB of accumulators afterwards), then the column parameters
-  __shared__ __align__(1024) char smem[8 * G_STG_WAVE_BYTES + 3 * G_BN * 4];
-  static_assert(4 * W4_DUMP_WAVE_BYTES <= 8 * G_STG_WAVE_BYTES, "accumulator regions overlap the column parameters");
-  float *colp = reinterpret_cast<float *>(smem + 8 * G_STG_WAVE_BYTES);
+  // one array: the rings, afterwards the waves' accumulator regions and the column parameters behind them
+  __shared__ __align__(1024) char smem[RING > EPILOGUE ? RING : EPILOGUE];
+  float *colp = reinterpret_cast<float *>(smem + 4 * DUMP_WAVE);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1518,14 +1561,28 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
   const int wm = wave >> 1, wn = wave & 1;
   const int r16 = lane & 15, g16 = lane >> 4;
 
-  const int tiles_m = (int)((p.M + G_BM - 1) / G_BM), tiles_n = (int)((p.N + G_BN - 1) / G_BN); // edge tiles stick out
+  const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN); // edge tiles stick out
   int tm, tn;
   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, p.group_m, tm, tn);
   // integer division runs on the vector unit; the operand addresses below must be in scalar registers
   tm = __builtin_amdgcn_readfirstlane(tm), tn = __builtin_amdgcn_readfirstlane(tn);
-  const int64_t m0 = (int64_t)tm * G_BM, n0 = (int64_t)tn * G_BN;
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   const int64_t lda_b = p.lda * ES, ldb_b = p.ldb * ES;
-  {
+  const int64_t b_step = TB ? 64 : BK * ldb_b; // from k-block to k-block
+  // (a row of A is shorter than 2^31 bytes, so K fits 32 bits)
+  const int all_groups = (int)((p.K + 4 * BK - 1) / (4 * BK));
+  int k_left = (int)(p.K & (4 * BK - 1)), groups = all_groups;
+  int64_t k_first = 0; // first k of this workgroup
+  if (p.splits > 1) {
+    // K slices: blockIdx.y is the slice, whole groups each (they differ by at most one); its f32 sums go
+    // to the workspace as they are, the second kernel adds the slices and runs the epilogue
+    const int slice = blockIdx.y;
+    const int g0 = (int)((int64_t)slice * all_groups / p.splits), g1 = (int)((int64_t)(slice + 1) * all_groups / p.splits);
+    k_first = (int64_t)g0 * 4 * BK, groups = g1 - g0;
+    k_left = g1 == all_groups ? k_left : 0;
+    p.C = p.partial + (int64_t)slice * p.M * p.N, p.ldc = p.N, p.out_dt = DT_F32;
+    p.bias = nullptr, p.act = ACT_NONE, p.residual = nullptr;
+  } else {
     const int64_t bz = blockIdx.y; // strided batch
     p.A = reinterpret_cast<const char *>(p.A) + bz * p.a_bs * ES;
     p.B = reinterpret_cast<const char *>(p.B) + bz * p.b_bs * ES;
@@ -1534,50 +1591,65 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
       p.residual = reinterpret_cast<const char *>(p.residual) + bz * p.c_bs * (p.residual_dt == DT_BF16 ? 2 : 4);
   }
 
-  // per-lane source offsets of the wave's DMA instructions, as in gemm_tile256_fast_kernel.  An edge tile's rows past
+  // Per-lane source offsets of the wave's DMA instructions, 1 KiB each: 8 rows by 128 bytes of A (or of B stored [N,K]), the
+  // chunk that fills position c of row r is c ^ (r / 2 % 8); k-rows of a block of B stored [K,N].  An edge tile's rows past
   // M and columns past N are fetched from the last row / the last 16-byte chunk inside (N is a multiple of the
   // chunk's columns): their products land in accumulators that the epilogue never stores.
-  const int rows_in = (int)min((int64_t)G_BM, p.M - m0), cols_in = (int)min((int64_t)G_BN, p.N - n0);
-  i32x4_t a_off, b_off;
-  int a_k[4], b_k[4]; // the first k of the lane's 16 bytes inside a k-block
+  const int rows_in = (int)min((int64_t)BM, p.M - m0), cols_in = (int)min((int64_t)BN, p.N - n0);
+  // k-row k of B keeps chunk c at c ^ b_swz(k): the RG k-rows that a transposing read takes lie in different banks
+  auto b_swz = [](int k) { return ES == 2 ? (k % 4) * 4 : BN == 256 ? (k % 8) * 2 : ((k % 8) >> 1) * 2; };
+  int a_off[8] = {}, b_off[8] = {}, a_k[MI], b_k[NB]; // *_k: the first k of the lane's 16 bytes inside a pair / block
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int row = (wave * 4 + i) * FG::A_ROWS_PER_DMA + lane / FG::A_CPR;
-    const int c = (lane % FG::A_CPR) ^ FG::a_swz(row);
+  for (int i = 0; i < MI; i++) {
+    const int row = (wave * MI + i) * 8 + lane / 8, c = (lane % 8) ^ ((row >> 1) & 7);
     a_off[i] = (int)(min(row, rows_in - 1) * lda_b + c * 16);
-    const int krow = (wave * 4 + i) * FG::B_ROWS_PER_DMA + lane / FG::B_CPR;
-    const int cb = min((lane % FG::B_CPR) ^ ((krow % FG::RG) * FG::CW), cols_in * ES / 16 - 1);
-    b_off[i] = TB ? (int)(min(row, cols_in - 1) * ldb_b + c * 16) : (int)(krow * ldb_b + cb * 16);
-    a_k[i] = c * 16 / ES, b_k[i] = TB ? a_k[i] : krow;
+    a_k[i] = c * 16 / ES;
   }
-  // fragment addresses as in gemm_tile256_mi16_kernel: A tile `it` = rows wm*128 + 16*it .., B tile `jt` = columns
-  // wn*128 + 16*jt ..; slots 2 and 3 through a second base (an instruction's offset field has 16 bits)
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(GCMI_LDS char *)smem;
-  typedef int i32x8_t __attribute__((ext_vector_type(8)));
-  i32x2_t a_ld;
-  i32x8_t b_ld0, b_ld2;
-  {
-    const int row_a = wm * 128 + r16;
-    a_ld[0] = (int)(lds0 + row_a * FG::KB + ((g16 ^ FG::a_swz(row_a)) << 4));
-    a_ld[1] = a_ld[0] + 65536;
-    const int kk = ES == 2 ? (r16 >> 2) : (r16 >> 1);
-    const int cc = ES == 2 ? (r16 & 3) : (r16 & 1);
 #pragma unroll
-    for (int jt = 0; jt < 8; jt++) {
-      const int chunk = ES == 2 ? (wn * 8 + jt) * 2 + (cc >> 1) : (wn * 8 + jt);
-      const int sub = ES == 2 ? (cc & 1) * 8 : cc * 8;
-      int at = FG::A_BYTES + (2 * FG::RG * g16 + kk) * FG::B_ROW_BYTES + ((chunk ^ (kk * FG::CW)) << 4) + sub;
-      if (TB) {
-        const int row_b = wn * 128 + jt * 16 + r16;
-        at = FG::A_BYTES + row_b * FG::KB + ((g16 ^ FG::a_swz(row_b)) << 4);
+  for (int i = 0; i < NB; i++) {
+    if constexpr (TB) {
+      const int row = (wave * NB + i) * 8 + lane / 8, c = (lane % 8) ^ ((row >> 1) & 7);
+      b_off[i] = (int)(min(row, cols_in - 1) * ldb_b + c * 16);
+      b_k[i] = c * 16 / ES;
+    } else {
+      const int at = (wave * NB + i) * 64 + lane, krow = at / B_CPR;
+      b_off[i] = (int)(krow * ldb_b + min((at % B_CPR) ^ b_swz(krow), cols_in * ES / 16 - 1) * 16);
+      b_k[i] = krow;
+    }
+  }
+  typedef int i32x8_t __attribute__((ext_vector_type(8)));
+  i32x8_t a_src, b_src;
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    a_src[i] = a_off[i], b_src[i] = b_off[i];
+  // fragment addresses: A tile `it` = rows wm*16*MI + 16*it .., B tile `jt` = columns wn*16*NJ + 16*jt ..
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(GCMI_LDS char *)smem, lds_b = lds0 + Ring::DA * A_PAIR;
+  i32x2_t a_ld;
+  i32x4_t b_ld = {0, 0, 0, 0};
+  {
+    const int row_a = wm * 16 * MI + r16, row_b = wn * 16 * NJ + r16;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      a_ld[h] = (int)(lds0 + row_a * 128 + (((4 * h + g16) ^ ((row_a >> 1) & 7)) << 4));
+      if (TB)
+        b_ld[h] = (int)(lds_b + row_b * 128 + (((4 * h + g16) ^ ((row_b >> 1) & 7)) << 4));
+    }
+    if (!TB) {
+      // the 16 lanes of a group hand the transposing read RG k-rows x 16 columns in 8-byte pieces (bf16: k row
+      // lane%16/4, 4 columns at lane%4; int8: k row lane%16/2, 8 columns at lane%2) and get back column lane%16;
+      // tiles 2j and 2j + 1 differ in a chunk bit that b_swz leaves alone
+      const int kk = ES == 2 ? (r16 >> 2) : (r16 >> 1), cc = ES == 2 ? (r16 & 3) : (r16 & 1);
+#pragma unroll
+      for (int j = 0; j < NJ / 2; j++) {
+        const int chunk = ES == 2 ? (wn * NJ + 2 * j) * 2 + (cc >> 1) : wn * NJ + 2 * j;
+        const int sub = ES == 2 ? (cc & 1) * 8 : cc * 8;
+        b_ld[j] = (int)(lds_b + (2 * RG * g16 + kk) * B_ROW + ((chunk ^ b_swz(kk)) << 4) + sub);
       }
-      b_ld0[jt] = (int)(lds0 + at);
-      b_ld2[jt] = (int)(lds0 + at + 65536);
     }
   }
 
-  // column parameters of this tile (see gemm_tile256_fast_kernel): 256 threads, one column each
-  float cp_bias = -0.0f, cp_scale = 1.0f;
+  // column parameters of this tile: 256 threads, one column each
+  float cp_bias = -0.0f, cp_scale = 1.0f; // an absent bias adds nothing, not even to -0.0
   int cp_cs = 0;
   if (tid < cols_in) {
     if (p.bias)
@@ -1591,66 +1663,84 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
     }
   }
 
-  uint64_t a_ptr = (uint64_t)(reinterpret_cast<const char *>(p.A) + m0 * lda_b);
-  uint64_t b_ptr = (uint64_t)(reinterpret_cast<const char *>(p.B) + (TB ? n0 * ldb_b : n0 * ES));
-  uint64_t b_step = TB ? (uint64_t)FG::KB : (uint64_t)(FG::BK * ldb_b);
-  // (a row of A is shorter than 2^31 bytes, so K fits 32 bits; inputs of the assembly in scalar registers)
-  const int K32 = (int)p.K;
-  int trips = __builtin_amdgcn_readfirstlane((K32 - 1) >> (ES == 2 ? 7 : 8)); // ring groups of four k-blocks, less the last one
-  const int k_left = __builtin_amdgcn_readfirstlane(K32 & (4 * FG::BK - 1));
-  const int ring_filled = k_left;
-  if (k_left) {
-    const int64_t k_full = p.K - k_left;
-    fill_ring_k_tail<ES, TB, 4, 4, FG::STAGE_BYTES, FG::A_BYTES>(
-        smem, wave, lane, reinterpret_cast<const char *>(a_ptr) + k_full * ES,
-        reinterpret_cast<const char *>(b_ptr) + (TB ? k_full * ES : k_full * ldb_b), (int64_t)b_step, k_left, a_off, b_off, a_k, b_k);
-  }
-  const uint32_t dma_lds = lds0 + (uint32_t)wave * 4096u;
+  // (inputs of the assembly in scalar registers)
+  const char *const a0 = reinterpret_cast<const char *>(p.A) + m0 * lda_b + k_first * ES;
+  const char *const b0 = reinterpret_cast<const char *>(p.B) + (TB ? n0 * ldb_b + k_first * ES : n0 * ES + k_first * ldb_b);
+  uint64_t a_ptr = (uint64_t)a0, b_ptr = (uint64_t)b0;
+  int pairs = __builtin_amdgcn_readfirstlane(2 * groups);
+  const int tail_group = __builtin_amdgcn_readfirstlane(k_left);
+  const uint32_t a_dma = lds0 + (uint32_t)(wave * MI * 1024), b_dma = lds_b + (uint32_t)(wave * NB * 1024);
   const uint32_t a_xor = p.a_xor;
   // where this lane writes its accumulators for the epilogue: row lane%16 (+ 16*it), 16-byte chunk lane/16 (+ 4*jt)
   // of the wave's region
-  const uint32_t dump_ld = lds0 + (uint32_t)wave * W4_DUMP_WAVE_BYTES + (uint32_t)(r16 * W4_DUMP_PITCH + g16 * 16);
+  const uint32_t dump_ld = lds0 + (uint32_t)wave * DUMP_WAVE + (uint32_t)(r16 * W4_DUMP_PITCH + g16 * 16);
 
-#define GCMI_W4_OPERANDS                                                                                              \
-  : "+{s[40:41]}"(a_ptr), "+{s[42:43]}"(b_ptr), "+{s46}"(trips)                                                       \
-  : "{v[0:3]}"(a_off), "{v[4:7]}"(b_off), "{v[8:9]}"(a_ld), "{v[10:17]}"(b_ld0), "{v[18:25]}"(b_ld2),                \
-    "{s[44:45]}"(b_step), "{s47}"(dma_lds), "{s48}"(a_xor), "{s50}"(ring_filled), "{v26}"(dump_ld)                   \
-  : "memory", "scc", "s49", GCMI_W4_CLOBBERS
+#define GCMI_W4_FILL(TEXT)                                                                                            \
+  asm volatile(TEXT : "+{s[40:41]}"(a_ptr), "+{s[42:43]}"(b_ptr)                                                      \
+               : "{v[0:7]}"(a_src), "{v[8:15]}"(b_src), "{s[44:45]}"(b_step), "{s46}"(pairs), "{s47}"(a_dma),         \
+                 "{s51}"(b_dma), "{s50}"(tail_group)                                                                  \
+               : "memory", "scc", "s49")
+#define GCMI_W4_MAIN(TEXT, CLOBBERS)                                                                                  \
+  asm volatile(TEXT : "+{s[40:41]}"(a_ptr), "+{s[42:43]}"(b_ptr), "+{s46}"(pairs)                                     \
+               : "{v[0:7]}"(a_src), "{v[8:15]}"(b_src), "{v[16:17]}"(a_ld), "{v[20:23]}"(b_ld),                       \
+                 "{s[44:45]}"(b_step), "{s47}"(a_dma), "{s51}"(b_dma), "{s48}"(a_xor), "{v28}"(dump_ld)               \
+               : "memory", "scc", "s49", "s52", "s53", "s54", "s55", "s56", CLOBBERS)
+#define GCMI_W4_OF(STEP)                                                                                              \
+  if constexpr (ES == 1 && MI == 8 && NJ == 8) STEP(I8_8x8, 8x8)                                                      \
+  else if constexpr (ES == 1 && MI == 8) STEP(I8_8x4, 8x4)                                                            \
+  else if constexpr (ES == 1) STEP(I8_6x4, 6x4)                                                                       \
+  else if constexpr (TB && MI == 8 && NJ == 8) STEP(BF16_TB_8x8, 8x8)                                                 \
+  else if constexpr (TB && MI == 8) STEP(BF16_TB_8x4, 8x4)                                                            \
+  else if constexpr (TB) STEP(BF16_TB_6x4, 6x4)                                                                       \
+  else if constexpr (MI == 8 && NJ == 8) STEP(BF16_8x8, 8x8)                                                          \
+  else if constexpr (MI == 8) STEP(BF16_8x4, 8x4)                                                                     \
+  else STEP(BF16_6x4, 6x4)
+#define GCMI_W4_STEP_FILL(NAME, TILES) GCMI_W4_FILL(GCMI_W4_FILL_##NAME);
+#define GCMI_W4_STEP_MAIN(NAME, TILES) GCMI_W4_MAIN(GCMI_W4_ASM_##NAME, GCMI_W4_CLOBBERS_##TILES);
+  GCMI_W4_OF(GCMI_W4_STEP_FILL)
+  if (tail_group) {
+    const int64_t k_full = p.K - k_left - k_first;
+    w4_fill_k_tail<ES, TB, MI, NJ>(smem, wave, lane, a0 + k_full * ES, b0 + (TB ? k_full * ES : k_full * ldb_b), b_step, k_left,
+                                   a_off, b_off, a_k, b_k);
+  }
 #ifdef GCMI_W4_TIMING // measurement builds: core clock cycles and 100 MHz ticks spent in the main loop
   const long long tick0 = clock64(), wall0 = wall_clock64();
 #endif
-  if constexpr (ES == 1)
-    asm volatile(GCMI_W4_ASM_I8 GCMI_W4_OPERANDS);
-  else if constexpr (TB)
-    asm volatile(GCMI_W4_ASM_BF16_TB GCMI_W4_OPERANDS);
-  else
-    asm volatile(GCMI_W4_ASM_BF16 GCMI_W4_OPERANDS);
-#undef GCMI_W4_OPERANDS
+  GCMI_W4_OF(GCMI_W4_STEP_MAIN)
+#undef GCMI_W4_OF
+#undef GCMI_W4_STEP_FILL
+#undef GCMI_W4_STEP_MAIN
+#undef GCMI_W4_FILL
+#undef GCMI_W4_MAIN
 #ifdef GCMI_W4_TIMING
   const long long tick1 = clock64(), wall1 = wall_clock64();
 #endif
   // the column parameters were requested before the main loop and are first needed here
   colp[tid] = cp_bias;
-  colp[G_BN + tid] = cp_scale;
-  reinterpret_cast<int *>(colp)[2 * G_BN + tid] = cp_cs;
+  if (ES == 1) {
+    colp[256 + tid] = cp_scale;
+    reinterpret_cast<int *>(colp)[512 + tid] = cp_cs;
+  }
   __syncthreads();
 
   const int out_kind = p.out_dt == DT_BF16 ? 0 : ((ES == 1 && p.out_dt == DT_S32) ? 2 : 1);
   const int kind = (out_kind == 2 ? (int)ACT_NONE : p.act) + 8 * out_kind;
-  const char *dump = smem + wave * W4_DUMP_WAVE_BYTES;
+  const char *dump = smem + wave * DUMP_WAVE;
   // a tile that sticks out of C takes the same code with every row and lane tested against the edge
-  const int rows_c = (int)min((int64_t)G_BM, p.M - m0), cols_c = (int)min((int64_t)G_BN, p.N - n0);
-  const bool edge_tile = rows_c < G_BM || cols_c < G_BN; // the same for the whole workgroup
+  const bool edge_tile = rows_in < BM || cols_in < BN; // the same for the whole workgroup
   if (edge_tile)
-    w4_epilogue_half_any<ES, true>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, rows_c, cols_c);
+    w4_epilogue_half_any<ES, true, 16 * MI, 16 * NJ>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, rows_in, cols_in);
   else
-    w4_epilogue_half_any<ES, false>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, G_BM, G_BN);
-  // the right half: the accumulators of column tiles 4-7 are still where the main loop left them
-  asm volatile(GCMI_W4_ASM_DUMP_HI : : "{v26}"(dump_ld) : "memory");
-  if (edge_tile)
-    w4_epilogue_half_any<ES, true>(p, kind, 1, m0, n0, wm, wn, lane, dump, colp, rows_c, cols_c);
-  else
-    w4_epilogue_half_any<ES, false>(p, kind, 1, m0, n0, wm, wn, lane, dump, colp, G_BM, G_BN);
+    w4_epilogue_half_any<ES, false, 16 * MI, 16 * NJ>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, BM, BN);
+  if constexpr (NJ > 4) {
+    // the right half: the accumulators of column tiles 4-7 are still where the main loop left them
+    static_assert(MI == 8 && NJ == 8, "the dump's tiles");
+    asm volatile(GCMI_W4_ASM_DUMP_HI_8x8 : : "{v28}"(dump_ld) : "memory");
+    if (edge_tile)
+      w4_epilogue_half_any<ES, true, 16 * MI, 16 * NJ>(p, kind, 1, m0, n0, wm, wn, lane, dump, colp, rows_in, cols_in);
+    else
+      w4_epilogue_half_any<ES, false, 16 * MI, 16 * NJ>(p, kind, 1, m0, n0, wm, wn, lane, dump, colp, BM, BN);
+  }
 #ifdef GCMI_W4_TIMING
   const long long wall_issued = wall_clock64();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1661,6 +1751,10 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gem
   }
 #endif
 }
+
+template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gemm_tile256_w4_kernel(GemmParams p) { w4_body<ES, TB, 8, 8>(p); }
+// 192 or 256 rows by 128 columns (instantiated beside the 128 x 128 kernel)
+template <bool TB, int ES, int MI> __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams p) { w4_body<ES, TB, MI, 4>(p); }
 
 
 // Four results of row m, columns n .. n+3, from their f32 sums: the rounding points of a bf16 graph (after the
