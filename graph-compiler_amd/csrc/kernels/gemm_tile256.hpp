@@ -1339,6 +1339,8 @@ __device__ __forceinline__ void w4_epilogue_half(const GemmParams &p, int half, 
   const int64_t n = n0 + col;
   if (MASKED && col >= cols_in)
     return;
+  if (WC % 64 != 0 && half * 64 + 4 * cc >= WC) // the last 32 columns of a wave tile of 96
+    return;
   const int row0 = wm * WR + rr; // + 4 * (i0 + u)
   const f32x4_t bias4 = *reinterpret_cast<const f32x4_t *>(colp + col); // -0.0 where there is no bias
   f32x4_t scale4 = {1.f, 1.f, 1.f, 1.f};
@@ -1597,7 +1599,8 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
   // chunk's columns): their products land in accumulators that the epilogue never stores.
   const int rows_in = (int)min((int64_t)BM, p.M - m0), cols_in = (int)min((int64_t)BN, p.N - n0);
   // k-row k of B keeps chunk c at c ^ b_swz(k): the RG k-rows that a transposing read takes lie in different banks
-  auto b_swz = [](int k) { return ES == 2 ? (k % 4) * 4 : BN == 256 ? (k % 8) * 2 : ((k % 8) >> 1) * 2; };
+  // (192 columns: rows of 384 bytes, k and k + 1 lie half the banks apart by themselves)
+  auto b_swz = [](int k) { return BN == 192 ? ((k >> 1) & 1) * 4 : ES == 2 ? (k % 4) * 4 : BN == 256 ? (k % 8) * 2 : ((k % 8) >> 1) * 2; };
   int a_off[8] = {}, b_off[8] = {}, a_k[MI], b_k[NB]; // *_k: the first k of the lane's 16 bytes inside a pair / block
 #pragma unroll
   for (int i = 0; i < MI; i++) {
@@ -1686,15 +1689,20 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
                  "{s[44:45]}"(b_step), "{s47}"(a_dma), "{s51}"(b_dma), "{s48}"(a_xor), "{v28}"(dump_ld)               \
                : "memory", "scc", "s49", "s52", "s53", "s54", "s55", "s56", CLOBBERS)
 #define GCMI_W4_OF(STEP)                                                                                              \
-  if constexpr (ES == 1 && MI == 8 && NJ == 8) STEP(I8_8x8, 8x8)                                                      \
+  if constexpr (ES == 1 && NJ == 8) STEP(I8_8x8, 8x8)                                                                 \
   else if constexpr (ES == 1 && MI == 8) STEP(I8_8x4, 8x4)                                                            \
-  else if constexpr (ES == 1) STEP(I8_6x4, 6x4)                                                                       \
-  else if constexpr (TB && MI == 8 && NJ == 8) STEP(BF16_TB_8x8, 8x8)                                                 \
+  else if constexpr (ES == 1 && MI == 6) STEP(I8_6x4, 6x4)                                                            \
+  else if constexpr (ES == 1) STEP(I8_4x4, 4x4)                                                                       \
+  else if constexpr (TB && NJ == 8) STEP(BF16_TB_8x8, 8x8)                                                            \
+  else if constexpr (TB && NJ == 6) STEP(BF16_TB_8x6, 8x6)                                                            \
   else if constexpr (TB && MI == 8) STEP(BF16_TB_8x4, 8x4)                                                            \
-  else if constexpr (TB) STEP(BF16_TB_6x4, 6x4)                                                                       \
-  else if constexpr (MI == 8 && NJ == 8) STEP(BF16_8x8, 8x8)                                                          \
+  else if constexpr (TB && MI == 6) STEP(BF16_TB_6x4, 6x4)                                                            \
+  else if constexpr (TB) STEP(BF16_TB_4x4, 4x4)                                                                       \
+  else if constexpr (NJ == 8) STEP(BF16_8x8, 8x8)                                                                     \
+  else if constexpr (NJ == 6) STEP(BF16_8x6, 8x6)                                                                     \
   else if constexpr (MI == 8) STEP(BF16_8x4, 8x4)                                                                     \
-  else STEP(BF16_6x4, 6x4)
+  else if constexpr (MI == 6) STEP(BF16_6x4, 6x4)                                                                     \
+  else STEP(BF16_4x4, 4x4)
 #define GCMI_W4_STEP_FILL(NAME, TILES) GCMI_W4_FILL(GCMI_W4_FILL_##NAME);
 #define GCMI_W4_STEP_MAIN(NAME, TILES) GCMI_W4_MAIN(GCMI_W4_ASM_##NAME, GCMI_W4_CLOBBERS_##TILES);
   GCMI_W4_OF(GCMI_W4_STEP_FILL)
@@ -1733,9 +1741,12 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
   else
     w4_epilogue_half_any<ES, false, 16 * MI, 16 * NJ>(p, kind, 0, m0, n0, wm, wn, lane, dump, colp, BM, BN);
   if constexpr (NJ > 4) {
-    // the right half: the accumulators of column tiles 4-7 are still where the main loop left them
-    static_assert(MI == 8 && NJ == 8, "the dump's tiles");
-    asm volatile(GCMI_W4_ASM_DUMP_HI_8x8 : : "{v28}"(dump_ld) : "memory");
+    // the right part: the accumulators of column tiles 4 and up are still where the main loop left them
+    static_assert(MI == 8 && (NJ == 8 || NJ == 6), "the dumps there are");
+    if constexpr (NJ == 8)
+      asm volatile(GCMI_W4_ASM_DUMP_HI_8x8 : : "{v28}"(dump_ld) : "memory");
+    else
+      asm volatile(GCMI_W4_ASM_DUMP_HI_8x6 : : "{v28}"(dump_ld) : "memory");
     if (edge_tile)
       w4_epilogue_half_any<ES, true, 16 * MI, 16 * NJ>(p, kind, 1, m0, n0, wm, wn, lane, dump, colp, rows_in, cols_in);
     else
@@ -1753,9 +1764,22 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
 }
 
 template <int ES, bool TB = false> __global__ __launch_bounds__(256, 1) void gemm_tile256_w4_kernel(GemmParams p) { w4_body<ES, TB, 8, 8>(p); }
-// 192 or 256 rows by 128 columns (instantiated beside the 128 x 128 kernel)
-template <bool TB, int ES, int MI> __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams p) { w4_body<ES, TB, MI, 4>(p); }
+// 128, 192 or 256 rows by 128 columns, 256 rows by 192
+template <bool TB, int ES, int MI, int NJ = 4> __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams p) { w4_body<ES, TB, MI, NJ>(p); }
 
+template <bool TB, int ES> static int launch_tall(const GemmParams &p, int rows, int cols, dim3 grid, hipStream_t stream) {
+  if (rows == 128 && cols == 128)
+    hipLaunchKernelGGL((gemm_tall_kernel<TB, ES, 4>), grid, dim3(256), 0, stream, p);
+  else if (rows == 192 && cols == 128)
+    hipLaunchKernelGGL((gemm_tall_kernel<TB, ES, 6>), grid, dim3(256), 0, stream, p);
+  else if (rows == 256 && cols == 128)
+    hipLaunchKernelGGL((gemm_tall_kernel<TB, ES, 8>), grid, dim3(256), 0, stream, p);
+  else if constexpr (ES == 2)
+    hipLaunchKernelGGL((gemm_tall_kernel<TB, ES, 8, 6>), grid, dim3(256), 0, stream, p);
+  else
+    return 2;
+  return hipGetLastError() == hipSuccess ? 0 : 5;
+}
 
 // Four results of row m, columns n .. n+3, from their f32 sums: the rounding points of a bf16 graph (after the
 // matmul and after every op, lib/gc/Transforms/Pipeline.cpp:79-95), or one f32 epilogue.
@@ -1897,7 +1921,7 @@ static void launch_splitk_reduce(const GemmParams &p, hipStream_t stream) {
 static constexpr int T128_B = 128, T128_KB = 64, T128_NST = 4;
 
 } // namespace gcmi
-extern "C" int gcmi_launch_tile128(const gcmi::GemmParams *p, int es, int rows, unsigned grid_x, unsigned grid_y, hipStream_t stream);
+extern "C" int gcmi_launch_tile128(const gcmi::GemmParams *p, int es, int rows, int cols, unsigned grid_x, unsigned grid_y, hipStream_t stream);
 namespace gcmi {
 
 // Host-side launch of the 256x256 tile kernels for one element size.
@@ -2137,7 +2161,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     p.partial = ws;
     if constexpr (ES == 2) {
       if (by128) { // the kernel cuts K itself: blockIdx.y = slice
-        const int rc = gcmi_launch_tile128(&p, ES, rows128, (unsigned)tiles, (unsigned)splits, stream);
+        const int rc = gcmi_launch_tile128(&p, ES, rows128, 128, (unsigned)tiles, (unsigned)splits, stream);
         if (rc)
           return rc;
       } else if (by256) { // equal slices as a strided batch with f32 results
@@ -2169,7 +2193,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
       *cfg = c;
     if (dry)
       return 0;
-    return gcmi_launch_tile128(&p, ES, rows128, (unsigned)nblk128, (unsigned)nbatch, stream);
+    return gcmi_launch_tile128(&p, ES, rows128, 128, (unsigned)nblk128, (unsigned)nbatch, stream);
   }
   // Whole tiles: 4 waves of 128 x 128 unless the caller asks for 8 waves of 128 x 64.  Results of 8-bit operands
   // leave the 4-wave kernel as bf16, f32 or as the raw s32 accumulators (same main loop, the epilogue is a plain
@@ -2236,7 +2260,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     } else {
       hipLaunchKernelGGL(gemm_tile256_w4_kernel<ES>, hgrid, dim3(256), 0, stream, head);
     }
-    return gcmi_launch_tile128(&rest, ES, 128, (unsigned)(4 * (nblk % n_cu)), 1, stream);
+    return gcmi_launch_tile128(&rest, ES, 128, 128, (unsigned)(4 * (nblk % n_cu)), 1, stream);
   }
   dim3 grid((unsigned)nblk, (unsigned)nbatch), block(G_THREADS);
   if (use_w4) {

@@ -363,6 +363,8 @@ CONFIGS = [
     Cfg("BF16_8x8", 2, False, 8, 8, 3, 2), Cfg("BF16_TB_8x8", 2, True, 8, 8, 3, 2), Cfg("I8_8x8", 1, False, 8, 8, 3, 2),
     Cfg("BF16_8x4", 2, False, 8, 4, 3, 3), Cfg("BF16_TB_8x4", 2, True, 8, 4, 3, 3), Cfg("I8_8x4", 1, False, 8, 4, 3, 3),
     Cfg("BF16_6x4", 2, False, 6, 4, 4, 3), Cfg("BF16_TB_6x4", 2, True, 6, 4, 4, 4), Cfg("I8_6x4", 1, False, 6, 4, 4, 3),
+    Cfg("BF16_4x4", 2, False, 4, 4, 4, 3), Cfg("BF16_TB_4x4", 2, True, 4, 4, 4, 4), Cfg("I8_4x4", 1, False, 4, 4, 4, 3),
+    Cfg("BF16_8x6", 2, False, 8, 6, 3, 2), Cfg("BF16_TB_8x6", 2, True, 8, 6, 3, 2),
 ]
 
 

@@ -8,15 +8,16 @@ import torch
 pytestmark = pytest.mark.gpu
 
 CASES = [(256, 260, 520, K) for K in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 384, 392, 512, 520, 640, 648)]
+CASES += [(128, 260, 520, K) for K in (256, 264, 320, 384, 392, 512, 520, 640, 648, 1032)] + [(128, 2100, 2104, K) for K in (264, 640)]
 CASES += [(192, 1237, 4096, K) for K in (264, 320, 384, 392, 512, 520, 640)] + [(256128, 1000, 8192, K) for K in (1024, 1032, 1152)]
 
 
 @pytest.mark.parametrize("tile,M,N,K", CASES)
 @pytest.mark.parametrize("trans_b", [0, 1])
 def test_exact_on_integers(gc, dev, tile, M, N, K, trans_b):
-    cfg = [1, 1, 1, 256, 256, 64, 128, 128, 32] if tile == 256 else None
+    cfg = {256: [1, 1, 1, 256, 256, 64, 128, 128, 32], 128: [1, 1, 1, 128, 128, 64, 64, 64, 32]}.get(tile)
     c = gc.tile_config(M, N, K, trans_b=bool(trans_b), out_dtype=gc.F32, matmul_config=cfg)[0]
-    assert (c.kernel, c.bm, c.bn) == {256: (2, 256, 256), 192: (5, 192, 128), 256128: (5, 256, 128)}[tile]
+    assert (c.kernel, c.bm, c.bn) == {256: (2, 256, 256), 128: (5, 128, 128), 192: (5, 192, 128), 256128: (5, 256, 128)}[tile]
     g = torch.Generator(device=dev).manual_seed(K)
     ints = lambda *s: torch.randint(-2, 3, s, device=dev, generator=g, dtype=torch.int32).to(torch.bfloat16)  # noqa: E731
     A = torch.full((M, K + 64), float("nan"), device=dev, dtype=torch.bfloat16)
