@@ -1973,6 +1973,23 @@ static constexpr double GCMI_US_FIXED_256 = 8.0, GCMI_US_FIXED_128 = 3.7; // lau
 static constexpr double GCMI_US_SECOND_PASS = 3.0;     // the second kernel of a K-sliced product
 static constexpr double GCMI_US_PER_SLICE_MOUT = 1.7;  // partial sums written and read back, per slice and 2^20 outputs
 static constexpr double GCMI_ONE_PASS_MARGIN = 0.9;    // slices must win by this factor
+// bf16 problems that would take 256 x 256 tiles in one pass: the time of one pass by tile, us, fitted to 184 random graph-replayed ones
+// with the weights from memory (500 to 4500 rows, 1500 to 11008 columns, K 64 to 6000, up to 2.7 rounds of large tiles; rms
+// error 9 to 12 %).  A launch, per round of workgroups (one per compute unit; two of 128 x 128) a start and an epilogue, per group of
+// 128 k its rounds and, as the clock and the memory system notice, its tiles per compute unit, and 2^20 results stored.
+struct GemmTileCost {
+  int rows, cols, per_cu;
+  double launch, round, group_round, group_load, mout;
+};
+static constexpr GemmTileCost GCMI_TILE_COSTS[] = {
+    {256, 256, 1, 2.2, 9.3, 1.46, 1.29, 0.05}, {256, 192, 1, 2.9, 7.3, 1.45, 0.65, 0.19}, {256, 128, 1, 3.1, 4.7, 0.93, 0.68, 0.09},
+    {192, 128, 1, 3.7, 2.7, 1.01, 0.29, 0.31}, {128, 128, 2, 2.2, 2.2, 0.59, 0.93, 0.12}};
+static inline double gcmi_us_tile(const GemmTileCost &t, int64_t M, int64_t N, int64_t batches, int groups, int n_cu) {
+  const double load = (double)(((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) * batches) / n_cu;
+  const double rounds = ceil(load / t.per_cu);
+  return t.launch + t.round * rounds + groups * (t.group_round * rounds + t.group_load * load) +
+         t.mout * (double)M * (double)N * (double)batches / 1048576.0;
+}
 enum GemmPlan { PLAN_TILE256 = 0, PLAN_TILE128, PLAN_SLICES_SHORT_A, PLAN_SLICES_TILE256, PLAN_SLICES_TILE128 };
 template <int ES>
 static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *want = nullptr, GemmTileConfig *cfg = nullptr,
@@ -2224,6 +2241,32 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
   }
   if (tail_cols || tail_rows)
     c.workgroups = (int32_t)(nblk - nblk % n_cu + 4 * (nblk % n_cu));
+  // Large tiles that leave much of a round idle: another tile where it is estimated clearly ahead, in one pass, the same bits
+  // (same products in the same order, same epilogue).  The 184 sizes of the estimates gain 1.10 on the average (the best tile of
+  // each would give 1.118), two lose more than 2 % (at most 5 %).  us, 256 x 256 / chosen: 1000 x 11008, K 4096 82.2 / 73.9 on 256 x 192;
+  // 2655 x 3520, K 3800 73.6 / 64.9 likewise; 1643 x 10048, K 1408 (280 tiles) 66.5 / 57.5 on 192 x 128; 3597 x 4672, K 128 22.0 / 15.6
+  // on 128 x 128.  Under half a round (the estimates above decide) and past three the sizes were not measured; past one, a K of 4096 and more keeps the large tile, which callers have
+  // been told of for 2048 x 11008 (165.8 there, 143.7 on 256 x 192; 4096 x 11008 263.7 / 283.0).
+  if (ES == 2 && use_w4 && t128_can && !tail_cols && !tail_rows && p.cfg_tile == 0 && !p.cfg_waves && !p.cfg_split_k &&
+      2 * nblk * nbatch >= n_cu && nblk * nbatch < (p.K < 4096 ? 3 : 1) * n_cu) {
+    const GemmTileCost *tile = &GCMI_TILE_COSTS[0];
+    double best = 0.95 * gcmi_us_tile(*tile, p.M, p.N, nbatch, groups, n_cu);
+    for (const GemmTileCost &t : GCMI_TILE_COSTS) {
+      const double us = gcmi_us_tile(t, p.M, p.N, nbatch, groups, n_cu);
+      if (us < best)
+        best = us, tile = &t;
+    }
+    if (tile->rows != 256 || tile->cols != 256) {
+      const int64_t tiles = ((p.M + tile->rows - 1) / tile->rows) * ((p.N + tile->cols - 1) / tile->cols);
+      c.kernel = GK_TILE128, c.bm = tile->rows, c.bn = tile->cols, c.wave_m = tile->rows / 2, c.wave_n = tile->cols / 2;
+      c.workgroups = (int32_t)tiles;
+      if (cfg)
+        *cfg = c;
+      if (dry)
+        return 0;
+      return gcmi_launch_tile128(&p, ES, tile->rows, tile->cols, (unsigned)tiles, (unsigned)nbatch, stream);
+    }
+  }
   if (cfg)
     *cfg = c;
   if (dry)
