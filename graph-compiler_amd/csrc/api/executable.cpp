@@ -12,12 +12,14 @@
 
 #include "gc_hip_kernels.h"
 #include "kernels/eltwise_params.h"
+#include "kernels/gemm_params.h"
 
 extern "C" {
 int gcmi_launch_eltwise(const gcmi::EltParams *p, hipStream_t stream);
 int gcmi_launch_reduce(const gcmi::ReduceParams *p, hipStream_t stream);
 int gcmi_launch_fused(const gcmi::FusedParams *p, hipStream_t stream);
 int gcmi_launch_softmax(const gcmi::SoftmaxParams *p, hipStream_t stream);
+int gcmi_launch_gemm_gated(const gcmi::GemmParams *p, const void *up, hipStream_t stream, int dry, gcmi::GemmTileConfig *cfg);
 }
 
 namespace gcapi {
@@ -199,6 +201,7 @@ Executable::Executable(Graph g, bool dry) : g_(std::move(g)) { init(dry); }
 void Executable::init(bool dry) {
   verify_graph(g_);
   plan();
+  plan_gates();
   plan_workspaces();
   layout_arena();
   if (dry)
@@ -240,8 +243,78 @@ char *Executable::staging() {
 // slot of the step's own, alive for that step only, so it shares arena space with other temporaries.  Nothing is
 // shared between executables or streams: two executables may run side by side, as the reference's may
 // (thread-local scratch, lib/gc/ExecutionEngine/CPURuntime/Microkernel/BrgemmOnednn.cpp:70).
+// silu(x . Wg^T) * (x . Wu^T), the gate of a feed-forward layer: two GEMMs of one operand and the point-wise group that
+// reads nothing but them become one step where a kernel takes them (gemm_gated.hip).  A MatmulConfig on either keeps
+// both as they are.
+static gcmi::GemmParams gated_params(const Step &s) {
+  gcmi::GemmParams p{};
+  p.M = s.M, p.N = s.N, p.K = s.K, p.lda = s.lda, p.ldb = s.ldb, p.ldc = s.ldc;
+  p.out_dt = p.bias_dt = p.residual_dt = GCMI_BF16, p.trans_b = 1, p.batch = 1;
+  return p;
+}
+
+void Executable::plan_gates() {
+  auto refs = [&](int slot) {
+    int n = 0;
+    for (const Step &s : steps_) {
+      for (int x : {s.a, s.b, s.c, s.out, s.bias, s.mask, s.aux, s.ws, s.scale_slot, s.scales_slot, s.zps_slot})
+        n += x == slot;
+      n += (int)std::count(s.f_in.begin(), s.f_in.end(), slot);
+    }
+    return n;
+  };
+  for (size_t i = 0; i < steps_.size(); i++) {
+    const Step &f = steps_[i];
+    if (f.kind != Step::Fused || f.sum_ins >= 0 || f.row_end >= 0 || f.f_in.size() != 2 || f.f_ins.size() != 3 || f.once ||
+        f.out_dt != GCMI_BF16 || f.red_reg != 4 || f.f_str[0] != dense_strides(f.dims) || f.f_str[1] != f.f_str[0])
+      continue;
+    // registers 0 and 1: the inputs; 2: sigmoid(gate); 3: silu(gate); 4: the result
+    const Step::FIns &sig = f.f_ins[0], &silu = f.f_ins[1], &mul = f.f_ins[2];
+    const int gate = sig.a, up = 1 - gate;
+    auto product = [](const Step::FIns &x, int a, int b) {
+      return x.op == gcmi::ELT_MUL && x.dt == GCMI_BF16 && ((x.a == a && x.b == b) || (x.a == b && x.b == a));
+    };
+    if (sig.op != gcmi::ELT_SIGMOID || sig.dt != GCMI_BF16 || gate < 0 || gate > 1 || !product(silu, 2, gate) || !product(mul, 3, up))
+      continue;
+    int at[2] = {-1, -1}; // the GEMMs behind inputs 0 and 1
+    bool ok = true;
+    for (int k = 0; k < 2 && ok; k++) {
+      const int slot = f.f_in[(size_t)k];
+      const Slot &sl = slots_[(size_t)slot];
+      for (size_t j = 0; j < i; j++)
+        if (steps_[j].out == slot)
+          at[k] = (int)j;
+      ok = at[k] >= 0 && f.f_in_dt[(size_t)k] == GCMI_BF16 && !sl.is_input && !sl.is_output && sl.init.empty() && refs(slot) == 2;
+      if (!ok)
+        break;
+      const Step &g = steps_[(size_t)at[k]];
+      ok = g.kind == Step::GemmBf16 && g.batch <= 1 && !g.ta && g.tb && !g.once && g.a_off == 0 && g.b_off == 0 && g.out_off == 0 &&
+           g.bias < 0 && g.c < 0 && g.act == 0 && g.out_dt == GCMI_BF16 && g.mm_cfg.empty() && g.ldc == g.N &&
+           prod(f.dims, 0, f.dims.size()) == g.M * g.N;
+    }
+    if (!ok)
+      continue;
+    const Step &g = steps_[(size_t)at[gate]], &u = steps_[(size_t)at[up]];
+    if (g.a != u.a || g.M != u.M || g.N != u.N || g.K != u.K || g.lda != u.lda || g.ldb != u.ldb)
+      continue;
+    Step s;
+    s.kind = Step::GemmGated, s.note = "MatMul x2 + " + f.note + " fused";
+    s.a = g.a, s.b = g.b, s.c = u.b, s.out = f.out;
+    s.M = g.M, s.N = g.N, s.K = g.K, s.lda = g.lda, s.ldb = g.ldb, s.ldc = g.N, s.tb = true, s.out_dt = GCMI_BF16;
+    const gcmi::GemmParams p = gated_params(s);
+    if (gcmi_launch_gemm_gated(&p, nullptr, nullptr, 1, nullptr) < 0)
+      continue;
+    s.parts = {g, u, f};
+    const size_t first = (size_t)std::min(at[0], at[1]), second = (size_t)std::max(at[0], at[1]);
+    steps_[i] = std::move(s);
+    steps_.erase(steps_.begin() + (long)second);
+    steps_.erase(steps_.begin() + (long)first);
+    i -= 2;
+  }
+}
+
 void Executable::plan_workspaces() {
-  for (Step &s : steps_) {
+  auto plan = [&](Step &s) {
     size_t bytes = 0;
     if (s.kind == Step::GemmBf16 && s.batch <= 1)
       bytes = gcmi_gemm_bf16_workspace_bytes_cfg(s.M, s.N, s.K, s.tb ? 1 : 0, s.mm_cfg.size() == 9 ? s.mm_cfg.data() : nullptr);
@@ -249,14 +322,13 @@ void Executable::plan_workspaces() {
       bytes = gcmi_mha_fwd_workspace_bytes_bh(s.BH, s.Sq, s.Sk, s.D, s.mask >= 0 ? 1 : 0);
     if (bytes)
       s.ws = new_slot(bytes);
+  };
+  for (Step &s : steps_) {
+    plan(s);
+    for (Step &part : s.parts)
+      plan(part);
   }
 }
-
-// One allocation per executable, temporaries with disjoint lifetimes share memory: the tick-based merge
-// of the reference (lib/gc/Transforms/MergeAllocTickBased.cpp, docs/memref_schedule.md) with the step
-// index as the tick.  A slot lives from the first step that names it to the last; graph inputs and
-// outputs, constants and the results of once-only steps live for the whole executable.  Temporaries
-// are placed in order of their first tick at the lowest offset that is free for their whole lifetime.
 void Executable::layout_arena() {
   const int n = (int)slots_.size();
   std::vector<int> first(n, -1), last(n, -1);
@@ -270,10 +342,15 @@ void Executable::layout_arena() {
   };
   for (int i = 0; i < (int)steps_.size(); i++) {
     const Step &s = steps_[i];
-    for (int slot : {s.a, s.b, s.c, s.out, s.bias, s.mask, s.aux, s.ws, s.scale_slot, s.scales_slot, s.zps_slot})
-      touch(slot, i);
-    for (int slot : s.f_in)
-      touch(slot, i);
+    auto touch_all = [&](const Step &x) {
+      for (int slot : {x.a, x.b, x.c, x.out, x.bias, x.mask, x.aux, x.ws, x.scale_slot, x.scales_slot, x.zps_slot})
+        touch(slot, i);
+      for (int slot : x.f_in)
+        touch(slot, i);
+    };
+    touch_all(s);
+    for (const Step &part : s.parts)
+      touch_all(part);
     if (s.once || (s.kind == Step::ColSum && s.op == 1))
       if (s.out >= 0)
         pinned[s.out] = 1;
@@ -1521,6 +1598,17 @@ void Executable::launch(const Step &s) {
                                stream_),
              "MatMul bf16");
     break;
+  case Step::GemmGated: {
+    gcmi::GemmParams p = gated_params(s);
+    p.A = P(s.a), p.B = P(s.b), p.C = P(s.out);
+    const int rc = gcmi_launch_gemm_gated(&p, P(s.c), stream_, 0, nullptr);
+    if (rc >= 0)
+      gc_check(rc, "gated MatMul bf16");
+    else // addresses that its kernels do not take
+      for (const Step &part : s.parts)
+        launch(part);
+    break;
+  }
   case Step::ColSum:
     if (s.op == 1 && colsum_valid_[s.out])
       break; // constant weight: already summed
@@ -1770,12 +1858,17 @@ void Executable::run(dnnl_graph_compiler_tensor *inputs, dnnl_graph_compiler_ten
 
 std::string Executable::describe() const {
   static const char *names[] = {"gemm_f32", "gemm_bf16", "gemm_int8", "colsum", "attention", "eltwise", "reduce", "softmax",
-                                "fused", "attention mask"};
+                                "fused", "attention mask", "gemm_bf16"};
   std::ostringstream os;
   static const char *kernels[] = {"bounds-checked tile", "whole tiles, 8 waves", "whole tiles, 4 waves (one per SIMD)",
                                   "K slices + second pass", "weight streaming (+ second pass)",
                                   "small tiles, 4 waves, two workgroups per compute unit", "f32",
                                   "few rows, K over the waves of a workgroup"};
+  auto tile_line = [&](const auto &c) {
+    os << "  tile: " << kernels[c.kernel] << ", " << c.bm << "x" << c.bn << " per workgroup, " << c.kbytes << " B of K per stage x "
+       << c.stages << " stages, waves " << c.waves_m << "x" << c.waves_n << " of " << c.wave_m << "x" << c.wave_n << ", mfma " << c.mfma_m
+       << "x" << c.mfma_n << "x" << c.mfma_k << ", split_k " << c.split_k << ", " << c.workgroups << " workgroups";
+  };
   for (auto &s : steps_) {
     os << (s.kind == Step::Fused ? (s.sum_ins >= 0 ? "reduce" : "fused") : names[(int)s.kind]) << ": " << s.note << "\n";
     if ((s.kind == Step::GemmBf16 && s.batch <= 1 && !s.ta) || s.kind == Step::GemmInt8) {
@@ -1785,10 +1878,7 @@ std::string Executable::describe() const {
       const int a_dt = s.kind == Step::GemmInt8 ? s.a_dt : GCMI_BF16;
       if (gcmi_gemm_tile_config_query(a_dt, s.M, s.N, s.K, s.tb ? 1 : 0, s.out_dt, s.mm_cfg.size() == 9 ? s.mm_cfg.data() : nullptr,
                                       &c, why, sizeof(why)) == 0) {
-        os << "  tile: " << kernels[c.kernel] << ", " << c.bm << "x" << c.bn << " per workgroup, " << c.kbytes
-           << " B of K per stage x " << c.stages << " stages, waves " << c.waves_m << "x" << c.waves_n << " of " << c.wave_m << "x"
-           << c.wave_n << ", mfma " << c.mfma_m << "x" << c.mfma_n << "x" << c.mfma_k << ", split_k " << c.split_k << ", "
-           << c.workgroups << " workgroups";
+        tile_line(c);
         if (c.split_k > 1) // the slot the partial sums of the slices were planned into
           os << ", workspace " << (s.ws >= 0 ? slots_[(size_t)s.ws].bytes : 0) << " B";
         if (c.from_attrs)
@@ -1799,6 +1889,13 @@ std::string Executable::describe() const {
           os << " [MatmulConfig attributes leave the default]";
         os << "\n";
       }
+    }
+    if (s.kind == Step::GemmGated) {
+      const gcmi::GemmParams p = gated_params(s);
+      gcmi::GemmTileConfig c{};
+      gcmi_launch_gemm_gated(&p, nullptr, nullptr, 1, &c);
+      tile_line(c);
+      os << "\n";
     }
   }
   if (!g_.target_hints.empty()) {

@@ -29,7 +29,7 @@
 namespace gcapi {
 
 struct Step {
-  enum Kind { GemmF32, GemmBf16, GemmInt8, ColSum, Mha, Elt, Reduce, Softmax, Fused, MhaClassify } kind;
+  enum Kind { GemmF32, GemmBf16, GemmInt8, ColSum, Mha, Elt, Reduce, Softmax, Fused, MhaClassify, GemmGated } kind;
   std::string note; // what was fused, for introspection
   bool once = false; // depends on constant tensors only: runs in the first execute, its result is kept
   // operands are arena slot indices (-1 = none)
@@ -84,6 +84,9 @@ struct Step {
   hipFunction_t jit_fn = nullptr;
   unsigned jit_grid = 0, jit_block = 0;
   bool jit_vectors = false; // it moves 16-byte vectors: the operands must be aligned
+  // gated pair of GEMMs (a . b and a . c, then their point-wise group): the steps it stands for, which run where its kernels
+  // do not take the operands' addresses
+  std::vector<Step> parts;
 };
 
 struct Slot {
@@ -150,6 +153,7 @@ private:
   int const_slot(const void *data, size_t bytes);
   void init(bool dry);
   void plan();
+  void plan_gates();
   void plan_workspaces();
   void layout_arena();
   void plan_generic(const Op &op);

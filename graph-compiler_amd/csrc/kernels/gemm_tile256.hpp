@@ -1445,6 +1445,76 @@ __device__ __forceinline__ void w4_epilogue_half_any(const GemmParams &p, int ki
 #undef GCMI_W4_CASE
 }
 
+// 1 / (1 + exp(-x)) of a bf16 value x for a bf16 result: the hardware's exponential and reciprocal, each good to an ulp of f32
+// or two, in place of expf and a correctly rounded division (20 issue slots fewer per result).  The sum is a sixteenth of the
+// true one, so that no reciprocal is below the smallest normal number, which the instruction would make 0.  Rounded to bf16 it is
+// what those give for every bf16 x (all 65536 compared on the GPU) but -89 to -91.5, where expf(-x) is infinite and they give 0.
+__device__ __forceinline__ float sigmoid_of_bf16(float x) {
+  return 0.0625f * __builtin_amdgcn_rcpf(0.0625f + __builtin_amdgcn_exp2f(fmaf(x, -1.4426950408889634f, -4.0f)));
+}
+
+// What a gated pair of products ends in, silu(gate) * up, for four results of a row: both sums rounded to bf16, then the
+// graph's three ops (x / (1 + exp(-x)) as sigmoid and product, the product with up), each rounded as a bf16 tensor would
+// be.  A NaN stays a NaN through the ops, so only the last conversion gives it 0x7FC0.
+__device__ __forceinline__ uint2 gated_silu4(const f32x4_t &gate, const f32x4_t &up) {
+  auto rnd = [](float(&x)[4]) {
+    const uint32_t a = pack_bf16x2(x[0], x[1]), b = pack_bf16x2(x[2], x[3]);
+    x[0] = __uint_as_float(a << 16), x[1] = __uint_as_float(a & 0xffff0000u);
+    x[2] = __uint_as_float(b << 16), x[3] = __uint_as_float(b & 0xffff0000u);
+  };
+  float g[4] = {gate[0], gate[1], gate[2], gate[3]}, u[4] = {up[0], up[1], up[2], up[3]}, x[4];
+  rnd(g), rnd(u);
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    x[e] = sigmoid_of_bf16(g[e]);
+  rnd(x);
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    x[e] = x[e] * g[e];
+  rnd(x);
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    x[e] = x[e] * u[e];
+  uint32_t p0 = pack_bf16x2(x[0], x[1]), p1 = pack_bf16x2(x[2], x[3]);
+  const float any_nan = (x[0] + x[1]) + (x[2] + x[3]);
+  if (__builtin_expect(any_nan != any_nan, 0)) {
+    p0 = f32_to_bf16_bits(x[0]) | ((uint32_t)f32_to_bf16_bits(x[1]) << 16);
+    p1 = f32_to_bf16_bits(x[2]) | ((uint32_t)f32_to_bf16_bits(x[3]) << 16);
+  }
+  return make_uint2(p0, p1);
+}
+
+// Epilogue of a gated tile: the left wave column holds the gate's sums, the right one those of up, for the same rows and
+// columns of C.  Each of the two waves of a wave row takes every other group of four rows of both their regions, up to 64 columns at a time.
+template <int WR, int WC>
+__device__ __forceinline__ void w4_gated_half(const GemmParams &p, int half, int64_t m0, int64_t n0, int wm, int wn, int lane,
+                                              const char *gate, const char *up, int rows_in, int cols_in) {
+  const int rr = lane >> 4, cc = lane & 15, col = half * 64 + 4 * cc; // this lane's four columns of C, from n0 on
+  if (col >= cols_in || (WC % 64 != 0 && col >= WC))
+    return;
+  constexpr int U = 4; // rows in flight per lane
+#pragma unroll 1
+  for (int i0 = wn; i0 < WR / 4; i0 += 2 * U) {
+    f32x4_t g[U], v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int at = ((i0 + 2 * u) * 4 + rr) * W4_DUMP_PITCH + cc * 16;
+      g[u] = *reinterpret_cast<const f32x4_t *>(gate + at);
+      v[u] = *reinterpret_cast<const f32x4_t *>(up + at);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int row = wm * WR + (i0 + 2 * u) * 4 + rr;
+      if (row >= rows_in)
+        continue;
+      typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+      const uint2 o = gated_silu4(g[u], v[u]);
+      __builtin_nontemporal_store(u32x2_t{o.x, o.y}, reinterpret_cast<u32x2_t *>(reinterpret_cast<uint16_t *>(p.C) +
+                                                                                 (m0 + row) * p.ldc + n0 + col));
+    }
+  }
+}
+
 // K not a whole number of ring groups (four k-blocks of 64 bytes): the incomplete group [k_full, K) is the FIRST one
 // computed, and this puts it into the ring's four slots before the main loop starts: whole k-blocks by DMA, the block
 // that K ends in through registers with zeros behind K (in both operands, so no product of theirs counts, whatever the
@@ -1539,7 +1609,10 @@ __device__ __forceinline__ void w4_fill_k_tail(char *smem, int wave, int lane, c
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 }
 
-template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_body(GemmParams p) {
+// GATED: silu(A . B^T) * (A . up^T) of two weights [N,K]: the left half of a tile's columns are columns of B, the right half
+// the same columns of `up`, so each wave column has one of the two products (bf16, one pass, a single GEMM).
+template <int ES, bool TB, int MI, int NJ, bool GATED = false> __device__ __forceinline__ void w4_body(GemmParams p, const void *up = nullptr) {
+  static_assert(!GATED || (TB && ES == 2), "gated: bf16 weights stored [N,K]");
   // B stored [N,K]: bf16 only.  (The same loop for 8-bit operands -- plain 16-byte fragment reads in place of the
   // transposing ones -- was measured against [K,N] on one board and is no faster: 166.9-168.9 against 167.2-168.6 us
   // for the 4096 x 4096 x 11008 layer; an 8-bit weight stored [N,K] is copied once instead.)
@@ -1548,6 +1621,7 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
   constexpr int BM = 32 * MI, BN = 32 * NJ, BK = 64 / ES, NB = TB ? NJ : NJ / 2;
   constexpr int A_PAIR = BM * 128, B_PAIR = BN * 128, RING = Ring::DA * A_PAIR + Ring::DB * B_PAIR;
   constexpr int DUMP_WAVE = 16 * MI * W4_DUMP_PITCH, EPILOGUE = 4 * DUMP_WAVE + 3 * 256 * 4;
+  constexpr int CN = GATED ? BN / 2 : BN; // columns of C
   constexpr int B_ROW = BN * ES, B_CPR = B_ROW / 16, RG = ES == 2 ? 4 : 8; // B stored [K,N]: bytes and chunks of a k-row, k-rows per transposing read
 #ifdef GCMI_W4_TIMING
   const long long wall_entry = wall_clock64();
@@ -1563,12 +1637,12 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
   const int wm = wave >> 1, wn = wave & 1;
   const int r16 = lane & 15, g16 = lane >> 4;
 
-  const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN); // edge tiles stick out
+  const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + CN - 1) / CN); // edge tiles stick out
   int tm, tn;
   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, p.group_m, tm, tn);
   // integer division runs on the vector unit; the operand addresses below must be in scalar registers
   tm = __builtin_amdgcn_readfirstlane(tm), tn = __builtin_amdgcn_readfirstlane(tn);
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * CN;
   const int64_t lda_b = p.lda * ES, ldb_b = p.ldb * ES;
   const int64_t b_step = TB ? 64 : BK * ldb_b; // from k-block to k-block
   // (a row of A is shorter than 2^31 bytes, so K fits 32 bits)
@@ -1597,7 +1671,7 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
   // chunk that fills position c of row r is c ^ (r / 2 % 8); k-rows of a block of B stored [K,N].  An edge tile's rows past
   // M and columns past N are fetched from the last row / the last 16-byte chunk inside (N is a multiple of the
   // chunk's columns): their products land in accumulators that the epilogue never stores.
-  const int rows_in = (int)min((int64_t)BM, p.M - m0), cols_in = (int)min((int64_t)BN, p.N - n0);
+  const int rows_in = (int)min((int64_t)BM, p.M - m0), cols_in = (int)min((int64_t)CN, p.N - n0);
   // k-row k of B keeps chunk c at c ^ b_swz(k): the RG k-rows that a transposing read takes lie in different banks
   // (192 columns: rows of 384 bytes, k and k + 1 lie half the banks apart by themselves)
   auto b_swz = [](int k) { return BN == 192 ? ((k >> 1) & 1) * 4 : ES == 2 ? (k % 4) * 4 : BN == 256 ? (k % 8) * 2 : ((k % 8) >> 1) * 2; };
@@ -1612,7 +1686,7 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
   for (int i = 0; i < NB; i++) {
     if constexpr (TB) {
       const int row = (wave * NB + i) * 8 + lane / 8, c = (lane % 8) ^ ((row >> 1) & 7);
-      b_off[i] = (int)(min(row, cols_in - 1) * ldb_b + c * 16);
+      b_off[i] = (int)(min(GATED ? row % CN : row, cols_in - 1) * ldb_b + c * 16);
       b_k[i] = c * 16 / ES;
     } else {
       const int at = (wave * NB + i) * 64 + lane, krow = at / B_CPR;
@@ -1668,7 +1742,8 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
 
   // (inputs of the assembly in scalar registers)
   const char *const a0 = reinterpret_cast<const char *>(p.A) + m0 * lda_b + k_first * ES;
-  const char *const b0 = reinterpret_cast<const char *>(p.B) + (TB ? n0 * ldb_b + k_first * ES : n0 * ES + k_first * ldb_b);
+  // (gated: waves 0 and 1 request the rows of the left half, 2 and 3 those of the right one)
+  const char *const b0 = reinterpret_cast<const char *>(GATED && wave >= 2 ? up : p.B) + (TB ? n0 * ldb_b + k_first * ES : n0 * ES + k_first * ldb_b);
   uint64_t a_ptr = (uint64_t)a0, b_ptr = (uint64_t)b0;
   int pairs = __builtin_amdgcn_readfirstlane(2 * groups);
   const int tail_group = __builtin_amdgcn_readfirstlane(k_left);
@@ -1723,6 +1798,21 @@ template <int ES, bool TB, int MI, int NJ> __device__ __forceinline__ void w4_bo
 #ifdef GCMI_W4_TIMING
   const long long tick1 = clock64(), wall1 = wall_clock64();
 #endif
+  if constexpr (GATED) {
+    const char *const gate = smem + 2 * wm * DUMP_WAVE, *const other = gate + DUMP_WAVE;
+    __syncthreads();
+    w4_gated_half<16 * MI, 16 * NJ>(p, 0, m0, n0, wm, wn, lane, gate, other, rows_in, cols_in);
+    if constexpr (NJ > 4) {
+      __syncthreads(); // the other wave has read this one's region
+      if constexpr (NJ == 8)
+        asm volatile(GCMI_W4_ASM_DUMP_HI_8x8 : : "{v28}"(dump_ld) : "memory");
+      else
+        asm volatile(GCMI_W4_ASM_DUMP_HI_8x6 : : "{v28}"(dump_ld) : "memory");
+      __syncthreads();
+      w4_gated_half<16 * MI, 16 * NJ>(p, 1, m0, n0, wm, wn, lane, gate, other, rows_in, cols_in);
+    }
+    return;
+  }
   // the column parameters were requested before the main loop and are first needed here
   colp[tid] = cp_bias;
   if (ES == 1) {

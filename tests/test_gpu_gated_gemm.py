@@ -1,0 +1,99 @@
+"""silu(x . Wg^T) * (x . Wu^T) as one launch (gemm_gated.hip) against one launch per op, in every form that sizes select."""
+import importlib
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mm(gc):
+    return importlib.import_module("graph_compiler_amd.mlir_modules")
+
+
+def _module(mm, T, K, N):
+    f = mm._Fn()
+    tw = mm.ttype([T, N], "bf16")
+    gate = mm._matmul(f, "matmul_transpose_b", "%arg0", [T, K], "%arg1", [N, K], [T, N], "bf16")
+    one = mm._splat(f, 1.0, [T, N], "bf16")
+    ex = mm._named(f, "exp", [mm._named(f, "negf", [gate], [tw], [T, N], "bf16")], [tw], [T, N], "bf16")
+    sig = mm._binary(f, "div", one, mm._binary(f, "add", one, ex, [T, N], "bf16"), [T, N], "bf16")
+    silu = mm._binary(f, "mul", sig, gate, [T, N], "bf16")
+    up = mm._matmul(f, "matmul_transpose_b", "%arg0", [T, K], "%arg2", [N, K], [T, N], "bf16")
+    out = mm._binary(f, "mul", silu, up, [T, N], "bf16")
+    args = [mm.ttype([T, K], "bf16"), mm.ttype([N, K], "bf16"), mm.ttype([N, K], "bf16")]
+    return mm._module(args, [tw], f, [out])
+
+
+def _run(ga, text, ins, out):
+    comp = ga.Compiler()
+    st, exe = comp.compile_mlir(text)
+    assert st == 0, ga.api().dnnl_graph_compiler_last_error().decode()
+    try:
+        assert exe.bind(list(enumerate(ins)), [(len(ins), out)], torch.cuda.current_stream().cuda_stream)() == 0
+        torch.cuda.synchronize()
+    finally:
+        exe.close()
+        comp.close()
+
+
+def _exact(dev, T, K, N, seed):
+    """Small integers times a power of two: every sum is exact in f32 in any order, so both ways have the same bits."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    r = lambda s, *shape: (torch.randint(-3, 4, shape, device=dev, generator=g) * s).bfloat16()  # noqa: E731
+    return [r(1.0, T, K), r(2.0 ** -6, N, K), r(2.0 ** -6, N, K)]
+
+
+# few rows: 1 to 4 column tiles per product, whole and cut workgroups, more than one round of them; tiles of 128 to 256 rows
+# by 64 to 128 columns, rows and columns off the tile, a K that ends inside a group
+FEW = [(1, 512, 4096), (31, 512, 4108), (32, 640, 11008), (33, 512, 13000), (64, 512, 4100), (64, 512, 16900), (17, 1024, 2816)]
+TILES = [(65, 512, 4108), (128, 520, 4100), (129, 512, 11008), (200, 1032, 2816), (257, 512, 11004), (300, 640, 5632),
+         (513, 512, 8200), (700, 520, 8204), (1000, 512, 11008), (1000, 1024, 5632)]
+
+
+@pytest.mark.parametrize("T,K,N", FEW + TILES)
+def test_bits_of_single_ops(ga, mm, dev, monkeypatch, T, K, N):
+    text = _module(mm, T, K, N)
+    ins = _exact(dev, T, K, N, T + K + N)
+    ins[0][0, 3] = float("inf")  # a row of infinities and NaNs, and no other
+    full = torch.full((T + 1, N), 7.0, device=dev, dtype=torch.bfloat16)
+    fused, single = full[:T], torch.empty(T, N, device=dev, dtype=torch.bfloat16)
+    st, plan = ga.explain_mlir(text)
+    assert st == 0
+    _run(ga, text, ins, fused)
+    monkeypatch.setenv("GCMI_NO_POINTWISE_FUSION", "1")
+    _run(ga, text, ins, single)
+    assert "MatMul x2" in plan and "MatMul x2" not in ga.explain_mlir(text)[1]
+    assert torch.equal(fused.view(torch.int16), single.view(torch.int16))
+    assert (full[T] == 7.0).all() and not fused[1:].isnan().any()
+
+
+@pytest.mark.parametrize("T,K,N", [(32, 4096, 11008), (200, 2048, 5632)])
+def test_error(ga, mm, dev, T, K, N):
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(T, K, device=dev, generator=g).bfloat16()
+    Wg, Wu = ((torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16() for _ in range(2))
+    out = torch.empty(T, N, device=dev, dtype=torch.bfloat16)
+    _run(ga, _module(mm, T, K, N), [x, Wg, Wu], out)
+    xd, gd, ud = x.double(), Wg.double(), Wu.double()
+    gate, up = xd @ gd.t(), xd @ ud.t()
+    eg, eu = ((K + 1) * 2.0 ** -24 * (xd.abs() @ w.abs().t()) for w in (gd, ud))  # f32 sums in any order
+    silu = gate * torch.sigmoid(gate)
+    # five roundings to bf16, half an ulp each: up, sigmoid, silu, the result, and gate, whose error silu passes on by a factor
+    # of up to 1 + |gate|; no slope of silu above 1.1
+    bound = 1.01 * (2.0 ** -9 * (5 + gate.abs()) * (silu * up).abs() + 1.1 * up.abs() * eg + silu.abs() * eu)
+    assert ((out.double() - silu * up).abs() <= bound).all()
+
+
+def test_operands_off_16_bytes_take_the_separate_steps(ga, mm, dev):
+    T, K, N = 32, 512, 4100
+    ins = _exact(dev, T, K, N, 1)
+    text = _module(mm, T, K, N)
+    want, out = (torch.empty(T, N, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    _run(ga, text, ins, want)
+    off = torch.empty(N * K + 4, device=dev, dtype=torch.bfloat16)[4:].view(N, K)
+    off.copy_(ins[2])
+    assert off.data_ptr() % 16 == 8
+    _run(ga, text, [ins[0], ins[1], off], out)
+    assert torch.equal(out, want)
