@@ -19,6 +19,9 @@ int gcmi_launch_eltwise(const gcmi::EltParams *p, hipStream_t stream);
 int gcmi_launch_reduce(const gcmi::ReduceParams *p, hipStream_t stream);
 int gcmi_launch_fused(const gcmi::FusedParams *p, hipStream_t stream);
 int gcmi_launch_softmax(const gcmi::SoftmaxParams *p, hipStream_t stream);
+int gcmi_gemm_bf16_slices(const void *A, const void *B, void *C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                          int trans_b, const void *residual, int64_t ldr, void *workspace, size_t workspace_bytes, int splits,
+                          int32_t *left, void *stream);
 int gcmi_launch_gemm_gated(const gcmi::GemmParams *p, const void *up, hipStream_t stream, int dry, gcmi::GemmTileConfig *cfg);
 }
 
@@ -203,6 +206,7 @@ void Executable::init(bool dry) {
   plan();
   plan_gates();
   plan_workspaces();
+  plan_slices();
   layout_arena();
   if (dry)
     return;
@@ -246,6 +250,8 @@ char *Executable::staging() {
 // silu(x . Wg^T) * (x . Wu^T), the gate of a feed-forward layer: two GEMMs of one operand and the point-wise group that
 // reads nothing but them become one step where a kernel takes them (gemm_gated.hip).  A MatmulConfig on either keeps
 // both as they are.
+static gcjit::FusedKernelSource generate_step(const Step &s, size_t i);
+
 static gcmi::GemmParams gated_params(const Step &s) {
   gcmi::GemmParams p{};
   p.M = s.M, p.N = s.N, p.K = s.K, p.lda = s.lda, p.ldb = s.ldb, p.ldc = s.ldc;
@@ -329,6 +335,33 @@ void Executable::plan_workspaces() {
       plan(part);
   }
 }
+// A GEMM cut into K slices whose result the next step normalises: the row kernel adds the slices (and the residual) as it
+// reads its row and stores the GEMM's result beside its own, so the GEMM's second pass is left out.  One launch in
+// place of two and the row is not read back, us: 32 x 4096 (4 slices) 3.8 + 4.1 / 4.7, 1000 x 4096 (2 slices) 12.9 + 6.8 / 12.5.
+void Executable::plan_slices() {
+  const char *off = getenv("GCMI_NO_GENERATED_KERNELS");
+  if (off && off[0] == '1')
+    return;
+  for (size_t i = 0; i + 1 < steps_.size(); i++) {
+    Step &g = steps_[i], &r = steps_[i + 1];
+    if (g.kind != Step::GemmBf16 || g.ws < 0 || g.batch > 1 || g.ta || g.once || r.once || g.bias >= 0 || g.act != 0 || g.out_dt != GCMI_BF16 ||
+        (g.c >= 0 && g.b_dt != GCMI_BF16) || !g.mm_cfg.empty() || g.a_off || g.b_off || g.out_off || g.ldc != g.N || r.kind != Step::Fused ||
+        r.sum_ins < 0 || r.row_end < 0 || r.n_red != g.N || g.out == g.c || r.out == g.out || r.out == g.c)
+      continue;
+    const auto in = std::find(r.f_in.begin(), r.f_in.end(), g.out);
+    gcmi_gemm_tile_config c{};
+    if (in == r.f_in.end() || prod(r.dims, 0, r.dims.size()) != g.M * g.N ||
+        gcmi_gemm_tile_config_query(GCMI_BF16, g.M, g.N, g.K, g.tb ? 1 : 0, g.out_dt, nullptr, &c, nullptr, 0) != 0 || c.split_k < 2 ||
+        slots_[(size_t)g.ws].bytes < (size_t)c.split_k * (size_t)(g.M * g.N) * 4)
+      continue;
+    r.sliced_in = (int)(in - r.f_in.begin()), r.sliced_splits = c.split_k, r.ws = g.ws, r.c = g.c;
+    if (generate_step(r, i + 1).sliced)
+      g.next_splits = c.split_k;
+    else
+      r.sliced_in = r.ws = r.c = -1, r.sliced_splits = 0;
+  }
+}
+
 void Executable::layout_arena() {
   const int n = (int)slots_.size();
   std::vector<int> first(n, -1), last(n, -1);
@@ -1517,6 +1550,31 @@ static int fused_registers(const Step &s) {
   return gcmi::fused_allocate(p);
 }
 
+// The kernel of a fused step; an empty source where the generator does not cover it.
+static gcjit::FusedKernelSource generate_step(const Step &s, size_t i) {
+  gcmi::FusedParams p{};
+  fill_fused_params(s, p);
+  int same_as[gcmi::FUSED_MAX_IN];
+  for (int k = 0; k < p.n_in; k++) {
+    same_as[k] = -1;
+    for (int j = 0; j < k && same_as[k] < 0; j++)
+      if (s.f_in[(size_t)j] == s.f_in[(size_t)k] && s.f_str[(size_t)j] == s.f_str[(size_t)k] && p.in_dt[j] == p.in_dt[k])
+        same_as[k] = j;
+  }
+  gcjit::SlicedInput sliced;
+  if (s.sliced_in >= 0) {
+    sliced.k = s.sliced_in, sliced.splits = s.sliced_splits, sliced.residual = s.c >= 0;
+    for (int k = 0; k < p.n_in; k++) // the same tensor read in another way would be read from memory
+      if (k != sliced.k && s.f_in[(size_t)k] == s.f_in[(size_t)sliced.k] && same_as[k] != sliced.k)
+        return {};
+  }
+  gcjit::FusedKernelSource k;
+  if (!gcjit::generate_fused(p, same_as, "gcmi_fused_step" + std::to_string(i), k, sliced))
+    return {};
+  k.source = "// " + s.note + "\n" + k.source;
+  return k;
+}
+
 // Kernels specialised for the fused groups of this plan (jit/fused_jit.h).  GCMI_NO_GENERATED_KERNELS=1 keeps the
 // library's interpreter kernels, which compute the same bits (tests compare the two).  A group the generator does not
 // cover, or a compiler that is missing or fails, also leaves the interpreter in place.
@@ -1534,20 +1592,9 @@ std::vector<gcjit::FusedKernelSource> Executable::generated_kernels() const {
     }
     if (s.kind != Step::Fused)
       continue;
-    gcmi::FusedParams p{};
-    fill_fused_params(s, p);
-    int same_as[gcmi::FUSED_MAX_IN];
-    for (int k = 0; k < p.n_in; k++) {
-      same_as[k] = -1;
-      for (int j = 0; j < k && same_as[k] < 0; j++)
-        if (s.f_in[(size_t)j] == s.f_in[(size_t)k] && s.f_str[(size_t)j] == s.f_str[(size_t)k] && p.in_dt[j] == p.in_dt[k])
-          same_as[k] = j;
-    }
-    gcjit::FusedKernelSource k;
-    if (gcjit::generate_fused(p, same_as, "gcmi_fused_step" + std::to_string(i), k)) {
-      k.source = "// " + s.note + "\n" + k.source;
+    gcjit::FusedKernelSource k = generate_step(s, i);
+    if (!k.source.empty())
       ks.push_back(std::move(k));
-    }
   }
   return ks;
 }
@@ -1578,6 +1625,17 @@ void Executable::build_generated_kernels() {
   }
 }
 
+// The generated kernel of a fused step is there and takes its operands' addresses.
+bool Executable::generated_takes(const Step &s) const {
+  if (!s.jit_fn)
+    return false;
+  auto aligned = [&](int slot) { return slot < 0 || (reinterpret_cast<uintptr_t>(ptr_[(size_t)slot]) & 15) == 0; };
+  bool all = aligned(s.out) && (s.sliced_in < 0 || (aligned(s.ws) && aligned(s.c)));
+  for (int slot : s.f_in)
+    all = all && aligned(slot);
+  return all || !s.jit_vectors;
+}
+
 // ---------------------------------------------------------------------------
 void Executable::launch(const Step &s) {
   auto P = [&](int slot) -> char * { return slot < 0 ? nullptr : (char *)ptr_[(size_t)slot]; };
@@ -1589,6 +1647,13 @@ void Executable::launch(const Step &s) {
              "MatMul f32");
     break;
   case Step::GemmBf16:
+    slices_left_ = 0;
+    if (s.next_splits && generated_takes(*(&s + 1))) { // (steps_ in their order)
+      gc_check(gcmi_gemm_bf16_slices(P(s.a), P(s.b), P(s.out), s.M, s.N, s.K, s.lda, s.ldb, s.ldc, s.tb ? 1 : 0, P(s.c), s.N, P(s.ws),
+                                     slots_[(size_t)s.ws].bytes, s.next_splits, &slices_left_, stream_),
+               "MatMul bf16");
+      break;
+    }
     // s.c: the residual tensor (same shape as the result), s.b_dt its type
     gc_check(gcmi_gemm_bf16_ws(P(s.a) + s.a_off * 2, P(s.b) + s.b_off * 2,
                                P(s.out) + s.out_off * (s.out_dt == GCMI_BF16 ? 2 : 4), s.batch, s.M, s.N, s.K, s.lda, s.ldb,
@@ -1697,19 +1762,19 @@ void Executable::launch(const Step &s) {
     }
     if ((size_t)(second_pass ? p.n : p.n / p.n_red) * (size_t)esz(p.out_dt) > slots_[(size_t)s.out].bytes)
       throw std::runtime_error("fused group: the result does not fit its buffer (" + s.note + ")");
-    if (s.jit_fn) {
-      bool aligned = (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+    // (a kernel that adds K slices is of no use where they were added already)
+    if (generated_takes(s) && (s.sliced_in < 0 || slices_left_)) {
+      void *args[gcmi::FUSED_MAX_IN + 4], *part = P(s.ws), *addend = P(s.c), *result = nullptr;
       for (int k = 0; k < p.n_in; k++)
-        aligned = aligned && (reinterpret_cast<uintptr_t>(p.in[k]) & 15) == 0;
-      if (aligned || !s.jit_vectors) {
-        void *args[gcmi::FUSED_MAX_IN + 1];
-        for (int k = 0; k < p.n_in; k++)
-          args[k] = (void *)&p.in[k];
-        args[p.n_in] = (void *)&p.out;
-        hip_check(hipModuleLaunchKernel(s.jit_fn, s.jit_grid, 1, 1, s.jit_block, 1, 1, 0, stream_, args, nullptr), s.note.c_str());
-        g_generated_launches++;
-        break;
+        args[k] = (void *)&p.in[k];
+      args[p.n_in] = (void *)&p.out;
+      if (s.sliced_in >= 0) {
+        result = P(s.f_in[(size_t)s.sliced_in]);
+        args[p.n_in + 1] = &part, args[p.n_in + 2] = &addend, args[p.n_in + 3] = &result;
       }
+      hip_check(hipModuleLaunchKernel(s.jit_fn, s.jit_grid, 1, 1, s.jit_block, 1, 1, 0, stream_, args, nullptr), s.note.c_str());
+      g_generated_launches++;
+      break;
     }
     gc_check(gcmi_launch_fused(&p, stream_) ? 5 : 0, s.note.c_str());
     break;
@@ -1890,6 +1955,8 @@ std::string Executable::describe() const {
         os << "\n";
       }
     }
+    if (s.sliced_in >= 0)
+      os << "  adds the " << s.sliced_splits << " K slices of the GEMM before it\n";
     if (s.kind == Step::GemmGated) {
       const gcmi::GemmParams p = gated_params(s);
       gcmi::GemmTileConfig c{};

@@ -84,6 +84,9 @@ struct Step {
   hipFunction_t jit_fn = nullptr;
   unsigned jit_grid = 0, jit_block = 0;
   bool jit_vectors = false; // it moves 16-byte vectors: the operands must be aligned
+  // a GEMM whose K slices the next step, a row kernel, adds itself (next_splits of them), and that row kernel: which of its inputs
+  // they are, how many, and the GEMM's residual (slot c) and workspace (slot ws)
+  int next_splits = 0, sliced_in = -1, sliced_splits = 0;
   // gated pair of GEMMs (a . b and a . c, then their point-wise group): the steps it stands for, which run where its kernels
   // do not take the operands' addresses
   std::vector<Step> parts;
@@ -125,6 +128,7 @@ private:
   std::vector<Step> steps_;
   std::vector<Slot> slots_;
   std::unordered_map<size_t, int> slot_of_tensor_;
+  int32_t slices_left_ = 0; // the GEMM just launched left its K slices to the next step (guarded by run_mu_)
   std::vector<void *> ptr_; // per-slot device pointer during execute (guarded by run_mu_)
   // execute() may be called from several host threads (the reference's execute is const and re-entrant,
   // src/dnnl/dnnl_graph_compiler.cpp:214-226): calls on one executable take turns, since they share its arena
@@ -155,6 +159,8 @@ private:
   void plan();
   void plan_gates();
   void plan_workspaces();
+  void plan_slices();
+  bool generated_takes(const Step &s) const;
   void layout_arena();
   void plan_generic(const Op &op);
   void plan_fusion(std::vector<bool> &skip, const std::vector<bool> &claimed, std::map<size_t, std::vector<Step>> &emit_at,

@@ -280,7 +280,7 @@ int gemm_bf16_any(bool trans_b, const void *A, const void *B, void *C, int64_t M
                   int64_t ldb, int64_t ldc, const void *bias, int bias_dtype, int act, int out_dtype, void *stream,
                   int64_t batch = 1, int64_t a_bs = 0, int64_t b_bs = 0, int64_t c_bs = 0, const void *residual = nullptr,
                   int64_t ldr = 0, int residual_dtype = 0, Ws ws_from = Ws::Library, void *ws = nullptr,
-                  size_t ws_bytes = 0, const int64_t *matmul_config = nullptr);
+                  size_t ws_bytes = 0, const int64_t *matmul_config = nullptr, int leave_splits = 0, int32_t *left = nullptr);
 }
 
 extern "C" int gcmi_gemm_bf16(const void *A, const void *B, void *C, int64_t M, int64_t N, int64_t K, int64_t lda,
@@ -338,7 +338,8 @@ namespace {
 int gemm_bf16_any(bool trans_b, const void *A, const void *B, void *C, int64_t M, int64_t N, int64_t K, int64_t lda,
                   int64_t ldb, int64_t ldc, const void *bias, int bias_dtype, int act, int out_dtype, void *stream,
                   int64_t batch, int64_t a_bs, int64_t b_bs, int64_t c_bs, const void *residual, int64_t ldr,
-                  int residual_dtype, Ws ws_from, void *ws, size_t ws_bytes, const int64_t *matmul_config) {
+                  int residual_dtype, Ws ws_from, void *ws, size_t ws_bytes, const int64_t *matmul_config, int leave_splits,
+                  int32_t *left) {
   if (M < 0 || N < 0 || K < 0)
     return fail(ST_INVALID, "gemm_bf16: negative size");
   if (M == 0 || N == 0)
@@ -373,6 +374,7 @@ int gemm_bf16_any(bool trans_b, const void *A, const void *B, void *C, int64_t M
     if (ws && (reinterpret_cast<uintptr_t>(ws) & 15) != 0)
       return fail(ST_INVALID, "gemm_bf16: workspace is not 16-byte aligned");
     p.partial = ws_bytes >= 4 ? (float *)ws : nullptr, p.partial_cap = (int64_t)(ws_bytes / 4);
+    p.leave_splits = left ? leave_splits : 0, p.left = left;
     return launched(gcmi_launch_gemm_bf16(&p, (hipStream_t)stream), "gemm_bf16");
   }
   if (ws_from == Ws::Static) {
@@ -454,6 +456,17 @@ extern "C" int gcmi_gemm_bf16_ws(const void *A, const void *B, void *C, int64_t 
   return gemm_bf16_any(trans_b != 0, A, B, C, M, N, K, lda, ldb, ldc, bias, bias_dtype, act, out_dtype, stream, batch,
                        stride_a, stride_b, stride_c, residual, ldr, residual_dtype, Ws::Caller, workspace,
                        workspace_bytes, matmul_config);
+}
+
+// C = A . B (+ residual, bf16 like all of them) in a compiled partition, for a next kernel that can add `splits` K slices itself:
+// *left = 1 where the call was cut into just that many and their sums are in the workspace, C not written; else 0 and C is
+// the result.
+extern "C" int gcmi_gemm_bf16_slices(const void *A, const void *B, void *C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                                     int64_t ldb, int64_t ldc, int trans_b, const void *residual, int64_t ldr, void *workspace,
+                                     size_t workspace_bytes, int splits, int32_t *left, void *stream) {
+  *left = 0;
+  return gemm_bf16_any(trans_b != 0, A, B, C, M, N, K, lda, ldb, ldc, nullptr, GCMI_BF16, GCMI_ACT_NONE, GCMI_BF16, stream, 1, 0, 0,
+                       0, residual, ldr, GCMI_BF16, Ws::Caller, workspace, workspace_bytes, nullptr, splits, left);
 }
 
 extern "C" int gcmi_gemm_tile_config_query(int a_dtype, int64_t M, int64_t N, int64_t K, int trans_b, int out_dtype,

@@ -186,11 +186,13 @@ struct Gen {
     }
   }
 
+  bool sliced = false;
   void signature(const std::string &name, int threads) {
     o << "extern \"C\" __global__ __launch_bounds__(" << threads << ") void " << name << "(";
     for (int k = 0; k < p.n_in; k++)
       o << "const void *__restrict__ in" << k << ", ";
-    o << "void *__restrict__ out) {\n";
+    o << "void *__restrict__ out" << (sliced ? ", const float *__restrict__ part, const void *__restrict__ addend, void *__restrict__ result" : "")
+      << ") {\n";
   }
 };
 
@@ -213,7 +215,8 @@ bool wide_indices(const FusedParams &p) {
 
 } // namespace
 
-bool generate_fused(const FusedParams &raw, const int *same_as, const std::string &name, FusedKernelSource &out) {
+bool generate_fused(const FusedParams &raw, const int *same_as, const std::string &name, FusedKernelSource &out,
+                    const SlicedInput &sliced) {
   FusedParams p = raw;
   if (p.n <= 0 || gcmi::fused_prepare(p, true) != 0)
     return false;
@@ -226,6 +229,8 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
   std::ostringstream &o = g.o;
   out.name = name, out.n_in = p.n_in, out.quad = p.quad != 0;
 
+  if (!has_sum && sliced.k >= 0)
+    return false;
   if (!has_sum) {
     const int threads = 256;
     const int64_t chunk = 4 * threads, steps = (p.n + chunk - 1) / chunk;
@@ -290,6 +295,24 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
   for (int j = p.sum_ins + 1; j < p.row_end; j++)
     g.widths[(size_t)(p.n_in + j)] = 1;
 
+  const int64_t step_elems = (int64_t)tpr * 4, trips = (p.n_red + step_elems - 1) / step_elems;
+  if (sliced.k >= 0) {
+    // a first-pass input in dense bf16 rows that nothing else reads but a second pass from registers, and few enough loads to
+    // have all in flight (16 bytes per slice and trip)
+    const int k = sliced.k;
+    bool ok = p.quad && k < p.n_in_pre && p.in_dt[k] == gcmi::DT_BF16 && ((p.vec_mask >> k) & 1) && trips <= 8 && second_pass && same_as &&
+              trips * sliced.splits <= 24;
+    int64_t dense = 1;
+    for (int d = last; d >= d0; d--) {
+      ok = ok && p.in_str[k][d] == dense;
+      dense *= p.dims[d];
+    }
+    for (int j = 0; j < p.n_in; j++)
+      ok = ok && (j == k || (same_as[j] != k && same_as[k] != j) || (same_as[j] == k && j >= p.n_in_row));
+    if (!ok)
+      return false;
+    g.sliced = out.sliced = true;
+  }
   g.signature(name, threads);
   if (tpr > 64)
     o << "  __shared__ float wave_sum[" << threads / 64 << "];\n";
@@ -312,7 +335,6 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
     }
     g.offsets("row", d0, d_row, t, "  ");
   }
-  const int64_t step_elems = (int64_t)tpr * 4, trips = (p.n_red + step_elems - 1) / step_elems;
   // A second-pass input that is a first-pass input again (the row that is normalised) is not read twice when a
   // thread's share of the row is small enough to stay in registers.
   g.keep_from.assign((size_t)p.n_in, -1);
@@ -389,6 +411,10 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
     for (int k = 0; k < p.n_in; k++) {
       const bool pass1 = k < p.n_in_pre, pass2 = second_pass && k >= p.n_in_row && g.keep_from[(size_t)k] < 0;
       const int need = (int)trips * (p.in_dt[k] == gcmi::DT_F32 ? 4 : 2);
+      if (k == sliced.k) {
+        regs += need, g.ahead[(size_t)k] = 1;
+        continue;
+      }
       if ((!pass1 && !pass2) || !((p.vec_mask >> k) & 1) || regs + need > 64)
         continue;
       regs += need;
@@ -402,6 +428,26 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
       o << "      raw" << k << "[it_] = *reinterpret_cast<const " << t << " *>(reinterpret_cast<const " << Gen::ctype(p.in_dt[k])
         << " *>(in" << k << ") + off" << k << ");\n    }\n  }\n";
     }
+  }
+  if (sliced.k >= 0) {
+    const std::string n = std::to_string(sliced.k), off = "base" + n + " + e", S = std::to_string(sliced.splits);
+    const std::string head = "#pragma unroll\n  for (int it_ = 0; it_ < " + std::to_string(trips) + "; it_++) {\n    const " + g.idx + " e = (" +
+                             g.idx + ")it_ * " + std::to_string(step_elems) + " + 4 * (" + g.idx + ")sub;\n    if (e < (" + g.idx + ")" +
+                             Gen::num(p.n_red) + ") {\n";
+    o << "  f4_ part_[" << trips << "][" << S << "] = {};\n  u2_ add_[" << trips << "] = {}, raw" << n << "[" << trips << "] = {};\n";
+    o << head << "#pragma unroll\n      for (int s_ = 0; s_ < " << S << "; s_++)\n        part_[it_][s_] = *reinterpret_cast<const f4_ *>(part + s_ * "
+      << p.n << "ll + " << off << ");\n";
+    if (sliced.residual)
+      o << "      add_[it_] = *reinterpret_cast<const u2_ *>(reinterpret_cast<const unsigned short *>(addend) + " << off << ");\n";
+    o << "    }\n  }\n" << head << "      f4_ v_ = part_[it_][0];\n#pragma unroll\n      for (int s_ = 1; s_ < " << S
+      << "; s_++)\n        v_ += part_[it_][s_];\n      float q_[4] = {v_[0], v_[1], v_[2], v_[3]};\n      gcmi::round_bf16_quad(q_);\n";
+    if (sliced.residual)
+      o << "      q_[0] += gcmi::bf16_bits_to_f32((unsigned short)add_[it_][0]); q_[1] += gcmi::bf16_bits_to_f32((unsigned short)(add_[it_][0] >> 16));\n"
+           "      q_[2] += gcmi::bf16_bits_to_f32((unsigned short)add_[it_][1]); q_[3] += gcmi::bf16_bits_to_f32((unsigned short)(add_[it_][1] >> 16));\n"
+           "      gcmi::round_bf16_quad(q_);\n";
+    o << "      raw" << n << "[it_] = u2_{(__float_as_uint(q_[0]) >> 16) | (__float_as_uint(q_[1]) & 0xffff0000u), (__float_as_uint(q_[2]) >> 16) | "
+         "(__float_as_uint(q_[3]) & 0xffff0000u)};\n      if (live)\n        *reinterpret_cast<u2_ *>(reinterpret_cast<unsigned short *>(result) + "
+      << off << ") = raw" << n << "[it_];\n    }\n  }\n";
   }
   o << "  float acc = 0.0f;\n";
   row_loop(0, p.n_in_pre, 0, p.sum_ins, false);

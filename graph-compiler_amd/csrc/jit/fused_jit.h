@@ -28,13 +28,24 @@ struct FusedKernelSource {
   std::string name, source;
   unsigned grid = 0, block = 0;
   int n_in = 0;
+  bool sliced = false; // has the arguments of a SlicedInput
   bool quad = false; // moves 16- or 8-byte vectors: every operand address must be 16-byte aligned
+};
+
+// A first-pass input of a row kernel that a K-sliced bf16 GEMM leaves as its partial sums: the kernel adds the slices in
+// ascending order, rounds, adds the residual, rounds (what the GEMM's second pass does), and stores that result too.  Three
+// arguments more behind `out`: the sums [splits][rows][row length] f32, the residual or null, the result.
+struct SlicedInput {
+  int k = -1; // which input; -1: none
+  int splits = 0;
+  bool residual = false;
 };
 
 // Writes the kernel for `p` (pointers are not read: they become kernel arguments in[0] .. in[n_in-1], out).
 // same_as[k] = j < k: input k is the same tensor, read through the same strides, as input j (-1: not known to be).
 // Returns false when the program is not one the generator covers (the caller keeps the interpreter).
-bool generate_fused(const gcmi::FusedParams &p, const int *same_as, const std::string &name, FusedKernelSource &out);
+bool generate_fused(const gcmi::FusedParams &p, const int *same_as, const std::string &name, FusedKernelSource &out,
+                    const SlicedInput &sliced = SlicedInput());
 
 // The kernel for a softmax along the innermost axis of a [rows, len] view (arguments: in0, out).  Returns false for
 // rows too long to keep in registers (the library's kernel runs those).

@@ -39,6 +39,10 @@ struct GemmParams {
   int32_t cfg_waves;    // 4 or 8 waves per workgroup on whole tiles
   int32_t cfg_split_k;  // number of K slices (1: none) where the shape can be sliced
   int32_t cfg_tile;     // 128: the 128 x 128 tile kernel where the shape allows it; 256: never that kernel
+  // a caller whose next kernel adds the K slices itself: cut into exactly this many, the partial sums stay in `partial`
+  // ([slice][M][N]), C is not written and *left (host memory) becomes 1
+  int32_t leave_splits; // 0: never
+  int32_t *left;
 };
 
 // What the launcher decides for one GEMM call: the GPU's counterpart of the reference's MatmulConfig

@@ -1987,6 +1987,10 @@ template <int ACT> __global__ __launch_bounds__(256) void gemm_splitk_reduce_ker
 
 // second pass of every K-sliced GEMM: one thread per four outputs, the activation as a template argument
 static void launch_splitk_reduce(const GemmParams &p, hipStream_t stream) {
+  if (p.leave_splits > 1 && p.leave_splits == p.splits) {
+    *p.left = 1;
+    return;
+  }
   const dim3 grid((unsigned)((p.M * (p.N / 4) + 255) / 256)), block(256);
   switch (p.act) {
   case ACT_RELU:
