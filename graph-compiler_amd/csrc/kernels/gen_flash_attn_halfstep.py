@@ -26,9 +26,12 @@ Fixed registers (the kernel binds its variables to them with register constraint
   %[koff]     immediate: byte offset of the K half tile (stage * 32768 + half * 8192)
   %[voff]     immediate: byte offset of the V half tile (stage * 32768 + 16384 + half * 8192)
 
-Head dim 64 (the second pair of macros): 4 d slices and 2 d tiles, i.e. 4 S + 4 PV MFMAs for the same vector work;
-O^T in v[0:31], Q fragments in v[96:111], K addresses in v[128:131], V addresses in v[136:137], V rows 128 bytes
-apart.  That half step is bound by the vector ALU: its first four slots carry ten vector instructions each.
+Head dim 64 (the second pair of macros): 4 d slices and 2 d tiles, i.e. 4 S + 4 PV MFMAs for the same vector work, V rows
+128 bytes apart.  That half step is bound by the vector ALU: its first four slots carry ten vector instructions each.  Its
+registers are packed so that four waves fit a SIMD (what one wave waits for, the others' vector work fills):
+  v[0:31]  O^T     v[32:47], v[48:63]  score tiles     v[64:79]  Q     v[80:83]  K addresses     v[84:85]  V addresses
+  v86 row sum   v87 offset of the exponent   v88 out: maximum   v[90:105]  K fragments   v[106:113]  V fragments of the first
+  16 keys (those of the others follow the K fragments of d slices 0 and 1, multiplied by then)   v89  scratch
 
 Wait states kept by construction (the assembler does not add them inside an asm statement):
   LDS data        -> MFMA       s_waitcnt lgkmcnt(n), counted here
@@ -42,12 +45,17 @@ import os
 import sys
 
 OPTS = set(filter(None, os.environ.get("GCMI_FA_OPTS", "").split(",")))  # experiments: nolds noexp novalu nomax nowait
-O, SA, SB, QF, KA, VA, L, NM, MRAW, ONES, KF, VF, TMP = 0, 64, 80, 96, 128, 136, 140, 141, 142, 143, 144, 176, 208
+O = 0
+#           score tiles  Q   K, V addresses  sum  offset  maximum  K frags  V frags of chunks 0, 1  scratch
+MAP = {128: (64, 80,     96, 128, 136,       140, 141,    142,     144,     (176, 192),             208),
+       64:  (32, 48,     64, 80,  84,        86,  87,     88,      90,      (106, 90),              89)}
 
 
-def gen(cur, nxt, D=128):
+def gen(second, D=128):
     """D = 128: 16 MFMAs (8 S, 8 PV) per half step.  D = 64: 4 d slices and 2 d tiles, i.e. 8 MFMAs for the same vector
     work -- that variant is bound by the vector ALU, and its slots take eight vector instructions each."""
+    SA, SB, QF, KA, VA, L, NM, MRAW, KF, VF, TMP = MAP[D]
+    cur, nxt = (SB, SA) if second else (SA, SB)
     out = []
     emit = out.append
     lds = []  # LDS reads in issue order (names)
@@ -60,7 +68,7 @@ def gen(cur, nxt, D=128):
         lds.append("k%d" % ds)
 
     def read_v(ch, dt):  # chunk ch = 16 keys = 16 rows of the V tile; the second read is 8 rows further
-        r = VF + 16 * ch + 4 * dt
+        r = VF[ch] + 4 * dt
         emit("ds_read_b64_tr_b16 v[%d:%d], v%d offset:%%[voff]+%d" % (r, r + 1, VA + dt, ch * 16 * ROWB))
         emit("ds_read_b64_tr_b16 v[%d:%d], v%d offset:%%[voff]+%d" % (r + 2, r + 3, VA + dt, ch * 16 * ROWB + 8 * ROWB))
         lds.append("v%d%d_lo" % (ch, dt))
@@ -134,7 +142,7 @@ def gen(cur, nxt, D=128):
             wait_for("v%d%d" % (ch, dt))
             acc = "v[%d:%d]" % (O + 16 * dt, O + 16 * dt + 15)
             pw = cur + 8 * ch
-            emit("v_mfma_f32_32x32x16_bf16 %s, v[%d:%d], v[%d:%d], %s" % (acc, VF + 16 * ch + 4 * dt, VF + 16 * ch + 4 * dt + 3, pw,
+            emit("v_mfma_f32_32x32x16_bf16 %s, v[%d:%d], v[%d:%d], %s" % (acc, VF[ch] + 4 * dt, VF[ch] + 4 * dt + 3, pw,
                                                                       pw + 3, acc))
         if k_ahead + slot < NDS:
             read_k(k_ahead + slot)
@@ -204,11 +212,12 @@ def main():
     with open(path, "w") as f:
         f.write("// generated by gen_flash_attn_halfstep.py -- do not edit\n")
         for D, tag in ((128, "FA"), (64, "FA64")):
-            for name, cur, nxt in (("CUR_B", SB, SA), ("CUR_A", SA, SB)):
+            for name, second in (("CUR_B", True), ("CUR_A", False)):
                 f.write("#define GCMI_%s_HALF_%s \\\n" % (tag, name))
-                f.write(" \\\n".join('  "%s\\n"' % ln for ln in gen(cur, nxt, D)))
+                f.write(" \\\n".join('  "%s\\n"' % ln for ln in gen(second, D)))
                 f.write("\n\n")
-        f.write("#define GCMI_FA_HALF_CLOBBERS %s\n" % ", ".join('"v%d"' % r for r in range(KF, TMP + 1)))
+        f.write("#define GCMI_FA_HALF_CLOBBERS %s\n" % ", ".join('"v%d"' % r for r in range(144, 209)))
+        f.write("#define GCMI_FA64_HALF_CLOBBERS %s\n" % ", ".join('"v%d"' % r for r in range(89, 114)))
 
 
 if __name__ == "__main__":
