@@ -84,6 +84,22 @@ __device__ __forceinline__ float gelu_erf_bf16_result(float x) {
   return fmaxf(x, -0.0f) - fabsf(g);
 }
 
+// The same for any bf16 x, q of degree 6: of the 65280 finite x all but 91 give the bf16 value nearest to the true one, those a
+// neighbour (erf_rational + 1, * x, * 0.5 misses 337, in the negative tail by up to the whole value, where 1 + erf cancels), in 15
+// issue slots against 19.  An infinite x times e = 0 must not be a NaN where x > 0 (with x < 0 the reference's (erf + 1) * x is one).
+__device__ __forceinline__ float gelu_erf_of_bf16(float x) {
+  const float a = fabsf(x);
+  float q = 8.261797574959928e-07f;
+  q = fmaf(q, a, -3.6872435885015875e-05f);
+  q = fmaf(q, a, 6.939342711120844e-04f);
+  q = fmaf(q, a, -7.395347114652395e-03f);
+  q = fmaf(q, a, 5.1314398646354675e-02f);
+  q = fmaf(q, a, 4.613657295703888e-01f);
+  q = fmaf(q, a, 1.150178074836731f);
+  const float g = fminf(x, 3.4028234663852886e+38f) * __builtin_amdgcn_exp2f(fmaf(-a, q, -1.0f));
+  return fmaxf(x, -0.0f) - fabsf(g);
+}
+
 // tanh for the GELU below, where it is added to 1: 1 - 2 / (e^(2|t|) + 1) with the sign of t, absolute error about
 // 2e-7 (relative accuracy near 0 is not kept: the math library's tanhf keeps it with a polynomial branch per element,
 // which costs the epilogues what the conditional in erf did).  Infinite and NaN arguments come out as +-1 and NaN.
@@ -116,6 +132,9 @@ __device__ __forceinline__ float apply_act(float x, int act) {
     return x;
   }
 }
+
+// the activation of a bf16 graph's GEMM: of a value that was rounded to bf16, rounded to bf16 after it
+__device__ __forceinline__ float apply_act_of_bf16(float x, int act) { return act == ACT_GELU_ERF ? gelu_erf_of_bf16(x) : apply_act(x, act); }
 
 // one point-wise op in f32 (shared by the single-op kernel and the fused programs)
 __device__ __forceinline__ float round_to_storage(float v, int dt) {

@@ -139,7 +139,7 @@ template <int MT> __global__ __launch_bounds__(SK_WAVES * 64, 2) void gemm_skinn
         if (p.bias)
           x = round_bf16(x + b);
         if (p.act != ACT_NONE)
-          x = round_bf16(apply_act(x, p.act));
+          x = round_bf16(apply_act_of_bf16(x, p.act));
         if (p.residual)
           x = round_bf16(x + r);
       } else {

@@ -256,7 +256,7 @@ __device__ __forceinline__ void gemm_epilogue_act(const GemmParams &p, typename 
           if (ACT != ACT_NONE) {
 #pragma unroll
             for (int e = 0; e < 4; e++)
-              x[e] = act_const<ACT>(x[e]);
+              x[e] = apply_act_of_bf16(x[e], ACT);
             if (ACT == ACT_RELU) { // max(x, 0) of a bf16 value is a bf16 value: nothing to round
               p0 = (__float_as_uint(x[0]) >> 16) | (__float_as_uint(x[1]) & 0xffff0000u);
               p1 = (__float_as_uint(x[2]) >> 16) | (__float_as_uint(x[3]) & 0xffff0000u);
@@ -315,7 +315,7 @@ __device__ __forceinline__ void gemm_epilogue_act(const GemmParams &p, typename 
               if (p.bias)
                 x = round_bf16(x + bias4[e]);
               if (ACT != ACT_NONE)
-                x = round_bf16(act_const<ACT>(x));
+                x = round_bf16(apply_act_of_bf16(x, ACT));
               if (p.residual)
                 x = round_bf16(x + r);
               o16[e] = f32_to_bf16_bits(x);
@@ -1297,8 +1297,8 @@ __device__ __forceinline__ void w4_epilogue_row(const GemmParams &p, const acc4_
     }
     if constexpr (ACT != ACT_NONE) {
 #pragma unroll
-      for (int e = 0; e < 4; e++)
-        x[e] = act_const<ACT>(x[e]);
+      for (int e = 0; e < 4; e++) // (GELU by erf / so, us: 1237 x 4096, K 1376 23.4 / 22.2; 2048 x 8192, K 512 29.3 / 25.6)
+        x[e] = apply_act_of_bf16(x[e], ACT);
       if constexpr (ACT == ACT_RELU) { // max(x, 0) of a bf16 value is a bf16 value: nothing to round
         p0 = (__float_as_uint(x[0]) >> 16) | (__float_as_uint(x[1]) & 0xffff0000u);
         p1 = (__float_as_uint(x[2]) >> 16) | (__float_as_uint(x[3]) & 0xffff0000u);
@@ -1353,6 +1353,7 @@ __device__ __forceinline__ void w4_epilogue_half(const GemmParams &p, int half, 
   const bool bias_finite = fabsf((bias4[0] + bias4[1]) + (bias4[2] + bias4[3])) < __builtin_inff() || // the usual case
                            (fabsf(bias4[0]) < __builtin_inff() && fabsf(bias4[1]) < __builtin_inff() &&
                             fabsf(bias4[2]) < __builtin_inff() && fabsf(bias4[3]) < __builtin_inff());
+  const bool bias_tame = fabsf(bias4[0]) < 0x1p120f && fabsf(bias4[1]) < 0x1p120f && fabsf(bias4[2]) < 0x1p120f && fabsf(bias4[3]) < 0x1p120f;
   bool cols_tame = true;
   if constexpr (ES == 1) {
 #pragma unroll
@@ -1377,6 +1378,20 @@ __device__ __forceinline__ void w4_epilogue_half(const GemmParams &p, int half, 
         for (int u = 0; u < U; u++)
           t += ((float)c[u][0] + (float)c[u][1]) + ((float)c[u][2] + (float)c[u][3]);
         if (__builtin_expect(bias_finite && fabsf(t) < __builtin_inff(), 1)) {
+#pragma unroll
+          for (int u = 0; u < U; u++)
+            w4_epilogue_row<ES, ACT, OUT, HB, HR, MASKED, true>(p, c[u], m0 + row0 + (i0 + u) * 4, n, bias4, scale4, cs4,
+                                                                row0 + (i0 + u) * 4 < rows_in);
+          return;
+        }
+      }
+      // GELU: a sum of magnitudes, since it makes a NaN of -inf
+      if constexpr (ES == 2 && OUT == DT_BF16 && !HR && ACT == ACT_GELU_ERF) {
+        float t = 0.0f;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          t += (fabsf((float)c[u][0]) + fabsf((float)c[u][1])) + (fabsf((float)c[u][2]) + fabsf((float)c[u][3]));
+        if (__builtin_expect(bias_tame && t < 0x1p120f, 1)) {
 #pragma unroll
           for (int u = 0; u < U; u++)
             w4_epilogue_row<ES, ACT, OUT, HB, HR, MASKED, true>(p, c[u], m0 + row0 + (i0 + u) * 4, n, bias4, scale4, cs4,
@@ -1916,7 +1931,7 @@ __device__ __forceinline__ void epilogue_store4(const GemmParams &p, const f32x4
       if (p.bias)
         x = round_bf16(x + b);
       if (p.act != ACT_NONE)
-        x = round_bf16(apply_act(x, p.act));
+        x = round_bf16(apply_act_of_bf16(x, p.act));
       if (p.residual)
         x = round_bf16(x + r);
     } else {
@@ -1982,7 +1997,7 @@ template <int ACT> __global__ __launch_bounds__(256) void gemm_splitk_reduce_ker
       if (p.bias)
         x = round_bf16(x + bias4[e]);
       if (ACT != ACT_NONE)
-        x = round_bf16(act_const<ACT>(x));
+        x = round_bf16(apply_act_of_bf16(x, ACT));
       if (p.residual)
         x = round_bf16(x + r);
     } else {
