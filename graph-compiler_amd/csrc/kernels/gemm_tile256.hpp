@@ -1609,8 +1609,8 @@ __device__ __forceinline__ void k_tail_requests(char *to, const char *from, cons
 // K not a whole number of groups (two pairs of k-blocks, 256 bytes): the incomplete group [k_full, K) is the FIRST one
 // computed, and this puts it into slots 0 and 1 of the rings before the main loop's own requests go out: chunks before K by DMA,
 // zeros behind it (in both operands, so no product of theirs counts, whatever the memory behind K holds) by the lanes whose
-// chunks those are, which take no part in that request.  Nothing is waited for here: the caller waits for these requests, the
-// oldest, when the next ones are on their way.  (The pair that K ends in used to go through registers, behind the next requests,
+// chunks those are, which take no part in that request.  Nothing is waited for here: the main loop waits for these requests, the
+// oldest, when the next ones are on their way and its accumulators are cleared.  (The pair that K ends in used to go through registers, behind the next requests,
 // and everything in flight was waited for: 852 x 1728, K 1104 of 8 bits 11.05 -> 10.37 us, 1796 x 192, K 1176 13.3 -> 12.6,
 // 3106 x 3840, K 280 18.5 -> 17.7; 37 random sizes with such a K 1.023 times, none slower.)
 template <int ES, bool TB, int MI, int NJ>
@@ -1788,7 +1788,7 @@ template <int ES, bool TB, int MI, int NJ, bool GATED = false> __device__ __forc
 #define GCMI_W4_MAIN(TEXT, CLOBBERS)                                                                                  \
   asm volatile(TEXT : "+{s[40:41]}"(a_ptr), "+{s[42:43]}"(b_ptr), "+{s46}"(pairs)                                     \
                : "{v[0:7]}"(a_src), "{v[8:15]}"(b_src), "{v[16:17]}"(a_ld), "{v[20:23]}"(b_ld),                       \
-                 "{s[44:45]}"(b_step), "{s47}"(a_dma), "{s51}"(b_dma), "{s48}"(a_xor), "{v28}"(dump_ld)               \
+                 "{s[44:45]}"(b_step), "{s47}"(a_dma), "{s51}"(b_dma), "{s48}"(a_xor), "{s50}"(tail_group), "{v28}"(dump_ld) \
                : "memory", "scc", "s49", "s52", "s53", "s54", "s55", "s56", CLOBBERS)
 #define GCMI_W4_OF(STEP)                                                                                              \
   if constexpr (ES == 1 && NJ == 8) STEP(I8_8x8, 8x8)                                                                 \
@@ -1813,13 +1813,6 @@ template <int ES, bool TB, int MI, int NJ, bool GATED = false> __device__ __forc
                                       a_off, b_off, a_k, b_k);
   }
   GCMI_W4_OF(GCMI_W4_STEP_FILL)
-  if (tail_group) { // its requests have landed; those behind them (none where there is nothing but the tail) may be in flight
-    constexpr int BEHIND = (Ring::DA > 2 ? Ring::DA - 2 : 0) * MI + (Ring::DB > 2 ? Ring::DB - 2 : 0) * NB * (TB ? 1 : 2);
-    if (pairs > 2)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(BEHIND) : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
 #ifdef GCMI_W4_TIMING // measurement builds: core clock cycles and 100 MHz ticks spent in the main loop
   const long long tick0 = clock64(), wall0 = wall_clock64();
 #endif

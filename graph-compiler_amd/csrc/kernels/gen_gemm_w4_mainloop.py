@@ -29,7 +29,8 @@ Register contract with the kernel (inputs in fixed registers, see the constraint
   s48         int8: 0x80808080 when A is u8 (the bytes are flipped to s8 on the way into the MFMA), else 0
   s49         scratch (keeps m0);  s52..s57 slot bookkeeping, scratch
   s50         not 0: the first two pairs are an incomplete group of K that the set-up puts into slots 0 and 1 itself
-              (between the two statements), and s[40:43] point at the pair behind them
+              (in front of FILL, its requests are the oldest), and s[40:43] point at the pair behind them.  MAIN waits for
+              them, with its accumulators cleared meanwhile
   a[0:..]     out: accumulator tile (jt, it) = a[(jt*MI+it)*4 : +4]
   v[32:..]    A fragments (MI row tiles x 4 registers) of first / second blocks, then B fragments likewise
 
@@ -314,6 +315,16 @@ def gen(c):
             for it in range(c.mi):
                 out.extend(xor_tile(it, 0))
 
+    def tail_group(behind):
+        """an incomplete group's requests have landed; those FILL sent behind them may be in flight"""
+        emit("s_cmp_eq_u32 s50, 0")
+        emit("s_cbranch_scc1 .LW4_%s_WHOLE%d_%%=" % (tag, behind))
+        emit("s_waitcnt vmcnt(%d)" % behind)
+        emit(".LW4_%s_WHOLE%d_%%=:" % (tag, behind))
+
+    behind = max(c.da - 2, 0) * c.mi + max(c.db - 2, 0) * c.nb * (1 if c.tb else 2)
+    assert behind > 0
+    tail_group(behind)
     first_block(38)
     w0 = min(p.wait[0] for P, p in plans.items() if P >= 4)
     stage(0, w0 if not c.tb else None, big.fills[0], True, True)
@@ -338,6 +349,7 @@ def gen(c):
     out.extend(dump(c, 0))
     emit("s_branch .LW4_%s_END_%%=" % tag)
     emit(".LW4_%s_SHORT_%%=:" % tag)
+    tail_group(0)
     first_block(2)
     for t in range(4):
         stage(t, plans[2].wait[t] if (t or not c.tb) else None, [], t < 3, t in (0, 2))

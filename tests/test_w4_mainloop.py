@@ -25,11 +25,14 @@ class Wave:
         self.lds = {}         # (operand, KiB of the wave's shares) -> [pair or k-block, landed, visible]
         self.last_read = {}   # (operand, slot) -> when
         self.mfmas, self.reads = 0, {}
-        if tail_group:        # the set-up has filled the first two pairs of both rings; the loop's requests start at pair 2
-            for op, n in (("a", c.mi), ("b", c.nb if c.tb else 2 * c.nb)):
+        if tail_group:        # the set-up has put the first two pairs into both rings: a number of requests, the oldest, and zeros
+            for op, n in (("a", c.mi), ("b", c.nb if c.tb else 2 * c.nb)):  # for the rest; the loop's requests start at pair 2
                 for q in range(2):
                     for i in range(n):
-                        self.lds[op, q * n + i] = [q if op == "a" or c.tb else 2 * q + i // c.nb, True, True]
+                        cell = [q if op == "a" or c.tb else 2 * q + i // c.nb, len(self.queue) >= tail_group, False]
+                        self.lds[op, q * n + i] = cell
+                        if not cell[1]:
+                            self.queue.append(cell)
 
     def val(self, x):
         return self.m0 if x == "m0" else self.s[int(x[1:])] if x[0] == "s" else int(x)
@@ -140,7 +143,7 @@ class Wave:
 
 @pytest.mark.parametrize("c", G.CONFIGS, ids=lambda c: c.name)
 @pytest.mark.parametrize("pairs", [2, 4, 6, 8, 10, 22, 64])
-@pytest.mark.parametrize("tail_group", [0, 1])
+@pytest.mark.parametrize("tail_group", [0, 1, 10 ** 6])  # an incomplete group in front: one request of it, all of them
 def test_every_read_finds_its_block(c, pairs, tail_group):
     fill, main = G.gen(c)
     w = Wave(c, pairs, tail_group)
