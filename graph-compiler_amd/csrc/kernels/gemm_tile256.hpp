@@ -1363,6 +1363,9 @@ __device__ __forceinline__ void w4_epilogue_half(const GemmParams &p, int half, 
   constexpr int U = 8; // rows in flight per lane
 #pragma unroll 1
   for (int i0 = 0; i0 < WR / 4; i0 += U) {
+    // none of the wave's 4 * U rows from here on lies inside (passed over: 3 x 2312, K 96 with GELU 13.3 us -> 9.9; 2 x 1192, K 136 14.6 -> 11.4)
+    if (MASKED && wm * WR + 4 * i0 >= rows_in)
+      return;
     acc4_t c[U];
 #pragma unroll
     for (int u = 0; u < U; u++)
@@ -2157,8 +2160,8 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     fast = false; // every batch's operands must keep the alignment the fast path loads with
   // Any M, N and K whole numbers of 16-byte chunks: the 4-wave kernel still takes it; its edge tiles clamp their loads
   // and store what lies inside C.
-  // Not worth it for a K of 64 bf16 or less under fewer than 32 rows, where nothing but set-up and epilogue is left: 10.4 us
-  // on the bounds-checked kernel, 12.5 here (16 x 4416, K 16; from K 65 on this one is the faster by 5 %).
+  // A K of 64 bf16 or less under fewer than 32 rows stays with the bounds-checked kernel, which is no line by speed: 11.1 us there, 9.3
+  // here (16 x 20000, K 64), since the 4-wave epilogue passes over rows outside C (before that 12.4; from K 65 on this one was ahead).
   const bool tiny = ES == 2 && !k_whole && p.K <= 64 && p.M < 32 && p.cfg_tile == 0;
   const bool ragged = !fast && !tiny && aligned && p.N % (16 / ES) == 0 && (p.M % G_BM != 0 || p.N % G_BN != 0 || !k_whole) &&
                       (nbatch == 1 || ((p.a_bs * ES) % 16 == 0 && (p.b_bs * ES) % 16 == 0 && (p.c_bs * out_es) % 16 == 0 &&
