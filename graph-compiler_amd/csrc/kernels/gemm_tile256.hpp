@@ -1464,11 +1464,11 @@ __device__ __forceinline__ void w4_epilogue_half_any(const GemmParams &p, int ki
 }
 
 // 1 / (1 + exp(-x)) of a bf16 value x for a bf16 result: the hardware's exponential and reciprocal, each good to an ulp of f32
-// or two, in place of expf and a correctly rounded division (20 issue slots fewer per result).  The sum is a sixteenth of the
-// true one, so that no reciprocal is below the smallest normal number, which the instruction would make 0.  Rounded to bf16 it is
-// what those give for every bf16 x (all 65536 compared on the GPU) but -89 to -91.5, where expf(-x) is infinite and they give 0.
+// or two, in place of expf and a correctly rounded division (20 issue slots fewer per result).  The sum is a quarter of the true
+// one: the reciprocal makes a result below the smallest normal number 0, which is then just where expf(-x) is infinite (2^128
+// and more, x = -89 and below).  Rounded to bf16 it is what those give for every bf16 x.
 __device__ __forceinline__ float sigmoid_of_bf16(float x) {
-  return 0.0625f * __builtin_amdgcn_rcpf(0.0625f + __builtin_amdgcn_exp2f(fmaf(x, -1.4426950408889634f, -4.0f)));
+  return 0.25f * __builtin_amdgcn_rcpf(0.25f + __builtin_amdgcn_exp2f(fmaf(x, -1.4426950408889634f, -2.0f)));
 }
 
 // What a gated pair of products ends in, silu(gate) * up, for four results of a row: both sums rounded to bf16, then the

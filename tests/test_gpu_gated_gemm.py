@@ -69,6 +69,24 @@ def test_bits_of_single_ops(ga, mm, dev, monkeypatch, T, K, N):
     assert (full[T] == 7.0).all() and not fused[1:].isnan().any()
 
 
+def test_sigmoid_of_every_value(ga, mm, dev, monkeypatch):
+    """Identity weights make the gate's sums the operand itself, every finite bf16 value; up's are 1."""
+    T, K, N = 128, 640, 4096
+    values = torch.arange(65536, device=dev, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    values = torch.where(values.isfinite(), values, torch.zeros_like(values)).view(T, 512)
+    ins = [torch.zeros(T, K, device=dev, dtype=torch.bfloat16)] + [torch.zeros(N, K, device=dev, dtype=torch.bfloat16) for _ in range(2)]
+    ins[0][:, :512], ins[0][:, K - 1] = values, 1.0
+    ins[1][torch.arange(N), torch.arange(N) % 512] = 1.0
+    ins[2][:, K - 1] = 1.0
+    text = _module(mm, T, K, N)
+    fused, single = (torch.empty(T, N, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    assert "MatMul x2" in ga.explain_mlir(text)[1]
+    _run(ga, text, ins, fused)
+    monkeypatch.setenv("GCMI_NO_POINTWISE_FUSION", "1")
+    _run(ga, text, ins, single)
+    assert torch.equal(fused.view(torch.int16), single.view(torch.int16))
+
+
 @pytest.mark.parametrize("T,K,N", [(32, 4096, 11008), (200, 2048, 5632)])
 def test_error(ga, mm, dev, T, K, N):
     g = torch.Generator(device=dev).manual_seed(3)
