@@ -937,6 +937,11 @@ int pointwise_code(const Op &op) {
   auto it = more.find(k);
   return it == more.end() ? -1 : it->second;
 }
+// ... for operand and result of these types
+int pointwise_code(const Op &op, int in_dt, int out_dt) {
+  const int code = pointwise_code(op);
+  return code == gcmi::ELT_GELU_ERF && in_dt == GCMI_BF16 && out_dt == GCMI_BF16 ? gcmi::ELT_GELU_ERF_OF_BF16 : code;
+}
 bool storage_float(DT d) { return d == DT::f32 || d == DT::bf16 || d == DT::f16; }
 } // namespace
 
@@ -1228,10 +1233,10 @@ void Executable::plan_fusion(std::vector<bool> &skip, const std::vector<bool> &c
     auto emit_member = [&](size_t m, const std::vector<Use> &u, int phase, std::string &names) {
       const Op &o = g_.ops[m];
       Step::FIns f;
-      f.op = pointwise_code(o);
       f.a = reg_of(u[0], phase);
       f.b = u.size() > 1 ? reg_of(u[1], phase) : f.a;
       f.dt = dt_dnnl(T(o.out[0]).dt);
+      f.op = pointwise_code(o, dt_dnnl(T(o.in[0]).dt), f.dt);
       f.imm = o.kind == "Pow" ? o.attr_f32("beta", 1.0f) : 0.0f;
       reg_of_op[m] = n_in + (int)s.f_ins.size();
       s.f_ins.push_back(f);
@@ -1454,7 +1459,7 @@ void Executable::plan_generic(const Op &op) {
     s.a_dt = dt_dnnl(T(op.in[0]).dt), s.b_dt = dt_dnnl(T(op.in[1]).dt), s.out_dt = dt_dnnl(out.dt);
     s.dims = out.shape, s.sa = bstrides(T(op.in[0])), s.sb = bstrides(T(op.in[1]));
   } else if (pointwise_code(op) >= 0 && op.in.size() == 1) {
-    s.op = pointwise_code(op);
+    s.op = pointwise_code(op, dt_dnnl(T(op.in[0]).dt), dt_dnnl(out.dt));
     s.alpha = k == "Pow" ? op.attr_f32("beta", 1.0f) : 0.0f;
     s.a = slot_for(op.in[0]), s.out = slot_for(op.out[0]);
     s.a_dt = dt_dnnl(T(op.in[0]).dt), s.out_dt = dt_dnnl(out.dt);

@@ -84,9 +84,11 @@ __device__ __forceinline__ float gelu_erf_bf16_result(float x) {
   return fmaxf(x, -0.0f) - fabsf(g);
 }
 
-// The same for any bf16 x, q of degree 6: of the 65280 finite x all but 91 give the bf16 value nearest to the true one, those a
-// neighbour (erf_rational + 1, * x, * 0.5 misses 337, in the negative tail by up to the whole value, where 1 + erf cancels), in 15
-// issue slots against 19.  An infinite x times e = 0 must not be a NaN where x > 0 (with x < 0 the reference's (erf + 1) * x is one).
+// The same for any bf16 x, q of degree 6, wherever operand and result are bf16 tensors: in a GEMM's epilogue and as an op of its
+// own, so that the bits do not depend on what the planner fuses.  Of the 65280 finite x all but 91 give the bf16 value nearest to
+// the true one; down to x = -9.7 those are a neighbour, below it (|result| < 1e-20) up to 4 % of the value, ten steps, and below
+// about -13, where the exponential is under the smallest normal number, 0.  (erf_rational + 1, * x, * 0.5 misses 337 and gives 0 from
+// -5.5 down, where 1 + erf cancels.)  15 issue slots against 19.  An infinite x times e = 0 must not be a NaN where x > 0 (with x < 0 the reference's (erf + 1) * x is one).
 __device__ __forceinline__ float gelu_erf_of_bf16(float x) {
   const float a = fabsf(x);
   float q = 8.261797574959928e-07f;
@@ -133,7 +135,8 @@ __device__ __forceinline__ float apply_act(float x, int act) {
   }
 }
 
-// the activation of a bf16 graph's GEMM: of a value that was rounded to bf16, rounded to bf16 after it
+// the activation of a bf16 graph's GEMM: of a value that was rounded to bf16, rounded to bf16 after it (ELT_GELU_ERF_OF_BF16 is the
+// same for a GELU that stands alone or in a point-wise group)
 __device__ __forceinline__ float apply_act_of_bf16(float x, int act) { return act == ACT_GELU_ERF ? gelu_erf_of_bf16(x) : apply_act(x, act); }
 
 // one point-wise op in f32 (shared by the single-op kernel and the fused programs)
@@ -157,6 +160,7 @@ __device__ __forceinline__ float fused_op(int op, float x, float y, float imm) {
   case ELT_RELU: return apply_act(x, ACT_RELU);
   case ELT_SIGMOID: return apply_act(x, ACT_SIGMOID);
   case ELT_GELU_ERF: return apply_act(x, ACT_GELU_ERF);
+  case ELT_GELU_ERF_OF_BF16: return gelu_erf_of_bf16(x);
   case ELT_GELU_TANH: return apply_act(x, ACT_GELU_TANH);
   case ELT_POW: return imm == 2.0f ? x * x : (imm == 1.0f ? x : (imm == 0.5f ? sqrtf(x) : powf(x, imm)));
   case ELT_MIN: return (x != x || y != y) ? x + y : fminf(x, y); // arith.minimumf: NaN propagates

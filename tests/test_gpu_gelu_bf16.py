@@ -1,4 +1,5 @@
-"""GELU of a bf16 GEMM's epilogue for every finite bf16 value: the product with the identity is the value itself."""
+"""GELU of bf16 for every finite bf16 value, in a GEMM's epilogue (the product with the identity is the value itself) and as an
+op of its own."""
 import pytest
 import torch
 
@@ -35,3 +36,45 @@ def test_infinities(gc, dev):
     out = gc.gemm_bf16(A, B, act="gelu_erf")
     assert (out[:, 0] == float("inf")).all() and out[:, 1:3].isnan().all() and not out[:, 3:].isnan().any()
     assert ((out[:, 5].float() - 1.953125).abs() < 1e-6).all() and (out[:, 6:] == 0).all()
+
+
+def _graph(ga, kinds, inner=()):
+    """x -> kinds[0] -> kinds[1] ...; MatMul has the identity for its second operand, inner results are outputs too"""
+    ops, last = [], 0
+    for i, kind in enumerate(kinds):
+        t = {"dtype": "bf16", "shape": [512, 128]}
+        ins = [dict(t, id=last)] + ([{"id": 100, "dtype": "bf16", "shape": [128, 128]}] if kind == "MatMul" else [])
+        attrs = {"attrs": {"mode": {"type": "string", "value": "gelu_erf"}}} if kind == "GELU" else {}
+        ops.append(dict({"kind": kind, "inputs": ins, "outputs": [dict(t, id=i + 1)]}, **attrs))
+        last = i + 1
+    matmul = "MatMul" in kinds
+    return ga._graph(ops, [0] + [100] * matmul, list(inner) + [last]), [0] + [100] * matmul, list(inner) + [last]
+
+
+def _run(ga, graph, x, eye):
+    text, ins, outs = graph
+    comp = ga.Compiler()
+    st, exe = comp.compile(text)
+    assert st == 0, ga.api().dnnl_graph_compiler_last_error().decode()
+    res = [torch.empty_like(x) for _ in outs]
+    try:
+        call = exe.bind([(i, x if i == 0 else eye) for i in ins], list(zip(outs, res)), torch.cuda.current_stream().cuda_stream)
+        assert call() == 0
+        torch.cuda.synchronize()
+    finally:
+        exe.close()
+        comp.close()
+    return res[-1]
+
+
+@pytest.mark.parametrize("kinds,inner,env", [
+    (["GELU"], (), None), (["MatMul", "GELU"], (1,), None),                                # a step of its own, alone and behind a GEMM
+    (["GELU", "Abs"], (), None), (["GELU", "Abs"], (), "GCMI_NO_GENERATED_KERNELS"),  # in a group: generated, interpreted
+    (["GELU", "Abs"], (), "GCMI_NO_POINTWISE_FUSION")])
+def test_bits_of_the_epilogue(ga, dev, monkeypatch, kinds, inner, env):
+    x, eye = _values(dev), torch.eye(128, device=dev, dtype=torch.bfloat16)
+    want = _run(ga, _graph(ga, ["MatMul", "GELU"]), x, eye)
+    if env:
+        monkeypatch.setenv(env, "1")
+    got = _run(ga, _graph(ga, kinds, inner), x, eye)
+    assert torch.equal(got, want.abs() if "Abs" in kinds else want)  # (the sum of a product makes -0 a 0)
