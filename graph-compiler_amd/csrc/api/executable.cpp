@@ -1595,9 +1595,9 @@ std::vector<gcjit::FusedKernelSource> Executable::generated_kernels() const {
       }
       continue;
     }
-    if (s.kind != Step::Fused)
+    if (s.kind != Step::Fused && s.kind != Step::GemmGated)
       continue;
-    gcjit::FusedKernelSource k = generate_step(s, i);
+    gcjit::FusedKernelSource k = generate_step(s.kind == Step::Fused ? s : s.parts.back(), i); // (a gate's point-wise group is its last part)
     if (!k.source.empty())
       ks.push_back(std::move(k));
   }
@@ -1624,18 +1624,18 @@ void Executable::build_generated_kernels() {
   }
   for (const gcjit::FusedKernelSource &k : ks) {
     const size_t i = (size_t)std::stoul(k.name.substr(strlen("gcmi_fused_step")));
-    Step &s = steps_[i];
+    Step &s = steps_[i].kind == Step::GemmGated ? steps_[i].parts.back() : steps_[i];
     s.jit_fn = jit_module_->function(k.name);
     s.jit_grid = k.grid, s.jit_block = k.block, s.jit_vectors = k.quad;
   }
 }
 
-// The generated kernel of a fused step is there and takes its operands' addresses.
-bool Executable::generated_takes(const Step &s) const {
+// The generated kernel of a fused step is there and takes its operands' addresses; `slices`: and adds the K slices of the GEMM in front.
+bool Executable::generated_takes(const Step &s, bool slices) const {
   if (!s.jit_fn)
     return false;
   auto aligned = [&](int slot) { return slot < 0 || (reinterpret_cast<uintptr_t>(ptr_[(size_t)slot]) & 15) == 0; };
-  bool all = aligned(s.out) && (s.sliced_in < 0 || (aligned(s.ws) && aligned(s.c)));
+  bool all = aligned(s.out) && (!slices || (aligned(s.ws) && aligned(s.c)));
   for (int slot : s.f_in)
     all = all && aligned(slot);
   return all || !s.jit_vectors;
@@ -1653,7 +1653,7 @@ void Executable::launch(const Step &s) {
     break;
   case Step::GemmBf16:
     slices_left_ = 0;
-    if (s.next_splits && generated_takes(*(&s + 1))) { // (steps_ in their order)
+    if (s.next_splits && generated_takes(*(&s + 1), true)) { // (steps_ in their order)
       gc_check(gcmi_gemm_bf16_slices(P(s.a), P(s.b), P(s.out), s.M, s.N, s.K, s.lda, s.ldb, s.ldc, s.tb ? 1 : 0, P(s.c), s.N, P(s.ws),
                                      slots_[(size_t)s.ws].bytes, s.next_splits, &slices_left_, stream_),
                "MatMul bf16");
@@ -1767,9 +1767,8 @@ void Executable::launch(const Step &s) {
     }
     if ((size_t)(second_pass ? p.n : p.n / p.n_red) * (size_t)esz(p.out_dt) > slots_[(size_t)s.out].bytes)
       throw std::runtime_error("fused group: the result does not fit its buffer (" + s.note + ")");
-    // (a kernel that adds K slices is of no use where they were added already)
-    if (generated_takes(s) && (s.sliced_in < 0 || slices_left_)) {
-      void *args[gcmi::FUSED_MAX_IN + 4], *part = P(s.ws), *addend = P(s.c), *result = nullptr;
+    if (generated_takes(s)) {
+      void *args[gcmi::FUSED_MAX_IN + 4], *part = slices_left_ ? P(s.ws) : nullptr, *addend = P(s.c), *result = nullptr;
       for (int k = 0; k < p.n_in; k++)
         args[k] = (void *)&p.in[k];
       args[p.n_in] = (void *)&p.out;

@@ -160,7 +160,7 @@ private:
   void plan_gates();
   void plan_workspaces();
   void plan_slices();
-  bool generated_takes(const Step &s) const;
+  bool generated_takes(const Step &s, bool slices = false) const;
   void layout_arena();
   void plan_generic(const Op &op);
   void plan_fusion(std::vector<bool> &skip, const std::vector<bool> &claimed, std::map<size_t, std::vector<Step>> &emit_at,

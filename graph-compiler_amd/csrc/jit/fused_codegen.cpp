@@ -435,6 +435,8 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
                              g.idx + ")it_ * " + std::to_string(step_elems) + " + 4 * (" + g.idx + ")sub;\n    if (e < (" + g.idx + ")" +
                              Gen::num(p.n_red) + ") {\n";
     o << "  f4_ part_[" << trips << "][" << S << "] = {};\n  u2_ add_[" << trips << "] = {}, raw" << n << "[" << trips << "] = {};\n";
+    o << "  if (part == nullptr) {\n" << head << "      raw" << n << "[it_] = *reinterpret_cast<const u2_ *>(reinterpret_cast<const unsigned short *>(in" << n
+      << ") + " << off << ");\n    }\n  }\n  } else {\n";
     o << head << "#pragma unroll\n      for (int s_ = 0; s_ < " << S << "; s_++)\n        part_[it_][s_] = *reinterpret_cast<const f4_ *>(part + s_ * "
       << p.n << "ll + " << off << ");\n";
     if (sliced.residual)
@@ -447,7 +449,7 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
            "      gcmi::round_bf16_quad(q_);\n";
     o << "      raw" << n << "[it_] = u2_{(__float_as_uint(q_[0]) >> 16) | (__float_as_uint(q_[1]) & 0xffff0000u), (__float_as_uint(q_[2]) >> 16) | "
          "(__float_as_uint(q_[3]) & 0xffff0000u)};\n      if (live)\n        *reinterpret_cast<u2_ *>(reinterpret_cast<unsigned short *>(result) + "
-      << off << ") = raw" << n << "[it_];\n    }\n  }\n";
+      << off << ") = raw" << n << "[it_];\n    }\n  }\n  }\n";
   }
   o << "  float acc = 0.0f;\n";
   row_loop(0, p.n_in_pre, 0, p.sum_ins, false);

@@ -34,7 +34,8 @@ struct FusedKernelSource {
 
 // A first-pass input of a row kernel that a K-sliced bf16 GEMM leaves as its partial sums: the kernel adds the slices in
 // ascending order, rounds, adds the residual, rounds (what the GEMM's second pass does), and stores that result too.  Three
-// arguments more behind `out`: the sums [splits][rows][row length] f32, the residual or null, the result.
+// arguments more behind `out`: the sums [splits][rows][row length] f32, the residual or null, the result.  With null for the sums
+// the input is read like any other (the GEMM ran in one pass, or added its slices itself).
 struct SlicedInput {
   int k = -1; // which input; -1: none
   int splits = 0;

@@ -68,3 +68,23 @@ def test_a_residual_off_16_bytes_takes_the_second_pass(ga, mm, dev):
     ins[2] = off
     for a, b in zip(_run(ga, text, ins, T, H), want):
         assert torch.allclose(a.float(), b.float(), rtol=2.0 ** -6, atol=2.0 ** -6)  # another kernel's sums: a rounding or two apart
+
+
+@pytest.mark.parametrize("which", ["residual", "operand", "weights of the gate"])
+def test_operands_off_16_bytes_keep_the_generated_kernels(ga, mm, dev, monkeypatch, which):
+    """The norm behind a GEMM that added its slices itself or ran in one pass, the point-wise group of a gate run in parts."""
+    T, H, F = 32, 2048, 2048
+    text, ins = mm.decoder_mlp_block(T, H, F), _inputs(dev, T, H, F)
+    before = ga.generated_kernel_launches()
+    _run(ga, text, ins, T, H)
+    per_call = ga.generated_kernel_launches() - before
+    at = {"residual": 2, "operand": 0, "weights of the gate": 5}[which]
+    off = torch.empty(ins[at].numel() + 4, device=dev, dtype=torch.bfloat16)[4:].view(ins[at].shape)
+    off.copy_(ins[at])
+    ins[at] = off
+    before = ga.generated_kernel_launches()
+    got = _run(ga, text, ins, T, H)
+    assert ga.generated_kernel_launches() - before == per_call + (2 if at == 5 else 0)
+    monkeypatch.setenv("GCMI_NO_GENERATED_KERNELS", "1")
+    for a, b in zip(got, _run(ga, text, ins, T, H)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
