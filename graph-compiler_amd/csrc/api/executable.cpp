@@ -1930,11 +1930,14 @@ std::string Executable::describe() const {
                                 "fused", "attention mask", "gemm_bf16"};
   std::ostringstream os;
   static const char *kernels[] = {"bounds-checked tile", "whole tiles, 8 waves", "whole tiles, 4 waves (one per SIMD)",
-                                  "K slices + second pass", "weight streaming (+ second pass)",
+                                  "K slices + second pass", "weight streaming",
                                   "small tiles, 4 waves, two workgroups per compute unit", "f32",
                                   "few rows, K over the waves of a workgroup"};
   auto tile_line = [&](const auto &c) {
-    os << "  tile: " << kernels[c.kernel] << ", " << c.bm << "x" << c.bn << " per workgroup, " << c.kbytes << " B of K per stage x "
+    // 128 x 128 tiles in pairs on a compute unit have a ring of four stages; alone, and taller or wider, they have more or are not 128 x 128
+    const bool alone = c.kernel == gcmi::GK_TILE128 && (c.bm != 128 || c.bn != 128 || c.stages != 4);
+    os << "  tile: " << (alone ? "small tiles, 4 waves (one per SIMD)" : kernels[c.kernel])
+       << (c.kernel == gcmi::GK_STREAM && c.split_k > 1 ? " + second pass" : "") << ", " << c.bm << "x" << c.bn << " per workgroup, " << c.kbytes << " B of K per stage x "
        << c.stages << " stages, waves " << c.waves_m << "x" << c.waves_n << " of " << c.wave_m << "x" << c.wave_n << ", mfma " << c.mfma_m
        << "x" << c.mfma_n << "x" << c.mfma_k << ", split_k " << c.split_k << ", " << c.workgroups << " workgroups";
   };

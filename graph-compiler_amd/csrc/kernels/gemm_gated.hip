@@ -21,9 +21,13 @@ static constexpr int GR_KB = 256; // bytes of K per row and stage
 // us, weights from memory, the two products on the kernels they get alone and the ops between them / this: 32 x 11008, K 4096
 // 48.6 / 39.4 (180 MB: 4.6 TB/s), 64 x 11008 58.8 / 40.7, 32 x 5632, K 2048 27.2 / 11.9, 32 x 2816, K 1024 13.9 / 5.4; random
 // sizes of up to 64 rows 2.0 times (74 of them, at least 1.14), of 65 to 128 rows and up to 8192 columns 2.05 (41, 1.28).
+constexpr int gated_rows_stages(int mt, int nt) {
+  const int stage = 16 * (mt + 2 * nt) * GR_KB;
+  return 160 * 1024 / stage < 4 ? 160 * 1024 / stage : 4;
+}
 template <int MT, int NT> __global__ __launch_bounds__(512, 1) void gemm_gated_rows_kernel(GemmParams p, const void *up, int cols) {
   constexpr int KB = GR_KB, A_BYTES = 16 * MT * KB, W_BYTES = 16 * NT * KB, STAGE = A_BYTES + 2 * W_BYTES;
-  constexpr int NST = 160 * 1024 / STAGE < 4 ? 160 * 1024 / STAGE : 4;
+  constexpr int NST = gated_rows_stages(MT, NT);
   constexpr int NA = MT / 2, PER = NA + NT; // requests of 4 rows per wave and stage
   static_assert(NST >= 3 && 2 * NT * MT * 4096 <= NST * STAGE, "a ring, and room for the partial sums");
   __shared__ __align__(1024) char smem[NST * STAGE];
@@ -211,7 +215,7 @@ extern "C" int gcmi_launch_gemm_gated(const GemmParams *p, const void *up, hipSt
   const int64_t rounds = (p->N + 64 * (int64_t)n_cu - 1) / (64 * (int64_t)n_cu), per = (p->N + n_cu * rounds - 1) / (n_cu * rounds);
   const int cols = (int)((per + 3) / 4 * 4);
   if (p->K % 128 == 0 && p->K >= 512 && (p->M <= 64 || (p->M <= 128 && cols <= 32))) {
-    c.kernel = GK_STREAM, c.bm = p->M <= 32 ? 32 : p->M <= 64 ? 64 : 128, c.bn = cols, c.kbytes = GR_KB, c.stages = 4;
+    c.kernel = GK_STREAM, c.bm = p->M <= 32 ? 32 : p->M <= 64 ? 64 : 128, c.bn = cols, c.kbytes = GR_KB, c.stages = gated_rows_stages(c.bm / 16, (cols + 15) / 16);
     c.waves_m = 1, c.waves_n = 2, c.wave_m = c.bm, c.wave_n = cols, c.group_m = 1, c.workgroups = (int32_t)((p->N + cols - 1) / cols);
     if (cfg)
       *cfg = c;
@@ -230,7 +234,7 @@ extern "C" int gcmi_launch_gemm_gated(const GemmParams *p, const void *up, hipSt
   }
   if (tiles > 0x7fffffff || (4 * tiles < n_cu && p->K > 1536))
     return -1;
-  c.kernel = GK_WAVES4, c.bm = tile->rows, c.bn = tile->cols, c.kbytes = 64, c.stages = 4, c.group_m = 4, c.workgroups = (int32_t)tiles;
+  c.kernel = GK_WAVES4, c.bm = tile->rows, c.bn = tile->cols, c.kbytes = 64, c.stages = w4_ring_blocks<2, true>(tile->rows, 2 * tile->cols), c.group_m = 4, c.workgroups = (int32_t)tiles;
   c.waves_m = c.waves_n = 2, c.wave_m = tile->rows / 2, c.wave_n = tile->cols;
   if (cfg)
     *cfg = c;

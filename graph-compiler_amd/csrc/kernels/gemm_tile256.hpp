@@ -2044,6 +2044,38 @@ static void launch_splitk_reduce(const GemmParams &p, hipStream_t stream) {
 // 128 columns, 128 rows or more: gemm_tile128.hpp
 static constexpr int T128_B = 128, T128_KB = 64, T128_NST = 4;
 
+// Whether tiles of rows x cols run on the kernel that puts two of them on a compute unit, or alone on the 4-wave kernels' hand-placed loop.
+// Two 128 x 128 tiles per compute unit only where there are more than a round of them, or two groups of K or less, which are
+// set-up and epilogue mostly.  Else the hand-placed loop with its deeper ring, the whole LDS to itself, us, two per unit / this,
+// weights from memory: 1000 x 4096, K 4096 [N,K] 48.2 / 37.2, 2048^3 27.8 / 23.7, 1422 x 2384, K 1280 [N,K] 16.3 / 12.9, 1086 x 144,
+// K 272 7.6 / 7.4, 8-bit 1024 x 4096, K 4096 31.5 / 26.9; but 746 x 944, K 160 7.4 / 7.6, 8-bit 1425 x 1168, K 208 7.9 / 8.3, and in more
+// than a round 2498 x 2544, K 512 13.3 / 14.2.
+static inline bool tile128_in_pairs(int es, int rows, int cols, int64_t K, int splits, int64_t workgroups) {
+  return rows == 128 && cols == 128 && (workgroups > gcmi_num_cus() || K * es <= 512 * (int64_t)(splits > 1 ? splits : 1));
+}
+
+// How many k-blocks (64 bytes of K per row) of both operands the LDS rings of the 4-wave kernel of rows x cols hold.
+template <int ES, bool TB, int MI, int NJ> constexpr int w4_ring_blocks() {
+  return 2 * (W4Ring<ES, TB, MI, NJ>::DA < W4Ring<ES, TB, MI, NJ>::DB ? W4Ring<ES, TB, MI, NJ>::DA : W4Ring<ES, TB, MI, NJ>::DB);
+}
+template <int ES, bool TB> static inline int w4_ring_blocks(int rows, int cols) {
+  if (cols == 128)
+    return rows == 128 ? w4_ring_blocks<ES, TB, 4, 4>() : rows == 192 ? w4_ring_blocks<ES, TB, 6, 4>() : w4_ring_blocks<ES, TB, 8, 4>();
+  if constexpr (ES == 2)
+    if (cols == 192)
+      return w4_ring_blocks<ES, TB, 8, 6>();
+  return w4_ring_blocks<ES, TB, 8, 8>();
+}
+// ... of the kernel that runs tiles of 128 x 128 to 256 x 192
+template <int ES> static inline int tile128_stages(int rows, int cols, int64_t K, int trans_b, int splits, int64_t workgroups) {
+  if (tile128_in_pairs(ES, rows, cols, K, splits, workgroups))
+    return T128_NST;
+  if constexpr (ES == 2)
+    if (trans_b)
+      return w4_ring_blocks<2, true>(rows, cols);
+  return w4_ring_blocks<ES, false>(rows, cols);
+}
+
 } // namespace gcmi
 extern "C" int gcmi_launch_tile128(const gcmi::GemmParams *p, int es, int rows, int cols, unsigned grid_x, unsigned grid_y, hipStream_t stream);
 namespace gcmi {
@@ -2284,7 +2316,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     const int tiles = (int)(by128 ? nblk128 : nblk);
     c.kernel = GK_SPLITK, c.split_k = splits, c.workgroups = tiles * splits;
     if (by128) {
-      c.bm = rows128, c.bn = 128, c.kbytes = T128_KB, c.stages = T128_NST;
+      c.bm = rows128, c.bn = 128, c.kbytes = T128_KB, c.stages = tile128_stages<ES>(rows128, 128, p.K, p.trans_b, splits, nblk128 * splits);
       c.waves_m = c.waves_n = 2, c.wave_m = rows128 / 2, c.wave_n = 64, c.mfma_m = c.mfma_n = 16, c.mfma_k = 32;
     } else if (by256) {
       c.kbytes = 64, c.stages = 4, c.waves_m = 2, c.waves_n = 2, c.wave_m = 128, c.wave_n = 128;
@@ -2327,7 +2359,8 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     return hipGetLastError() == hipSuccess ? 0 : 5;
   }
   if (plan == PLAN_TILE128) {
-    c.kernel = GK_TILE128, c.bm = rows128, c.bn = 128, c.kbytes = T128_KB, c.stages = T128_NST;
+    c.kernel = GK_TILE128, c.bm = rows128, c.bn = 128, c.kbytes = T128_KB;
+    c.stages = tile128_stages<ES>(rows128, 128, p.K, p.trans_b, 1, nblk128 * nbatch);
     c.waves_m = c.waves_n = 2, c.wave_m = rows128 / 2, c.wave_n = 64, c.mfma_m = c.mfma_n = 16, c.mfma_k = 64 / ES;
     c.workgroups = (int32_t)nblk128;
     if (cfg)
@@ -2383,7 +2416,7 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
     if (tile->rows != 256 || tile->cols != 256) {
       const int64_t tiles = ((p.M + tile->rows - 1) / tile->rows) * ((p.N + tile->cols - 1) / tile->cols);
       c.kernel = GK_TILE128, c.bm = tile->rows, c.bn = tile->cols, c.wave_m = tile->rows / 2, c.wave_n = tile->cols / 2;
-      c.workgroups = (int32_t)tiles;
+      c.workgroups = (int32_t)tiles, c.stages = tile128_stages<ES>(tile->rows, tile->cols, p.K, p.trans_b, 1, tiles * nbatch);
       if (cfg)
         *cfg = c;
       if (dry)

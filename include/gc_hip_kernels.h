@@ -160,7 +160,8 @@ int gcmi_gemm_bf16_ws(const void *A, const void *B, void *C, int64_t batch, int6
  * kernel (up to 128 rows of A against wide weights in either layout; bn = 64:
  * the 8-wave kernel with the LDS ring, with split_k > 1 followed by the second
  * pass), 5 tiles of 128 x 128 with 4 waves
- * of 64 x 64, or of 192 or 256 x 128 with one workgroup per compute unit
+ * of 64 x 64, two workgroups per compute unit (stages = 4) or one (more
+ * stages), or of 192 or 256 x 128 or 256 x 192 with one
  * (problems of few 256 x 256 tiles; with split_k > 1 kind 3 is reported and
  * bn = 128 tells), 6 the f32 kernels (a_dtype GCMI_F32, A
  * stored [M,K]: bm = bn = 16, 32, 64 or 128, mfma_m = 0 for the vector kernel of
