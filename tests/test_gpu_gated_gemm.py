@@ -45,22 +45,26 @@ def _exact(dev, T, K, N, seed):
     return [r(1.0, T, K), r(2.0 ** -6, N, K), r(2.0 ** -6, N, K)]
 
 
-# few rows: 1 to 4 column tiles per product, whole and cut workgroups, more than one round of them; tiles of 128 to 256 rows
-# by 64 to 128 columns, rows and columns off the tile, a K that ends inside a group
-FEW = [(1, 512, 4096), (31, 512, 4108), (32, 640, 11008), (33, 512, 13000), (64, 512, 4100), (64, 512, 16900), (17, 1024, 2816)]
-TILES = [(65, 512, 4108), (128, 520, 4100), (129, 512, 11008), (200, 1032, 2816), (257, 512, 11004), (300, 640, 5632),
-         (513, 512, 8200), (700, 520, 8204), (1000, 512, 11008), (1000, 1024, 5632)]
+# The kernel each size selects: rows x columns of C per workgroup.  Few rows: 1 to 4 column tiles per product for up to 32 and 64 rows, 1
+# and 2 up to 128, whole and cut workgroups, more than one round of them; tiles of 128 to 256 rows by 64 to 128 columns, rows and
+# columns off the tile, a K that ends inside a group.
+FEW = [(1, 512, 4096, "32x16"), (31, 512, 4108, "32x20"), (32, 640, 11008, "32x44"), (20, 512, 13000, "32x52"), (17, 1024, 2816, "32x12"),
+       (40, 1024, 2816, "64x12"), (64, 512, 4100, "64x20"), (64, 512, 16900, "64x36"), (33, 512, 13000, "64x52"), (100, 1024, 2816, "128x12"),
+       (65, 512, 4108, "128x20")]
+TILES = [(128, 520, 4100, "128x64"), (129, 512, 11008, "192x64"), (200, 1032, 2816, "128x64"), (250, 512, 11008, "256x64"),
+         (250, 520, 11008, "256x64"), (257, 512, 11004, "128x64"), (300, 640, 5632, "192x64"), (513, 520, 8200, "192x64"),
+         (700, 520, 8204, "256x128"), (1000, 512, 11008, "256x96"), (1000, 1024, 5632, "256x96"), (1000, 520, 11008, "256x96")]
 
 
-@pytest.mark.parametrize("T,K,N", FEW + TILES)
-def test_bits_of_single_ops(ga, mm, dev, monkeypatch, T, K, N):
+@pytest.mark.parametrize("T,K,N,tile", FEW + TILES)
+def test_bits_of_single_ops(ga, mm, dev, monkeypatch, T, K, N, tile):
     text = _module(mm, T, K, N)
     ins = _exact(dev, T, K, N, T + K + N)
     ins[0][0, 3] = float("inf")  # a row of infinities and NaNs, and no other
     full = torch.full((T + 1, N), 7.0, device=dev, dtype=torch.bfloat16)
     fused, single = full[:T], torch.empty(T, N, device=dev, dtype=torch.bfloat16)
     st, plan = ga.explain_mlir(text)
-    assert st == 0
+    assert st == 0 and ", %s per workgroup" % tile in plan and ("weight streaming" in plan) == (T <= 100), plan
     _run(ga, text, ins, fused)
     monkeypatch.setenv("GCMI_NO_POINTWISE_FUSION", "1")
     _run(ga, text, ins, single)

@@ -39,7 +39,7 @@ def _run(ga, text, ins, T, H):
     return [f[:T].clone() for f in full]
 
 
-# one row and more, 4 and 8 slices of the weight stream; slices of tiles; a K that ends inside a group; rows off 512 and 1024
+# two rows and more (of one row the residual is a bias to the planner, and the GEMM adds its slices itself), 4 and 8 slices of the weight stream; slices of tiles; a K that ends inside a group; rows off 512 and 1024
 # elements, one and several to a workgroup
 @pytest.mark.parametrize("T,H,F,special", [(2, 2048, 2560, False), (32, 2048, 5632, True), (32, 4096, 1024, False), (50, 4100, 4096, False),
                                            (100, 2048, 2560, False), (200, 2056, 8200, True), (300, 776, 6152, False),
@@ -56,6 +56,14 @@ def test_bits(ga, mm, dev, monkeypatch, T, H, F, special):
     assert "K slices of the GEMM before it" not in ga.explain_mlir(text)[1]
     want = _run(ga, text, ins, T, H)
     for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+def test_bits_of_one_row(ga, mm, dev, monkeypatch):
+    text, ins = mm.decoder_mlp_block(1, 2048, 2560), _inputs(dev, 1, 2048, 2560)
+    got = _run(ga, text, ins, 1, 2048)
+    monkeypatch.setenv("GCMI_NO_GENERATED_KERNELS", "1")
+    for a, b in zip(got, _run(ga, text, ins, 1, 2048)):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
