@@ -1363,8 +1363,9 @@ __device__ __forceinline__ void w4_epilogue_half(const GemmParams &p, int half, 
   constexpr int U = 8; // rows in flight per lane
 #pragma unroll 1
   for (int i0 = 0; i0 < WR / 4; i0 += U) {
-    // none of the wave's 4 * U rows from here on lies inside (passed over: 3 x 2312, K 96 with GELU 13.3 us -> 9.9; 2 x 1192, K 136 14.6 -> 11.4)
-    if (MASKED && wm * WR + 4 * i0 >= rows_in)
+    // none of the wave's 4 * U rows from here on lies inside (passed over: 3 x 2312, K 96 with GELU 13.3 us -> 9.9; 2 x 1192, K 136 14.6 -> 11.4).
+    // Waves of 64 rows have two groups and only pay for the question: 8-bit 63 x 544, K 64 with GELU 6.95 us -> 7.1, 1437 x 976, K 112 7.15 -> 7.28
+    if (MASKED && WR > 64 && wm * WR + 4 * i0 >= rows_in)
       return;
     acc4_t c[U];
 #pragma unroll
