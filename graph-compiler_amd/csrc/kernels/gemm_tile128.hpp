@@ -26,7 +26,8 @@ struct T128 {
   static_assert(T128_NST * STAGE_BYTES <= 4 * DUMP_WAVE_BYTES, "the ring overlaps the column parameters");
 };
 
-template <bool TB, int ES> __global__ __launch_bounds__(256, 2) void gemm_tile128_kernel(GemmParams p) {
+// RUNS: tiles are dealt to the XCDs in runs, else they are taken in the hardware's order.
+template <bool TB, int ES, bool RUNS = true> __global__ __launch_bounds__(256, 2) void gemm_tile128_kernel(GemmParams p) {
   static_assert(!TB || ES == 2, "B stored [N,K]: bf16 only");
   constexpr int KB = T128_KB, BK = KB / ES, NST = T128_NST, MI = T128::MI, BM = T128::BM, A_BYTES = T128::A_BYTES, STAGE = T128::STAGE_BYTES;
   constexpr int NA = MI / 2, NB = 2, PER = NA + NB; // requests of 1 KiB per wave and stage
@@ -46,7 +47,7 @@ template <bool TB, int ES> __global__ __launch_bounds__(256, 2) void gemm_tile12
 
   const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + T128_B - 1) / T128_B);
   int tm, tn;
-  tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, p.group_m, tm, tn);
+  tile_of_id(RUNS ? xcd_run(blockIdx.x, gridDim.x) : (int)blockIdx.x, tiles_m, tiles_n, p.group_m, tm, tn);
   tm = __builtin_amdgcn_readfirstlane(tm), tn = __builtin_amdgcn_readfirstlane(tn);
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * T128_B;
   const int64_t lda_b = p.lda * ES, ldb_b = p.ldb * ES;

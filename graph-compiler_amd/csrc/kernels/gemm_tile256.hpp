@@ -111,10 +111,12 @@ __device__ __forceinline__ uint4 load_chunk(const char *base, int64_t row, int64
 // rectangle of tiles and share A/B panels in that XCD's L2.  Workgroups bid, bid + 8, ... take one run of tiles each; where
 // their number is no multiple of 8 the first nblk % 8 runs are one longer (such numbers used to keep the hardware's order, every
 // XCD then reads nearly every panel: a decoder layer's 1000 tokens, with 172 tiles of 256 x 256 each for gate and up, 415 us, now 392).
-__device__ __forceinline__ void tile_of_block(int bid, int nblk, int tiles_m, int tiles_n, int group_m, int &tm,
-                                              int &tn) {
+__device__ __forceinline__ int xcd_run(int bid, int nblk) {
   const int run = bid & 7;
-  const int id = run * (nblk >> 3) + min(run, nblk & 7) + (bid >> 3);
+  return run * (nblk >> 3) + min(run, nblk & 7) + (bid >> 3);
+}
+// tile `id` in groups of group_m tile rows, each walked column by column
+__device__ __forceinline__ void tile_of_id(int id, int tiles_m, int tiles_n, int group_m, int &tm, int &tn) {
   int per_group = group_m * tiles_n;
   int g = id / per_group;
   int first_m = g * group_m;
@@ -122,6 +124,10 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblk, int tiles_m, in
   int in_g = id - g * per_group;
   tm = first_m + in_g % gm;
   tn = in_g / gm;
+}
+__device__ __forceinline__ void tile_of_block(int bid, int nblk, int tiles_m, int tiles_n, int group_m, int &tm,
+                                              int &tn) {
+  tile_of_id(xcd_run(bid, nblk), tiles_m, tiles_n, group_m, tm, tn);
 }
 
 // compile-time loop: the body receives std::integral_constant<int, I>, so every
