@@ -242,11 +242,6 @@ char *Executable::staging() {
   return staging_;
 }
 
-// Scratch of the steps whose kernels need some (partial sums of K-sliced GEMMs, mask tile classes of attention, partial
-// results of attention whose keys are cut over workgroups): a
-// slot of the step's own, alive for that step only, so it shares arena space with other temporaries.  Nothing is
-// shared between executables or streams: two executables may run side by side, as the reference's may
-// (thread-local scratch, lib/gc/ExecutionEngine/CPURuntime/Microkernel/BrgemmOnednn.cpp:70).
 // silu(x . Wg^T) * (x . Wu^T), the gate of a feed-forward layer: two GEMMs of one operand and the point-wise group that
 // reads nothing but them become one step where a kernel takes them (gemm_gated.hip).  A MatmulConfig on either keeps
 // both as they are.
@@ -319,6 +314,11 @@ void Executable::plan_gates() {
   }
 }
 
+// Scratch of the steps whose kernels need some (partial sums of K-sliced GEMMs, mask tile classes of attention, partial
+// results of attention whose keys are cut over workgroups): a
+// slot of the step's own, alive for that step only (slices that the next step adds: for both), so it shares arena space with other temporaries.  Nothing is
+// shared between executables or streams: two executables may run side by side, as the reference's may
+// (thread-local scratch, lib/gc/ExecutionEngine/CPURuntime/Microkernel/BrgemmOnednn.cpp:70).
 void Executable::plan_workspaces() {
   auto plan = [&](Step &s) {
     size_t bytes = 0;
@@ -362,6 +362,11 @@ void Executable::plan_slices() {
   }
 }
 
+// One allocation per executable, temporaries with disjoint lifetimes share memory: the tick-based merge
+// of the reference (lib/gc/Transforms/MergeAllocTickBased.cpp, docs/memref_schedule.md) with the step
+// index as the tick (the parts of a gated pair have its tick).  A slot lives from the first step that names it to the last; graph
+// inputs and outputs, constants and the results of once-only steps live for the whole executable.  Temporaries
+// are placed in order of their first tick at the lowest offset that is free for their whole lifetime.
 void Executable::layout_arena() {
   const int n = (int)slots_.size();
   std::vector<int> first(n, -1), last(n, -1);

@@ -67,7 +67,8 @@ enum GemmKernel : int32_t {
   GK_WAVES4 = 2,  // whole tiles, 4 waves of 128 x 128 (one per SIMD), 16x16 MFMAs, hand-placed main loop
   GK_SPLITK = 3,  // too few tiles for the GPU: K slices over workgroups + second pass
   GK_STREAM = 4,  // a short A against wide weights: weight-streaming kernel (+ second pass where K is sliced)
-  GK_TILE128 = 5, // 128 x 128 tiles, 4 waves of 64 x 64, two workgroups per compute unit: problems of few 256 x 256 tiles
+  GK_TILE128 = 5, // problems of few 256 x 256 tiles: 128 x 128, 4 waves of 64 x 64, two workgroups per compute unit (4 stages); or alone
+                  // on a compute unit (more stages), up to 256 x 128 and 256 x 192, on the hand-placed main loop
   GK_FEW_ROWS = 7, // up to 256 rows, one launch: K over the waves of a workgroup, tiles of 16 to 64 rows and columns
   GK_F32 = 6,     // f32 operands: bm tells the tile, mfma_m 0 the vector kernel (asked for, never launched through this)
 };

@@ -1205,7 +1205,6 @@ template <int ES, bool TB = false> __global__ __launch_bounds__(512, 1) void gem
 // same work was ten times the code, all of it executed once per workgroup and fetched cold: 12 us of a 100 us
 // kernel went into instruction-cache misses.
 static constexpr int W4_DUMP_PITCH = 272;                   // 64 f32 / s32 + 16 bytes: conflict-free for the 16-byte writes
-static constexpr int W4_DUMP_WAVE_BYTES = 128 * W4_DUMP_PITCH; // 34816 per wave, 139264 per workgroup
 
 // Four results of one row: c = the raw accumulators of columns n .. n+3 of row m.  HAS_BIAS / HAS_RES are
 // compile-time so that the eight rows of an unrolled group are straight-line code (their LDS reads go out together).
@@ -2105,10 +2104,9 @@ static inline double gcmi_us_per_group_256(double load) { // one workgroup per c
   return 2.75;
 }
 // Taller tiles of 128 columns (one workgroup per compute unit): fewer fragment reads per product than 128 rows, so where 128
-// rows make more than a round and 192 or 256 do not, they are ahead (64 random such sizes: 1.14 times on the average, at most
-// 1.5; 8-bit ones with K 1056 to 8112, 123 of them, 1.17, at least 0.95 from the cache and 0.81 from memory).  128 / 192 / 256 rows in one pass, us: 1237 x 4096, K 1376 29.3 / 22.5 / 27.5;
-// 305 x 11008, K 4096 69.5 / 56.3 / 63.8; 483 x 11008 73.1 / - / 67.3; where 128 rows fit one round they stay: 1000 x 4096,
-// K 4096 38.6 / 47.8 / 59.4.
+// rows make more than a round and 192 or 256 do not, they are ahead; where 128 rows fit one round they stay.  These rates, and those of
+// 128 rows up to a load of 1, were fitted to a main loop that the compiler had scheduled.  The hand-placed one is about an
+// eighth faster (GCMI_TILE_COSTS below rates it), which the comparison with K slices and with 256 x 256 tiles here does not have yet.
 static inline double gcmi_us_per_group_tall(int rows) { return rows == 192 ? 1.5 : 1.85; }
 static inline double gcmi_us_fixed_tall(int rows, int es) { return (rows == 192 ? 5.0 : 6.0) + (es == 1 ? 1.0 : 0.0); } // (8-bit: the longer epilogue, alone on its unit)
 // A long K beside wide weights costs 128 rows more per group than the estimate has, which was fitted to weights that the
@@ -2409,8 +2407,9 @@ static int launch_tile256(const GemmParams *pp, hipStream_t stream, int64_t *wan
   // (same products in the same order, same epilogue).  The 184 sizes of the estimates gain 1.10 on the average (the best tile of
   // each would give 1.118), two lose more than 2 % (at most 5 %).  us, 256 x 256 / chosen: 1000 x 11008, K 4096 82.2 / 73.9 on 256 x 192;
   // 2655 x 3520, K 3800 73.6 / 64.9 likewise; 1643 x 10048, K 1408 (280 tiles) 66.5 / 57.5 on 192 x 128; 3597 x 4672, K 128 22.0 / 15.6
-  // on 128 x 128.  Under half a round (the estimates above decide) and past three the sizes were not measured; past one, a K of 4096 and more keeps the large tile, which callers have
-  // been told of for 2048 x 11008 (165.8 there, 143.7 on 256 x 192; 4096 x 11008 263.7 / 283.0).
+  // on 128 x 128.  Under half a round (the estimates above decide) and past three the sizes were not measured.  Past one, a K of 4096 and
+  // more was not fitted either and keeps the large tile, which is no line by speed: 2048 x 11008 165.8 there, 143.7 on 256 x 192, 4096 x
+  // 11008 263.7 / 283.0.
   if (ES == 2 && use_w4 && t128_can && !tail_cols && !tail_rows && p.cfg_tile == 0 && !p.cfg_waves && !p.cfg_split_k &&
       2 * nblk * nbatch >= n_cu && nblk * nbatch < (p.K < 4096 ? 3 : 1) * n_cu) {
     const GemmTileCost *tile = &GCMI_TILE_COSTS[0];
