@@ -121,9 +121,9 @@ def time_launches(torch, fn, nsets, steps, warmup):
 # bytes the main kernel of a decode-shaped GEMM fetches per launch (FETCH_SIZE, scaled as above), by (N, K)
 DECODE_TRAFFIC = {(4096, 4096): 35_800_000, (11008, 4096): 92_500_000, (4096, 11008): 95_900_000}
 TRAFFIC = {  # (bytes per launch of the dominant kernel, the committed profile they come from)
-    "gemm": (235414490, "profiles/gemm_tile256_w4_bf16_4096cubed.md"),
-    "int8": (384693096, "profiles/gemm_tile256_w4_int8_mlp_layer.md"),
-    "chain": (684027008 + 575145347, "profiles/gemm_tile256_w4_bf16_mlp_chain.md"),  # both launches
+    "gemm": (235475251, "profiles/gemm_tile256_w4_bf16_4096cubed.md"),
+    "int8": (384744857, "profiles/gemm_tile256_w4_int8_mlp_layer.md"),
+    "chain": (678247424 + 575204454, "profiles/gemm_tile256_w4_bf16_mlp_chain.md"),  # both launches
     "mha": (362734179, "profiles/mha_fwd_fast_b4_h32_s2048_d128_every_block.md"),
     "mha_skip": (330983112, "profiles/mha_fwd_fast_b4_h32_s2048_d128.md"),
 }
