@@ -429,6 +429,7 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
         << " *>(in" << k << ") + off" << k << ");\n    }\n  }\n";
     }
   }
+  std::ostringstream store_result;
   if (sliced.k >= 0) {
     const std::string n = std::to_string(sliced.k), off = "base" + n + " + e", S = std::to_string(sliced.splits);
     const std::string head = "#pragma unroll\n  for (int it_ = 0; it_ < " + std::to_string(trips) + "; it_++) {\n    const " + g.idx + " e = (" +
@@ -448,8 +449,11 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
            "      q_[2] += gcmi::bf16_bits_to_f32((unsigned short)add_[it_][1]); q_[3] += gcmi::bf16_bits_to_f32((unsigned short)(add_[it_][1] >> 16));\n"
            "      gcmi::round_bf16_quad(q_);\n";
     o << "      raw" << n << "[it_] = u2_{(__float_as_uint(q_[0]) >> 16) | (__float_as_uint(q_[1]) & 0xffff0000u), (__float_as_uint(q_[2]) >> 16) | "
-         "(__float_as_uint(q_[3]) & 0xffff0000u)};\n      if (live)\n        *reinterpret_cast<u2_ *>(reinterpret_cast<unsigned short *>(result) + "
-      << off << ") = raw" << n << "[it_];\n    }\n  }\n  }\n";
+         "(__float_as_uint(q_[3]) & 0xffff0000u)};\n    }\n  }\n  }\n";
+    // stored behind the last use: in the branch above, its end would wait for the store (1000 x 4096, 2 slices 12.0 us without the
+    // branch, 12.4 with the store inside it)
+    store_result << "  if (part != nullptr && live) {\n" << head << "      *reinterpret_cast<u2_ *>(reinterpret_cast<unsigned short *>(result) + " << off
+                 << ") = raw" << n << "[it_];\n    }\n  }\n  }\n";
   }
   o << "  float acc = 0.0f;\n";
   row_loop(0, p.n_in_pre, 0, p.sum_ins, false);
@@ -483,7 +487,7 @@ bool generate_fused(const FusedParams &raw, const int *same_as, const std::strin
   }
   if (second_pass)
     row_loop(p.n_in_row, p.n_in, p.row_end, p.n_ins, true);
-  o << "}\n";
+  o << store_result.str() << "}\n";
   out.source = o.str();
   return true;
 }
